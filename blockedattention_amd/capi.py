@@ -19,7 +19,8 @@ SYMBOLS = (
     "ba_status_string", "ba_abi_version", "ba_plan_bytes", "ba_plan_gemm", "ba_plan_softmax", "ba_plan_read",
     "ba_plan_read_into", "ba_plan_gemm_notify", "ba_plan_softmax_notify", "ba_plan_wait",
     "ba_varlen_gemm", "ba_blocked_softmax", "ba_blocked_softmax_backward", "ba_gemm_softmax",
-    "ba_varlen_attention", "ba_gemm_softmax_static", "ba_static_read", "ba_varlen_gemm_two",
+    "ba_varlen_attention", "ba_attention_rows", "ba_varlen_attention_train", "ba_varlen_attention_backward",
+    "ba_gemm_softmax_static", "ba_static_read", "ba_varlen_gemm_two",
 )
 MAILBOX_BYTES = 320
 STATIC_MAX_SEGMENTS = 4096   # BA_STATIC_MAX_SEGMENTS
@@ -36,6 +37,7 @@ class PlanInfo(ctypes.Structure):
         ("list_rest", ctypes.c_int32), ("small_max_N", ctypes.c_int32), ("small_max_M", ctypes.c_int32),
         ("list_rows", ctypes.c_int32), ("att_blocks64", ctypes.c_int32), ("att_blocks128", ctypes.c_int32),
         ("list_mini", ctypes.c_int32), ("list_pipe", ctypes.c_int32), ("pipe_groups", ctypes.c_int32), ("min_N", ctypes.c_int32), ("min_K", ctypes.c_int32), ("ring_groups", ctypes.c_int32), ("wide_groups", ctypes.c_int32),
+        ("att_cols64", ctypes.c_int32),
     ]
 
     def as_dict(self):
@@ -91,6 +93,12 @@ def load():
     lib.ba_gemm_softmax.argtypes = [vp, ctypes.POINTER(PlanInfo), i64, i32, vp, vp, vp, i32, i64, i64, i64, i64, f32, vp]
     lib.ba_varlen_attention.restype = i32
     lib.ba_varlen_attention.argtypes = [vp, ctypes.POINTER(PlanInfo), i64, i32, vp, vp, vp, vp, i64, i64, i64, i64, f32, vp]
+    lib.ba_attention_rows.restype = i64
+    lib.ba_attention_rows.argtypes = [ctypes.POINTER(PlanInfo), i64]
+    lib.ba_varlen_attention_train.restype = i32
+    lib.ba_varlen_attention_train.argtypes = [vp, ctypes.POINTER(PlanInfo), i64, i32, vp, vp, vp, vp, vp, i64, i64, i64, i64, f32, vp]
+    lib.ba_varlen_attention_backward.restype = i32
+    lib.ba_varlen_attention_backward.argtypes = [vp, ctypes.POINTER(PlanInfo), i64, i32, *[vp] * 10, i64, i64, i64, i64, f32, vp]
     lib.ba_gemm_softmax_static.restype = i32
     lib.ba_gemm_softmax_static.argtypes = [i64, i32, vp, vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, i64, i64, i64, i64, f32, vp]
     lib.ba_static_read.restype = i32
@@ -284,3 +292,24 @@ def varlen_attention(plan, Q, K, V, out, H, Dm1, Dm2, Dout, scale=1.0):
                                     _ptr(out), H, Dm1, Dm2, Dout, float(scale), _stream())
     check(st, "ba_varlen_attention")
     return out
+
+
+def varlen_attention_train(plan, Q, K, V, out, lse, H, Dm1, Dm2, Dout, scale=1.0):
+    """As varlen_attention, also writing ``lse`` (fp32, see attention_rows) for the backward pass."""
+    st = load().ba_varlen_attention_train(plan.ptr, plan._hint(), plan.nseg, dtype_code(Q.dtype), _ptr(Q), _ptr(K), _ptr(V),
+                                          _ptr(out), _ptr(lse), H, Dm1, Dm2, Dout, float(scale), _stream())
+    check(st, "ba_varlen_attention_train")
+    return out
+
+
+def attention_rows(plan, Dm1):
+    """Entries per head of the ``lse`` and ``delta`` arrays of a plan whose summary has been read."""
+    return load().ba_attention_rows(plan._hint(), Dm1)
+
+
+def varlen_attention_backward(plan, Q, K, V, out, dO, lse, delta, dQ, dK, dV, H, Dm1, Dm2, Dout, scale=1.0):
+    """dQ, dK, dV of varlen_attention_train for the gradient dO of its output (see ba_varlen_attention_backward)."""
+    st = load().ba_varlen_attention_backward(plan.ptr, plan._hint(), plan.nseg, dtype_code(Q.dtype), _ptr(Q), _ptr(K), _ptr(V),
+                                             _ptr(out), _ptr(dO), _ptr(lse), _ptr(delta), _ptr(dQ), _ptr(dK), _ptr(dV), H,
+                                             Dm1, Dm2, Dout, float(scale), _stream())
+    check(st, "ba_varlen_attention_backward")

@@ -1,0 +1,65 @@
+// What the one-pass attention (attention.hip) and its backward (attention_backward.hip) share: counted LDS operand
+// reads, element-wise operand loads, the rows of the per-query arrays.
+#pragma once
+#include <type_traits>
+#include <utility>
+
+#include "ba_gemm_common.hpp"
+
+namespace ba {
+
+constexpr int kAttKeys = 64;                          // keys (backward: or queries) staged in LDS at a time
+
+// LDS operand reads as inline assembly, so that kAttRing of them are in flight under the matrix instructions
+// (left to itself the compiler, short of registers, issues each read right before its use and every matrix
+// instruction waits a full LDS round trip).  The compiler does not count these reads: lds_wait<n> waits until at
+// most n of them are outstanding and hands the register on, so the use cannot move above the wait.  Counting is
+// conservative when other LDS or scalar loads are in flight: the counter is then higher, the wait longer.
+template <int OFF> __device__ __forceinline__ void lds_read128(u32x4 &dst, uint32_t addr) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF) : "memory");
+}
+template <int N> __device__ __forceinline__ void lds_wait(u32x4 &x) {
+    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(x) : "n"(N) : "memory");
+}
+template <typename F, int... I> __device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
+    static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+__device__ __forceinline__ uint32_t lds_offset(const void *p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
+}
+
+// Eight consecutive elements k0 .. k0+7 of a row of K elements, zeros at and past K, for rows whose
+// length is not a multiple of 8 (pieces straddle nothing, but the row may end inside one): element by
+// element, one load in flight, few registers -- the slow path must not set the register count of the
+// kernel.  Each step shifts the 128-bit value down by one element and puts the new one on top.
+__device__ __forceinline__ u32x4 load8_slow(const uint16_t *row, int k0, int K) {
+    uint32_t r0 = 0, r1 = 0, r2 = 0, r3 = 0;
+#pragma nounroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t x = row[min(k0 + i, K - 1)];
+        r0 = (r0 >> 16) | (r1 << 16);
+        r1 = (r1 >> 16) | (r2 << 16);
+        r2 = (r2 >> 16) | (r3 << 16);
+        r3 = (r3 >> 16) | ((k0 + i < K ? x : 0u) << 16);
+    }
+    return u32x4{r0, r1, r2, r3};
+}
+
+// a * b + c for a, b below 2^24: one instruction
+__device__ __forceinline__ uint32_t mad24(uint32_t a, uint32_t b, uint32_t c) { return __umul24(a, b) + c; }
+
+// Where the rows of a segment lie in a per-query array of the backward pass: ceil(Dm1 / min_K) floats per head, row r
+// of segment g at ceil(off1 / min_K) + r.  Segments do not overlap there because none has fewer than min_K elements a
+// row (segments without keys, which min_K does not count, have no entry).
+__host__ __device__ inline int64_t att_rows_per_head(int min_K, int64_t Dm1) {
+    const int64_t k = min_K > 1 ? min_K : 1;
+    return (Dm1 + k - 1) / k;
+}
+__device__ __forceinline__ int64_t att_row_base(int min_K, int64_t Dm1, int64_t h, int64_t off1) {
+    return h * att_rows_per_head(min_K, Dm1) + att_rows_per_head(min_K, off1);
+}
+
+}  // namespace ba

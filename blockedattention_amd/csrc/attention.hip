@@ -24,18 +24,13 @@
 #include <stdlib.h>
 
 #include <algorithm>
-#include <type_traits>
-#include <utility>
 
-#include "ba_device.hpp"
-#include "ba_gemm_common.hpp"
-#include "ba_host.hpp"
+#include "att_common.hpp"
 
 namespace ba {
 
 constexpr int kAttThreads = 256;
 constexpr int kAttWaves = kAttThreads / 64;
-constexpr int kAttKeys = 64;                          // keys per block
 constexpr int kAttRows = 16 * kAttWaves;              // queries per workgroup round
 static_assert(kAttRows == kAttBlockRows, "the plan's row-block prefixes count blocks of kAttRows and 2 kAttRows");
 // LDS row pitches.  A 16-byte operand read of a wavefront is served 32 lanes at a time, 512 bytes wide (measured:
@@ -49,53 +44,12 @@ constexpr int kAttPitchV = kAttKeys * 2 + 32;
 // workgroup there: 256 segments of 32..128 rows, 31.3 -> 29.0 us)
 constexpr int att_ring(int nk, int qt) { return qt == 1 && nk <= 2 ? 3 : 6; }
 
-// LDS operand reads as inline assembly, so that kAttRing of them are in flight under the matrix instructions
-// (left to itself the compiler, short of registers, issues each read right before its use and every matrix
-// instruction waits a full LDS round trip).  The compiler does not count these reads: lds_wait<n> waits until at
-// most n of them are outstanding and hands the register on, so the use cannot move above the wait.  Counting is
-// conservative when other LDS or scalar loads are in flight: the counter is then higher, the wait longer.
-template <int OFF> __device__ __forceinline__ void lds_read128(u32x4 &dst, uint32_t addr) {
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF) : "memory");
-}
-template <int N> __device__ __forceinline__ void lds_wait(u32x4 &x) {
-    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(x) : "n"(N) : "memory");
-}
-template <typename F, int... I> __device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
-    static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-__device__ __forceinline__ uint32_t lds_offset(const void *p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
-}
-
-// Eight consecutive elements k0 .. k0+7 of a row of K elements, zeros at and past K, for rows whose
-// length is not a multiple of 8 (pieces straddle nothing, but the row may end inside one): element by
-// element, one load in flight, few registers -- the slow path must not set the register count of the
-// kernel.  Each step shifts the 128-bit value down by one element and puts the new one on top.
-__device__ __forceinline__ u32x4 load8_slow(const uint16_t *row, int k0, int K) {
-    uint32_t r0 = 0, r1 = 0, r2 = 0, r3 = 0;
-#pragma nounroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t x = row[min(k0 + i, K - 1)];
-        r0 = (r0 >> 16) | (r1 << 16);
-        r1 = (r1 >> 16) | (r2 << 16);
-        r2 = (r2 >> 16) | (r3 << 16);
-        r3 = (r3 >> 16) | ((k0 + i < K ? x : 0u) << 16);
-    }
-    return u32x4{r0, r1, r2, r3};
-}
-
-// a * b + c for a, b below 2^24: one instruction
-__device__ __forceinline__ uint32_t mad24(uint32_t a, uint32_t b, uint32_t c) { return __umul24(a, b) + c; }
-
 // NK = 32-wide k steps (head dimension padded to 32 * NK).  VEC: the segment's K is a multiple of 8, its
 // rows come as 16-byte loads; otherwise element by element.  The two are separate instances of the whole
 // body so that the slow loads do not sit inside the fast path's loops.
-template <int DT, int NK, int QT, bool VEC>
-__device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbuf, const SegRec &rec, int64_t h, int zblock,
-                                               unsigned char *sK, unsigned char *sV) {
+template <int DT, int NK, int QT, bool VEC, bool LSE>
+__device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbuf, float *lse_rows, const SegRec &rec, int64_t h,
+                                               int zblock, unsigned char *sK, unsigned char *sV) {
     constexpr int KP = 32 * NK;                       // padded head dimension
     constexpr int kPitchK = KP * 2 + 32;              // bytes per LDS row of keys
     constexpr int kPieces = KP / 8;                   // 16-byte pieces per row
@@ -357,6 +311,8 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
             const int qr = r0 + kAttRows * q + j;
             const float l = quad_column_sum(lsum[q]);
             const float inv = N > 0 ? 1.0f / l : 0.f;
+            // base-2 logarithm of the row's sum of exponentials, for the backward pass
+            if (LSE && rg == 0 && qr < M && N > 0) lse_rows[qr] = fmaf(m[q], c, __builtin_amdgcn_logf(l));
             if (qr < M) {
                 uint16_t *orow = os + (int64_t)qr * K;
 #pragma unroll
@@ -377,8 +333,10 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
     }
 }
 
-template <int DT, int NK, int QT>
-__global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void attention_kernel(RunArgs a, const void *Vbuf) {
+// LSE: the build for training, which also writes the rows' sums (as a run-time choice it cost the plain one 2 % on 512
+// segments of 16 .. 256 rows and columns: 23.1 -> 23.6 us).
+template <int DT, int NK, int QT, bool LSE>
+__global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void attention_kernel(RunArgs a, const void *Vbuf, float *lse) {
     constexpr int KP = 32 * NK;
     __shared__ __attribute__((aligned(16))) unsigned char sK[kAttKeys * (KP * 2 + 32)];
     __shared__ __attribute__((aligned(16))) unsigned char sV[KP * kAttPitchV];
@@ -428,26 +386,32 @@ __global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void at
             atomicAdd(&reinterpret_cast<PlanHeader *>(a.plan)->run_errors, 1);
         return;
     }
-    if ((K & 7) == 0) attention_body<DT, NK, QT, true>(a, Vbuf, rec, h, zblock, sK, sV);
-    else attention_body<DT, NK, QT, false>(a, Vbuf, rec, h, zblock, sK, sV);
+    float *lse_rows = LSE ? lse + att_row_base(((ConstHdr)(uintptr_t)a.plan)->min_K, a.Dm1, h, rec.off1) : nullptr;
+    if ((K & 7) == 0) attention_body<DT, NK, QT, true, LSE>(a, Vbuf, lse_rows, rec, h, zblock, sK, sV);
+    else attention_body<DT, NK, QT, false, LSE>(a, Vbuf, lse_rows, rec, h, zblock, sK, sV);
 }
 
-template <int DT, int QT>
-static void launch_nk(int nk, dim3 grid, hipStream_t stream, const RunArgs &args, const void *V) {
+template <int DT, int QT, bool LSE>
+static void launch_nk(int nk, dim3 grid, hipStream_t stream, const RunArgs &args, const void *V, float *lse) {
     // args.ride_slots = 1: work items from the plan's row-block prefix; else args.tile_zdim = row blocks per
     // (segment, head) pair, tile_groups = pairs per die
     switch (nk) {
-        case 1: hipLaunchKernelGGL((attention_kernel<DT, 1, QT>), grid, dim3(kAttThreads), 0, stream, args, V); break;
-        case 2: hipLaunchKernelGGL((attention_kernel<DT, 2, QT>), grid, dim3(kAttThreads), 0, stream, args, V); break;
-        case 3: hipLaunchKernelGGL((attention_kernel<DT, 3, QT>), grid, dim3(kAttThreads), 0, stream, args, V); break;
-        default: hipLaunchKernelGGL((attention_kernel<DT, 4, QT>), grid, dim3(kAttThreads), 0, stream, args, V); break;
+        case 1: hipLaunchKernelGGL((attention_kernel<DT, 1, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse); break;
+        case 2: hipLaunchKernelGGL((attention_kernel<DT, 2, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse); break;
+        case 3: hipLaunchKernelGGL((attention_kernel<DT, 3, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse); break;
+        default: hipLaunchKernelGGL((attention_kernel<DT, 4, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse); break;
     }
+}
+template <int DT, int QT>
+static void launch_build(int nk, dim3 grid, hipStream_t stream, const RunArgs &args, const void *V, float *lse) {
+    if (lse) launch_nk<DT, QT, true>(nk, grid, stream, args, V, lse);
+    else launch_nk<DT, QT, false>(nk, grid, stream, args, V, lse);
 }
 
 // Strips per wavefront: two where segments are tall (each operand read from LDS then feeds two matrix
 // instructions and a block of keys is staged half as often), one otherwise (more, lighter workgroups).
 
-int launch_attention(int dtype, const RunArgs &args, const void *V, int64_t nseg, const ba_plan_info *info,
+int launch_attention(int dtype, const RunArgs &args, const void *V, float *lse, int64_t nseg, const ba_plan_info *info,
                      hipStream_t stream) {
     if (dtype != BA_F16 && dtype != BA_BF16) return BA_ERR_UNSUPPORTED;
     static const int forced = [] { const char *e = getenv("BLOCKEDATTN_ATT_STRIPS"); return e ? atoi(e) : 0; }();
@@ -486,8 +450,8 @@ int launch_attention(int dtype, const RunArgs &args, const void *V, int64_t nseg
         run.tile_groups = (int)pairs8;
         grid = dim3((unsigned)(pairs8 * z * 8));
     }
-    if (dtype == BA_F16) { if (qt == 2) launch_nk<0, 2>(nk, grid, stream, run, V); else launch_nk<0, 1>(nk, grid, stream, run, V); }
-    else { if (qt == 2) launch_nk<1, 2>(nk, grid, stream, run, V); else launch_nk<1, 1>(nk, grid, stream, run, V); }
+    if (dtype == BA_F16) { if (qt == 2) launch_build<0, 2>(nk, grid, stream, run, V, lse); else launch_build<0, 1>(nk, grid, stream, run, V, lse); }
+    else { if (qt == 2) launch_build<1, 2>(nk, grid, stream, run, V, lse); else launch_build<1, 1>(nk, grid, stream, run, V, lse); }
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
 }
 

@@ -1,0 +1,537 @@
+// Backward of the one-pass varlen attention (attention.hip): dQ, dK and dV per segment and head from dO, with the
+// probabilities recomputed from the row sums the forward pass kept (base-2 logarithms, one float per query) and never
+// written to memory.  It is what a caller of the reference gets from the backward passes of blockGEMM, blockSoftmax
+// and blockGEMM (csrc/sparseBlockedAttention.cpp:52-72, 95-114): that chain writes and reads six M x N arrays.
+//
+//   P  = 2^(c Q K^T - lse)      dP = dO V^T      dS = P o (dP - delta),  delta = sum over columns of dO o O
+//   dV = P^T dO                 dK = scale dS^T Q                        dQ = scale dS K
+//
+// Two kernels, each owning its results (no atomics, the same sums every time): attention_dq_kernel walks the keys for a
+// block of queries and leaves delta for attention_dkdv_kernel, which walks the queries for a block of keys.  The scores
+// and dP are computed in both, seven products instead of five; adding dQ to memory from the second kernel instead
+// would move N / 128 times the size of dQ in fp32 atomics.
+//
+// Measured on 16 segments x 16 heads of 1024 .. 4096 rows, K = 128, bf16: dQ 1.37 ms (1.08 PFLOP/s over its three
+// products), dK and dV 2.10 ms (0.94 over four), 3.5 ms together against 9.3 ms of the chain; every operand read from LDS
+// feeds two matrix instructions, which puts the LDS port at 80 to 100 % of the matrix unit's rate: the next limit.
+//
+// Operands lie in LDS as rows (one copy of each): a matrix operand whose reduction runs over the head dimension is read
+// 16 bytes per lane, one whose reduction runs over the rows by the transposing read (ds_read_b64_tr_b16).  The lane that
+// holds scores of (row 16 t + 4 rg + e, column 16 u + j) packs them, over two row tiles, into the second operand of the
+// product that reduces over those rows, so that P and dS stay where they are.
+#include <algorithm>
+
+#include "att_common.hpp"
+#include "ba_host.hpp"
+
+namespace ba {
+
+constexpr uint32_t kNowhere = 0xfffffff0u;            // byte offset no segment reaches
+
+typedef __attribute__((address_space(3))) unsigned char *LdsPtr;
+__device__ __forceinline__ LdsPtr lds_ptr(void *p) { return (LdsPtr)p; }
+__device__ __forceinline__ u32x4 lds_row16(LdsPtr p, int off) {
+    return *reinterpret_cast<__attribute__((address_space(3))) const u32x4 *>(p + off);
+}
+// Eight rows of one column (see lds_tr8 in gemm_any16.hip): four rows from p + off, four from `next` bytes on.
+__device__ __forceinline__ u32x4 lds_col8(LdsPtr p, int off, int next) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4 *Ptr;
+    const u32x2 l = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((Ptr)(p + off)));
+    const u32x2 h = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((Ptr)(p + off + next)));
+    return u32x4{l[0], l[1], h[0], h[1]};
+}
+// Barrier that waits for this wavefront's LDS traffic only (the loads of the next block stay in flight).
+__device__ __forceinline__ void att_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Rows of K elements read as 16-byte pieces (eight elements from column 8 p on) through a buffer descriptor that spans
+// the segment.  VEC: K is a multiple of 8, every piece lies inside a row, rows past the last read as zeros.  Otherwise a
+// piece may reach past its row's end (those elements are cleared) and the last ones past the segment's end: they are
+// read from the last 16 bytes of the segment and shifted down.  A segment of fewer than eight elements is read element by element.
+template <bool VEC> struct RowPieces {
+    __amdgpu_buffer_rsrc_t res;
+    uint32_t bytes, row_bytes;
+    int K;
+    __device__ __forceinline__ RowPieces(const uint16_t *seg, int rows, int K_) {
+        K = K_;
+        row_bytes = 2u * (uint32_t)K_;
+        bytes = (uint32_t)rows * row_bytes;
+        res = __builtin_amdgcn_make_buffer_rsrc((void *)seg, 0, bytes, kRsrcFlags);
+    }
+    __device__ __forceinline__ uint32_t offset(int row, int piece) const {
+        return 8 * piece < K ? (uint32_t)row * row_bytes + 16u * (uint32_t)piece : kNowhere;
+    }
+    __device__ __forceinline__ u32x4 load(uint32_t off) const {
+        if constexpr (VEC) return __builtin_amdgcn_raw_buffer_load_b128(res, off, 0, 0);
+        if (bytes >= 16) return __builtin_amdgcn_raw_buffer_load_b128(res, min(off, bytes - 16), 0, 0);
+        u32x4 x = {0u, 0u, 0u, 0u};
+#pragma nounroll
+        for (int i = 0; i < 8; ++i) {                 // each step shifts the piece down and puts an element on top
+            const uint32_t e = __builtin_amdgcn_raw_buffer_load_b16(res, off + 2 * i, 0, 0);
+            x = u32x4{__builtin_amdgcn_alignbit(x[1], x[0], 16), __builtin_amdgcn_alignbit(x[2], x[1], 16),
+                      __builtin_amdgcn_alignbit(x[3], x[2], 16), (x[3] >> 16) | (e << 16)};
+        }
+        return x;
+    }
+    // what load(off) returned -> the piece (no-op for VEC)
+    __device__ __forceinline__ u32x4 finish(u32x4 x, uint32_t off, int piece) const {
+        if constexpr (VEC) return x;
+        if (bytes >= 16) {
+            const uint32_t behind = off <= bytes - 16 ? 0u : (min(off, bytes) - (bytes - 16)) >> 1;    // elements 0 .. 8
+            if (__any(behind != 0)) {
+                if (behind & 8) x = u32x4{0u, 0u, 0u, 0u};
+                if (behind & 4) x = u32x4{x[2], x[3], 0u, 0u};
+                if (behind & 2) x = u32x4{x[1], x[2], x[3], 0u};
+                if (behind & 1)
+                    x = u32x4{__builtin_amdgcn_alignbit(x[1], x[0], 16), __builtin_amdgcn_alignbit(x[2], x[1], 16),
+                              __builtin_amdgcn_alignbit(x[3], x[2], 16), x[3] >> 16};
+            }
+        }
+        const int left = K - 8 * piece;               // elements of the row from this piece on
+        if (left < 8) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) x[w] &= left >= 2 * w + 2 ? 0xffffffffu : left == 2 * w + 1 ? 0xffffu : 0u;
+        }
+        return x;
+    }
+    __device__ __forceinline__ u32x4 get(int row, int piece) const {
+        const uint32_t off = offset(row, piece);
+        return finish(load(off), off, piece);
+    }
+};
+
+template <int DT> __device__ __forceinline__ float lo16(uint32_t w) { return Elem<DT>::to_float((uint16_t)w); }
+template <int DT> __device__ __forceinline__ float hi16(uint32_t w) { return Elem<DT>::to_float((uint16_t)(w >> 16)); }
+
+// Four consecutive results (columns c0 .. c0 + 3 of a row of K) to memory.
+template <int DT> __device__ __forceinline__ void store4(uint16_t *row, int c0, int K, f32x4 v, float f) {
+    if (c0 + 4 <= K) {
+        *reinterpret_cast<u32x2_unaligned *>(row + c0) =
+            u32x2{Elem<DT>::pack2(v[0] * f, v[1] * f), Elem<DT>::pack2(v[2] * f, v[3] * f)};
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (c0 + e < K) row[c0 + e] = Elem<DT>::from_float(v[e] * f);
+    }
+}
+
+// LDS pitch of staged rows: 16 * (2 * odd) bytes, the 16-byte operand reads and the transposing reads meet no conflict
+constexpr int att_pitch(int nk) { return 64 * nk + 32; }
+
+struct AttBwdArgs {
+    const void *V, *O, *dO;
+    const float *lse;
+    float *delta;
+    void *dQ, *dK, *dV;
+};
+
+// The ROWS rows of an array staged per block: thread -> (row, piece), kSteps pieces an array.
+template <int NK, int THREADS, int ROWS = kAttKeys> struct AttStage {
+    static constexpr int kPieces = 4 * NK;
+    static constexpr int kLpr = NK == 3 ? 16 : kPieces;      // lanes per row (a power of two)
+    static constexpr int kRowsStep = THREADS / kLpr;
+    static constexpr int kSteps = ROWS / kRowsStep > 0 ? ROWS / kRowsStep : 1;
+};
+
+// ---------------------------------------------------------------------------------------------------------- dQ
+// Workgroup = 4 wavefronts; a wavefront owns QT strips of 16 queries (64 apart), their Q and dO fragments in registers,
+// and walks the keys in blocks of 64 staged in LDS (K and V rows), 32 at a time: scores and dP transposed (lane = query
+// j, keys 4 rg + e), dS packed over two key tiles, dQ^T += K^T dS^T.
+template <int DT, int NK, int QT, bool VEC>
+__device__ __forceinline__ void att_dq_body(const RunArgs &a, const AttBwdArgs &w, const SegRec &rec, int64_t h, int64_t row0,
+                                            int block, unsigned char *sK, unsigned char *sV) {
+    using St = AttStage<NK, 256>;
+    constexpr int kPitch = att_pitch(NK);
+    constexpr int kOutTiles = 2 * NK;
+    const int M = rec.M, N = rec.N, K = rec.K;
+    const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = lane_id(), j = lane & 15, rg = lane >> 4;
+    const int64_t o1 = h * a.Dm1 + rec.off1, o2 = h * a.Dm2 + rec.off2;
+    const RowPieces<VEC> pq((const uint16_t *)a.A + o1, M, K), pg((const uint16_t *)w.dO + o1, M, K), po((const uint16_t *)w.O + o1, M, K);
+    const RowPieces<VEC> pk((const uint16_t *)a.B + o2, N, K), pv((const uint16_t *)w.V + o2, N, K);
+    const float c = a.scale * kLog2e;
+
+    const int s_row = tid / St::kLpr, s_piece = tid % St::kLpr;
+    u32x4 kw[St::kSteps], vw[St::kSteps];
+    auto fetch = [&](int kb) {
+#pragma unroll
+        for (int s = 0; s < St::kSteps; ++s) {
+            const uint32_t off = pk.offset(kb + s * St::kRowsStep + s_row, s_piece);
+            kw[s] = pk.load(off);
+            vw[s] = pv.load(off);
+        }
+    };
+    if (N > 0) fetch(0);
+
+    const int r0 = block * kAttBlockRows * QT + wave * 16;
+    u32x4 qf[QT][NK], gf[QT][NK];
+    float lse[QT], delta[QT];
+    f32x4 acc[QT][kOutTiles];
+#pragma unroll
+    for (int q = 0; q < QT; ++q) {
+        const int row = r0 + kAttBlockRows * q + j;
+        float d = 0.f;
+#pragma unroll
+        for (int s = 0; s < NK; ++s) {
+            qf[q][s] = pq.get(row, 4 * s + rg);
+            gf[q][s] = pg.get(row, 4 * s + rg);
+            const u32x4 of = po.get(row, 4 * s + rg);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                d = fmaf(lo16<DT>(gf[q][s][i]), lo16<DT>(of[i]), d);
+                d = fmaf(hi16<DT>(gf[q][s][i]), hi16<DT>(of[i]), d);
+            }
+        }
+        delta[q] = quad_column_sum(d);
+        lse[q] = row < M && N > 0 ? w.lse[row0 + row] : INFINITY;        // 2^-inf: rows that do not exist have no probabilities
+        if (row < M && N > 0 && rg == 0) w.delta[row0 + row] = delta[q];
+#pragma unroll
+        for (int t = 0; t < kOutTiles; ++t) acc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const LdsPtr k_row = lds_ptr(sK) + j * kPitch + rg * 16, v_row = lds_ptr(sV) + j * kPitch + rg * 16;
+    const LdsPtr k_col = lds_ptr(sK) + (4 * rg + (j >> 2)) * kPitch + (j & 3) * 8;
+
+    for (int kb = 0; kb < N; kb += kAttKeys) {
+        att_lds_barrier();                             // the previous block is consumed
+        if (St::kLpr == St::kPieces || s_piece < St::kPieces) {
+#pragma unroll
+            for (int s = 0; s < St::kSteps; ++s) {
+                const int row = s * St::kRowsStep + s_row;
+                const uint32_t off = pk.offset(kb + row, s_piece);
+                *reinterpret_cast<u32x4 *>(sK + row * kPitch + s_piece * 16) = pk.finish(kw[s], off, s_piece);
+                *reinterpret_cast<u32x4 *>(sV + row * kPitch + s_piece * 16) = pv.finish(vw[s], off, s_piece);
+            }
+        }
+        att_lds_barrier();
+        if (kb + kAttKeys < N) fetch(kb + kAttKeys);
+        if (r0 >= M) continue;                         // the wavefront only stages
+        const int left = N - kb;
+        auto half = [&](auto h_tag) {                  // (a strip whose rows do not exist runs along: one code path)
+            constexpr int NQ = QT, H0 = decltype(h_tag)::value;       // key tiles 2 H0, 2 H0 + 1
+            f32x4 s[NQ][2], dp[NQ][2];
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) s[q][t] = dp[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int st = 0; st < NK; ++st)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const u32x4 kf = lds_row16(k_row, 16 * (2 * H0 + t) * kPitch + 64 * st);
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) s[q][t] = Elem<DT>::mfma(kf, qf[q][st], s[q][t]);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int st = 0; st < NK; ++st)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const u32x4 vf = lds_row16(v_row, 16 * (2 * H0 + t) * kPitch + 64 * st);
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) dp[q][t] = Elem<DT>::mfma(vf, gf[q][st], dp[q][t]);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            u32x4 ds[NQ];
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[q][t][e] = __builtin_amdgcn_exp2f(fmaf(s[q][t][e], c, -lse[q]));
+                if (left < kAttKeys) {                 // keys past the last one (their scores are zeros, lse may be anything)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) s[q][t][e] = 16 * (2 * H0 + t) + 4 * rg + e < left ? s[q][t][e] : 0.f;
+                }
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[q][t][e] *= dp[q][t][e] - delta[q];
+                    ds[q][2 * t] = Elem<DT>::pack2(s[q][t][0], s[q][t][1]);
+                    ds[q][2 * t + 1] = Elem<DT>::pack2(s[q][t][2], s[q][t][3]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < kOutTiles; ++t) {
+                const u32x4 kc = lds_col8(k_col, 32 * H0 * kPitch + 32 * t, 16 * kPitch);
+#pragma unroll
+                for (int q = 0; q < NQ; ++q) acc[q][t] = Elem<DT>::mfma(kc, ds[q], acc[q][t]);
+            }
+        };
+        half(std::integral_constant<int, 0>{});
+        if (left > 32) half(std::integral_constant<int, 1>{});
+    }
+    uint16_t *dq = (uint16_t *)w.dQ + o1;
+#pragma unroll
+    for (int q = 0; q < QT; ++q) {
+        const int row = r0 + kAttBlockRows * q + j;
+        if (row >= M) continue;
+#pragma unroll
+        for (int t = 0; t < kOutTiles; ++t) store4<DT>(dq + (int64_t)row * K, 16 * t + 4 * rg, K, acc[q][t], a.scale);
+    }
+}
+
+// Work item of a workgroup: item u of the (head, segment, block) items, head-major, cut into eight contiguous shares, one
+// per die (as in attention_kernel: the blocks of a pair read the same rows and run side by side on one die).
+// prefix: blocks of the segments before each segment; per_head: all of them.
+__device__ __forceinline__ bool att_item(const RunArgs &a, int which, int64_t per_head, int64_t &h, int &g, int &block) {
+    const unsigned id = blockIdx.x, die = id & 7u, kk = id >> 3;
+    const int32_t *pfx = plan_rowblocks(a.plan, a.nseg, which);
+    const int64_t items = per_head * a.H, share = (items + 7) >> 3;
+    const int64_t u = (int64_t)die * share + kk;
+    // a grid too small for the plan's items: the summary the launch was sized from is not this plan's
+    if (id == 0 && threadIdx.x == 0 && share * 8 > (int64_t)gridDim.x)
+        atomicAdd(&reinterpret_cast<PlanHeader *>(a.plan)->run_errors, 1);
+    if (kk >= share || u >= items) return false;
+    h = u / per_head;
+    const int item = (int)(u % per_head);
+    g = prefix_search(pfx, a.nseg, item);
+    block = item - ((ConstI32)(uintptr_t)pfx)[g];
+    return true;
+}
+// The head dimension fits the build and every byte offset inside the segment fits 32 bits.
+__device__ __forceinline__ bool att_fits(const RunArgs &a, const SegRec &rec, int kp, int64_t h, int block) {
+    if (rec.K <= kp && ((int64_t)max(rec.M, rec.N) + kAttKeys) * rec.K < (int64_t(1) << 31)) return true;
+    if (h == 0 && block == 0 && threadIdx.x == 0) atomicAdd(&reinterpret_cast<PlanHeader *>(a.plan)->run_errors, 1);
+    return false;
+}
+
+template <int DT, int NK, int QT>
+__global__ __launch_bounds__(256, 2) void attention_dq_kernel(RunArgs a, AttBwdArgs w) {
+    __shared__ __attribute__((aligned(16))) unsigned char sK[kAttKeys * att_pitch(NK)];
+    __shared__ __attribute__((aligned(16))) unsigned char sV[kAttKeys * att_pitch(NK)];
+    const ConstHdr hdr = (ConstHdr)(uintptr_t)a.plan;
+    const int64_t per_head = QT == 2 ? hdr->att_blocks128 : hdr->att_blocks64;
+    const int min_K = hdr->min_K;
+    if (!header_ok(a)) { report_mismatch(a); return; }
+    int64_t h;
+    int g, block;
+    if (!att_item(a, QT - 1, per_head, h, g, block)) return;
+    const SegRec rec = load_rec(plan_ro(a.plan, a.nseg).recs, g);
+    if (rec.M < 1 || rec.K < 1 || !att_fits(a, rec, 32 * NK, h, block)) return;
+    const int64_t row0 = att_row_base(min_K, a.Dm1, h, rec.off1);
+    if ((rec.K & 7) == 0) att_dq_body<DT, NK, QT, true>(a, w, rec, h, row0, block, sK, sV);
+    else att_dq_body<DT, NK, QT, false>(a, w, rec, h, row0, block, sK, sV);
+}
+
+// ------------------------------------------------------------------------------------------------------- dK and dV
+// Workgroup = PAIRS pairs of wavefronts; a pair owns 32 keys and walks the queries in blocks of QB staged in LDS (Q and
+// dO rows, two stages).  One wavefront of a pair (side 0) holds K's fragments and dV's sums, the other (side 1) V's
+// fragments and dK's sums, which keeps either within the registers of two wavefronts per SIMD at a head dimension of 128
+// (both sums and both operands in one wavefront would take 192 registers before the first score):
+//   step 1   side 0: P = 2^(c Q K^T - lse), packed, handed over through LDS;   side 1: dP = dO V^T
+//   step 2   side 0: dV^T += dO^T P;                                           side 1: dS = P o (dP - delta), dK^T += Q^T dS
+// Both sides run the same code on the two arrays in exchanged roles, two products each.
+template <int DT, int NK, int PAIRS, int QB, bool VEC>
+__device__ __forceinline__ void att_dkdv_body(const RunArgs &a, const AttBwdArgs &w, const SegRec &rec, int64_t h, int64_t row0,
+                                              int block, unsigned char *lds) {
+    constexpr int kThreads = 128 * PAIRS;
+    using St = AttStage<NK, kThreads, QB>;
+    constexpr int kTiles = QB / 16;
+    constexpr int kPitch = att_pitch(NK);
+    constexpr int kArray = QB * kPitch;          // bytes of one staged array
+    constexpr int kStage = 2 * kArray + 8 * QB;        // Q, dO, lse, delta
+    constexpr int kOutTiles = 2 * NK;
+    const int M = rec.M, N = rec.N, K = rec.K;
+    const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = lane_id(), j = lane & 15, rg = lane >> 4;
+    const int side = wave / PAIRS, pair = wave % PAIRS;
+    const int64_t o1 = h * a.Dm1 + rec.off1, o2 = h * a.Dm2 + rec.off2;
+    const RowPieces<VEC> pq((const uint16_t *)a.A + o1, M, K), pg((const uint16_t *)w.dO + o1, M, K);
+    const RowPieces<VEC> pf((const uint16_t *)(side ? w.V : a.B) + o2, N, K);
+    const float c = a.scale * kLog2e;
+
+    const int s_row = tid / St::kLpr, s_piece = tid % St::kLpr;
+    u32x4 qw[St::kSteps], gw[St::kSteps];
+    float aux = 0.f;                                   // threads 0 .. QB - 1: lse, QB .. 2 QB - 1: delta of a row of the block
+    auto fetch = [&](int qb) {
+#pragma unroll
+        for (int s = 0; s < St::kSteps; ++s) {
+            const uint32_t off = pq.offset(qb + s * St::kRowsStep + s_row, s_piece);
+            qw[s] = pq.load(off);
+            gw[s] = pg.load(off);
+        }
+        if (tid < 2 * QB) {
+            const int row = qb + (tid & (QB - 1));
+            // 2^-inf: rows that do not exist have no probabilities
+            aux = row < M ? (tid < QB ? w.lse : w.delta)[row0 + row] : tid < QB ? INFINITY : 0.f;
+        }
+    };
+    auto put = [&](int qb, unsigned char *stage) {
+        if ((St::kLpr == St::kPieces || s_piece < St::kPieces) && (St::kRowsStep <= QB || s_row < QB)) {
+#pragma unroll
+            for (int s = 0; s < St::kSteps; ++s) {
+                const int row = s * St::kRowsStep + s_row;
+                const uint32_t off = pq.offset(qb + row, s_piece);
+                *reinterpret_cast<u32x4 *>(stage + row * kPitch + s_piece * 16) = pq.finish(qw[s], off, s_piece);
+                *reinterpret_cast<u32x4 *>(stage + kArray + row * kPitch + s_piece * 16) = pg.finish(gw[s], off, s_piece);
+            }
+        }
+        if (tid < 2 * QB) *reinterpret_cast<float *>(stage + 2 * kArray + 4 * tid) = aux;
+    };
+    if (M > 0) fetch(0);
+
+    const int key0 = block * 32 * PAIRS + 32 * pair;
+    const bool alive = key0 < N;
+    u32x4 kf[2][NK];
+    f32x4 acc[kOutTiles][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int s = 0; s < NK; ++s) kf[u][s] = pf.get(key0 + 16 * u + j, 4 * s + rg);
+#pragma unroll
+        for (int t = 0; t < kOutTiles; ++t) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    // this side's arrays: rows for the scores (Q / dO), columns for the sums (dO / Q)
+    const LdsPtr row_base = lds_ptr(lds) + side * kArray + j * kPitch + rg * 16;
+    const LdsPtr col_base = lds_ptr(lds) + (1 - side) * kArray + (4 * rg + (j >> 2)) * kPitch + (j & 3) * 8;
+    const LdsPtr aux_base = lds_ptr(lds) + 2 * kArray + side * 4 * QB + rg * 16;
+    unsigned char *hand = lds + 2 * kStage + pair * (64 * QB) + lane * 16;        // kTiles 16-byte slots of 64 lanes a pair
+    if (M > 0) put(0, lds);
+    att_lds_barrier();
+
+    for (int qb = 0, stage = 0; qb < M; qb += QB, stage ^= 1) {
+        const bool more = qb + QB < M;
+        if (more) fetch(qb + QB);
+        f32x4 s[kTiles][2];
+        u32x4 pk[kTiles / 2][2];                                // [row tile pair][key tile]
+        if (alive) {
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) s[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int st = 0; st < NK; ++st)
+#pragma unroll
+                for (int t = 0; t < kTiles; ++t) {
+                    const u32x4 rf = lds_row16(row_base, stage * kStage + 16 * t * kPitch + 64 * st);
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) s[t][u] = Elem<DT>::mfma(rf, kf[u][st], s[t][u]);
+                }
+            if (side == 0) {
+#pragma unroll
+                for (int t = 0; t < kTiles; ++t) {
+                    const f32x4 l = __builtin_bit_cast(f32x4, lds_row16(aux_base, stage * kStage + 64 * t));
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) s[t][u][e] = __builtin_amdgcn_exp2f(fmaf(s[t][u][e], c, -l[e]));
+                        pk[t >> 1][u][2 * (t & 1)] = Elem<DT>::pack2(s[t][u][0], s[t][u][1]);
+                        pk[t >> 1][u][2 * (t & 1) + 1] = Elem<DT>::pack2(s[t][u][2], s[t][u][3]);
+                    }
+                }
+#pragma unroll
+                for (int tt = 0; tt < kTiles / 2; ++tt)
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) *reinterpret_cast<u32x4 *>(hand + (2 * tt + u) * 1024) = pk[tt][u];
+            }
+        }
+        att_lds_barrier();
+        if (alive) {
+            if (side == 1) {
+#pragma unroll
+                for (int tt = 0; tt < kTiles / 2; ++tt)
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) pk[tt][u] = *reinterpret_cast<const u32x4 *>(hand + (2 * tt + u) * 1024);
+#pragma unroll
+                for (int t = 0; t < kTiles; ++t) {
+                    const f32x4 d = __builtin_bit_cast(f32x4, lds_row16(aux_base, stage * kStage + 64 * t));
+#pragma unroll
+                    for (int u = 0; u < 2; ++u)
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            const uint32_t p = pk[t >> 1][u][2 * (t & 1) + i];
+                            pk[t >> 1][u][2 * (t & 1) + i] =
+                                Elem<DT>::pack2(lo16<DT>(p) * (s[t][u][2 * i] - d[2 * i]),
+                                                hi16<DT>(p) * (s[t][u][2 * i + 1] - d[2 * i + 1]));
+                        }
+                }
+            }
+#pragma unroll
+            for (int tt = 0; tt < kTiles / 2; ++tt)
+#pragma unroll
+                for (int t = 0; t < kOutTiles; ++t) {
+                    const u32x4 cf = lds_col8(col_base, stage * kStage + 32 * tt * kPitch + 32 * t, 16 * kPitch);
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) acc[t][u] = Elem<DT>::mfma(cf, pk[tt][u], acc[t][u]);
+                }
+        }
+        if (more) put(qb + QB, lds + (stage ^ 1) * kStage);
+        att_lds_barrier();
+    }
+    uint16_t *out = (uint16_t *)(side ? w.dK : w.dV) + o2;
+    const float f = side ? a.scale : 1.0f;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int key = key0 + 16 * u + j;
+        if (key >= N) continue;
+#pragma unroll
+        for (int t = 0; t < kOutTiles; ++t) store4<DT>(out + (int64_t)key * K, 16 * t + 4 * rg, K, acc[t][u], f);
+    }
+}
+
+constexpr int att_dkdv_lds(int nk, int pairs, int qb) { return 2 * (2 * qb * att_pitch(nk) + 8 * qb) + pairs * 64 * qb; }
+
+template <int DT, int NK, int PAIRS, int QB>
+__global__ __launch_bounds__(128 * PAIRS, 2) void attention_dkdv_kernel(RunArgs a, AttBwdArgs w) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    static_assert(PAIRS == 2 || PAIRS == 4, "the plan's column-block prefixes count blocks of 64 and of 128");
+    const ConstHdr hdr = (ConstHdr)(uintptr_t)a.plan;
+    const int64_t per_head = PAIRS == 4 ? hdr->att_cols128 : hdr->att_cols64;
+    const int min_K = hdr->min_K;
+    if (!header_ok(a)) return;                         // reported by the dQ kernel
+    int64_t h;
+    int g, block;
+    if (!att_item(a, PAIRS == 4 ? 3 : 2, per_head, h, g, block)) return;
+    const SegRec rec = load_rec(plan_ro(a.plan, a.nseg).recs, g);
+    if (rec.N < 1 || rec.K < 1 || !att_fits(a, rec, 32 * NK, h, block)) return;
+    const int64_t row0 = att_row_base(min_K, a.Dm1, h, rec.off1);
+    if ((rec.K & 7) == 0) att_dkdv_body<DT, NK, PAIRS, QB, true>(a, w, rec, h, row0, block, lds);
+    else att_dkdv_body<DT, NK, PAIRS, QB, false>(a, w, rec, h, row0, block, lds);
+}
+
+template <int DT, int NK, int QT, int PAIRS, int QB>
+static int launch_bwd(const RunArgs &args, const AttBwdArgs &w, const ba_plan_info *info, hipStream_t stream) {
+    constexpr int kLds = att_dkdv_lds(NK, PAIRS, QB);
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&attention_dkdv_kernel<DT, NK, PAIRS, QB>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    if (attr != hipSuccess) return BA_ERR_LAUNCH;
+    const int64_t rows = ((QT == 2 ? info->att_blocks128 : info->att_blocks64) * args.H + 7) / 8 * 8;
+    // (blocks of 128 columns: at most half of the blocks of 64 and a half more for every segment)
+    const int64_t blocks = PAIRS == 4 ? ((int64_t)info->att_cols64 + info->nseg) / 2 : info->att_cols64;
+    const int64_t cols = (blocks * args.H + 7) / 8 * 8;
+    if (rows > 0x7fffffff || cols > 0x7fffffff) return BA_ERR_UNSUPPORTED;
+    if (rows > 0) hipLaunchKernelGGL((attention_dq_kernel<DT, NK, QT>), dim3((unsigned)rows), dim3(256), 0, stream, args, w);
+    if (cols > 0)
+        hipLaunchKernelGGL((attention_dkdv_kernel<DT, NK, PAIRS, QB>), dim3((unsigned)cols), dim3(128 * PAIRS), kLds, stream, args, w);
+    return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
+}
+
+template <int DT, int QT, int PAIRS, int QB>
+static int launch_bwd_nk(int nk, const RunArgs &args, const AttBwdArgs &w, const ba_plan_info *info, hipStream_t stream) {
+    switch (nk) {
+        case 1: return launch_bwd<DT, 1, QT, PAIRS, QB>(args, w, info, stream);
+        case 2: return launch_bwd<DT, 2, QT, PAIRS, QB>(args, w, info, stream);
+        case 3: return launch_bwd<DT, 3, QT, PAIRS, QB>(args, w, info, stream);
+        default: return launch_bwd<DT, 4, QT, PAIRS, QB>(args, w, info, stream);
+    }
+}
+
+int launch_attention_backward(int dtype, const RunArgs &args, const void *V, const void *O, const void *dO, const float *lse,
+                              float *delta, void *dQ, void *dK, void *dV, const ba_plan_info *info, hipStream_t stream) {
+    if (info->max_K > 128 || info->nseg <= 0) return info->nseg <= 0 ? BA_OK : BA_ERR_UNSUPPORTED;
+    const AttBwdArgs w{V, O, dO, lse, delta, dQ, dK, dV};
+    const int nk = std::max(1, (info->max_K + 31) / 32);
+    // Segments of 256 rows and more on average: wavefronts of two query strips, and workgroups of 128 keys that stage 64
+    // queries (16 x 16 pairs of 1024 .. 4096 rows: dK and dV 2.10 ms; 64 keys and 32 queries 2.78 ms, 128 keys and 32
+    // queries 2.44 ms: every query block is staged once per workgroup).  Shorter ones: 64 keys and 32 queries, two to
+    // three times as many resident workgroups (1024 x 4 pairs of 2 .. 512 rows: 127 us; 64 queries 184 us, 128 keys 168 us).
+    const bool tall = info->total_rows >= 256 * std::max<int64_t>(info->nseg, 1);
+    if (dtype == BA_F16)
+        return tall ? launch_bwd_nk<0, 2, 4, 64>(nk, args, w, info, stream) : launch_bwd_nk<0, 1, 2, 32>(nk, args, w, info, stream);
+    if (dtype == BA_BF16)
+        return tall ? launch_bwd_nk<1, 2, 4, 64>(nk, args, w, info, stream) : launch_bwd_nk<1, 1, 2, 32>(nk, args, w, info, stream);
+    return BA_ERR_UNSUPPORTED;
+}
+
+}  // namespace ba

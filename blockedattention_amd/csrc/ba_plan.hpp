@@ -4,8 +4,9 @@
 //   PlanHeader                    (256 bytes)
 //   SegRec recs[cap]              one 48-byte record per segment: offsets and shape
 //   SegRec lists[5][cap]          the records of each launch class once more, compacted (work lists)
-//   int32  rowblocks[2][cap + 4]  GEMM plans: exclusive prefix over the segments of their row blocks of 64 and of
-//                                 128 rows (the one-pass attention's work items); entry nseg = all of them
+//   int32  rowblocks[4][cap + 4]  GEMM plans: exclusive prefix over the segments of their row blocks of 64 and of
+//                                 128 rows and of their column blocks of 64 and of 128 (the work items of the
+//                                 one-pass attention and of its backward); entry nseg = all of them
 //
 // cap = nseg rounded up so that every array starts 16-byte aligned.  The
 // compute kernels read the plan through scalar loads (it is never written
@@ -64,11 +65,16 @@ enum PrefixKind {
     kPfxPack = 10,  // 1 for the first segment of a pack of tiny segments, else 0
     kPfxSlow = 11,  // ceil(M/16) for segments the 16-byte operand loads cannot serve
     kPfxAtt64 = 12,   // GEMM plans: ceil(M/64) for every segment with rows (one-pass attention, any-layout GEMM)
-    kPfxAtt128 = 13,  // the same in row blocks of 128
+    kPfxAttCols = 13, // GEMM plans: ceil(N/64) for every segment with columns (backward of the one-pass attention)
     kPfxMini = 14,    // 1 for a segment of the strip kernel's main list that is small enough for one wavefront
-    kPfxPipe = 15,    // 1 for a segment of the tile list that the pipelined row-block kernel can take (fused call)
-    kNumPrefix = 16
+    kNumPrefix = 15
 };
+// Three of the flags share their scanned word with a second one (a pass holds at most 1024 segments, 16 bits suffice):
+//   kPfxMini   2^16 for a segment of the tile list that the pipelined row-block kernel can take (fused call)
+//   kPfxPack   2^16 for a segment with an odd number of row blocks of 64
+//   kListRows  2^16 for a segment with an odd number of column blocks of 64
+// The blocks of 128 before a segment are half of the blocks of 64 and the odd segments before it.
+enum SecondFlag { kTwoPipe = 0, kTwoOddRows = 1, kTwoOddCols = 2, kNumTwo = 3 };
 
 // "Mini" segments: strip-class segments of at most 64 rows whose B_g needs at most kMiniBlocks LDS blocks and at most
 // eight column tiles.  One wavefront can take such a segment on its own (a quarter of a 64 KiB window), so four of
@@ -82,7 +88,7 @@ __host__ __device__ inline bool mini_shape(int M, int N, int K) {
     return M >= 1 && M <= kMiniRows && b >= 1 && b <= kMiniBlocks && fast_strip_tiles(N) <= 8;
 }
 constexpr int kMailboxTicket = 256;   // byte offset of the ticket word in a scheduler mailbox (behind the header copy)
-constexpr int kAttBlockRows = 64;   // kPfxAtt64 counts blocks of this many rows, kPfxAtt128 of twice as many
+constexpr int kAttBlockRows = 64;   // kPfxAtt64 counts blocks of this many rows, kPfxAttCols of as many columns
 
 // A segment is "aligned" when K % 8 == 0 and its A and B offsets are multiples
 // of 8 elements: every operand row then starts on a 16-byte boundary (given
@@ -102,14 +108,15 @@ struct PlanHeader {
     int32_t bad_segments;
     int32_t run_errors;      // bumped by kernels that refuse to run
     int32_t small_max_N, small_max_M;   // maxima over the segments of the strip kernel's main launch
-    int32_t att_blocks64, att_blocks128;   // totals of kPfxAtt64 / kPfxAtt128: the one-pass attention's row blocks per head
+    int32_t att_blocks64, att_blocks128;   // row blocks of 64 and of 128 per head: the one-pass attention's work items
     int32_t mini_count;      // total of kPfxMini
-    int32_t pipe_count;      // total of kPfxPipe
+    int32_t pipe_count;      // segments of the tile list that the pipelined row-block kernel can take
     int32_t pipe_groups;     // bumped by every workgroup of the pipelined row-block kernel that found work in this plan
     int32_t min_N, min_K;    // smallest N and K over the segments that have rows and columns (0: there is none)
     int32_t ring_groups;     // bumped by every workgroup of the any-layout GEMM that wrote its rows through the LDS ring
     int32_t wide_groups;     // bumped by every workgroup of the row-block kernel's build for 128 < K <= 256 that found work
-    int32_t pad_[12];
+    int32_t att_cols64, att_cols128;   // column blocks of 64 and of 128 per head: its backward's
+    int32_t pad_[10];
 };
 static_assert(sizeof(PlanHeader) == 256, "PlanHeader must stay 256 bytes");
 
@@ -179,10 +186,10 @@ __host__ __device__ constexpr size_t plan_lists_end(int64_t nseg) {
     return sizeof(PlanHeader) + (1 + kNumLists) * (size_t)plan_cap(nseg) * sizeof(SegRec);
 }
 __host__ __device__ constexpr size_t plan_bytes_for(int64_t nseg) {
-    return plan_lists_end(nseg) + 2 * ((size_t)plan_cap(nseg) + 4) * sizeof(int32_t);     // cap is a multiple of 4
+    return plan_lists_end(nseg) + 4 * ((size_t)plan_cap(nseg) + 4) * sizeof(int32_t);     // cap is a multiple of 4
 }
-// Row-block prefix `which` (0: blocks of 64 rows, 1: of 128): entry g = blocks of the segments before g,
-// entry nseg = all.
+// Row-block prefix `which` (0: blocks of 64 rows, 1: of 128 rows, 2: of 64 columns, 3: of 128): entry g = blocks of the segments
+// before g, entry nseg = all.
 __host__ __device__ inline int32_t *plan_rowblocks(void *buf, int64_t nseg, int which) {
     return (int32_t *)((char *)buf + plan_lists_end(nseg)) + (size_t)which * ((size_t)plan_cap(nseg) + 4);
 }

@@ -7,6 +7,7 @@
 #include <chrono>
 #include <mutex>
 
+#include "att_common.hpp"
 #include "ba_host.hpp"
 
 // Plan buffer of ba_gemm_softmax_static: one array per GPU the library runs on, held until the process ends.
@@ -129,6 +130,7 @@ static int info_from_header(const PlanHeader &h, ba_plan_info *info) {
     info->min_N = h.min_N; info->min_K = h.min_K;
     info->ring_groups = h.ring_groups;
     info->wide_groups = h.wide_groups;
+    info->att_cols64 = h.att_cols64;
     return (h.bad_segments || h.run_errors) ? BA_ERR_BAD_METADATA : BA_OK;
 }
 
@@ -326,7 +328,37 @@ __attribute__((visibility("default"))) int ba_varlen_attention(void *plan, const
     if (H == 0 || Dm1 == 0 || nseg == 0) return BA_OK;
     if (!out || !Q || (Dm2 > 0 && (!K || !V))) return BA_ERR_INVALID_ARG;
     RunArgs args{plan, Q, K, out, H, Dm1, Dm2, Dout, scale, 0, 0, 0, (int)nseg};
-    return launch_attention(dtype, args, V, nseg, info, (hipStream_t)stream);
+    return launch_attention(dtype, args, V, nullptr, nseg, info, (hipStream_t)stream);
+}
+
+__attribute__((visibility("default"))) int64_t ba_attention_rows(const ba_plan_info *info, int64_t Dm1) {
+    return info && Dm1 > 0 ? att_rows_per_head(info->min_K, Dm1) : 0;
+}
+
+__attribute__((visibility("default"))) int ba_varlen_attention_train(void *plan, const ba_plan_info *info, int64_t nseg,
+                                                                     int dtype, const void *Q, const void *K,
+                                                                     const void *V, void *out, float *lse, int64_t H,
+                                                                     int64_t Dm1, int64_t Dm2, int64_t Dout, float scale,
+                                                                     ba_stream_t stream) {
+    if (!plan || nseg < 0 || nseg > (int64_t(1) << 30) || bad_sizes(H, Dm1, Dm2, Dout)) return BA_ERR_INVALID_ARG;
+    if (dtype != BA_F16 && dtype != BA_BF16) return BA_ERR_UNSUPPORTED;
+    if (H == 0 || Dm1 == 0 || nseg == 0) return BA_OK;
+    if (!out || !lse || !Q || (Dm2 > 0 && (!K || !V))) return BA_ERR_INVALID_ARG;
+    RunArgs args{plan, Q, K, out, H, Dm1, Dm2, Dout, scale, 0, 0, 0, (int)nseg};
+    return launch_attention(dtype, args, V, lse, nseg, info, (hipStream_t)stream);
+}
+
+__attribute__((visibility("default"))) int ba_varlen_attention_backward(
+    void *plan, const ba_plan_info *info, int64_t nseg, int dtype, const void *Q, const void *K, const void *V,
+    const void *out, const void *dO, const float *lse, float *delta, void *dQ, void *dK, void *dV, int64_t H, int64_t Dm1,
+    int64_t Dm2, int64_t Dout, float scale, ba_stream_t stream) {
+    if (!plan || !info || nseg < 0 || nseg > (int64_t(1) << 30) || bad_sizes(H, Dm1, Dm2, Dout)) return BA_ERR_INVALID_ARG;
+    if (dtype != BA_F16 && dtype != BA_BF16) return BA_ERR_UNSUPPORTED;
+    if (H == 0 || nseg == 0) return BA_OK;
+    if (Dm1 > 0 && (!Q || !out || !dO || !dQ || !lse || !delta)) return BA_ERR_INVALID_ARG;
+    if (Dm2 > 0 && (!K || !V || !dK || !dV)) return BA_ERR_INVALID_ARG;
+    RunArgs args{plan, Q, K, nullptr, H, Dm1, Dm2, Dout, scale, 0, 0, 0, (int)info->nseg};
+    return launch_attention_backward(dtype, args, V, out, dO, lse, delta, dQ, dK, dV, info, (hipStream_t)stream);
 }
 
 }  // extern "C"

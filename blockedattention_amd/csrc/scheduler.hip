@@ -130,11 +130,11 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedArgs a) {
     PlanView pv = plan_view(a.plan, nseg);
 
     int64_t base64[3] = {0, 0, 0};
-    int32_t base32[kNumPrefix] = {};
+    int32_t base32[kNumPrefix] = {}, base_two[kNumTwo] = {};
     int32_t maxM = 0, maxN = 0, maxK = 0, nbad = 0;
     int32_t maxSmallN = 0, maxSmallM = 0;       // widest / tallest segment of the strip kernel's main launch
     int32_t maxInvN = 0, maxInvK = 0;           // INT32_MAX - the smallest N and K of the segments that have rows and columns
-    // Every scanned count of a segment is at most max(rows, strips x chunks): while the sum of these weights stays
+    // Every scanned count of a segment is at most max(rows, column blocks, strips x chunks): while the sum of these weights stays
     // below 2^31, none of the int32 scans can overflow; a batch beyond that is rejected as a whole.
     int64_t weight = 0;
     const bool offsets_given = a.mode != 0;   // prefix sums are inputs
@@ -230,25 +230,26 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedArgs a) {
         int32_t v32[kNumScan], t32[kNumScan];
 #pragma unroll
         for (int q = 0; q < kNumLists; ++q) v32[q] = (cls == q && !mini) ? 1 : 0;
-        v32[kPfxMini] = mini ? 1 : 0;
-        v32[kPfxPipe] = (cls == kListTile && pipe_segment(seg_kind, ni, ki)) ? 1 : 0;
+        v32[kPfxMini] = (mini ? 1 : 0) + ((cls == kListTile && pipe_segment(seg_kind, ni, ki)) ? 1 << 16 : 0);
         const bool wide_rows = mi >= 1 && ni > kRunCols;      // the softmax row kernel's, whatever the plan kind
-        v32[kListRows] = wide_rows ? 1 : 0;
-        weight += max((int64_t)mi, (int64_t)strips * chunks) + 1;
+        const int32_t row_blocks = mi >= 1 ? (mi + kAttBlockRows - 1) / kAttBlockRows : 0;   // of every segment with rows, whatever N and K are
+        const int32_t col_blocks = ni >= 1 ? (ni + kAttBlockRows - 1) / kAttBlockRows : 0;
+        weight += max(max((int64_t)mi, (int64_t)col_blocks), (int64_t)strips * chunks) + 1;
         v32[kPfxGemm] = (mfma_ok && ni > kWaveCols) ? strips * chunks : 0;
         v32[kPfxStrip] = (mfma_ok && ni <= kWaveCols) ? strips : 0;
         v32[kPfxSplit] = (mfma_ok && ni > kWaveCols && ni <= kSplitCols) ? strips : 0;
         v32[kPfxWide] = (mfma_ok && ni > kSplitCols) ? strips : 0;
         v32[kPfxRows] = ni >= 1 ? mi : 0;
-        v32[kPfxPack] = pack > 0 ? 1 : 0;
+        v32[kListRows] = (wide_rows ? 1 : 0) + ((col_blocks & 1) << 16);
+        v32[kPfxPack] = (pack > 0 ? 1 : 0) + ((row_blocks & 1) << 16);
         v32[kPfxSlow] = aligned ? 0 : strips;
-        const bool att_rows = mi >= 1;                         // row blocks of every segment with rows, whatever N and K are
-        v32[kPfxAtt64] = att_rows ? (mi + kAttBlockRows - 1) / kAttBlockRows : 0;
-        v32[kPfxAtt128] = att_rows ? (mi + 2 * kAttBlockRows - 1) / (2 * kAttBlockRows) : 0;
+        v32[kPfxAtt64] = row_blocks;
+        v32[kPfxAttCols] = col_blocks;
         if (a.kind == 1) {
 #pragma unroll
             for (int q = 0; q < kNumPrefix; ++q)
                 if (q >= kNumLists && q != kPfxRows) v32[q] = 0;
+            v32[kListRows] &= 0xffff;
         }
         // The main strip launch's list is kept in eight buckets of decreasing work (16-row strips x column
         // tiles / 8, clipped): workgroups that start together then take about equally long and the longest
@@ -261,6 +262,13 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedArgs a) {
                 v32[kNumPrefix + wd] = (bucket >> 1) == wd ? 1 << (16 * (bucket & 1)) : 0;
         }
         block_exclusive_scan<int32_t, kNumScan, kSchedWaves>(v32, t32, sScan32);
+        constexpr int kTwoWord[kNumTwo] = {kPfxMini, kPfxPack, kListRows};
+        int32_t v_two[kNumTwo], t_two[kNumTwo];
+#pragma unroll
+        for (int q = 0; q < kNumTwo; ++q) {
+            v_two[q] = (int32_t)((uint32_t)v32[kTwoWord[q]] >> 16); v32[kTwoWord[q]] &= 0xffff;
+            t_two[q] = (int32_t)((uint32_t)t32[kTwoWord[q]] >> 16); t32[kTwoWord[q]] &= 0xffff;
+        }
         int32_t small_pos = v32[kListSmall];                  // position in the list among this pass's entries
         if constexpr (kBucketed) {
             small_pos = 0;
@@ -285,8 +293,11 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedArgs a) {
             if (mini) pv.list[kListSmall][plan_cap(nseg) - 1 - (base32[kPfxMini] + v32[kPfxMini])] = rec;
             if (wide_rows) pv.list[kListRows][base32[kListRows] + v32[kListRows]] = rec;
             if (a.kind == 0) {
-                plan_rowblocks(a.plan, nseg, 0)[g] = base32[kPfxAtt64] + v32[kPfxAtt64];
-                plan_rowblocks(a.plan, nseg, 1)[g] = base32[kPfxAtt128] + v32[kPfxAtt128];
+                const int32_t rows64 = base32[kPfxAtt64] + v32[kPfxAtt64], cols64 = base32[kPfxAttCols] + v32[kPfxAttCols];
+                plan_rowblocks(a.plan, nseg, 0)[g] = rows64;
+                plan_rowblocks(a.plan, nseg, 1)[g] = (rows64 + base_two[kTwoOddRows] + v_two[kTwoOddRows]) >> 1;
+                plan_rowblocks(a.plan, nseg, 2)[g] = cols64;
+                plan_rowblocks(a.plan, nseg, 3)[g] = (cols64 + base_two[kTwoOddCols] + v_two[kTwoOddCols]) >> 1;
             }
             if (!offsets_given) {
                 if (a.a1) a.a1[g] = o1;
@@ -304,6 +315,8 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedArgs a) {
         if (mi >= 1 && ni >= 1) { maxInvN = max(maxInvN, INT32_MAX - ni); maxInvK = max(maxInvK, INT32_MAX - ki); }
 #pragma unroll
         for (int q = 0; q < kNumPrefix; ++q) base32[q] += t32[q];
+#pragma unroll
+        for (int q = 0; q < kNumTwo; ++q) base_two[q] += t_two[q];
         if (!offsets_given) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) base64[q] += t64[q];
@@ -355,17 +368,22 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedArgs a) {
         h->small_max_N = rSN; h->small_max_M = rSM;
         h->bad_segments = rBad + ((D1 < 0 || D2 < 0 || DO < 0) ? 1 : 0) + (total_weight >= (int64_t(1) << 31) ? 1 : 0);
         h->run_errors = 0;
+        const int32_t rows128 = (base32[kPfxAtt64] + base_two[kTwoOddRows]) >> 1, cols128 = (base32[kPfxAttCols] + base_two[kTwoOddCols]) >> 1;
         h->att_blocks64 = base32[kPfxAtt64];
-        h->att_blocks128 = base32[kPfxAtt128];
+        h->att_blocks128 = rows128;
         h->mini_count = base32[kPfxMini];
-        h->pipe_count = base32[kPfxPipe];
+        h->pipe_count = base_two[kTwoPipe];
+        h->att_cols64 = base32[kPfxAttCols];
+        h->att_cols128 = cols128;
         h->pipe_groups = 0;
         h->min_N = rInvN ? INT32_MAX - rInvN : 0;
         h->min_K = rInvK ? INT32_MAX - rInvK : 0;
         h->ring_groups = 0;
         h->wide_groups = 0;
         plan_rowblocks(a.plan, nseg, 0)[nseg] = base32[kPfxAtt64];     // zero for softmax plans
-        plan_rowblocks(a.plan, nseg, 1)[nseg] = base32[kPfxAtt128];
+        plan_rowblocks(a.plan, nseg, 1)[nseg] = rows128;
+        plan_rowblocks(a.plan, nseg, 2)[nseg] = base32[kPfxAttCols];
+        plan_rowblocks(a.plan, nseg, 3)[nseg] = cols128;
         if (a.mailbox) {
             // the summary for a host that waits on the ticket instead of copying and synchronising: the header
             // first, visible system-wide, then the ticket behind it

@@ -459,30 +459,86 @@ Tensor sparseBlockedGEMMSoftmax_op(const Tensor &mat1, const Tensor &mat2, const
     return out;
 }
 
-// softmax(scale * Q_g K_g^T) V_g in one pass: forward only, the probabilities are never written.
-// Q is the M x K operand of the segments, K and V are both N x K; the result has Q's shape.
-Tensor sparseBlockedAttention_op(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mat1Accum,
-                                 const OptTensor &mat2Accum, const OptTensor &outAccum, const OptTensor &MList,
-                                 const OptTensor &NList, const OptTensor &KList, double scale) {
-    check_data(q, "q"); check_data(k, "k"); check_data(v, "v");
-    c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
-    TORCH_CHECK(q.scalar_type() == k.scalar_type() && q.scalar_type() == v.scalar_type(),
-                "q, k and v must have the same dtype");
-    TORCH_CHECK(q.scalar_type() == at::kHalf || q.scalar_type() == at::kBFloat16,
-                "the one-pass attention takes fp16 or bf16 operands");
-    TORCH_CHECK(q.device() == k.device() && q.device() == v.device(), "q, k and v must be on the same device");
-    Schedule s = schedule_gemm(q, mat1Accum, mat2Accum, outAccum, MList, NList, KList);
+// softmax(scale * Q_g K_g^T) V_g in one pass, the probabilities never written.  Q is the M x K operand of the segments,
+// K and V are both N x K; the result is [H, Dm1].  With lse, the rows' sums for the backward pass too.
+Tensor attention_launch(const Tensor &q, const Tensor &k, const Tensor &v, Schedule &s, double scale, Tensor *lse) {
     TORCH_CHECK(q.size(-1) == s.info.Dm1 && k.size(-1) == s.info.Dm2 && v.size(-1) == s.info.Dm2,
                 "operand sizes do not match the segments: need ", s.info.Dm1, " (q) and ", s.info.Dm2, " (k, v)");
     TORCH_CHECK(s.info.max_K <= 128, "the one-pass attention takes head dimensions up to 128, got ", s.info.max_K);
     const int64_t H = leading(q);
     TORCH_CHECK(leading(k) == H && leading(v) == H, "q, k and v disagree on the number of heads");
     Tensor out = at::empty({H, s.info.Dm1}, q.options());
-    check_status(ba_varlen_attention(s.plan.data_ptr(), &s.info, s.info.nseg, dtype_code(q, "attention"), q.data_ptr(),
-                                     k.data_ptr(), v.data_ptr(), out.data_ptr(), H, s.info.Dm1, s.info.Dm2,
-                                     s.info.Dout, (float)scale, current_stream(q)),
-                 "ba_varlen_attention");
+    const int dt = dtype_code(q, "attention");
+    void *stream = current_stream(q);
+    if (!lse) {
+        check_status(ba_varlen_attention(s.plan.data_ptr(), &s.info, s.info.nseg, dt, q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                         out.data_ptr(), H, s.info.Dm1, s.info.Dm2, s.info.Dout, (float)scale, stream),
+                     "ba_varlen_attention");
+        return out;
+    }
+    *lse = at::empty({H, ba_attention_rows(&s.info, s.info.Dm1)}, q.options().dtype(at::kFloat));
+    check_status(ba_varlen_attention_train(s.plan.data_ptr(), &s.info, s.info.nseg, dt, q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                           out.data_ptr(), lse->data_ptr<float>(), H, s.info.Dm1, s.info.Dm2, s.info.Dout,
+                                           (float)scale, stream),
+                 "ba_varlen_attention_train");
     return out;
+}
+
+Schedule attention_schedule(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &a1, const OptTensor &a2,
+                            const OptTensor &aO, const OptTensor &M, const OptTensor &N, const OptTensor &K) {
+    TORCH_CHECK(q.scalar_type() == k.scalar_type() && q.scalar_type() == v.scalar_type(),
+                "q, k and v must have the same dtype");
+    TORCH_CHECK(q.scalar_type() == at::kHalf || q.scalar_type() == at::kBFloat16,
+                "the one-pass attention takes fp16 or bf16 operands");
+    TORCH_CHECK(q.device() == k.device() && q.device() == v.device(), "q, k and v must be on the same device");
+    return schedule_gemm(q, a1, a2, aO, M, N, K);
+}
+
+// Differentiable form.  Between the passes it keeps the operands, the result, the rows' sums and the plan with its
+// summary: nothing of the size M x N, and the backward pass schedules nothing.
+class SparseBlockedAttention : public torch::autograd::Function<SparseBlockedAttention> {
+public:
+    static variable_list forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &a1,
+                                 const OptTensor &a2, const OptTensor &aO, const OptTensor &M, const OptTensor &N,
+                                 const OptTensor &K, double scale) {
+        Schedule s = attention_schedule(q, k, v, a1, a2, aO, M, N, K);
+        Tensor lse;
+        Tensor out = attention_launch(q, k, v, s, scale, &lse);
+        ctx->save_for_backward({q, k, v, out, lse, s.plan});
+        ctx->saved_data["info"] = std::string(reinterpret_cast<const char *>(&s.info), sizeof(s.info));
+        ctx->saved_data["scale"] = scale;
+        ctx->saved_data["lists"] = M.has_value() && N.has_value() && K.has_value();
+        return {out};
+    }
+
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
+        TORCH_CHECK(ctx->saved_data["lists"].toBool(), "blockFusedAttention: the backward pass needs MList, NList and KList");
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &plan = saved[5];
+        c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+        const Tensor grad = grads[0].to(q.scalar_type()).contiguous();
+        ba_plan_info info;
+        memcpy(&info, ctx->saved_data["info"].toStringRef().data(), sizeof(info));
+        Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), delta = at::empty_like(lse);
+        check_status(ba_varlen_attention_backward(plan.data_ptr(), &info, info.nseg, dtype_code(q, "attention backward"),
+                                                  q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), grad.data_ptr(),
+                                                  lse.data_ptr<float>(), delta.data_ptr<float>(), dq.data_ptr(),
+                                                  dk.data_ptr(), dv.data_ptr(), leading(q), info.Dm1, info.Dm2, info.Dout,
+                                                  (float)ctx->saved_data["scale"].toDouble(), current_stream(q)),
+                     "ba_varlen_attention_backward");
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+Tensor sparseBlockedAttention_op(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mat1Accum,
+                                 const OptTensor &mat2Accum, const OptTensor &outAccum, const OptTensor &MList,
+                                 const OptTensor &NList, const OptTensor &KList, double scale) {
+    check_data(q, "q"); check_data(k, "k"); check_data(v, "v");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+    if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
+        return SparseBlockedAttention::apply(q, k, v, mat1Accum, mat2Accum, outAccum, MList, NList, KList, scale)[0];
+    Schedule s = attention_schedule(q, k, v, mat1Accum, mat2Accum, outAccum, MList, NList, KList);
+    return attention_launch(q, k, v, s, scale, nullptr);
 }
 
 }  // namespace

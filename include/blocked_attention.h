@@ -98,6 +98,9 @@ typedef struct ba_plan_info {
     /* workgroups of the row-block kernel's build for 128 < K <= 256 (large segments, 16-bit results, whole-line
      * stores) that have found work in this plan since it was built */
     int32_t wide_groups;
+    /* GEMM plans: column blocks of 64 per head, summed over the segments with N >= 1 (backward of the one-pass
+     * attention).  In what was padding: the size of the structure is that of the version without it. */
+    int32_t att_cols64;
 } ba_plan_info;
 
 const char *ba_status_string(int status);
@@ -238,6 +241,28 @@ int ba_gemm_softmax(void *plan, const ba_plan_info *info, int64_t nseg, int dtyp
 int ba_varlen_attention(void *plan, const ba_plan_info *info, int64_t nseg, int dtype, const void *Q, const void *K,
                         const void *V, void *out, int64_t H, int64_t Dm1, int64_t Dm2, int64_t Dout, float scale,
                         ba_stream_t stream);
+
+/*
+ * Forward and backward of the one-pass attention for training.  The forward is
+ * ba_varlen_attention with one more result: `lse`, per query the base-2
+ * logarithm of its row's sum of 2^(scale log2(e) score).  The backward
+ * recomputes the probabilities from it and writes dQ ([H, Dm1]), dK and dV
+ * (both [H, Dm2]) for the gradient dO ([H, Dm1]) of the output O; with
+ * ba_varlen_gemm and ba_blocked_softmax_backward it stands in for the backward
+ * of the reference's chain (csrc/sparseBlockedAttention.cpp:52-72, 95-114)
+ * without its M x N arrays.  `lse` and the scratch array `delta` are fp32,
+ * H * ba_attention_rows(info, Dm1) entries each (one a row when all K_g are
+ * equal); entries of rows without keys are not touched.  `info` is required in
+ * the backward.  Types, limits and error codes as for ba_varlen_attention.
+ */
+int64_t ba_attention_rows(const ba_plan_info *info, int64_t Dm1);
+int ba_varlen_attention_train(void *plan, const ba_plan_info *info, int64_t nseg, int dtype, const void *Q, const void *K,
+                              const void *V, void *out, float *lse, int64_t H, int64_t Dm1, int64_t Dm2, int64_t Dout,
+                              float scale, ba_stream_t stream);
+int ba_varlen_attention_backward(void *plan, const ba_plan_info *info, int64_t nseg, int dtype, const void *Q,
+                                 const void *K, const void *V, const void *out, const void *dO, const float *lse,
+                                 float *delta, void *dQ, void *dK, void *dV, int64_t H, int64_t Dm1, int64_t Dm2,
+                                 int64_t Dout, float scale, ba_stream_t stream);
 
 /*
  * ba_gemm_softmax for callers that cannot allocate device memory (code under
