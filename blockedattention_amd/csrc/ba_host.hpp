@@ -85,7 +85,9 @@ int launch_gemm_any16(int dtype, const RunArgs &args, int64_t nseg, const ba_pla
 // where both take the 64 x 64 build; BA_ERR_UNSUPPORTED (nothing launched) otherwise.
 int launch_gemm_any16_two(int dtype, const RunArgs &a, const ba_plan_info *info_a, const RunArgs &b, const ba_plan_info *info_b,
                           hipStream_t stream);
-// fp32, fp64 and the integer types (gemm_generic.hip); dtype: ba_dtype
+// fp32 in any layout (gemm_f32.hip)
+int launch_gemm_f32(const RunArgs &args, int64_t nseg, const ba_plan_info *info, hipStream_t stream);
+// fp64 and the integer types (gemm_generic.hip); dtype: ba_dtype
 int launch_gemm_generic(int dtype, const RunArgs &args, int64_t nseg, const ba_plan_info *info, hipStream_t stream);
 int launch_softmax(int dtype, void *plan, int64_t nseg, const void *src, void *dst, int64_t H, int64_t Dsrc,
                    float scale, const ba_plan_info *info, hipStream_t stream);

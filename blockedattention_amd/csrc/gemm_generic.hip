@@ -1,9 +1,8 @@
 // Varlen GEMM for the element types without a kernel of their own (the reference's generic kernel,
-// csrc/cuda/spBlkGEMM.cu:120-271, instantiated by AT_DISPATCH_ALL_TYPES at :1010): fp32 and fp64 on the matrix
-// instructions of their type (v_mfma_f32_16x16x4_f32, v_mfma_f64_16x16x4_f64: products and sums in the element
-// type), the integer types with plain multiply-adds.  Like the reference, the accumulator has the element type:
+// csrc/cuda/spBlkGEMM.cu:120-271, instantiated by AT_DISPATCH_ALL_TYPES at :1010): fp64 on its matrix instruction
+// (v_mfma_f64_16x16x4_f64: products and sums in fp64), the integer types with plain multiply-adds.  Like the reference, the accumulator has the element type:
 // integers wrap modulo 2^bits, which is what unsigned arithmetic at 32 or 64 bits followed by a truncating store
-// yields bit for bit.  Any shape, offset and layout (transpose flags); fp16/bf16 have their own kernels.
+// yields bit for bit.  Any shape, offset and layout (transpose flags); fp16, bf16 and fp32 have their own kernels.
 //
 // Workgroup = 64 rows x 64 columns of one segment and head at a time, k in chunks of 64 (32 for the 8-byte
 // types).  A chunk of B_g (64 columns x chunk) is staged in LDS by the whole workgroup with coalesced loads along
@@ -24,8 +23,8 @@ constexpr int kGenCols = 64;                         // columns per block = lane
 constexpr int kGenRows = kStripRows * kGenWaves;     // rows per workgroup round
 
 // Element type T -> type S the operands are staged and accumulated in, chunk length, and where a lane's four
-// results of a 16 x 16 tile lie: lane (j = lane%16, q = lane/16) holds column j of rows 4q + e (fp32 matrix
-// instruction, and the layout the multiply-add path uses) or of rows 4e + q (fp64 matrix instruction).
+// results of a 16 x 16 tile lie: lane (j = lane%16, q = lane/16) holds column j of rows 4q + e (multiply-adds) or of
+// rows 4e + q (fp64 matrix instruction).
 template <typename T> struct Gen {
     typedef uint32_t S;
     static constexpr int kChunk = 64;
@@ -36,18 +35,12 @@ template <> struct Gen<int64_t> {
     static constexpr int kChunk = 32;
     static constexpr bool kMatrix = false, kRowsStrided = false;
 };
-template <> struct Gen<float> {
-    typedef float S;
-    static constexpr int kChunk = 64;
-    static constexpr bool kMatrix = true, kRowsStrided = false;
-};
 template <> struct Gen<double> {
     typedef double S;
     static constexpr int kChunk = 32;
     static constexpr bool kMatrix = true, kRowsStrided = true;
 };
 
-typedef float f32x4v __attribute__((ext_vector_type(4)));
 typedef double f64x4v __attribute__((ext_vector_type(4)));
 
 // grid (head, segment, z) with kFlagHeadFast (consecutive workgroups, which go to the dies in turn, are the heads
@@ -158,15 +151,9 @@ __global__ __launch_bounds__(kGenThreads) void gemm_generic_kernel(RunArgs a) {
 #pragma unroll
                         for (int t = 0; t < kGenCols / 16; ++t) {
                             const S bv = bcol[t * 16 * kPitchB + k4];
-                            if constexpr (sizeof(S) == 4) {
-                                f32x4v c = {acc[t][0], acc[t][1], acc[t][2], acc[t][3]};
-                                c = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, c, 0, 0, 0);
-                                acc[t][0] = c[0]; acc[t][1] = c[1]; acc[t][2] = c[2]; acc[t][3] = c[3];
-                            } else {
-                                f64x4v c = {acc[t][0], acc[t][1], acc[t][2], acc[t][3]};
-                                c = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, c, 0, 0, 0);
-                                acc[t][0] = c[0]; acc[t][1] = c[1]; acc[t][2] = c[2]; acc[t][3] = c[3];
-                            }
+                            f64x4v c = {acc[t][0], acc[t][1], acc[t][2], acc[t][3]};
+                            c = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, c, 0, 0, 0);
+                            acc[t][0] = c[0]; acc[t][1] = c[1]; acc[t][2] = c[2]; acc[t][3] = c[3];
                         }
                     }
                 } else {
@@ -222,7 +209,6 @@ int launch_gemm_generic(int dtype, const RunArgs &args, int64_t nseg, const ba_p
     const dim3 grid = head_fast ? dim3((unsigned)args.H, (unsigned)nseg, (unsigned)z)
                                 : dim3((unsigned)nseg, (unsigned)args.H, (unsigned)z);
     switch (dtype) {
-        case BA_F32: launch_generic_t<float>(run, grid, stream); break;
         case BA_F64: launch_generic_t<double>(run, grid, stream); break;
         case BA_U8: launch_generic_t<uint8_t>(run, grid, stream); break;
         case BA_I8: launch_generic_t<int8_t>(run, grid, stream); break;
