@@ -17,7 +17,7 @@ META_FROM_LISTS, META_FROM_ACCUM, META_GIVEN = 0, 1, 2
 
 SYMBOLS = (
     "ba_status_string", "ba_abi_version", "ba_plan_bytes", "ba_plan_gemm", "ba_plan_softmax", "ba_plan_read",
-    "ba_plan_read_into", "ba_plan_gemm_notify", "ba_plan_softmax_notify", "ba_plan_wait",
+    "ba_plan_read_into", "ba_plan_gemm_notify", "ba_plan_gemm_train_notify", "ba_plan_softmax_notify", "ba_plan_wait",
     "ba_varlen_gemm", "ba_blocked_softmax", "ba_blocked_softmax_backward", "ba_gemm_softmax",
     "ba_varlen_attention", "ba_attention_rows", "ba_varlen_attention_train", "ba_varlen_attention_backward",
     "ba_gemm_softmax_static", "ba_static_read", "ba_varlen_gemm_two",
@@ -79,6 +79,8 @@ def load():
     lib.ba_plan_read_into.argtypes = [vp, ctypes.POINTER(PlanInfo), vp, vp]
     lib.ba_plan_gemm_notify.restype = i32
     lib.ba_plan_gemm_notify.argtypes = [vp, ctypes.c_size_t, i64, i32, vp, vp, vp, vp, vp, vp, vp, u32, vp]
+    lib.ba_plan_gemm_train_notify.restype = i32
+    lib.ba_plan_gemm_train_notify.argtypes = [vp, vp, vp, ctypes.c_size_t, i64, i32, vp, vp, vp, vp, vp, vp, vp, u32, vp]
     lib.ba_plan_softmax_notify.restype = i32
     lib.ba_plan_softmax_notify.argtypes = [vp, ctypes.c_size_t, i64, vp, vp, vp, i32, vp, u32, vp]
     lib.ba_plan_wait.restype = i32

@@ -168,6 +168,16 @@ __attribute__((visibility("default"))) int ba_plan_gemm_notify(void *plan, size_
                            (hipStream_t)stream, mailbox, ticket);
 }
 
+__attribute__((visibility("default"))) int ba_plan_gemm_train_notify(void *plan, void *plan_dA, void *plan_dB,
+                                                                     size_t plan_bytes, int64_t nseg, int mode,
+                                                                     int64_t *MList, int64_t *NList, int64_t *KList,
+                                                                     int64_t *accum1, int64_t *accum2, int64_t *accumOut,
+                                                                     void *mailbox, uint32_t ticket, ba_stream_t stream) {
+    if (!mailbox) return BA_ERR_INVALID_ARG;
+    return launch_schedule_train(plan, plan_dA, plan_dB, plan_bytes, nseg, mode, MList, NList, KList, accum1, accum2,
+                                 accumOut, (hipStream_t)stream, (char *)mailbox, ticket);
+}
+
 __attribute__((visibility("default"))) int ba_plan_softmax_notify(void *plan, size_t plan_bytes, int64_t nseg,
                                                                   const int64_t *rowList, const int64_t *colList,
                                                                   int64_t *accum, int accum_given, void *mailbox,

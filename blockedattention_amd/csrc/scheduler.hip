@@ -109,10 +109,17 @@ __device__ __forceinline__ bool derive_lists(int64_t mk, int64_t nk, int64_t mn,
     return n * k == nk;
 }
 
+// Plans of one launch, a workgroup each: a training step's forward and backward products (see ba_plan_gemm_train_notify).
+constexpr int kSchedPlans = 3;
+struct SchedBatch {
+    SchedArgs plan[kSchedPlans];
+};
+
 constexpr int kSmallBuckets = 8;                          // work buckets of the main strip launch's list
 
 template <int kSchedThreads>
-__global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedArgs a) {
+__global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedBatch batch) {
+    const SchedArgs a = batch.plan[blockIdx.x];
     constexpr int kSchedWaves = kSchedThreads / 64;
     // Only the 256-thread build (65 to 256 segments) orders its list by work: smaller batches are resident at
     // once whatever their order, and in the larger builds, which are bound by instruction issue, the four more
@@ -395,9 +402,9 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedArgs a) {
     }
 }
 
-int launch_schedule(void *plan, size_t plan_bytes, int64_t nseg, int mode, int kind, int64_t *M, int64_t *N,
-                    int64_t *K, int64_t *a1, int64_t *a2, int64_t *aO, hipStream_t stream, void *mailbox,
-                    uint32_t ticket) {
+// Checks the arguments of one plan and fills `args`.
+static int schedule_args(SchedArgs &args, void *plan, size_t plan_bytes, int64_t nseg, int mode, int kind, int64_t *M, int64_t *N,
+                    int64_t *K, int64_t *a1, int64_t *a2, int64_t *aO, void *mailbox, uint32_t ticket) {
     if (!plan || nseg < 0 || nseg > (int64_t(1) << 30)) return BA_ERR_INVALID_ARG;
     if (plan_bytes < plan_bytes_for(nseg) || ((uintptr_t)plan & 15)) return BA_ERR_WORKSPACE;
     if (mode < 0 || mode > 2) return BA_ERR_INVALID_ARG;
@@ -410,12 +417,41 @@ int launch_schedule(void *plan, size_t plan_bytes, int64_t nseg, int mode, int k
         return BA_ERR_INVALID_ARG;
     }
     if (mailbox && ((uintptr_t)mailbox & 15)) return BA_ERR_INVALID_ARG;
-    SchedArgs args{plan, nseg, mode, kind, M, N, K, a1, a2, aO, mailbox, ticket};
-    if (nseg <= 64) hipLaunchKernelGGL(schedule_kernel<64>, dim3(1), dim3(64), 0, stream, args);
-    else if (nseg <= 256) hipLaunchKernelGGL(schedule_kernel<256>, dim3(1), dim3(256), 0, stream, args);
-    else if (nseg <= 512) hipLaunchKernelGGL(schedule_kernel<512>, dim3(1), dim3(512), 0, stream, args);
-    else hipLaunchKernelGGL(schedule_kernel<kSchedThreadsMax>, dim3(1), dim3(kSchedThreadsMax), 0, stream, args);
+    args = SchedArgs{plan, nseg, mode, kind, M, N, K, a1, a2, aO, mailbox, ticket};
+    return BA_OK;
+}
+
+static int launch_plans(const SchedBatch &args, unsigned plans, int64_t nseg, hipStream_t stream) {
+    if (nseg <= 64) hipLaunchKernelGGL(schedule_kernel<64>, dim3(plans), dim3(64), 0, stream, args);
+    else if (nseg <= 256) hipLaunchKernelGGL(schedule_kernel<256>, dim3(plans), dim3(256), 0, stream, args);
+    else if (nseg <= 512) hipLaunchKernelGGL(schedule_kernel<512>, dim3(plans), dim3(512), 0, stream, args);
+    else hipLaunchKernelGGL(schedule_kernel<kSchedThreadsMax>, dim3(plans), dim3(kSchedThreadsMax), 0, stream, args);
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
+}
+
+int launch_schedule(void *plan, size_t plan_bytes, int64_t nseg, int mode, int kind, int64_t *M, int64_t *N,
+                    int64_t *K, int64_t *a1, int64_t *a2, int64_t *aO, hipStream_t stream, void *mailbox, uint32_t ticket) {
+    SchedBatch args{};
+    const int st = schedule_args(args.plan[0], plan, plan_bytes, nseg, mode, kind, M, N, K, a1, a2, aO, mailbox, ticket);
+    return st != BA_OK ? st : launch_plans(args, 1, nseg, stream);
+}
+
+// The plans of a product and of its two gradients: dA = dS B is (M, K, N) over (dS, B, dA), dB = dS^T A is (N, K, M) over
+// (dS, A, dB).  The gradients' plans take the metadata from the caller's half of it, permuted, like the first one: they
+// need nothing that the first plan writes, so the three workgroups run side by side.
+int launch_schedule_train(void *plan, void *plan_dA, void *plan_dB, size_t plan_bytes, int64_t nseg, int mode, int64_t *M,
+                          int64_t *N, int64_t *K, int64_t *a1, int64_t *a2, int64_t *aO, hipStream_t stream, char *mailbox,
+                          uint32_t ticket) {
+    SchedBatch args{};
+    int st = schedule_args(args.plan[0], plan, plan_bytes, nseg, mode, 0, M, N, K, a1, a2, aO, mailbox, ticket);
+    const bool lists = mode != BA_META_FROM_ACCUM, accum = mode != BA_META_FROM_LISTS;
+    int64_t *m = lists ? M : nullptr, *n = lists ? N : nullptr, *k = lists ? K : nullptr;
+    int64_t *s1 = accum ? a1 : nullptr, *s2 = accum ? a2 : nullptr, *sO = accum ? aO : nullptr;
+    if (st == BA_OK) st = schedule_args(args.plan[1], plan_dA, plan_bytes, nseg, mode, 0, m, k, n, sO, s2, s1,
+                                        mailbox + BA_MAILBOX_BYTES, ticket);
+    if (st == BA_OK) st = schedule_args(args.plan[2], plan_dB, plan_bytes, nseg, mode, 0, n, k, m, sO, s1, s2,
+                                        mailbox + 2 * BA_MAILBOX_BYTES, ticket);
+    return st != BA_OK ? st : launch_plans(args, 3, nseg, stream);
 }
 
 }  // namespace ba

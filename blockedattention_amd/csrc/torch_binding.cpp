@@ -174,15 +174,15 @@ std::vector<int64_t> schedule_cache_stats() {
     return {c.hits, c.misses, (int64_t)c.entries.size(), (int64_t)c.capacity};
 }
 
-// Where a scheduler launch hands its summary to the host: BA_MAILBOX_BYTES of pinned, GPU-writable memory per
-// calling thread (allocated at the thread's first schedule, kept for the life of the process) and a ticket that
+// Where a scheduler launch hands its summaries to the host: BA_MAILBOX_BYTES of pinned, GPU-writable memory per
+// plan (up to three) and calling thread (allocated at the thread's first schedule, kept for the life of the process) and a ticket that
 // changes with every use.  The host then spins on the ticket instead of copying and synchronising the stream.
 struct Mailbox {
     void *mem = nullptr;
     uint32_t ticket = 0;
     Mailbox() {
-        if (hipHostMalloc(&mem, BA_MAILBOX_BYTES, hipHostMallocCoherent | hipHostMallocMapped | hipHostMallocPortable) != hipSuccess) mem = nullptr;
-        else memset(mem, 0, BA_MAILBOX_BYTES);
+        if (hipHostMalloc(&mem, 3 * BA_MAILBOX_BYTES, hipHostMallocCoherent | hipHostMallocMapped | hipHostMallocPortable) != hipSuccess) mem = nullptr;
+        else memset(mem, 0, 3 * BA_MAILBOX_BYTES);
     }
 };
 Mailbox &mailbox() {
@@ -192,7 +192,8 @@ Mailbox &mailbox() {
 
 // The three metadata cases of the reference (cpp:17-44), resolved on the device.
 Schedule schedule_gemm(const Tensor &like, const OptTensor &a1, const OptTensor &a2, const OptTensor &aO,
-                       const OptTensor &M, const OptTensor &N, const OptTensor &K, bool use_cache = true) {
+                       const OptTensor &M, const OptTensor &N, const OptTensor &K, bool use_cache = true,
+                       bool train = false) {
     const bool have_accum = a1.has_value() && a2.has_value() && aO.has_value();
     const bool have_lists = M.has_value() && N.has_value() && K.has_value();
     TORCH_CHECK(have_accum || have_lists,
@@ -234,12 +235,27 @@ Schedule schedule_gemm(const Tensor &like, const OptTensor &a1, const OptTensor 
     int st;
     if (mb.mem) {
         const uint32_t ticket = ++mb.ticket ? mb.ticket : ++mb.ticket;       // never 0, the mailbox's first content
-        check_status(ba_plan_gemm_notify(s.plan.data_ptr(), bytes, nseg, mode, s.M.data_ptr<int64_t>(),
-                                         s.N.data_ptr<int64_t>(), s.K.data_ptr<int64_t>(), s.accum1.data_ptr<int64_t>(),
-                                         s.accum2.data_ptr<int64_t>(), s.accumOut.data_ptr<int64_t>(), mb.mem, ticket,
-                                         stream),
-                     "ba_plan_gemm_notify");
-        st = ba_plan_wait(mb.mem, ticket, &s.info, 60 * 1000 * 1000);
+        int64_t *const m = s.M.data_ptr<int64_t>(), *const n = s.N.data_ptr<int64_t>(), *const k = s.K.data_ptr<int64_t>();
+        int64_t *const o1 = s.accum1.data_ptr<int64_t>(), *const o2 = s.accum2.data_ptr<int64_t>(),
+                *const oO = s.accumOut.data_ptr<int64_t>();
+        if (train) {
+            // the backward products' plans in the same launch (the same verdict and summaries as if made one by one)
+            auto g1 = std::make_shared<Schedule>(), g2 = std::make_shared<Schedule>();
+            g1->plan = at::empty_like(s.plan); g2->plan = at::empty_like(s.plan);
+            check_status(ba_plan_gemm_train_notify(s.plan.data_ptr(), g1->plan.data_ptr(), g2->plan.data_ptr(), bytes, nseg,
+                                                   mode, m, n, k, o1, o2, oO, mb.mem, ticket, stream),
+                         "ba_plan_gemm_train_notify");
+            st = ba_plan_wait(mb.mem, ticket, &s.info, 60 * 1000 * 1000);
+            char *const mem = static_cast<char *>(mb.mem);
+            const int st1 = ba_plan_wait(mem + BA_MAILBOX_BYTES, ticket, &g1->info, 60 * 1000 * 1000);
+            const int st2 = ba_plan_wait(mem + 2 * BA_MAILBOX_BYTES, ticket, &g2->info, 60 * 1000 * 1000);
+            if (st1 == BA_OK) s.derived->grad1 = std::move(g1);      // else the backward pass makes it, and reports
+            if (st2 == BA_OK) s.derived->grad2 = std::move(g2);
+        } else {
+            check_status(ba_plan_gemm_notify(s.plan.data_ptr(), bytes, nseg, mode, m, n, k, o1, o2, oO, mb.mem, ticket, stream),
+                         "ba_plan_gemm_notify");
+            st = ba_plan_wait(mb.mem, ticket, &s.info, 60 * 1000 * 1000);
+        }
     } else {
         check_status(ba_plan_gemm(s.plan.data_ptr(), bytes, nseg, mode, s.M.data_ptr<int64_t>(),
                                   s.N.data_ptr<int64_t>(), s.K.data_ptr<int64_t>(), s.accum1.data_ptr<int64_t>(),
@@ -325,14 +341,24 @@ Schedule &derived_schedule(const Schedule &s, std::shared_ptr<Schedule> Derived:
     return *p;
 }
 
+// A schedule that an autograd node keeps from its forward to its backward pass.
+struct KeptSchedule : torch::CustomClassHolder {
+    explicit KeptSchedule(const Schedule &schedule) : s(schedule) {}
+    const Schedule s;
+};
+const Schedule &kept_schedule(AutogradContext *ctx) {
+    return static_cast<const KeptSchedule *>(ctx->saved_data["schedule"].toCapsule().get())->s;
+}
+
 class SparseBlockedGEMM : public torch::autograd::Function<SparseBlockedGEMM> {
 public:
     static variable_list forward(AutogradContext *ctx, const Tensor &mat1, const Tensor &mat2, const OptTensor &a1,
                                  const OptTensor &a2, const OptTensor &aO, const OptTensor &M, const OptTensor &N,
-                                 const OptTensor &K, bool t1, bool t2) {
+                                 const OptTensor &K, bool t1, bool t2, bool train) {
         check_data(mat1, "mat1"); check_data(mat2, "mat2");
         c10::hip::HIPGuardMasqueradingAsCUDA guard(mat1.device());
-        Schedule s = schedule_gemm(mat1, a1, a2, aO, M, N, K);
+        Schedule s = schedule_gemm(mat1, a1, a2, aO, M, N, K, /*use_cache=*/true, train);
+        ctx->saved_data["schedule"] = c10::IValue::make_capsule(c10::make_intrusive<KeptSchedule>(s));
         ctx->save_for_backward({mat1, mat2, s.accum1, s.accum2, s.accumOut, s.M, s.N, s.K});
         ctx->saved_data["transpose1"] = t1;
         ctx->saved_data["transpose2"] = t2;
@@ -352,7 +378,7 @@ public:
         Tensor g1, g2;
         // dS and the saved operands are read as they lie: the products whose reduction runs over N or M take the
         // kernels for any layout and reduction length (two launches, like the reference)
-        Schedule fwd = schedule_gemm(grad, a1, a2, aO, M, N, K);          // the forward's, from the cache
+        const Schedule &fwd = kept_schedule(ctx);
         Schedule &s1 = derived_schedule(fwd, &Derived::grad1, grad, aO, a2, a1, M, K, N);
         Schedule &s2 = derived_schedule(fwd, &Derived::grad2, grad, aO, a1, a2, N, K, M);
         // batches of short segments: both products as ONE launch where the library offers it (layouts of the
@@ -376,7 +402,7 @@ public:
             g2 = gemm_launch(grad, mat1, s2, true, !t1);
         }
         return {g1.view_as(saved[0]), g2.view_as(saved[1]), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(),
-                Tensor(), Tensor(), Tensor()};
+                Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -396,6 +422,7 @@ public:
         check_status(ba_blocked_softmax(s.plan.data_ptr(), &s.info, s.info.nseg, dt, src.data_ptr(), out.data_ptr(), H,
                                         s.info.Dout, (float)scale, current_stream(src)),
                      "ba_blocked_softmax");
+        ctx->saved_data["schedule"] = c10::IValue::make_capsule(c10::make_intrusive<KeptSchedule>(s));
         ctx->save_for_backward({out, s.accumOut, s.M, s.N});
         ctx->saved_data["scale"] = scale;
         return {out};
@@ -406,7 +433,7 @@ public:
         const Tensor grad = grads[0].contiguous();
         c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
         const Tensor y = saved[0].to(grad.scalar_type());
-        Schedule s = schedule_softmax(grad, saved[2], saved[3], saved[1]);
+        const Schedule &s = kept_schedule(ctx);
         const int64_t H = leading(y);
         Tensor dx = at::empty_like(y);
         check_status(ba_blocked_softmax_backward(s.plan.data_ptr(), &s.info, s.info.nseg,
@@ -422,8 +449,9 @@ public:
 Tensor sparseBlockedGEMM_op(const Tensor &mat1, const Tensor &mat2, const OptTensor &mat1Accum,
                             const OptTensor &mat2Accum, const OptTensor &outAccum, const OptTensor &MList,
                             const OptTensor &NList, const OptTensor &KList, bool transpose1, bool transpose2) {
+    const bool train = at::GradMode::is_enabled() && (mat1.requires_grad() || mat2.requires_grad());
     return SparseBlockedGEMM::apply(mat1, mat2, mat1Accum, mat2Accum, outAccum, MList, NList, KList, transpose1,
-                                    transpose2)[0];
+                                    transpose2, train)[0];
 }
 
 Tensor sparseBlockedSoftmax_op(const Tensor &src, const OptTensor &rowList, const OptTensor &colList,

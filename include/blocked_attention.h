@@ -173,6 +173,14 @@ int ba_plan_gemm_notify(void *plan, size_t plan_bytes, int64_t nseg, int mode,
 int ba_plan_softmax_notify(void *plan, size_t plan_bytes, int64_t nseg,
                            const int64_t *rowList, const int64_t *colList,
                            int64_t *accum, int accum_given, void *mailbox, uint32_t ticket, ba_stream_t stream);
+/* ba_plan_gemm_notify for a training step: one launch makes the plan of the product and those of its two gradients,
+ * dA = dS B (plan_dA: metadata (M, K, N), operands dS and B) and dB = dS^T A (plan_dB: (N, K, M), dS and A), which the
+ * reference's backward derives again (csrc/sparseBlockedAttention.cpp:52-72).  All three buffers have plan_bytes; the
+ * mailbox holds three of BA_MAILBOX_BYTES, collected one by one with ba_plan_wait and the same ticket. */
+int ba_plan_gemm_train_notify(void *plan, void *plan_dA, void *plan_dB, size_t plan_bytes, int64_t nseg, int mode,
+                              int64_t *MList, int64_t *NList, int64_t *KList,
+                              int64_t *accum1, int64_t *accum2, int64_t *accumOut,
+                              void *mailbox, uint32_t ticket, ba_stream_t stream);
 int ba_plan_wait(const void *mailbox, uint32_t ticket, ba_plan_info *host_info, int64_t timeout_us);
 
 /*
