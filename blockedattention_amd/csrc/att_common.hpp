@@ -4,7 +4,7 @@
 #include <type_traits>
 #include <utility>
 
-#include "ba_gemm_common.hpp"
+#include "row_pieces.hpp"
 
 namespace ba {
 

@@ -10,7 +10,9 @@
 //   segment_kernel  everything that needs care instead of speed: packs of tiny
 //                   segments sharing one MFMA tile (wave_pack), segments that
 //                   break the 16-byte operand alignment (K % 8 != 0, odd segment
-//                   starts, transposed layouts: element-wise generic_rows),
+//                   starts: any_rows in the fused call, element by element in
+//                   the product alone, where few segments of a batch are of this
+//                   kind -- others take gemm_any16.hip),
 //                   strip-class leftovers whose B_g is walked in K slabs
 //                   (strips_from_lds).
 //
@@ -18,13 +20,14 @@
 // eight k-values are one 16-byte load straight into an MFMA operand register;
 // no transposition is ever needed.
 #include "strip_body.hpp"
+#include "any_rows.hpp"
 
 namespace ba {
 
 // ------------------------------------------------------------------ kernels
 // segment_kernel   grid (segment, head, z): one workgroup per segment and head;
-//                  its wavefronts take the segment's 16-row strips (N <= 256),
-//                  the pack it leads, or its rows on the element-wise path.
+//                  its wavefronts take the segment's 16-row strips (N <= 256, or
+//                  any N where it is not aligned), the pack it leads, or its rows on the element-wise path.
 //                  No search: the block index is the segment.
 // gemm_large_kernel  GEMM only, N > 256: one wavefront per 16 x 256 piece, found
 //                  by a search in the scanned piece counts.
@@ -35,8 +38,9 @@ namespace ba {
 // MAXNT = 8 is the build for batches whose widest segment has N <= 128: half the
 // accumulator registers, half again as many resident wavefronts.  The host picks it from
 // the plan summary; without a summary the 16-tile build runs.
-template <int DT, bool FUSED, bool F32OUT, int MAXNT>
-__global__ __launch_bounds__(kSegThreads, MAXNT <= 8 ? 6 : 4) void segment_kernel(RunArgs a) {
+// ANY: the build of the fused call for batches with segments of any alignment, which runs its strips through any_rows.
+template <int DT, bool FUSED, bool F32OUT, int MAXNT, bool ANY>
+__global__ __launch_bounds__(kSegThreads, ANY ? (MAXNT <= 8 ? 3 : 2) : MAXNT <= 8 ? 6 : 4) void segment_kernel(RunArgs a) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const PlanRO pv = plan_ro(a.plan, a.nseg);
     const int64_t h = blockIdx.y;
@@ -55,13 +59,21 @@ __global__ __launch_bounds__(kSegThreads, MAXNT <= 8 ? 6 : 4) void segment_kerne
     const bool mfma_ok = (a.flags & kFlagMfmaOk) != 0;
     if (kind == kSegEmpty) return;
     if (mfma_ok && a.list < 0 && launch_class(kind, s.M, s.N, s.K) != kListRest) return;   // another kernel's
-    if (!mfma_ok || kind == kSegSlow) {
-        // Element-wise path.  With MFMA ruled out for the whole launch this also
-        // covers the segments the list kernels would have taken.
-        for (int r = first; r < s.M; r += stride) generic_seg_rows<DT, FUSED>(s, a, r, r + 1, 0, s.N);
+    if constexpr (ANY) {
+        // With the 16-byte operand loads ruled out for the whole launch this also covers the segments the list
+        // kernels would have taken.
+        if (!mfma_ok || kind == kSegSlow || kind == kSegStrip) {
+            for (int base = blockIdx.z * kSegWaves * kStripRows; base < s.M; base += stride * kStripRows)
+                any_rows<DT, F32OUT, MAXNT>(s, a, lds, base + wave * kStripRows);
+            return;
+        }
+    } else if (!mfma_ok || kind == kSegSlow) {
+        // Element-wise path of the product alone (no fused launch of this build has such segments).
+        if constexpr (!FUSED)
+            for (int r = first; r < s.M; r += stride) generic_seg_rows<DT>(s, a, r, r + 1, 0, s.N);
         return;
     }
-    if (kind == kSegStrip) {
+    if (!ANY && kind == kSegStrip) {
         // One strip per wavefront; blockIdx.z selects the group of kSegWaves strips.
         const int strips = (s.M + kStripRows - 1) / kStripRows;
         const int nt = (s.N + 15) >> 4;
@@ -308,26 +320,34 @@ static int launch_set(int dtype, const RunArgs &args_in, int64_t nseg, const ba_
     if (n_rest > 0 && !packs_taken) {
         // z spreads the 16-row strips (or rows) of the largest segment over workgroups
         int64_t z = 4, blocks = 32;
+        const bool any = !info || !mfma_ok || info->slow_items > 0;
         if (info) {
-            const int64_t units = mfma_ok && info->slow_items == 0 ? ceil_div(std::min<int64_t>(info->max_M, 256), kStripRows)
-                                                                     : std::min<int64_t>(info->max_M, 4096);
+            // (segments of any alignment: strips of 16 rows in the fused call, single rows in the product alone)
+            const int64_t units = !any ? ceil_div(std::min<int64_t>(info->max_M, 256), kStripRows)
+                                : FUSED ? ceil_div(info->max_M, kStripRows) : std::min<int64_t>(info->max_M, 4096);
             z = std::max<int64_t>(1, std::min<int64_t>(64, ceil_div(units, kSegWaves)));
             // LDS window for B_g: whole B_g of the largest strip-class segment if it fits 64 KiB
             const int64_t nt = ceil_div(std::min<int64_t>(std::max<int64_t>(info->max_N, 1), kWaveCols), 16);
             const int64_t nks = ceil_div(std::max<int64_t>(info->max_K, 1), 32);
             blocks = std::max<int64_t>(nt, std::min<int64_t>(nt * nks, 64));
         }
+        if (FUSED && any) blocks = ceil_div(any_rows_lds(lean ? 8 : kMaxTiles), kLdsBlockBytes);
         RunArgs seg_args = args;
         seg_args.list = mfma_ok ? kListRest : -1;
         seg_args.lds_blocks = (int)blocks;
         const dim3 grid((unsigned)n_rest, H, (unsigned)z);
         const size_t lds_bytes = (size_t)blocks * kLdsBlockBytes;
-        if (lean)
-            hipLaunchKernelGGL((segment_kernel<DT, FUSED, F32OUT, 8>), grid, dim3(kSegThreads), lds_bytes, stream,
-                               seg_args);
-        else
-            hipLaunchKernelGGL((segment_kernel<DT, FUSED, F32OUT, 16>), grid, dim3(kSegThreads), lds_bytes, stream,
-                               seg_args);
+        auto launch = [&](auto any_tag) {
+            constexpr bool ANY = decltype(any_tag)::value;
+            if (lean)
+                hipLaunchKernelGGL((segment_kernel<DT, FUSED, F32OUT, 8, ANY>), grid, dim3(kSegThreads), lds_bytes, stream, seg_args);
+            else
+                hipLaunchKernelGGL((segment_kernel<DT, FUSED, F32OUT, 16, ANY>), grid, dim3(kSegThreads), lds_bytes, stream, seg_args);
+        };
+        if constexpr (FUSED) {
+            if (any) launch(std::true_type{});
+            else launch(std::false_type{});
+        } else launch(std::false_type{});
     }
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
 }

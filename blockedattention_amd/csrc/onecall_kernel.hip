@@ -1,6 +1,6 @@
 // Fused GEMM + softmax of a small batch (at most 512 segments) in ONE launch, without a plan: every
 // workgroup derives its own segment's offsets and class from the metadata arrays in registers, then runs
-// the same device bodies as the plan-driven kernels (strip, tile, leftover-strip or element-wise).
+// the same device bodies as the plan-driven kernels (strip, tile, leftover-strip or any-alignment rows).
 //
 // Grid (head, segment, z).  The first wavefront of a workgroup reads the whole metadata (one entry per lane
 // and round of 64 segments, every load issued before the first is used), applies the scheduler's acceptance
@@ -14,6 +14,7 @@
 // own), the segments run in index order, not in work order, and every workgroup has the 64 KiB window and the
 // 16-tile build's registers, whatever the widest segment is (the host does not know it).
 #include "strip_body.hpp"
+#include "any_rows.hpp"
 
 namespace ba {
 
@@ -160,7 +161,8 @@ __global__ __launch_bounds__(kSegThreads, 2) void onecall_kernel(RunArgs a, Meta
     const int first = bz * kSegWaves + wave, stride = gz * kSegWaves;
     if (!(a.flags & kFlagMfmaOk) || !aligned) {
         s.kind = kSegSlow;
-        for (int r = first; r < s.M; r += stride) generic_seg_rows<DT, true>(s, a, r, r + 1, 0, s.N);
+        for (int base = bz * kSegWaves * kStripRows; base < s.M; base += stride * kStripRows)
+            any_rows<DT, F32OUT, kMaxTiles>(s, a, lds, base + wave * kStripRows);
         return;
     }
     s.kind = s.N <= kWaveCols ? kSegStrip : s.N <= kSplitCols ? kSegSplit : kSegWide;
@@ -190,6 +192,7 @@ static int launch_oc(const RunArgs &args_in, const MetaArgs &meta, hipStream_t s
     args.lds_extra = 0;
     args.list = -1;
     const size_t lds_bytes = (size_t)kBigBlocks * kLdsBlockBytes;
+    static_assert(kBigBlocks * kLdsBlockBytes >= any_rows_lds(kMaxTiles), "the panel of any_rows fits the window");
     static_assert(kBigBlocks * kLdsBlockBytes >= kStages * kTileChunkBytes, "the tile body's stages fit the window");
     // two workgroups per compute unit's worth of (segment, head) pairs where the batch has that few; a z
     // beyond a segment's strips or row blocks costs a workgroup that reads the metadata and leaves

@@ -19,12 +19,11 @@ __device__ __forceinline__ u32x4 load_frag_fast(const uint16_t *__restrict__ row
 }
 
 // ------------------------------------------------------------ generic rows
-// Fallback for segments the 16-byte operand loads cannot serve (K % 8 != 0,
-// odd segment starts, transposed layouts): one wavefront walks rows
-// [r_begin, r_end), lanes own columns c_begin + lane + 64*j, fp32 multiply-add
-// in k order.  GEMM only writes the products; the fused form sweeps each row
-// twice (maximum and sum first, then recompute and store).  Never inlined, so
-// its registers do not add to the MFMA paths.
+// The product alone of segments the 16-byte operand loads cannot serve (K % 8
+// != 0, odd segment starts) where they are few among aligned ones: one wavefront
+// walks rows [r_begin, r_end), lanes own columns c_begin + lane + 64*j, fp32
+// multiply-add in k order.  Never inlined, so its registers do not add to the
+// MFMA paths.
 template <int DT> __device__ __forceinline__ float generic_dot(const uint16_t *__restrict__ aseg,
                                                                const uint16_t *__restrict__ bseg, int r, int col,
                                                                int M, int N, int K, bool t1, bool t2) {
@@ -42,38 +41,15 @@ template <int DT> __device__ __forceinline__ void store_one(void *out, int64_t e
     else reinterpret_cast<uint16_t *>(out)[e] = Elem<DT>::from_float(v);
 }
 
-template <int DT, bool FUSED>
+template <int DT>
 __device__ __attribute__((noinline)) void generic_rows(const uint16_t *aseg, const uint16_t *bseg, void *out,
                                                        int64_t o, int M, int N, int K, int r_begin, int r_end,
-                                                       int c_begin, int c_end, float scale, int flags) {
+                                                       int c_begin, int c_end, int flags) {
     const int lane = lane_id();
-    const bool t1 = flags & kFlagTranspose1, t2 = flags & kFlagTranspose2, f32out = flags & kFlagOutF32;
-    for (int r = r_begin; r < r_end; ++r) {
-        const int64_t e0 = o + (int64_t)r * N;
-        if (!FUSED) {
-            for (int col = c_begin + lane; col < c_end; col += 64)
-                store_one<DT>(out, e0 + col, generic_dot<DT>(aseg, bseg, r, col, M, N, K, t1, t2), false);
-        } else {
-            float c = scale * kLog2e;
-            const float sgn = c < 0.f ? -1.f : 1.f;
-            c *= sgn;
-            float mx = -INFINITY;
-            for (int col = lane; col < N; col += 64)
-                mx = fmaxf(mx, sgn * generic_dot<DT>(aseg, bseg, r, col, M, N, K, t1, t2));
-            mx = wave_max(mx);
-            const float bias = -((mx == -INFINITY) ? 0.f : mx) * c;
-            float sum = 0.f;
-            for (int col = lane; col < N; col += 64)
-                sum += __builtin_amdgcn_exp2f(fmaf(sgn * generic_dot<DT>(aseg, bseg, r, col, M, N, K, t1, t2), c, bias));
-            sum = wave_sum(sum);
-            const float inv = 1.f / sum;
-            for (int col = lane; col < N; col += 64)
-                store_one<DT>(out, e0 + col,
-                              __builtin_amdgcn_exp2f(
-                                  fmaf(sgn * generic_dot<DT>(aseg, bseg, r, col, M, N, K, t1, t2), c, bias)) * inv,
-                              f32out);
-        }
-    }
+    const bool t1 = flags & kFlagTranspose1, t2 = flags & kFlagTranspose2;
+    for (int r = r_begin; r < r_end; ++r)
+        for (int col = c_begin + lane; col < c_end; col += 64)
+            store_one<DT>(out, o + (int64_t)r * N + col, generic_dot<DT>(aseg, bseg, r, col, M, N, K, t1, t2), false);
 }
 
 // ------------------------------------------------------------ local softmax
@@ -190,11 +166,11 @@ __device__ __forceinline__ void store_rows(const f32x4 (&acc)[kMaxTiles], int nt
 }
 
 
-template <int DT, bool FUSED>
+template <int DT>
 __device__ __forceinline__ void generic_seg_rows(const Seg &s, const RunArgs &a, int r_begin, int r_end,
                                                  int c_begin, int c_end) {
-    generic_rows<DT, FUSED>((const uint16_t *)a.A + s.a, (const uint16_t *)a.B + s.b, a.out, s.o, s.M, s.N, s.K,
-                            r_begin, min(r_end, s.M), c_begin, min(c_end, s.N), a.scale, a.flags);
+    generic_rows<DT>((const uint16_t *)a.A + s.a, (const uint16_t *)a.B + s.b, a.out, s.o, s.M, s.N, s.K, r_begin,
+                     min(r_end, s.M), c_begin, min(c_end, s.N), a.flags);
 }
 
 // ---------------------------------------------------------------- pack item
