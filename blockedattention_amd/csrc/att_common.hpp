@@ -1,5 +1,5 @@
 // What the one-pass attention (attention.hip) and its backward (attention_backward.hip) share: counted LDS operand
-// reads, element-wise operand loads, the rows of the per-query arrays.
+// reads, the rows of the per-query arrays.
 #pragma once
 #include <type_traits>
 #include <utility>
@@ -29,23 +29,6 @@ template <int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
 }
 __device__ __forceinline__ uint32_t lds_offset(const void *p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
-}
-
-// Eight consecutive elements k0 .. k0+7 of a row of K elements, zeros at and past K, for rows whose
-// length is not a multiple of 8 (pieces straddle nothing, but the row may end inside one): element by
-// element, one load in flight, few registers -- the slow path must not set the register count of the
-// kernel.  Each step shifts the 128-bit value down by one element and puts the new one on top.
-__device__ __forceinline__ u32x4 load8_slow(const uint16_t *row, int k0, int K) {
-    uint32_t r0 = 0, r1 = 0, r2 = 0, r3 = 0;
-#pragma nounroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t x = row[min(k0 + i, K - 1)];
-        r0 = (r0 >> 16) | (r1 << 16);
-        r1 = (r1 >> 16) | (r2 << 16);
-        r2 = (r2 >> 16) | (r3 << 16);
-        r3 = (r3 >> 16) | ((k0 + i < K ? x : 0u) << 16);
-    }
-    return u32x4{r0, r1, r2, r3};
 }
 
 // a * b + c for a, b below 2^24: one instruction

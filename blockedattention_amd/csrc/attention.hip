@@ -45,8 +45,9 @@ constexpr int kAttPitchV = kAttKeys * 2 + 32;
 constexpr int att_ring(int nk, int qt) { return qt == 1 && nk <= 2 ? 3 : 6; }
 
 // NK = 32-wide k steps (head dimension padded to 32 * NK).  VEC: the segment's K is a multiple of 8, its
-// rows come as 16-byte loads; otherwise element by element.  The two are separate instances of the whole
-// body so that the slow loads do not sit inside the fast path's loops.
+// rows come as 16-byte loads that need no clearing; otherwise through RowPieces (element by element before: 256 x 8
+// pairs of 32 .. 128 rows, K = 61: 103 -> 48 us; 16 x 8 pairs of 512 .. 2048, K = 101: 764 -> 279 us).  The two are
+// separate instances of the whole body so that the clearing does not sit inside the fast path's loops.
 template <int DT, int NK, int QT, bool VEC, bool LSE>
 __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbuf, float *lse_rows, const SegRec &rec, int64_t h,
                                                int zblock, unsigned char *sK, unsigned char *sV) {
@@ -93,11 +94,12 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
     // out of range and stays there (its advance is multiplied by zero).
     const __amdgpu_buffer_rsrc_t resK = __builtin_amdgcn_make_buffer_rsrc((void *)ks, 0, VEC ? N * K * 2 : 0, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t resV = __builtin_amdgcn_make_buffer_rsrc((void *)vs, 0, VEC ? N * K * 2 : 0, kRsrcFlags);
-    constexpr uint32_t kNever = 0xfffffff0u;
+    // Other rows: 16-byte pieces at any alignment, cleared past the row's end on the way into LDS.
+    const RowPieces<false> pq(qs, M, K), pk(ks, N, K), pv(vs, N, K);
     const uint32_t row_bytes = 2u * (uint32_t)K;      // all advances below are under 2^24 (K <= 128)
     const uint32_t k_live = 8 * k_piece < K ? 1u : 0u, v_live = 8 * v_piece < K ? 1u : 0u;
-    const uint32_t k_byte0 = k_live ? (uint32_t)k_row * row_bytes + 16u * (uint32_t)k_piece : kNever;
-    const uint32_t v_byte0 = v_live ? (uint32_t)(4 * v_kg) * row_bytes + 16u * (uint32_t)v_piece : kNever;
+    const uint32_t k_byte0 = k_live ? (uint32_t)k_row * row_bytes + 16u * (uint32_t)k_piece : kNowhere;
+    const uint32_t v_byte0 = v_live ? (uint32_t)(4 * v_kg) * row_bytes + 16u * (uint32_t)v_piece : kNowhere;
 
     // operand reads: lane (j, rg) reads 16 bytes of key row 16 t + j at k = 32 s + 8 rg, of value row (output
     // column) 16 t + j at the lane group's eight keys of half cc
@@ -120,7 +122,7 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                     qf[q][s] = *reinterpret_cast<const u32x4_unaligned *>(qrow + min(32 * s + 8 * rg, K - 8));
             } else {
 #pragma unroll
-                for (int s = 0; s < NK; ++s) qf[q][s] = load8_slow(qrow, 32 * s + 8 * rg, K);
+                for (int s = 0; s < NK; ++s) qf[q][s] = pq.get(min(r0 + kAttRows * q + j, M - 1), 4 * s + rg);
             }
 #pragma unroll
             for (int s = 0; s < NK; ++s) {
@@ -159,22 +161,26 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
             } else {
 #pragma unroll
                 for (int step = 0; step < kSteps; ++step)
-                    kw[step] = load8_slow(ks + (int64_t)min(kb + step * kRowsStep + k_row, N - 1) * K, 8 * k_piece, K);
+                    kw[step] = pk.load(pk.offset(kb + step * kRowsStep + k_row, k_piece));
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    vw[i] = load8_slow(vs + (int64_t)min(kb + 4 * v_kg + i, N - 1) * K, 8 * v_piece, K);
-                // zeros past the head dimension and past the last key (values: their probabilities are zeros
-                // too, but 0 * stale bits could be NaN)
+                for (int i = 0; i < 4; ++i) vw[i] = pv.load(pv.offset(kb + 4 * v_kg + i, v_piece));
+            }
+        };
+        // what the loads of block kb brought -> pieces with zeros past the head dimension and past the last key
+        // (values: their probabilities are zeros too, but 0 * stale bits could be NaN)
+        auto finish = [&](int kb) {
+            if constexpr (!VEC) {
 #pragma unroll
                 for (int step = 0; step < kSteps; ++step)
-                    kw[step] = (kb + step * kRowsStep + k_row < N && 8 * k_piece < K) ? kw[step] : zero4;
+                    kw[step] = pk.finish(kw[step], pk.offset(kb + step * kRowsStep + k_row, k_piece), k_piece);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) vw[i] = (kb + 4 * v_kg + i < N && 8 * v_piece < K) ? vw[i] : zero4;
+                for (int i = 0; i < 4; ++i) vw[i] = pv.finish(vw[i], pv.offset(kb + 4 * v_kg + i, v_piece), v_piece);
             }
         };
         if (N > 0) fetch(0);
 
         for (int kb = 0; kb < N; kb += kAttKeys) {
+            finish(kb);
             __syncthreads();                           // the previous block (or round) is consumed
             // ---- keys: sK[key][k], one 16-byte piece per thread and step, pieces of a row on neighbouring lanes
             if (kLpr == kPieces || k_piece < kPieces) {
