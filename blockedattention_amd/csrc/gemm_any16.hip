@@ -404,17 +404,24 @@ __device__ __forceinline__ void any16_ring_round(__amdgpu_buffer_rsrc_t resX, __
 }
 
 // RT = 16-row tiles per wavefront (the workgroup's step covers 64 RT rows), CG = groups of 64 columns per step.
-// The loads of a step are issued two steps ahead into registers, the chunks alternate between two LDS buffers:
-// one barrier per step, and two steps' worth of loads in flight per workgroup while it computes.  The kernel is
+// 128 x 128: the loads of a step are issued two steps ahead into registers, the chunks alternate between two LDS
+// buffers: one barrier per step, and two steps' worth of loads in flight per workgroup while it computes.  The kernel is
 // bound by operand traffic out of L2 (a 64 x 64 step fetches 16 KiB for 32 matrix instructions), which the
 // 128 x 128 step halves per result.
-template <int DT, int RT, int CG, bool T1, bool T2>
+// 64 x 64 with few steps is bound by the life of a workgroup: what counts is how many are resident.  One step
+// ahead and ONE buffer (BUFS = 1, two barriers a step) take 64 registers and 20 KiB, eight workgroups to a compute unit
+// instead of four.  Both backward products of 256 x 8 pairs of 32 .. 128 rows, K = 64: 39.9 -> 31.3 us (five resident: 36.5, six:
+// 32.3); 300 x 4 pairs of 5 .. 200, K 20 .. 100: the product with both operands as they lie 29.7 -> 28.6, the one with a
+// k-major operand 29.7 -> 28.1 us.  (Lines that end behind a segment loaded as its last 32 bytes and shifted, as in
+// RowPieces, instead of element by element: slower, 34.0, 34.1 and 32.8 us.)  See any_one_buffer for longer streams of steps.
+template <int DT, int RT, int CG, int BUFS, bool T1, bool T2>
 __device__ __forceinline__ void any16_stream_rounds(__amdgpu_buffer_rsrc_t resX, __amdgpu_buffer_rsrc_t resY, uint16_t *os, int M,
                                                     int N, int K, int first_round, int round_step, int rounds,
                                                     unsigned char *any_lds) {
     constexpr int kRows = kAnyTile * RT, kCols = kAnyTile * CG;
     constexpr int kPitchXT = AnyBuf<kRows>::pitch_t, kPitchYT = AnyBuf<kCols>::pitch_t;
     constexpr int kBufBytes = AnyBuf<kRows>::bytes + AnyBuf<kCols>::bytes;
+    constexpr int kBufs = BUFS;
     const int tid = threadIdx.x;
     const int wave = uniform(tid >> 6);
     const int lane = lane_id(), n = lane & 15, q = lane >> 4;
@@ -471,9 +478,9 @@ __device__ __forceinline__ void any16_stream_rounds(__amdgpu_buffer_rsrc_t resX,
     };
     const int ncb = (N + kCols - 1) / kCols;
     const int steps = ncb * nkc;                     // (column block, chunk) pairs of one round, chunk fastest
-    // With at most two chunks of k (K <= 128) the X chunks of a round stay in LDS, one per buffer, and are fetched
+    // With no more chunks of k than buffers the X chunks of a round stay in LDS, one per buffer, and are fetched
     // once instead of once per column block; only Y streams.
-    const bool x_once = nkc <= 2;
+    const bool x_once = nkc <= kBufs;
     clear();
     // The workgroup's rounds (first_round, first_round + round_step, ... below `rounds`) are ONE stream of steps: the
     // loads of a round's first chunks are issued during the last steps of the round before, so only the first round
@@ -506,15 +513,16 @@ __device__ __forceinline__ void any16_stream_rounds(__amdgpu_buffer_rsrc_t resX,
     };
     Stage sa, sb;
     if (total > 0) { fetch(sa, f_round, f_cb, f_kc); advance(); }
-    if (total > 1) { fetch(sb, f_round, f_cb, f_kc); advance(); }
+    if (kBufs == 2 && total > 1) { fetch(sb, f_round, f_cb, f_kc); advance(); }
     int c_round = first_round, cb = 0, kc = 0;            // the chunk being computed
     auto do_step = [&](int gs, Stage &st) __attribute__((always_inline)) {
         const int step = cb * nkc + kc;                   // position inside the round: decides the buffers
         const int r0 = c_round * kRows;
         // a new round's X chunks go where the last one's lie: wait until every wavefront has read those
-        if (step == 0 && gs > 0) lds_barrier();
-        unsigned char *buf = any_lds + (step & 1) * kBufBytes;
-        unsigned char *xbuf = any_lds + (x_once ? kc : step & 1) * kBufBytes;
+        // (with one buffer: and the last step's chunks)
+        if ((kBufs == 1 || step == 0) && gs > 0) lds_barrier();
+        unsigned char *buf = any_lds + (kBufs == 1 ? 0 : step & 1) * kBufBytes;
+        unsigned char *xbuf = any_lds + (kBufs == 1 ? 0 : x_once ? kc : step & 1) * kBufBytes;
         if (!x_once || cb == 0) {
 #pragma unroll
             for (int i = 0; i < RT; ++i) {
@@ -530,8 +538,8 @@ __device__ __forceinline__ void any16_stream_rounds(__amdgpu_buffer_rsrc_t resX,
             put_chunk16<true, 4 * CG, kPitchYT>(l, t2, N, K, cb * kCols, kc * kAnyTile, buf + AnyBuf<kRows>::bytes,
                                                 tid + kAnyThreads * i);
         }
-        if (gs + 2 < total) { fetch(st, f_round, f_cb, f_kc); advance(); }   // in flight under two steps of matrix instructions
-        // every wavefront has written its part of this chunk, and is done reading the chunk before last,
+        if (gs + kBufs < total) { fetch(st, f_round, f_cb, f_kc); advance(); }   // in flight under the matrix instructions
+        // every wavefront has written its part of this chunk and (two buffers) is done reading the chunk before last,
         // whose buffer the NEXT step's writes go to
         lds_barrier();
         // the B operands are read two tiles ahead of the matrix instructions that use them (an LDS round trip
@@ -570,9 +578,9 @@ __device__ __forceinline__ void any16_stream_rounds(__amdgpu_buffer_rsrc_t resX,
             if (++cb == ncb) { cb = 0; c_round += round_step; }
         }
     };
-    for (int gs = 0; gs < total; gs += 2) {
+    for (int gs = 0; gs < total; gs += kBufs) {
         do_step(gs, sa);
-        if (gs + 1 < total) do_step(gs + 1, sb);
+        if (kBufs == 2 && gs + 1 < total) do_step(gs + 1, sb);
     }
     if (nkc == 0)                                                  // K = 0: the result is zeros
         for (int round = first_round; round < rounds; round += round_step)
@@ -584,7 +592,7 @@ __device__ __forceinline__ void any16_stream_rounds(__amdgpu_buffer_rsrc_t resX,
 // per segment: either round wants all 256 registers, and neither as a function called from the other's kernel nor
 // inlined beside it did they keep out of each other's way (spills in the streaming loop, saves around every call).
 // block_x: the workgroup's index in the flat grid of a launch with the totals on the host (ride_slots = 1).
-template <int DT, int RT, int CG, bool T1, bool T2, bool RING>
+template <int DT, int RT, int CG, int BUFS, bool T1, bool T2, bool RING>
 __device__ __forceinline__ void any16_workgroup(const RunArgs &a, unsigned block_x, unsigned char *any_lds) {
     static_assert(!RING || (RT == 2 && CG == 2), "the ring belongs to the 128 x 128 build");
     constexpr int kRows = kAnyTile * RT, kCols = kAnyTile * CG;
@@ -647,46 +655,56 @@ __device__ __forceinline__ void any16_workgroup(const RunArgs &a, unsigned block
             if (round + round_step < rounds) lds_barrier();        // the next round's X chunks go where the rings are
         }
     } else {
-        any16_stream_rounds<DT, RT, CG, T1, T2>(resX, resY, os, M, N, K, first_round, round_step, rounds, any_lds);
+        any16_stream_rounds<DT, RT, CG, BUFS, T1, T2>(resX, resY, os, M, N, K, first_round, round_step, rounds, any_lds);
     }
 }
 
-template <int DT, int RT, int CG, bool T1, bool T2, bool RING>
-__global__ __launch_bounds__(kAnyThreads, RT * CG >= 4 ? 2 : 4) void gemm_any16_kernel(RunArgs a) {
+template <int DT, int RT, int CG, int BUFS, bool T1, bool T2, bool RING>
+__global__ __launch_bounds__(kAnyThreads, RT * CG >= 4 ? 2 : BUFS == 1 ? 8 : 4) void gemm_any16_kernel(RunArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char any_lds[];
-    any16_workgroup<DT, RT, CG, T1, T2, RING>(a, blockIdx.x, any_lds);
+    any16_workgroup<DT, RT, CG, BUFS, T1, T2, RING>(a, blockIdx.x, any_lds);
 }
 
 // Two products in one launch (64 x 64 build, totals on the host): the first `split` workgroups are those of a launch
 // over `a`, the rest those of a launch over `b`.  For the two products of the backward pass of a batch of short
 // segments, dA = dS B (second operand k-major) and dB = dS^T A (both k-major): each alone is a few rounds of
 // workgroups that live for one or two steps, and two launches pay the ramps at both ends twice.
-template <int DT>
-__global__ __launch_bounds__(kAnyThreads, 4) void gemm_any16_two_kernel(RunArgs a, RunArgs b, unsigned split) {
+template <int DT, int BUFS>
+__global__ __launch_bounds__(kAnyThreads, BUFS == 1 ? 8 : 4) void gemm_any16_two_kernel(RunArgs a, RunArgs b, unsigned split) {
     extern __shared__ __attribute__((aligned(16))) unsigned char any_lds[];
-    if (blockIdx.x < split) any16_workgroup<DT, 1, 1, false, true, false>(a, blockIdx.x, any_lds);
-    else any16_workgroup<DT, 1, 1, true, true, false>(b, blockIdx.x - split, any_lds);
+    if (blockIdx.x < split) any16_workgroup<DT, 1, 1, BUFS, false, true, false>(a, blockIdx.x, any_lds);
+    else any16_workgroup<DT, 1, 1, BUFS, true, true, false>(b, blockIdx.x - split, any_lds);
 }
 
-template <int DT, int RT, int CG, bool T1, bool T2, bool RING>
+template <int DT, int RT, int CG, int BUFS, bool T1, bool T2, bool RING>
 static void launch_any_build(const RunArgs &run, dim3 grid, hipStream_t stream) {
-    constexpr int kLds = 2 * (AnyBuf<kAnyTile * RT>::bytes + AnyBuf<kAnyTile * CG>::bytes);
+    constexpr int kLds = BUFS * (AnyBuf<kAnyTile * RT>::bytes + AnyBuf<kAnyTile * CG>::bytes);
     if constexpr (kLds > 65536) {
         static const bool attr_set = [] {
-            return hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_any16_kernel<DT, RT, CG, T1, T2, RING>),
+            return hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_any16_kernel<DT, RT, CG, BUFS, T1, T2, RING>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLds) == hipSuccess;
         }();
         (void)attr_set;
     }
-    hipLaunchKernelGGL((gemm_any16_kernel<DT, RT, CG, T1, T2, RING>), grid, dim3(kAnyThreads), kLds, stream, run);
+    hipLaunchKernelGGL((gemm_any16_kernel<DT, RT, CG, BUFS, T1, T2, RING>), grid, dim3(kAnyThreads), kLds, stream, run);
 }
-template <int DT, int RT, int CG, bool RING = false>
+template <int DT, int RT, int CG, int BUFS, bool RING = false>
 static void launch_any(const RunArgs &run, dim3 grid, hipStream_t stream) {
     const bool t1 = run.flags & kFlagTranspose1, t2 = run.flags & kFlagTranspose2;
-    if (t1 && t2) launch_any_build<DT, RT, CG, true, true, RING>(run, grid, stream);
-    else if (t1) launch_any_build<DT, RT, CG, true, false, RING>(run, grid, stream);
-    else if (t2) launch_any_build<DT, RT, CG, false, true, RING>(run, grid, stream);
-    else launch_any_build<DT, RT, CG, false, false, RING>(run, grid, stream);
+    if (t1 && t2) launch_any_build<DT, RT, CG, BUFS, true, true, RING>(run, grid, stream);
+    else if (t1) launch_any_build<DT, RT, CG, BUFS, true, false, RING>(run, grid, stream);
+    else if (t2) launch_any_build<DT, RT, CG, BUFS, false, true, RING>(run, grid, stream);
+    else launch_any_build<DT, RT, CG, BUFS, false, false, RING>(run, grid, stream);
+}
+
+// The 64 x 64 build: one buffer where the steps of a mean row's round (blocks of 64 columns times chunks of 64 k) are at
+// most four.  Longer streams of steps keep two buffers, for the second step in flight and the X chunks that stay.
+// One / two buffers: 256 x 8 pairs of 32 .. 128 rows, K = 61 (2 steps) 34.4 / 39.4 us with the softmax behind it; 1024 x 4 power-law
+// pairs, K = 128 (4 steps), forward and backward 238 / 251; 128 x 8 pairs of 64 .. 250, K = 101 (6 steps) 73 / 69.
+static bool any_one_buffer(const ba_plan_info *info) {
+    if (!info || info->total_rows <= 0) return false;
+    auto blocks = [&](int64_t area) { return (area / info->total_rows + kAnyTile - 1) / kAnyTile; };
+    return blocks(info->Dout) * blocks(info->Dm1) <= 4;
 }
 
 int launch_gemm_any16(int dtype, const RunArgs &args, int64_t nseg, const ba_plan_info *info, hipStream_t stream) {
@@ -722,18 +740,21 @@ int launch_gemm_any16(int dtype, const RunArgs &args, int64_t nseg, const ba_pla
     static const bool ring_env = [] { const char *e = getenv("BLOCKEDATTN_ANY_RING"); return !e || atoi(e) != 0; }();
     bool stream_too = true;
     if (big && info && ring_env && info->min_K <= 2 * kAnyTile && info->max_N >= 2 * kAnyRingChunk) {
-        if (dtype == BA_F16) launch_any<0, 2, 2, true>(run, grid, stream);
-        else launch_any<1, 2, 2, true>(run, grid, stream);
+        if (dtype == BA_F16) launch_any<0, 2, 2, 2, true>(run, grid, stream);
+        else launch_any<1, 2, 2, 2, true>(run, grid, stream);
         run.flags |= kFlagRingToo | kFlagQuiet;
         stream_too = info->min_N < 2 * kAnyRingChunk || info->max_K > 2 * kAnyTile;
     }
     if (stream_too) {
+        const bool one = any_one_buffer(info);
         if (dtype == BA_F16) {
-            if (big) launch_any<0, 2, 2>(run, grid, stream);
-            else launch_any<0, 1, 1>(run, grid, stream);
+            if (big) launch_any<0, 2, 2, 2>(run, grid, stream);
+            else if (one) launch_any<0, 1, 1, 1>(run, grid, stream);
+            else launch_any<0, 1, 1, 2>(run, grid, stream);
         } else {
-            if (big) launch_any<1, 2, 2>(run, grid, stream);
-            else launch_any<1, 1, 1>(run, grid, stream);
+            if (big) launch_any<1, 2, 2, 2>(run, grid, stream);
+            else if (one) launch_any<1, 1, 1, 1>(run, grid, stream);
+            else launch_any<1, 1, 1, 2>(run, grid, stream);
         }
     }
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
@@ -760,13 +781,18 @@ int launch_gemm_any16_two(int dtype, const RunArgs &a, const ba_plan_info *info_
     ra.ride_slots = rb.ride_slots = 1;
     ra.nseg = (int)info_a->nseg;
     rb.nseg = (int)info_b->nseg;
-    constexpr int kLds = 2 * (AnyBuf<kAnyTile>::bytes + AnyBuf<kAnyTile>::bytes);
-    if (dtype == BA_F16)
-        hipLaunchKernelGGL((gemm_any16_two_kernel<0>), dim3((unsigned)(grid_a + grid_b)), dim3(kAnyThreads), kLds, stream, ra, rb,
-                           (unsigned)grid_a);
-    else
-        hipLaunchKernelGGL((gemm_any16_two_kernel<1>), dim3((unsigned)(grid_a + grid_b)), dim3(kAnyThreads), kLds, stream, ra, rb,
-                           (unsigned)grid_a);
+    auto launch = [&](auto kernel, int bufs) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(grid_a + grid_b)), dim3(kAnyThreads), bufs * 2 * AnyBuf<kAnyTile>::bytes, stream,
+                           ra, rb, (unsigned)grid_a);
+    };
+    const bool one = any_one_buffer(info_a) && any_one_buffer(info_b);
+    if (dtype == BA_F16) {
+        if (one) launch(gemm_any16_two_kernel<0, 1>, 1);
+        else launch(gemm_any16_two_kernel<0, 2>, 2);
+    } else {
+        if (one) launch(gemm_any16_two_kernel<1, 1>, 1);
+        else launch(gemm_any16_two_kernel<1, 2>, 2);
+    }
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
 }
 
