@@ -21,6 +21,14 @@ template <int OFF> __device__ __forceinline__ void lds_read128(u32x4 &dst, uint3
 template <int N> __device__ __forceinline__ void lds_wait(u32x4 &x) {
     asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(x) : "n"(N) : "memory");
 }
+// The same for the transposing read: four elements of one column from each of two groups of rows NEXT bytes apart.
+template <int OFF, int NEXT> __device__ __forceinline__ void lds_read_tr(u32x2 &lo, u32x2 &hi, uint32_t addr) {
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(lo) : "v"(addr), "n"(OFF) : "memory");
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(hi) : "v"(addr), "n"(OFF + NEXT) : "memory");
+}
+template <int N> __device__ __forceinline__ void lds_wait_tr(u32x2 &lo, u32x2 &hi) {
+    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(lo), "+v"(hi) : "n"(N) : "memory");
+}
 template <typename F, int... I> __device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
     (f(std::integral_constant<int, I>{}), ...);
 }

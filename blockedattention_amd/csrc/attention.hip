@@ -8,8 +8,8 @@
 // both with the per-head stride Dm2), O_g is M x K at off1 of a [H, Dm1] buffer.  K <= 128.
 //
 // Workgroup = 4 wavefronts = 64 queries of one segment and head; the keys go by in blocks of 64.
-// Per block the workgroup stages K_g's rows (as they lie, zero padded to a multiple of 32 in k) and
-// V_g's rows TRANSPOSED (one LDS row per output column, keys along the row) in LDS.  A wavefront owns
+// Per block the workgroup stages K_g's and V_g's rows as they lie, zero padded to a multiple of 32
+// columns, in LDS; the second product reads V through the transposing LDS read.  A wavefront owns
 // 16 queries:
 //   S^T block  = K_blk Q^T   (matrix instructions, A operand = key rows from LDS, B operand = the
 //                wavefront's query rows, held in registers for the whole pass); the lane
@@ -17,10 +17,14 @@
 //   online softmax: reference value m (a lazily raised row maximum) and row sum l per query (per lane;
 //                the four lanes of a query exchange the block maximum), accumulators rescaled by
 //                2^((m_old - m_new) c) when m is raised;
-//   O^T       += V_blk^T P^T (A operand = transposed value rows from LDS, B operand = the lane's own
+//   O^T       += V_blk^T P^T (A operand = columns of the value rows, gathered from LDS four keys at a
+//                time by ds_read_b64_tr_b16, B operand = the lane's own
 //                probabilities rounded to the 16-bit type: the k index of the instruction runs over
 //                keys in the order the score registers hold them, so P never moves between lanes).
 // The query index is lane%16 in scores and outputs alike, so m, l and the rescaling are per lane.
+// Value rows were transposed on the way into LDS before (32 v_perm and eight 8-byte writes a thread and block, two-way
+// conflicts): 512 pairs of 16 .. 256 rows and columns, K 32 .. 128, 23.2 -> 22.2 us; 16 x 16 pairs of 1024 .. 4096,
+// K = 128, 1084 -> 1069 us; 1024 x 4 power-law pairs with the backward 293 -> 284 us.
 #include <stdlib.h>
 
 #include <algorithm>
@@ -33,12 +37,10 @@ constexpr int kAttThreads = 256;
 constexpr int kAttWaves = kAttThreads / 64;
 constexpr int kAttRows = 16 * kAttWaves;              // queries per workgroup round
 static_assert(kAttRows == kAttBlockRows, "the plan's row-block prefixes count blocks of kAttRows and 2 kAttRows");
-// LDS row pitches.  A 16-byte operand read of a wavefront is served 32 lanes at a time, 512 bytes wide (measured:
-// lane * 16 and 288-byte rows run at 4.75 cycles per wavefront read, 272- and 144-byte rows at 8): the lanes
-// (j, rg) and (j, rg + 1) of sixteen rows j must land in 32 different 16-byte slots modulo 512 bytes, which a
-// pitch of 16 * (2 * odd) bytes does.  Keys: 64 NK + 32 bytes; transposed values (64 keys a row): 160 bytes.  The
-// staging writes take what is left (two-way conflicts on a quarter as many instructions).
-constexpr int kAttPitchV = kAttKeys * 2 + 32;
+// LDS row pitch, keys and values alike: 64 NK + 32 bytes.  A 16-byte operand read of a wavefront is served 32 lanes at
+// a time, 512 bytes wide (measured: lane * 16 and 288-byte rows run at 4.75 cycles per wavefront read, 272- and
+// 144-byte rows at 8): the lanes (j, rg) and (j, rg + 1) of sixteen rows j must land in 32 different 16-byte slots
+// modulo 512 bytes, which a pitch of 16 * (2 * odd) bytes does; the transposing reads meet no conflict there either.
 // LDS operand reads in flight per wavefront: six, or three in the builds for short segments and head dimensions
 // up to 64, which then fit 128 registers and run four wavefronts per SIMD (the launch is bound by the life of a
 // workgroup there: 256 segments of 32..128 rows, 31.3 -> 29.0 us)
@@ -76,19 +78,11 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
     const uint32_t keep = c_signed == 0.f ? 0u : 0xffffffffu;
     const u32x4 zero4 = u32x4{0u, 0u, 0u, 0u};
 
-    // Staging, per thread: kSteps 16-byte pieces of the key rows (kLpr neighbouring lanes share a row; step s
-    // takes rows s * kRowsStep ..) and 4 keys x 8 columns of values (key group tid % 16, piece tid / 16; a load
-    // instruction of a wavefront then covers 64 contiguous bytes of sixteen rows, a write 128 of one).  Element
-    // offsets inside a segment fit 32 bits (checked by the kernel).
-    constexpr int kLpr = NK == 3 ? 16 : kPieces;      // lanes per key row (a power of two; 12 pieces: 4 lanes idle)
+    // Staging, per thread: kSteps 16-byte pieces of the key rows and of the value rows (kLpr neighbouring lanes share
+    // a row; step s takes rows s * kRowsStep ..).  Element offsets inside a segment fit 32 bits (checked by the kernel).
+    constexpr int kLpr = NK == 3 ? 16 : kPieces;      // lanes per row (a power of two; 12 pieces: 4 lanes idle)
     constexpr int kSteps = kLpr / 4, kRowsStep = kAttThreads / kLpr;
     const int k_row = tid / kLpr, k_piece = tid % kLpr;
-    const int v_kg = tid & 15, v_piece = tid >> 4;    // sixteen lanes = the sixteen key groups of one piece
-    const bool v_thread = v_piece < kPieces;
-    // Keys along an LDS row of transposed values stand in the order the probabilities have in a lane's registers:
-    // the eight keys 32 cc + 16 h + 4 rg + e (h < 2, e < 4) of lane group rg are 16 contiguous bytes, one operand
-    // read.  The thread's four keys 4 v_kg .. + 3 (v_kg = 8 cc + 4 h + rg) go to the 8-byte slot 8 cc + 2 rg + h.
-    const int v_slot = (v_kg & 8) + 2 * (v_kg & 3) + ((v_kg >> 2) & 1);
     // VEC: the loads go through buffer descriptors that span exactly the segment's keys and values, so a row
     // past the last key reads as zeros with no code; a piece past the head dimension has an offset that is
     // out of range and stays there (its advance is multiplied by zero).
@@ -97,14 +91,13 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
     // Other rows: 16-byte pieces at any alignment, cleared past the row's end on the way into LDS.
     const RowPieces<false> pq(qs, M, K), pk(ks, N, K), pv(vs, N, K);
     const uint32_t row_bytes = 2u * (uint32_t)K;      // all advances below are under 2^24 (K <= 128)
-    const uint32_t k_live = 8 * k_piece < K ? 1u : 0u, v_live = 8 * v_piece < K ? 1u : 0u;
+    const uint32_t k_live = 8 * k_piece < K ? 1u : 0u;
     const uint32_t k_byte0 = k_live ? (uint32_t)k_row * row_bytes + 16u * (uint32_t)k_piece : kNowhere;
-    const uint32_t v_byte0 = v_live ? (uint32_t)(4 * v_kg) * row_bytes + 16u * (uint32_t)v_piece : kNowhere;
 
-    // operand reads: lane (j, rg) reads 16 bytes of key row 16 t + j at k = 32 s + 8 rg, of value row (output
-    // column) 16 t + j at the lane group's eight keys of half cc
+    // operand reads: lane (j, rg) reads 16 bytes of key row 16 t + j at k = 32 s + 8 rg; of the values it addresses four
+    // columns of key 4 rg + j / 4 and receives column j of the lane group's four keys
     const uint32_t k_addr = lds_offset(sK) + (uint32_t)(j * kPitchK + rg * 16);
-    const uint32_t v_addr = lds_offset(sV) + (uint32_t)(j * kAttPitchV + rg * 16);
+    const uint32_t v_addr = lds_offset(sV) + (uint32_t)((4 * rg + (j >> 2)) * kPitchK + (j & 3) * 8);
 
     constexpr int kRoundRows = kAttRows * QT;           // queries per workgroup round
     for (int round = zblock; (int64_t)round * kRoundRows < M; round += a.ride_slots ? (1 << 24) : a.tile_zdim) {
@@ -141,29 +134,27 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
         }
 
         // The loads run one block ahead of the arithmetic: the loads of block kb + 64 are issued before the
-        // matrix work on block kb and land in registers (kw: this thread's pieces of the key rows, vw: its
-        // 4 keys x 8 columns of values) while that work runs.  All loads of a block sit in one branch-free
+        // matrix work on block kb and land in registers (kw, vw: this thread's pieces of the key and value
+        // rows) while that work runs.  All loads of a block sit in one branch-free
         // sequence (index clamped, value selected afterwards): loads behind a branch wait one by one.
-        u32x4 kw[kSteps], vw[4];
-        uint32_t k_byte = k_byte0, v_byte = v_byte0;
+        u32x4 kw[kSteps], vw[kSteps];
+        uint32_t k_byte = k_byte0;
         auto fetch = [&](int kb) {                     // called for kb = 0, 64, 128, .. in turn
             if constexpr (VEC) {
 #pragma unroll
-                for (int step = 0; step < kSteps; ++step)
-                    kw[step] = __builtin_amdgcn_raw_buffer_load_b128(
-                        resK, mad24(k_live, (uint32_t)(step * kRowsStep) * row_bytes, k_byte), 0, 0);
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    vw[i] = __builtin_amdgcn_raw_buffer_load_b128(
-                        resV, mad24(v_live, (uint32_t)i * row_bytes, v_byte), 0, 0);
+                for (int step = 0; step < kSteps; ++step) {
+                    const uint32_t off = mad24(k_live, (uint32_t)(step * kRowsStep) * row_bytes, k_byte);
+                    kw[step] = __builtin_amdgcn_raw_buffer_load_b128(resK, off, 0, 0);
+                    vw[step] = __builtin_amdgcn_raw_buffer_load_b128(resV, off, 0, 0);
+                }
                 k_byte = mad24(k_live, (uint32_t)kAttKeys * row_bytes, k_byte);
-                v_byte = mad24(v_live, (uint32_t)kAttKeys * row_bytes, v_byte);
             } else {
 #pragma unroll
-                for (int step = 0; step < kSteps; ++step)
-                    kw[step] = pk.load(pk.offset(kb + step * kRowsStep + k_row, k_piece));
-#pragma unroll
-                for (int i = 0; i < 4; ++i) vw[i] = pv.load(pv.offset(kb + 4 * v_kg + i, v_piece));
+                for (int step = 0; step < kSteps; ++step) {
+                    const uint32_t off = pk.offset(kb + step * kRowsStep + k_row, k_piece);
+                    kw[step] = pk.load(off);
+                    vw[step] = pv.load(off);
+                }
             }
         };
         // what the loads of block kb brought -> pieces with zeros past the head dimension and past the last key
@@ -171,10 +162,11 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
         auto finish = [&](int kb) {
             if constexpr (!VEC) {
 #pragma unroll
-                for (int step = 0; step < kSteps; ++step)
-                    kw[step] = pk.finish(kw[step], pk.offset(kb + step * kRowsStep + k_row, k_piece), k_piece);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) vw[i] = pv.finish(vw[i], pv.offset(kb + 4 * v_kg + i, v_piece), v_piece);
+                for (int step = 0; step < kSteps; ++step) {
+                    const uint32_t off = pk.offset(kb + step * kRowsStep + k_row, k_piece);
+                    kw[step] = pk.finish(kw[step], off, k_piece);
+                    vw[step] = pv.finish(vw[step], off, k_piece);
+                }
             }
         };
         if (N > 0) fetch(0);
@@ -182,23 +174,13 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
         for (int kb = 0; kb < N; kb += kAttKeys) {
             finish(kb);
             __syncthreads();                           // the previous block (or round) is consumed
-            // ---- keys: sK[key][k], one 16-byte piece per thread and step, pieces of a row on neighbouring lanes
+            // ---- one 16-byte piece per thread, array and step, pieces of a row on neighbouring lanes
             if (kLpr == kPieces || k_piece < kPieces) {
 #pragma unroll
-                for (int step = 0; step < kSteps; ++step)
-                    *reinterpret_cast<u32x4 *>(sK + (step * kRowsStep + k_row) * kPitchK + k_piece * 16) = kw[step];
-            }
-            // ---- values, transposed: 8 runs of 4 keys, one per column of the thread's piece
-            if (v_thread) {
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {          // word w of the four rows = columns 2w and 2w + 1
-                    const uint32_t lo01 = __builtin_amdgcn_perm(vw[1][w], vw[0][w], 0x05040100u);
-                    const uint32_t lo23 = __builtin_amdgcn_perm(vw[3][w], vw[2][w], 0x05040100u);
-                    const uint32_t hi01 = __builtin_amdgcn_perm(vw[1][w], vw[0][w], 0x07060302u);
-                    const uint32_t hi23 = __builtin_amdgcn_perm(vw[3][w], vw[2][w], 0x07060302u);
-                    unsigned char *dst = sV + (8 * v_piece + 2 * w) * kAttPitchV + v_slot * 8;
-                    *reinterpret_cast<u32x2 *>(dst) = u32x2{lo01, lo23};
-                    *reinterpret_cast<u32x2 *>(dst + kAttPitchV) = u32x2{hi01, hi23};
+                for (int step = 0; step < kSteps; ++step) {
+                    const int at = (step * kRowsStep + k_row) * kPitchK + k_piece * 16;
+                    *reinterpret_cast<u32x4 *>(sK + at) = kw[step];
+                    *reinterpret_cast<u32x4 *>(sV + at) = vw[step];
                 }
             }
             __syncthreads();
@@ -291,19 +273,23 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                 // ---- O^T += V^T P^T; a value operand read serves every strip
                 {
                     constexpr int kReads = 2 * kOutTiles;  // read i: key half i / kOutTiles, output tile i % kOutTiles
+                    u32x2 lo[kAttRing], hi[kAttRing];      // keys 4 rg .. + 3 of the half's two key tiles
                     static_for<kAttRing>([&](auto ic) {
                         constexpr int I = decltype(ic)::value;
-                        if constexpr (I < kReads) lds_read128<16 * (I % kOutTiles) * kAttPitchV + 64 * (I / kOutTiles)>(ring[I], v_addr);
+                        if constexpr (I < kReads)
+                            lds_read_tr<32 * (I / kOutTiles) * kPitchK + 32 * (I % kOutTiles), 16 * kPitchK>(lo[I], hi[I], v_addr);
                     });
                     static_for<kReads>([&](auto ic) {
                         constexpr int I = decltype(ic)::value, R = I % kAttRing;
                         constexpr int kBehind = (I + kAttRing < kReads ? I + kAttRing : kReads) - (I + 1);
-                        lds_wait<kBehind>(ring[R]);
+                        lds_wait_tr<2 * kBehind>(lo[R], hi[R]);
+                        const u32x4 v = u32x4{lo[R][0], lo[R][1], hi[R][0], hi[R][1]};
     #pragma unroll
                         for (int q = 0; q < NQ; ++q)
-                            oacc[q][I % kOutTiles] = Elem<DT>::mfma(ring[R], pf[q][I / kOutTiles], oacc[q][I % kOutTiles]);
+                            oacc[q][I % kOutTiles] = Elem<DT>::mfma(v, pf[q][I / kOutTiles], oacc[q][I % kOutTiles]);
                         if constexpr (I + kAttRing < kReads)
-                            lds_read128<16 * ((I + kAttRing) % kOutTiles) * kAttPitchV + 64 * ((I + kAttRing) / kOutTiles)>(ring[R], v_addr);
+                            lds_read_tr<32 * ((I + kAttRing) / kOutTiles) * kPitchK + 32 * ((I + kAttRing) % kOutTiles), 16 * kPitchK>(
+                                lo[R], hi[R], v_addr);
                     });
                 }
             };
@@ -345,7 +331,7 @@ template <int DT, int NK, int QT, bool LSE>
 __global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void attention_kernel(RunArgs a, const void *Vbuf, float *lse) {
     constexpr int KP = 32 * NK;
     __shared__ __attribute__((aligned(16))) unsigned char sK[kAttKeys * (KP * 2 + 32)];
-    __shared__ __attribute__((aligned(16))) unsigned char sV[KP * kAttPitchV];
+    __shared__ __attribute__((aligned(16))) unsigned char sV[kAttKeys * (KP * 2 + 32)];
     // (the row blocks per head come with the header: one memory round trip less than the prefix's last entry)
     const int64_t per_head = QT == 2 ? ((ConstHdr)(uintptr_t)a.plan)->att_blocks128 : ((ConstHdr)(uintptr_t)a.plan)->att_blocks64;
     if (!header_ok(a)) { report_mismatch(a); return; }
