@@ -414,8 +414,10 @@ __device__ __forceinline__ void att_dkdv_body(const RunArgs &a, const AttBwdArgs
 
 constexpr int att_dkdv_lds(int nk, int pairs, int qb) { return 2 * (2 * qb * att_pitch(nk) + 8 * qb) + pairs * 64 * qb; }
 
+// The build for short segments is bound by the life of a workgroup: three wavefronts per SIMD, not the two that its 197
+// registers at a head dimension of 128 would leave (30 of them spilled), 1024 x 4 pairs of 2 .. 512 rows: 133 -> 110 us.
 template <int DT, int NK, int PAIRS, int QB>
-__global__ __launch_bounds__(128 * PAIRS, 2) void attention_dkdv_kernel(RunArgs a, AttBwdArgs w) {
+__global__ __launch_bounds__(128 * PAIRS, QB == 32 ? 3 : 2) void attention_dkdv_kernel(RunArgs a, AttBwdArgs w) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     static_assert(PAIRS == 2 || PAIRS == 4, "the plan's column-block prefixes count blocks of 64 and of 128");
     const ConstHdr hdr = (ConstHdr)(uintptr_t)a.plan;
@@ -467,7 +469,8 @@ int launch_attention_backward(int dtype, const RunArgs &args, const void *V, con
     // Segments of 256 rows and more on average: wavefronts of two query strips, and workgroups of 128 keys that stage 64
     // queries (16 x 16 pairs of 1024 .. 4096 rows: dK and dV 2.10 ms; 64 keys and 32 queries 2.78 ms, 128 keys and 32
     // queries 2.44 ms: every query block is staged once per workgroup).  Shorter ones: 64 keys and 32 queries, two to
-    // three times as many resident workgroups (1024 x 4 pairs of 2 .. 512 rows: 127 us; 64 queries 184 us, 128 keys 168 us).
+    // three times as many resident workgroups (1024 x 4 pairs of 2 .. 512 rows, at two wavefronts
+    // per SIMD: 127 us; 64 queries 184 us, 128 keys 168 us).
     const bool tall = info->total_rows >= 256 * std::max<int64_t>(info->nseg, 1);
     if (dtype == BA_F16)
         return tall ? launch_bwd_nk<0, 2, 4, 64>(nk, args, w, info, stream) : launch_bwd_nk<0, 1, 2, 32>(nk, args, w, info, stream);
