@@ -41,10 +41,11 @@ static_assert(kAttRows == kAttBlockRows, "the plan's row-block prefixes count bl
 // a time, 512 bytes wide (measured: lane * 16 and 288-byte rows run at 4.75 cycles per wavefront read, 272- and
 // 144-byte rows at 8): the lanes (j, rg) and (j, rg + 1) of sixteen rows j must land in 32 different 16-byte slots
 // modulo 512 bytes, which a pitch of 16 * (2 * odd) bytes does; the transposing reads meet no conflict there either.
-// LDS operand reads in flight per wavefront: six, or three in the builds for short segments and head dimensions
-// up to 64, which then fit 128 registers and run four wavefronts per SIMD (the launch is bound by the life of a
-// workgroup there: 256 segments of 32..128 rows, 31.3 -> 29.0 us)
-constexpr int att_ring(int nk, int qt) { return qt == 1 && nk <= 2 ? 3 : 6; }
+// LDS operand reads in flight per wavefront: six, or three in the builds for short segments, which are bound by the
+// life of a workgroup: head dimensions up to 64 then fit 128 registers and four wavefronts per SIMD (256 segments of
+// 32..128 rows, 31.3 -> 29.0 us), those up to 128 spill 7 registers instead of 17 at three wavefronts (512 pairs of
+// 16 .. 256 rows and columns, 22.2 -> 21.9 us)
+constexpr int att_ring(int nk, int qt) { return qt == 1 ? 3 : 6; }
 
 // NK = 32-wide k steps (head dimension padded to 32 * NK).  VEC: the segment's K is a multiple of 8, its
 // rows come as 16-byte loads that need no clearing; otherwise through RowPieces (element by element before: 256 x 8
