@@ -32,6 +32,25 @@ __device__ __forceinline__ int64_t readlane64(int64_t v, int l) {
 }
 __device__ __forceinline__ int64_t wave_total(int64_t v) { return readlane64(wave_inclusive_scan(v), 63); }
 
+// any_rows as a call: inlined, its descriptors and addresses cost the other bodies 30 more spilled scalars and every aligned
+// batch up to 0.3 us a launch (96 x 5 pairs of 4 .. 46 rows, inlined / called: 10.2 / 9.9 us; 152 x 5 of 6 .. 33: 12.1 / 11.9).
+// Unaligned ones pay for it: 26 pairs of 69 .. 226 rows, K 39 .. 79: 14.2 / 16.0 us (595 element by element).  Arguments of a
+// call lose their uniformity, hence uniform().
+typedef __attribute__((address_space(3))) unsigned char *AnyLds;
+template <int DT, bool F32OUT>
+__device__ __attribute__((noinline)) void any_rows_call(const uint16_t *A, const uint16_t *B, void *out, int64_t o, int M, int N,
+                                                        int K, float scale, AnyLds lds, int r0) {
+    RunArgs a{};
+    a.A = (const void *)uniform64((int64_t)A);
+    a.B = (const void *)uniform64((int64_t)B);
+    a.out = (void *)uniform64((int64_t)out);
+    a.scale = __builtin_bit_cast(float, uniform(__builtin_bit_cast(int, scale)));
+    Seg s{};
+    s.o = uniform64(o);
+    s.M = uniform(M); s.N = uniform(N); s.K = uniform(K);
+    any_rows<DT, F32OUT, kMaxTiles>(s, a, (unsigned char *)lds, uniform(r0));
+}
+
 template <int DT, bool F32OUT>
 __global__ __launch_bounds__(kSegThreads, 2) void onecall_kernel(RunArgs a, MetaArgs m) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -162,7 +181,8 @@ __global__ __launch_bounds__(kSegThreads, 2) void onecall_kernel(RunArgs a, Meta
     if (!(a.flags & kFlagMfmaOk) || !aligned) {
         s.kind = kSegSlow;
         for (int base = bz * kSegWaves * kStripRows; base < s.M; base += stride * kStripRows)
-            any_rows<DT, F32OUT, kMaxTiles>(s, a, lds, base + wave * kStripRows);
+            any_rows_call<DT, F32OUT>((const uint16_t *)a.A + s.a, (const uint16_t *)a.B + s.b, a.out, s.o, s.M, s.N, s.K, a.scale,
+                                      (AnyLds)lds, base + wave * kStripRows);
         return;
     }
     s.kind = s.N <= kWaveCols ? kSegStrip : s.N <= kSplitCols ? kSegSplit : kSegWide;
