@@ -9,7 +9,7 @@
 // which recomputes the scores.
 //
 // 256 x 8 pairs of 32 .. 128 rows and columns, K = 61: 4136 -> 36 us (K = 64 on the aligned path: 14.6); 128 x 4 pairs of
-// 64 .. 256, K = 101: 8667 -> 52 us; one launch, 128 x 4 pairs of 32 .. 128, K = 61: 1416 -> 20 us.  The loop was bound by
+// 64 .. 256, K = 101: 8667 -> 52 us; one launch (measured inlined there), 128 x 4 pairs of 32 .. 128, K = 61: 1416 -> 20 us.  The loop was bound by
 // 2-byte loads, one per multiply-add.  Now it is the life of a workgroup: load, barrier, matrix instructions, softmax,
 // stores one after the other, three or two workgroups to a compute unit by registers.  (128 and 168 registers, one
 // workgroup more, spill: 49 and 63 us.)
