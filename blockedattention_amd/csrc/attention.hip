@@ -345,7 +345,7 @@ __global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void at
     // not exist, except past the end of a share (the grid is sized from an upper bound of the item count).
     // Without it: pair = die + 8 (k mod pairs per die), row block k / pairs per die; a workgroup takes every
     // tile_zdim-th row block of its pair, and the workgroups that find no rows come last.
-    const unsigned id = blockIdx.x, die = id & 7u, kk = id >> 3;
+    const unsigned id = flat_block(), die = id & 7u, kk = id >> 3;
     int g, zblock;
     int64_t h;
     if (a.ride_slots) {
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void at
         const int64_t items = per_head * a.H, share = (items + 7) >> 3;
         const int64_t u = (int64_t)die * share + kk;
         // a grid too small for the plan's items: the host summary the launch was sized from is not this plan's
-        if (id == 0 && threadIdx.x == 0 && share * 8 > (int64_t)gridDim.x)
+        if (id == 0 && threadIdx.x == 0 && share * 8 > flat_blocks())
             atomicAdd(&reinterpret_cast<PlanHeader *>(a.plan)->run_errors, 1);
         if (kk >= share || u >= items) return;
         h = u / per_head;
@@ -364,6 +364,7 @@ __global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void at
         const unsigned pairs8 = (unsigned)a.tile_groups;
         const int64_t pair = (int64_t)die + 8 * (int64_t)(kk % pairs8);
         zblock = (int)(kk / pairs8);
+        if (zblock >= a.tile_zdim) return;             // (the last row of a flat grid)
         if (pair >= (int64_t)a.nseg * a.H) return;
         g = (int)(pair / a.H);
         h = pair % a.H;
@@ -435,13 +436,13 @@ int launch_attention(int dtype, const RunArgs &args, const void *V, float *lse, 
         const int64_t share = (items + 7) / 8;
         if (share * 8 > 0x7fffffff) return BA_ERR_UNSUPPORTED;
         run.ride_slots = 1;
-        grid = dim3((unsigned)(share * 8));
+        grid = flat_grid(share * 8);
     } else {
         const int64_t pairs8 = (nseg * args.H + 7) / 8;    // pairs per die, rounded up
         if (pairs8 * z * 8 > 0x7fffffff || pairs8 > 0x7fffffff) return BA_ERR_UNSUPPORTED;
         run.tile_zdim = (int)z;
         run.tile_groups = (int)pairs8;
-        grid = dim3((unsigned)(pairs8 * z * 8));
+        grid = flat_grid(pairs8 * z * 8);
     }
     if (dtype == BA_F16) { if (qt == 2) launch_build<0, 2>(nk, grid, stream, run, V, lse); else launch_build<0, 1>(nk, grid, stream, run, V, lse); }
     else { if (qt == 2) launch_build<1, 2>(nk, grid, stream, run, V, lse); else launch_build<1, 1>(nk, grid, stream, run, V, lse); }

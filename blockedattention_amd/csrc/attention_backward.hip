@@ -218,12 +218,12 @@ __device__ __forceinline__ void att_dq_body(const RunArgs &a, const AttBwdArgs &
 // per die (as in attention_kernel: the blocks of a pair read the same rows and run side by side on one die).
 // prefix: blocks of the segments before each segment; per_head: all of them.
 __device__ __forceinline__ bool att_item(const RunArgs &a, int which, int64_t per_head, int64_t &h, int &g, int &block) {
-    const unsigned id = blockIdx.x, die = id & 7u, kk = id >> 3;
+    const unsigned id = flat_block(), die = id & 7u, kk = id >> 3;
     const int32_t *pfx = plan_rowblocks(a.plan, a.nseg, which);
     const int64_t items = per_head * a.H, share = (items + 7) >> 3;
     const int64_t u = (int64_t)die * share + kk;
     // a grid too small for the plan's items: the summary the launch was sized from is not this plan's
-    if (id == 0 && threadIdx.x == 0 && share * 8 > (int64_t)gridDim.x)
+    if (id == 0 && threadIdx.x == 0 && share * 8 > flat_blocks())
         atomicAdd(&reinterpret_cast<PlanHeader *>(a.plan)->run_errors, 1);
     if (kk >= share || u >= items) return false;
     h = u / per_head;
@@ -445,9 +445,9 @@ static int launch_bwd(const RunArgs &args, const AttBwdArgs &w, const ba_plan_in
     const int64_t blocks = PAIRS == 4 ? ((int64_t)info->att_cols64 + info->nseg) / 2 : info->att_cols64;
     const int64_t cols = (blocks * args.H + 7) / 8 * 8;
     if (rows > 0x7fffffff || cols > 0x7fffffff) return BA_ERR_UNSUPPORTED;
-    if (rows > 0) hipLaunchKernelGGL((attention_dq_kernel<DT, NK, QT>), dim3((unsigned)rows), dim3(256), 0, stream, args, w);
+    if (rows > 0) hipLaunchKernelGGL((attention_dq_kernel<DT, NK, QT>), flat_grid(rows), dim3(256), 0, stream, args, w);
     if (cols > 0)
-        hipLaunchKernelGGL((attention_dkdv_kernel<DT, NK, PAIRS, QB>), dim3((unsigned)cols), dim3(128 * PAIRS), kLds, stream, args, w);
+        hipLaunchKernelGGL((attention_dkdv_kernel<DT, NK, PAIRS, QB>), flat_grid(cols), dim3(128 * PAIRS), kLds, stream, args, w);
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
 }
 

@@ -219,6 +219,10 @@ __device__ __forceinline__ Seg load_listed(const PlanRO &pv, int slot, int64_t h
     return s;
 }
 
+// Index of a workgroup in a flat grid and how many there are (see flat_grid()).
+__device__ __forceinline__ unsigned flat_block() { return blockIdx.y * kFlatRow + blockIdx.x; }
+__device__ __forceinline__ int64_t flat_blocks() { return (int64_t)gridDim.x * gridDim.y; }
+
 // The header fields every kernel checks, fetched as one batch of scalar loads
 // (no branch between them).  The segment count comes with the launch, so the
 // addresses of the plan's arrays do not wait for the header either.

@@ -108,6 +108,17 @@ int launch_attention(int dtype, const RunArgs &args, const void *V, float *lse, 
 int launch_attention_backward(int dtype, const RunArgs &args, const void *V, const void *O, const void *dO, const float *lse,
                               float *delta, void *dQ, void *dK, void *dV, const ba_plan_info *info, hipStream_t stream);
 
+// Flat grids.  A launch counts the threads of a grid dimension in 32 bits and cuts what does not fit without an error
+// (2^24 workgroups of 256 threads run as none at all): flat_grid() deals n workgroups to two dimensions, whole rows of
+// kFlatRow (a multiple of the eight dies, so the round-robin over them goes on); flat_block() is the index of a
+// workgroup, flat_blocks() how many there are, n or a little more.  Launches with another grid to fall back on take
+// that from kMaxFlatGroups on.
+constexpr unsigned kFlatRow = 1u << 20;
+constexpr int64_t kMaxFlatGroups = (int64_t(1) << 24) - 1024;
+inline dim3 flat_grid(int64_t n) {
+    return n <= (int64_t)kFlatRow ? dim3((unsigned)n) : dim3(kFlatRow, (unsigned)((n + kFlatRow - 1) / kFlatRow));
+}
+
 // Number of compute units of the current device (cached per device).
 int device_cu_count();
 

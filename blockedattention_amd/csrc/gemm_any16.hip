@@ -725,7 +725,7 @@ int launch_gemm_any16(int dtype, const RunArgs &args, int64_t nseg, const ba_pla
     // (one workgroup per existing round, not per (segment, head): a 64 x 64 x 64 step takes a workgroup about a
     // microsecond whatever is in flight, so the rounds of a segment are worth more side by side than one after the
     // other -- 512 segments of 16..256 rows: 20.8 us against 35 / 26 / 22 us with one / two / three workgroups per pair)
-    if (info && items < (int64_t(1) << 31) - 1024) {
+    if (info && items < kMaxFlatGroups) {
         if (items == 0) return BA_OK;                   // no segment has rows
         run.ride_slots = 1;
         const int64_t unit = (int64_t)kDies * kAnyDieBlock;           // whole blocks for every die
@@ -776,7 +776,7 @@ int launch_gemm_any16_two(int dtype, const RunArgs &a, const ba_plan_info *info_
     const int64_t items_a = (int64_t)info_a->att_blocks64 * a.H, items_b = (int64_t)info_b->att_blocks64 * b.H;
     if (items_a <= 0 || items_b <= 0) return BA_ERR_UNSUPPORTED;
     const int64_t grid_a = (items_a + unit - 1) / unit * unit, grid_b = (items_b + unit - 1) / unit * unit;
-    if (grid_a + grid_b >= (int64_t(1) << 31) - 1024) return BA_ERR_UNSUPPORTED;
+    if (grid_a + grid_b >= kMaxFlatGroups) return BA_ERR_UNSUPPORTED;
     RunArgs ra = a, rb = b;
     ra.ride_slots = rb.ride_slots = 1;
     ra.nseg = (int)info_a->nseg;

@@ -220,7 +220,7 @@ __device__ __forceinline__ void f32_round(const RunArgs &a, const SegRec &rec, i
 }
 
 // a.ride_slots = 1 (launches that know the batch's totals): one workgroup per existing (head, segment, row block) item,
-// head-major, cut into eight contiguous shares, one per die (as in attention_kernel).  Else grid (pair, z).
+// head-major, cut into eight contiguous shares, one per die (as in attention_kernel).  Else grid (pair, z), the pairs flat too.
 template <bool T1, bool T2>
 __global__ __launch_bounds__(kF32Threads, 4) void gemm_f32_kernel(RunArgs a) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -229,11 +229,11 @@ __global__ __launch_bounds__(kF32Threads, 4) void gemm_f32_kernel(RunArgs a) {
     int g, round, step;
     int64_t h;
     if (a.ride_slots) {
-        const unsigned id = blockIdx.x, die = id & 7u, kk = id >> 3;
+        const unsigned id = flat_block(), die = id & 7u, kk = id >> 3;
         const int32_t *pfx = plan_rowblocks(a.plan, a.nseg, 0);
         const int64_t items = per_head * a.H, share = (items + 7) >> 3;
         const int64_t u = (int64_t)die * share + kk;
-        if (id == 0 && threadIdx.x == 0 && share * 8 > (int64_t)gridDim.x)    // sized from another plan's summary
+        if (id == 0 && threadIdx.x == 0 && share * 8 > flat_blocks())    // sized from another plan's summary
             atomicAdd(&reinterpret_cast<PlanHeader *>(a.plan)->run_errors, 1);
         if (kk >= share || u >= items) return;
         h = u / per_head;
@@ -242,10 +242,11 @@ __global__ __launch_bounds__(kF32Threads, 4) void gemm_f32_kernel(RunArgs a) {
         round = item - ((ConstI32)(uintptr_t)pfx)[g];
         step = 1 << 24;
     } else {
-        g = (int)(blockIdx.x / (unsigned)a.H);
-        h = blockIdx.x % (unsigned)a.H;
-        round = blockIdx.y;
-        step = gridDim.y;
+        g = (int)(flat_block() / (unsigned)a.H);
+        h = flat_block() % (unsigned)a.H;
+        if (g >= a.nseg) return;                       // (the last row of a flat grid)
+        round = blockIdx.z;
+        step = gridDim.z;
     }
     const SegRec rec = load_rec(plan_ro(a.plan, a.nseg).recs, g);
     if (rec.N < 1) return;
@@ -276,10 +277,11 @@ int launch_gemm_f32(const RunArgs &args, int64_t nseg, const ba_plan_info *info,
         if (items <= 0) return BA_OK;
         if (items > 0x7ffffff0) return BA_ERR_UNSUPPORTED;
         run.ride_slots = 1;
-        grid = dim3((unsigned)((items + 7) / 8 * 8));
+        grid = flat_grid((items + 7) / 8 * 8);
     } else {
         if (nseg * args.H > 0x7fffffff) return BA_ERR_UNSUPPORTED;
-        grid = dim3((unsigned)(nseg * args.H), 4);
+        grid = flat_grid(nseg * args.H);
+        grid.z = 4;
     }
     switch (run.flags & (kFlagTranspose1 | kFlagTranspose2)) {
         case 0: return launch_f32<false, false>(run, grid, stream);

@@ -620,7 +620,7 @@ static int launch_softmax_t(const SoftmaxArgs &args, int64_t nseg, const ba_plan
         static const int both_env = [] { const char *e = getenv("BLOCKEDATTN_SOFTMAX_BOTH"); return e ? atoi(e) : -1; }();
         const int64_t rows_blocks = n_rows * args.H * z_rows, runs_blocks = nseg * args.H * z_runs;
         const bool both = info && rows_work && n_rows < nseg && info->max_N > 128 &&
-                          rows_blocks + runs_blocks < (int64_t(1) << 31) &&
+                          rows_blocks + runs_blocks < kMaxFlatGroups &&
                           (both_env >= 0 ? both_env != 0 : rows_blocks <= (int64_t)cus * 64);
         if (both) {
             const BothGrid bg{(unsigned)rows_blocks, (unsigned)z_rows, (unsigned)nseg, (unsigned)z_runs};
