@@ -29,10 +29,14 @@ constexpr int kF32Cols = 128;                        // columns of a step
 constexpr int kF32Pitch = kF32Tile * 4 + 32;         // bytes of an LDS row: 16 * (2 * odd), reads of 16 rows meet no conflict
 static_assert(kF32Rows == kAttBlockRows, "the plan's row-block prefix counts blocks of 64 rows");
 
-// Four consecutive words from byte `off` of a line on, through a descriptor that spans the segment (a load that would
-// cross its end is dropped whole).  EDGE: the piece may reach past the segment's end; the load is then moved back to its
-// last 16 bytes and shifted by finish().  A segment of fewer than four elements is read word by word.
+// Four consecutive words from byte `off` of a line on, through a descriptor that spans the segment; kNowhere, for pieces
+// that do not exist, reads as zeros.  EDGE: the piece may reach past the segment's end; the load is then moved back to its
+// last 16 bytes and shifted by finish().  A segment of fewer than four elements is read word by word (the compiler may
+// merge the four reads), the words past its end as zeros: offsets past it are held at 16, so that none of the four wraps.
 template <bool EDGE> struct Words4 {
+    // past every segment (areas are below 2^30 elements, multiples of four without EDGE); a 16-byte load at the one
+    // without EDGE ends where 32-bit offsets do
+    static constexpr uint32_t kNowhere = EDGE ? 0xfffffffcu : 0xfffffff0u;
     __amdgpu_buffer_rsrc_t res;
     uint32_t bytes;
     __device__ __forceinline__ Words4(const float *seg, int elements)
@@ -43,6 +47,7 @@ template <bool EDGE> struct Words4 {
         if (!EDGE || bytes >= 16)
             return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(res, EDGE ? min(off, bytes - 16) : off, 0, 0));
         f32x4 x;
+        off = min(off, 16u);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             x[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(res, off + 4 * i, 0, 0));
@@ -63,7 +68,6 @@ template <bool EDGE> struct Words4 {
         return x;
     }
 };
-constexpr uint32_t kF32Nowhere = 0xfffffffcu;       // no segment reaches it (areas are below 2^30 elements)
 
 // A 16 G (rows or columns of the result) x 64 (k) chunk of an operand on its way into LDS as [row][k], in pieces of four
 // words: kPieces a thread.  MAJOR: stored k-major (K lines of `rows`); EDGE as above.  `rows` x K operand, chunk at
@@ -84,7 +88,7 @@ template <bool MAJOR, bool EDGE, int G, bool DEALT> struct F32Chunk {
     static __device__ __forceinline__ uint32_t offset(int rows, int K, int r0, int k0, int tid, int i) {
         const int l = (MAJOR ? k0 : r0) + line(tid, i), pos = MAJOR ? r0 + col(tid, i) : k0 + 4 * (tid & 15);
         const int lines = MAJOR ? K : rows, len = MAJOR ? rows : K;
-        return l < lines && pos < len ? 4u * (uint32_t)(l * len + pos) : kF32Nowhere;
+        return l < lines && pos < len ? 4u * (uint32_t)(l * len + pos) : Words4<EDGE>::kNowhere;
     }
     __device__ __forceinline__ void fetch(const Words4<EDGE> &src, int rows, int K, int r0, int k0, int tid) {
 #pragma unroll
@@ -131,7 +135,7 @@ __device__ __forceinline__ void f32_block(const Words4<EDGE || T1> &pa, const Wo
     f32x4 av[4];                                       // !T1: four words of k = 16 b + 4 q of the lane's row
     auto aoff = [&](int k0, int b) {
         const int row = r0 + arow, k = k0 + 16 * b + 4 * q;
-        return row < M && k < K ? 4u * (uint32_t)(row * K + k) : kF32Nowhere;
+        return row < M && k < K ? 4u * (uint32_t)(row * K + k) : Words4<EDGE>::kNowhere;
     };
     auto fetch = [&](int k0) {
         cb.fetch(pb, N, K, c0, k0, tid);

@@ -43,3 +43,43 @@ def test_empty_dimensions_and_no_summary(dev):
     for summary in (True, False):
         run(dev, [4, 0, 9, 300, 5], [6, 5, 0, 70, 7], [16, 8, 24, 0, 3], 2, False, False, seed=2, summary=summary)
         run(dev, [700, 65], [20, 130], [17, 64], 3, True, True, seed=3, summary=summary)
+
+
+@pytest.mark.parametrize("t1,t2", [(False, False), (True, False), (False, True), (True, True)])
+def test_segments_below_four_elements(dev, t1, t2):
+    # every shape whose operands have one to three elements, each between larger neighbours: a piece of such an operand
+    # that does not exist (k past K above all, where both operands would have to be wrong) adds nothing
+    shapes = [(m, n, k) for m in (1, 2, 3) for n in (1, 2, 3) for k in (1, 2, 3)]
+    M, N, K = (np.array([x for s in shapes for x in (s[i], 20)]) for i in range(3))
+    run(dev, M, N, K, 2, t1, t2, seed=5)
+    run(dev, [2], [3], [1], 1, t1, t2, seed=6)
+
+
+@pytest.mark.parametrize("t1,t2", [(True, False), (False, True)])
+def test_infinity_stays_in_its_row(dev, t1, t2):
+    # K = 1, the k-major operand [inf, 2] (and [inf, 2, 3]): the rows or columns without the infinity are finite
+    for n in (2, 3):
+        x = torch.tensor([[float("inf"), 2.0, 3.0][:n]], device=dev)
+        y = torch.tensor([[1.0, -1.0]], device=dev)
+        M, N = (n, 2) if t1 else (2, n)
+        out = torch.full((1, 2 * n), float("nan"), device=dev)
+        print(f"fp32 infinity case {n} {t1} {t2}", flush=True)
+        capi.varlen_gemm(make_plan(dev, [M], [N], [1]), x if t1 else y, y if t1 else x, out, 1, M, N, M * N, t1, t2)
+        want = torch.outer(x[0], y[0]) if t1 else torch.outer(y[0], x[0])
+        assert torch.equal(out.view(M, N), want)
+
+
+def test_gradients_of_segments_below_four_elements(dev):
+    import blockedAttention
+    shapes = [(1, 2, 2), (1, 3, 3), (1, 2, 3), (5, 6, 7), (1, 3, 2), (2, 1, 1)]
+    M, N, K = (np.array([s[i] for s in shapes]) for i in range(3))
+    g = torch.Generator().manual_seed(9)
+    a, b, go = (torch.randn((2, int(x.sum())), generator=g) for x in (M * K, N * K, M * N))
+    ad, bd = a.to(dev).requires_grad_(), b.to(dev).requires_grad_()
+    blockedAttention.blockGEMM(ad, bd, None, None, None, *(torch.from_numpy(x).to(dev) for x in (M, N, K))).backward(go.to(dev))
+    o1, o2, oo = (np.concatenate([[0], np.cumsum(x)]) for x in (M * K, N * K, M * N))
+    for s, (m, n, k) in enumerate(shapes):
+        A, B, G = (t[:, o[s]:o[s + 1]].double().reshape(2, r, -1) for t, o, r in ((a, o1, m), (b, o2, n), (go, oo, m)))
+        for got, x, y, red in ((ad.grad[:, o1[s]:o1[s + 1]], G, B, n), (bd.grad[:, o2[s]:o2[s + 1]], G.transpose(1, 2), A, m)):
+            err = (got.cpu().double().reshape(2, x.shape[1], -1) - x @ y).abs()
+            assert (err <= (red + 2) * 2.0 ** -24 * (x.abs() @ y.abs())).all()
