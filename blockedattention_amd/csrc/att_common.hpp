@@ -44,7 +44,8 @@ __device__ __forceinline__ uint32_t mad24(uint32_t a, uint32_t b, uint32_t c) { 
 
 // Where the rows of a segment lie in a per-query array of the backward pass: ceil(Dm1 / min_K) floats per head, row r
 // of segment g at ceil(off1 / min_K) + r.  Segments do not overlap there because none has fewer than min_K elements a
-// row (segments without keys, which min_K does not count, have no entry).
+// row (segments without keys, which min_K does not count, have no entry).  The arrays are sized from the host's summary:
+// a kernel gets its min_K with the launch and touches them only if the plan has the same.
 __host__ __device__ inline int64_t att_rows_per_head(int min_K, int64_t Dm1) {
     const int64_t k = min_K > 1 ? min_K : 1;
     return (Dm1 + k - 1) / k;

@@ -329,13 +329,14 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
 // LSE: the build for training, which also writes the rows' sums (as a run-time choice it cost the plain one 2 % on 512
 // segments of 16 .. 256 rows and columns: 23.1 -> 23.6 us).
 template <int DT, int NK, int QT, bool LSE>
-__global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void attention_kernel(RunArgs a, const void *Vbuf, float *lse) {
+__global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void attention_kernel(RunArgs a, const void *Vbuf, float *lse, int min_K) {
     constexpr int KP = 32 * NK;
     __shared__ __attribute__((aligned(16))) unsigned char sK[kAttKeys * (KP * 2 + 32)];
     __shared__ __attribute__((aligned(16))) unsigned char sV[kAttKeys * (KP * 2 + 32)];
     // (the row blocks per head come with the header: one memory round trip less than the prefix's last entry)
     const int64_t per_head = QT == 2 ? ((ConstHdr)(uintptr_t)a.plan)->att_blocks128 : ((ConstHdr)(uintptr_t)a.plan)->att_blocks64;
-    if (!header_ok(a)) { report_mismatch(a); return; }
+    // (lse is sized by the min_K of the host's summary)
+    if (!header_ok(a) || (LSE && ((ConstHdr)(uintptr_t)a.plan)->min_K != min_K)) { report_mismatch(a); return; }
     // Workgroup -> (segment, head, row block).  Consecutive workgroup ids go to the eight dies of the chip in
     // turn, and each die has its own L2: id = die + 8 k.  All row blocks of one (segment, head) pair read the
     // same keys and values, so they should run on ONE die at about the same time.
@@ -380,26 +381,26 @@ __global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void at
             atomicAdd(&reinterpret_cast<PlanHeader *>(a.plan)->run_errors, 1);
         return;
     }
-    float *lse_rows = LSE ? lse + att_row_base(((ConstHdr)(uintptr_t)a.plan)->min_K, a.Dm1, h, rec.off1) : nullptr;
+    float *lse_rows = LSE ? lse + att_row_base(min_K, a.Dm1, h, rec.off1) : nullptr;
     if ((K & 7) == 0) attention_body<DT, NK, QT, true, LSE>(a, Vbuf, lse_rows, rec, h, zblock, sK, sV);
     else attention_body<DT, NK, QT, false, LSE>(a, Vbuf, lse_rows, rec, h, zblock, sK, sV);
 }
 
 template <int DT, int QT, bool LSE>
-static void launch_nk(int nk, dim3 grid, hipStream_t stream, const RunArgs &args, const void *V, float *lse) {
+static void launch_nk(int nk, dim3 grid, hipStream_t stream, const RunArgs &args, const void *V, float *lse, int min_K) {
     // args.ride_slots = 1: work items from the plan's row-block prefix; else args.tile_zdim = row blocks per
     // (segment, head) pair, tile_groups = pairs per die
     switch (nk) {
-        case 1: hipLaunchKernelGGL((attention_kernel<DT, 1, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse); break;
-        case 2: hipLaunchKernelGGL((attention_kernel<DT, 2, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse); break;
-        case 3: hipLaunchKernelGGL((attention_kernel<DT, 3, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse); break;
-        default: hipLaunchKernelGGL((attention_kernel<DT, 4, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse); break;
+        case 1: hipLaunchKernelGGL((attention_kernel<DT, 1, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
+        case 2: hipLaunchKernelGGL((attention_kernel<DT, 2, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
+        case 3: hipLaunchKernelGGL((attention_kernel<DT, 3, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
+        default: hipLaunchKernelGGL((attention_kernel<DT, 4, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
     }
 }
 template <int DT, int QT>
-static void launch_build(int nk, dim3 grid, hipStream_t stream, const RunArgs &args, const void *V, float *lse) {
-    if (lse) launch_nk<DT, QT, true>(nk, grid, stream, args, V, lse);
-    else launch_nk<DT, QT, false>(nk, grid, stream, args, V, lse);
+static void launch_build(int nk, dim3 grid, hipStream_t stream, const RunArgs &args, const void *V, float *lse, int min_K) {
+    if (lse) launch_nk<DT, QT, true>(nk, grid, stream, args, V, lse, min_K);
+    else launch_nk<DT, QT, false>(nk, grid, stream, args, V, lse, min_K);
 }
 
 // Strips per wavefront: two where segments are tall (each operand read from LDS then feeds two matrix
@@ -426,6 +427,7 @@ int launch_attention(int dtype, const RunArgs &args, const void *V, float *lse, 
     if (info) z = std::min<int64_t>(z, (4 * info->total_rows / std::max<int64_t>(nseg, 1) + round_rows - 1) / round_rows);
     z = std::max<int64_t>(z, 1);
     if (nseg <= 0) return BA_OK;
+    const int min_K = info ? info->min_K : 0;
     RunArgs run = args;
     dim3 grid;
     if (info && info->total_rows >= 0) {
@@ -444,8 +446,8 @@ int launch_attention(int dtype, const RunArgs &args, const void *V, float *lse, 
         run.tile_groups = (int)pairs8;
         grid = flat_grid(pairs8 * z * 8);
     }
-    if (dtype == BA_F16) { if (qt == 2) launch_build<0, 2>(nk, grid, stream, run, V, lse); else launch_build<0, 1>(nk, grid, stream, run, V, lse); }
-    else { if (qt == 2) launch_build<1, 2>(nk, grid, stream, run, V, lse); else launch_build<1, 1>(nk, grid, stream, run, V, lse); }
+    if (dtype == BA_F16) { if (qt == 2) launch_build<0, 2>(nk, grid, stream, run, V, lse, min_K); else launch_build<0, 1>(nk, grid, stream, run, V, lse, min_K); }
+    else { if (qt == 2) launch_build<1, 2>(nk, grid, stream, run, V, lse, min_K); else launch_build<1, 1>(nk, grid, stream, run, V, lse, min_K); }
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
 }
 

@@ -65,6 +65,7 @@ struct AttBwdArgs {
     const float *lse;
     float *delta;
     void *dQ, *dK, *dV;
+    int min_K;                                         // of the summary that lse and delta were sized from
 };
 
 // The ROWS rows of an array staged per block: thread -> (row, piece), kSteps pieces an array.
@@ -245,14 +246,14 @@ __global__ __launch_bounds__(256, 2) void attention_dq_kernel(RunArgs a, AttBwdA
     __shared__ __attribute__((aligned(16))) unsigned char sV[kAttKeys * att_pitch(NK)];
     const ConstHdr hdr = (ConstHdr)(uintptr_t)a.plan;
     const int64_t per_head = QT == 2 ? hdr->att_blocks128 : hdr->att_blocks64;
-    const int min_K = hdr->min_K;
-    if (!header_ok(a)) { report_mismatch(a); return; }
+    const bool rows_ok = hdr->min_K == w.min_K;
+    if (!header_ok(a) || !rows_ok) { report_mismatch(a); return; }
     int64_t h;
     int g, block;
     if (!att_item(a, QT - 1, per_head, h, g, block)) return;
     const SegRec rec = load_rec(plan_ro(a.plan, a.nseg).recs, g);
     if (rec.M < 1 || rec.K < 1 || !att_fits(a, rec, 32 * NK, h, block)) return;
-    const int64_t row0 = att_row_base(min_K, a.Dm1, h, rec.off1);
+    const int64_t row0 = att_row_base(w.min_K, a.Dm1, h, rec.off1);
     if ((rec.K & 7) == 0) att_dq_body<DT, NK, QT, true>(a, w, rec, h, row0, block, sK, sV);
     else att_dq_body<DT, NK, QT, false>(a, w, rec, h, row0, block, sK, sV);
 }
@@ -422,14 +423,14 @@ __global__ __launch_bounds__(128 * PAIRS, QB == 32 ? 3 : 2) void attention_dkdv_
     static_assert(PAIRS == 2 || PAIRS == 4, "the plan's column-block prefixes count blocks of 64 and of 128");
     const ConstHdr hdr = (ConstHdr)(uintptr_t)a.plan;
     const int64_t per_head = PAIRS == 4 ? hdr->att_cols128 : hdr->att_cols64;
-    const int min_K = hdr->min_K;
-    if (!header_ok(a)) return;                         // reported by the dQ kernel
+    const bool rows_ok = hdr->min_K == w.min_K;
+    if (!header_ok(a) || !rows_ok) return;            // reported by the dQ kernel
     int64_t h;
     int g, block;
     if (!att_item(a, PAIRS == 4 ? 3 : 2, per_head, h, g, block)) return;
     const SegRec rec = load_rec(plan_ro(a.plan, a.nseg).recs, g);
     if (rec.N < 1 || rec.K < 1 || !att_fits(a, rec, 32 * NK, h, block)) return;
-    const int64_t row0 = att_row_base(min_K, a.Dm1, h, rec.off1);
+    const int64_t row0 = att_row_base(w.min_K, a.Dm1, h, rec.off1);
     if ((rec.K & 7) == 0) att_dkdv_body<DT, NK, PAIRS, QB, true>(a, w, rec, h, row0, block, lds);
     else att_dkdv_body<DT, NK, PAIRS, QB, false>(a, w, rec, h, row0, block, lds);
 }
@@ -464,7 +465,7 @@ static int launch_bwd_nk(int nk, const RunArgs &args, const AttBwdArgs &w, const
 int launch_attention_backward(int dtype, const RunArgs &args, const void *V, const void *O, const void *dO, const float *lse,
                               float *delta, void *dQ, void *dK, void *dV, const ba_plan_info *info, hipStream_t stream) {
     if (info->max_K > 128 || info->nseg <= 0) return info->nseg <= 0 ? BA_OK : BA_ERR_UNSUPPORTED;
-    const AttBwdArgs w{V, O, dO, lse, delta, dQ, dK, dV};
+    const AttBwdArgs w{V, O, dO, lse, delta, dQ, dK, dV, info->min_K};
     const int nk = std::max(1, (info->max_K + 31) / 32);
     // Segments of 256 rows and more on average: wavefronts of two query strips, and workgroups of 128 keys that stage 64
     // queries (16 x 16 pairs of 1024 .. 4096 rows: dK and dV 2.10 ms; 64 keys and 32 queries 2.78 ms, 128 keys and 32

@@ -101,7 +101,7 @@ int launch_softmax_backward(int dtype, void *plan, int64_t nseg, const void *y, 
 
 // Varlen attention O = softmax(scale Q K^T) V without the probabilities in memory (see attention.hip).
 // args.A = Q, args.B = K, args.out = O ([H, Dm1]); V has K's layout.
-// lse: nullptr, or per query the base-2 logarithm of its row's sum of exponentials (see att_rows_per_head()).
+// lse: nullptr, or per query the base-2 logarithm of its row's sum of exponentials (see att_rows_per_head(); with info).
 int launch_attention(int dtype, const RunArgs &args, const void *V, float *lse, int64_t nseg, const ba_plan_info *info,
                      hipStream_t stream);
 // Its backward (attention_backward.hip): dQ, dK, dV from dO; delta is scratch of lse's size.

@@ -354,7 +354,7 @@ __attribute__((visibility("default"))) int ba_varlen_attention_train(void *plan,
     if (!plan || nseg < 0 || nseg > (int64_t(1) << 30) || bad_sizes(H, Dm1, Dm2, Dout)) return BA_ERR_INVALID_ARG;
     if (dtype != BA_F16 && dtype != BA_BF16) return BA_ERR_UNSUPPORTED;
     if (H == 0 || Dm1 == 0 || nseg == 0) return BA_OK;
-    if (!out || !lse || !Q || (Dm2 > 0 && (!K || !V))) return BA_ERR_INVALID_ARG;
+    if (!info || !out || !lse || !Q || (Dm2 > 0 && (!K || !V))) return BA_ERR_INVALID_ARG;
     RunArgs args{plan, Q, K, out, H, Dm1, Dm2, Dout, scale, 0, 0, 0, (int)nseg};
     return launch_attention(dtype, args, V, lse, nseg, info, (hipStream_t)stream);
 }

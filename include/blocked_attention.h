@@ -260,8 +260,10 @@ int ba_varlen_attention(void *plan, const ba_plan_info *info, int64_t nseg, int 
  * of the reference's chain (csrc/sparseBlockedAttention.cpp:52-72, 95-114)
  * without its M x N arrays.  `lse` and the scratch array `delta` are fp32,
  * H * ba_attention_rows(info, Dm1) entries each (one a row when all K_g are
- * equal); entries of rows without keys are not touched.  `info` is required in
- * the backward.  Types, limits and error codes as for ba_varlen_attention.
+ * equal); entries of rows without keys are not touched.  `info` is required
+ * (BA_ERR_INVALID_ARG without): a plan that those sizes do not fit is reported
+ * in run_errors and nothing is written.  Types, limits and error codes as for
+ * ba_varlen_attention.
  */
 int64_t ba_attention_rows(const ba_plan_info *info, int64_t Dm1);
 int ba_varlen_attention_train(void *plan, const ba_plan_info *info, int64_t nseg, int dtype, const void *Q, const void *K,

@@ -149,3 +149,32 @@ def test_given_prefix_sums_with_gaps_and_partial_gradients(dev):
             ref = torch.softmax(0.2 * qq @ kk.t(), -1).t() @ gg
             got = vd.grad.reshape(4, -1)[h, b].float().cpu().reshape(ref.shape)
             assert (got - ref).abs().max() <= 1e-2 * ref.abs().max()
+
+
+def test_summary_of_another_plan_is_reported(dev):
+    # equal segment count and totals, other smallest K: the per-query arrays sized from the summary are too short for
+    # the plan (one block of rows each, K = 16 against 8), and nothing is written to them or behind them
+    M = N = np.array([8, 8, 8]); K, K2 = np.array([8, 64, 24]), np.array([16, 64, 16])
+    plan, other = make_plan(dev, M, N, K), make_plan(dev, M, N, K2)
+    d, do = int((M * K).sum()), int((M * N).sum())
+    q, k, v, go = (torch.randn((2, d), generator=torch.Generator().manual_seed(i)).half().to(dev) for i in range(4))
+    own, short = capi.attention_rows(plan, d), capi.attention_rows(other, d)
+    assert short < own
+    info, dims = plan.info, (2, d, d, do, 0.5)
+    out, lse, delta = torch.full_like(q, 7.0), torch.full((2, own), 7.0, device=dev), torch.full((2, own), 7.0, device=dev)
+    grads = [torch.full_like(q, 7.0) for _ in range(3)]
+    plan.info = other.info
+    capi.varlen_attention_train(plan, q, k, v, out, lse, *dims)
+    assert plan.read(raise_on_bad=False).run_errors == 1
+    plan.info = other.info
+    capi.varlen_attention_backward(plan, q, k, v, out, go, lse, delta, *grads, *dims)
+    assert plan.read(raise_on_bad=False).run_errors == 2
+    for t in (out, lse, delta, *grads):
+        assert bool((t == 7.0).all())
+    # without a summary the arrays have no size: refused
+    plan.info = None
+    with pytest.raises(capi.BlockedAttentionError):
+        capi.varlen_attention_train(plan, q, k, v, out, lse, *dims)
+    with pytest.raises(capi.BlockedAttentionError):
+        capi.varlen_attention_backward(plan, q, k, v, out, go, lse, delta, *grads, *dims)
+    plan.info = info
