@@ -341,13 +341,29 @@ Schedule &derived_schedule(const Schedule &s, std::shared_ptr<Schedule> Derived:
     return *p;
 }
 
-// A schedule that an autograd node keeps from its forward to its backward pass.
-struct KeptSchedule : torch::CustomClassHolder {
-    explicit KeptSchedule(const Schedule &schedule) : s(schedule) {}
-    const Schedule s;
-};
-const Schedule &kept_schedule(AutogradContext *ctx) {
-    return static_cast<const KeptSchedule *>(ctx->saved_data["schedule"].toCapsule().get())->s;
+// What an autograd node keeps of a schedule from its forward to its backward pass: two tensors, the plan and a copy of
+// its summary, saved like the operands (a capsule or raw bytes in the node's other data would shut it out of compiled
+// autograd, which hashes those).
+void keep_schedule(variable_list &saved, const Schedule &s) {
+    Tensor info = at::empty({(int64_t)sizeof(ba_plan_info)}, at::TensorOptions().dtype(at::kByte).device(at::kCPU));
+    memcpy(info.data_ptr(), &s.info, sizeof(ba_plan_info));
+    saved.push_back(s.plan);
+    saved.push_back(info);
+}
+// The schedule of saved[at] and saved[at + 1].  Saved-tensor hooks may have put them anywhere (a summary that comes back
+// on the GPU is copied once more); what is not a plan and its summary any longer is refused.
+Schedule kept_schedule(const variable_list &saved, size_t at, const Tensor &like) {
+    Schedule s;
+    s.plan = saved[at];
+    const Tensor info = saved[at + 1].to(at::kCPU);
+    TORCH_CHECK(info.scalar_type() == at::kByte && info.is_contiguous() && info.numel() == (int64_t)sizeof(ba_plan_info),
+                "backward: the saved summary of the plan came back as ", info.toString(), info.sizes());
+    memcpy(&s.info, info.data_ptr(), sizeof(ba_plan_info));
+    check_data(s.plan, "backward: the saved plan");
+    TORCH_CHECK(s.plan.scalar_type() == at::kByte && s.plan.device() == like.device() && s.info.nseg >= 0 &&
+                    s.plan.numel() == (int64_t)ba_plan_bytes(s.info.nseg) && ((uintptr_t)s.plan.data_ptr() & 15) == 0,
+                "backward: the saved plan came back as ", s.plan.toString(), s.plan.sizes());
+    return s;
 }
 
 class SparseBlockedGEMM : public torch::autograd::Function<SparseBlockedGEMM> {
@@ -358,8 +374,15 @@ public:
         check_data(mat1, "mat1"); check_data(mat2, "mat2");
         c10::hip::HIPGuardMasqueradingAsCUDA guard(mat1.device());
         Schedule s = schedule_gemm(mat1, a1, a2, aO, M, N, K, /*use_cache=*/true, train);
-        ctx->saved_data["schedule"] = c10::IValue::make_capsule(c10::make_intrusive<KeptSchedule>(s));
-        ctx->save_for_backward({mat1, mat2, s.accum1, s.accum2, s.accumOut, s.M, s.N, s.K});
+        variable_list keep{mat1, mat2, s.accum1, s.accum2, s.accumOut, s.M, s.N, s.K};
+        if (train) {
+            std::lock_guard<std::mutex> lock(s.derived->mu);
+            if (s.derived->grad1 && s.derived->grad2) {
+                keep_schedule(keep, *s.derived->grad1);
+                keep_schedule(keep, *s.derived->grad2);
+            }
+        }
+        ctx->save_for_backward(keep);
         ctx->saved_data["transpose1"] = t1;
         ctx->saved_data["transpose2"] = t2;
         return {gemm_launch(mat1, mat2, s, t1, t2)};
@@ -378,19 +401,25 @@ public:
         Tensor g1, g2;
         // dS and the saved operands are read as they lie: the products whose reduction runs over N or M take the
         // kernels for any layout and reduction length (two launches, like the reference)
-        const Schedule &fwd = kept_schedule(ctx);
-        Schedule &s1 = derived_schedule(fwd, &Derived::grad1, grad, aO, a2, a1, M, K, N);
-        Schedule &s2 = derived_schedule(fwd, &Derived::grad2, grad, aO, a1, a2, N, K, M);
+        Schedule s1, s2;
+        if (saved.size() > 8) {
+            s1 = kept_schedule(saved, 8, grad);
+            s2 = kept_schedule(saved, 10, grad);
+        } else {                                       // the forward's schedule was made by a call without gradients
+            const Schedule fwd = schedule_gemm(grad, a1, a2, aO, M, N, K);
+            s1 = derived_schedule(fwd, &Derived::grad1, grad, aO, a2, a1, M, K, N);
+            s2 = derived_schedule(fwd, &Derived::grad2, grad, aO, a1, a2, N, K, M);
+        }
+        const int64_t heads = leading(grad);
         // batches of short segments: both products as ONE launch where the library offers it (layouts of the
         // untransposed forward), else one call each
         bool done = false;
         if (!t1 && !t2 && grad.dim() >= 1 && grad.size(-1) == s1.info.Dm1 && mat2.size(-1) == s1.info.Dm2 &&
-            grad.size(-1) == s2.info.Dm1 && mat1.size(-1) == s2.info.Dm2 && leading(mat1) == leading(grad) &&
-            leading(mat2) == leading(grad) && (grad.scalar_type() == at::kHalf || grad.scalar_type() == at::kBFloat16)) {
-            const int64_t H = leading(grad);
-            g1 = at::empty({H, s1.info.Dout}, grad.options());
-            g2 = at::empty({H, s2.info.Dout}, grad.options());
-            const int st = ba_varlen_gemm_two(dtype_code(grad, "sparseBlockedGEMM backward"), H, s1.plan.data_ptr(), &s1.info,
+            grad.size(-1) == s2.info.Dm1 && mat1.size(-1) == s2.info.Dm2 && leading(mat1) == heads && leading(mat2) == heads &&
+            (grad.scalar_type() == at::kHalf || grad.scalar_type() == at::kBFloat16)) {
+            g1 = at::empty({heads, s1.info.Dout}, grad.options());
+            g2 = at::empty({heads, s2.info.Dout}, grad.options());
+            const int st = ba_varlen_gemm_two(dtype_code(grad, "sparseBlockedGEMM backward"), heads, s1.plan.data_ptr(), &s1.info,
                                               grad.data_ptr(), mat2.data_ptr(), g1.data_ptr(), s1.info.Dm1, s1.info.Dm2,
                                               s1.info.Dout, s2.plan.data_ptr(), &s2.info, grad.data_ptr(), mat1.data_ptr(),
                                               g2.data_ptr(), s2.info.Dm1, s2.info.Dm2, s2.info.Dout, current_stream(grad));
@@ -422,8 +451,10 @@ public:
         check_status(ba_blocked_softmax(s.plan.data_ptr(), &s.info, s.info.nseg, dt, src.data_ptr(), out.data_ptr(), H,
                                         s.info.Dout, (float)scale, current_stream(src)),
                      "ba_blocked_softmax");
-        ctx->saved_data["schedule"] = c10::IValue::make_capsule(c10::make_intrusive<KeptSchedule>(s));
-        ctx->save_for_backward({out, s.accumOut, s.M, s.N});
+        // (the metadata only so that a change of it between the passes is refused by its version counter)
+        variable_list keep{out, s.accumOut, s.M, s.N};
+        keep_schedule(keep, s);
+        ctx->save_for_backward(keep);
         ctx->saved_data["scale"] = scale;
         return {out};
     }
@@ -433,8 +464,8 @@ public:
         const Tensor grad = grads[0].contiguous();
         c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
         const Tensor y = saved[0].to(grad.scalar_type());
-        const Schedule &s = kept_schedule(ctx);
-        const int64_t H = leading(y);
+        const Schedule s = kept_schedule(saved, 4, grad);
+        const int64_t H = leading(grad);
         Tensor dx = at::empty_like(y);
         check_status(ba_blocked_softmax_backward(s.plan.data_ptr(), &s.info, s.info.nseg,
                                                  dtype_code(y, "softmax backward"),
@@ -532,8 +563,9 @@ public:
         Schedule s = attention_schedule(q, k, v, a1, a2, aO, M, N, K);
         Tensor lse;
         Tensor out = attention_launch(q, k, v, s, scale, &lse);
-        ctx->save_for_backward({q, k, v, out, lse, s.plan});
-        ctx->saved_data["info"] = std::string(reinterpret_cast<const char *>(&s.info), sizeof(s.info));
+        variable_list keep{q, k, v, out, lse};
+        keep_schedule(keep, s);
+        ctx->save_for_backward(keep);
         ctx->saved_data["scale"] = scale;
         ctx->saved_data["lists"] = M.has_value() && N.has_value() && K.has_value();
         return {out};
@@ -542,16 +574,17 @@ public:
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
         TORCH_CHECK(ctx->saved_data["lists"].toBool(), "blockFusedAttention: the backward pass needs MList, NList and KList");
         const auto saved = ctx->get_saved_variables();
-        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &plan = saved[5];
-        c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4];
         const Tensor grad = grads[0].to(q.scalar_type()).contiguous();
-        ba_plan_info info;
-        memcpy(&info, ctx->saved_data["info"].toStringRef().data(), sizeof(info));
+        c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
+        const Schedule s = kept_schedule(saved, 5, grad);
+        const ba_plan_info &info = s.info;
+        const int64_t H = leading(grad);
         Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), delta = at::empty_like(lse);
-        check_status(ba_varlen_attention_backward(plan.data_ptr(), &info, info.nseg, dtype_code(q, "attention backward"),
+        check_status(ba_varlen_attention_backward(s.plan.data_ptr(), &info, info.nseg, dtype_code(q, "attention backward"),
                                                   q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), grad.data_ptr(),
                                                   lse.data_ptr<float>(), delta.data_ptr<float>(), dq.data_ptr(),
-                                                  dk.data_ptr(), dv.data_ptr(), leading(q), info.Dm1, info.Dm2, info.Dout,
+                                                  dk.data_ptr(), dv.data_ptr(), H, info.Dm1, info.Dm2, info.Dout,
                                                   (float)ctx->saved_data["scale"].toDouble(), current_stream(q)),
                      "ba_varlen_attention_backward");
         return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};

@@ -1,0 +1,99 @@
+"""What the operators' autograd nodes keep between the passes: compiled autograd takes it, saved-tensor hooks may move it."""
+import pytest
+import torch
+
+import blockedAttention
+from blockedattention_amd import blockAttention
+
+pytestmark = pytest.mark.gpu
+
+M, N, K = [5, 70, 9], [7, 40, 4], [16, 8, 24]
+
+
+def meta(dev):
+    return [torch.tensor(x, device=dev) for x in (M, N, K)]
+
+
+def operands(dev, n, dtype=torch.float16):
+    g = torch.Generator().manual_seed(3)
+    sizes = [sum(m * k for m, k in zip(M, K)), sum(a * k for a, k in zip(N, K))]
+    return [torch.randn((2, sizes[min(i, 1)]), generator=g).to(dtype).to(dev).requires_grad_() for i in range(n)]
+
+
+def product(q, k, m):
+    return blockedAttention.blockGEMM(q, k, None, None, None, *m)
+
+
+def pair(q, k, m):
+    return blockedAttention.blockSoftmax(product(q, k, m), m[0], m[1], scale=0.3)
+
+
+def attention(q, k, v, m):
+    return blockedAttention.blockFusedAttention(q, k, v, *m, scale=0.3)
+
+
+OPS = {"product": (product, 2), "pair": (pair, 2), "attention": (attention, 3)}
+
+
+def gradients(dev, op, backward=torch.Tensor.backward, hooks=None, m=None):
+    f, n = OPS[op]
+    ts = operands(dev, n)
+    m = m or meta(dev)
+    if hooks is None:
+        out = f(*ts, m)
+    else:
+        with torch.autograd.graph.saved_tensors_hooks(*hooks):
+            out = f(*ts, m)
+    backward(out.float().pow(2).sum())
+    return [t.grad for t in ts]
+
+
+@pytest.mark.parametrize("op", list(OPS))
+def test_compiled_autograd(dev, op):
+    import torch._dynamo.compiled_autograd as compiled
+
+    def backward(loss):
+        with compiled._enable(torch.compile(backend="eager")):
+            loss.backward()
+
+    want = gradients(dev, op)
+    for _ in range(2):                                         # new metadata, then again
+        assert all(torch.equal(a, b) for a, b in zip(gradients(dev, op, backward), want))
+
+
+@pytest.mark.parametrize("op", list(OPS))
+def test_hooks_that_move_and_copy(dev, op):
+    want = gradients(dev, op)
+    for hooks in ((lambda t: t.cpu(), lambda t: t.to(dev)),     # everything comes back on the GPU, the summary too
+                  (lambda t: t.clone(), lambda t: t.clone()),
+                  (lambda t: (t.cpu(), t.device), lambda p: p[0].to(p[1]))):
+        assert all(torch.equal(a, b) for a, b in zip(gradients(dev, op, hooks=hooks), want))
+
+
+@pytest.mark.parametrize("op", list(OPS))
+def test_more_batches_in_flight_than_the_cache_holds(dev, op):
+    f, n = OPS[op]
+    want = gradients(dev, op)
+    for capacity in (0, 2, 8):
+        blockAttention.set_schedule_cache(capacity)
+        try:
+            passes = []
+            for _ in range(5):
+                ts = operands(dev, n)
+                passes.append((ts, f(*ts, meta(dev))))
+            for ts, out in passes:
+                out.float().pow(2).sum().backward()
+                assert all(torch.equal(t.grad, b) for t, b in zip(ts, want))
+        finally:
+            blockAttention.set_schedule_cache(8)
+
+
+@pytest.mark.parametrize("op", list(OPS))
+def test_gradients_after_a_call_without(dev, op):
+    # the schedule of the first call has no plans for the gradients; two passes with gradients on the same metadata
+    f, n = OPS[op]
+    want, m = gradients(dev, op), meta(dev)
+    with torch.no_grad():
+        f(*operands(dev, n), m)
+    for _ in range(3):
+        assert all(torch.equal(a, b) for a, b in zip(gradients(dev, op, m=m), want))
