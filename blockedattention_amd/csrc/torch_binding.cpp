@@ -365,6 +365,12 @@ Schedule kept_schedule(const variable_list &saved, size_t at, const Tensor &like
                 "backward: the saved plan came back as ", s.plan.toString(), s.plan.sizes());
     return s;
 }
+// An operand or result that comes back for the backward pass (through whatever hooks there are), `last` elements a head.
+void check_kept(const Tensor &t, const char *name, const Tensor &like, int64_t H, int64_t last) {
+    check_data(t, name);
+    TORCH_CHECK(t.device() == like.device() && t.dim() >= 1 && t.size(-1) == last && leading(t) == H, "backward: the saved ", name,
+                " came back as ", t.toString(), t.sizes(), ", not ", H, " x ", last);
+}
 
 class SparseBlockedGEMM : public torch::autograd::Function<SparseBlockedGEMM> {
 public:
@@ -411,11 +417,12 @@ public:
             s2 = derived_schedule(fwd, &Derived::grad2, grad, aO, a1, a2, N, K, M);
         }
         const int64_t heads = leading(grad);
+        check_kept(mat1, "mat1", grad, heads, s2.info.Dm2);
+        check_kept(mat2, "mat2", grad, heads, s1.info.Dm2);
         // batches of short segments: both products as ONE launch where the library offers it (layouts of the
         // untransposed forward), else one call each
         bool done = false;
-        if (!t1 && !t2 && grad.dim() >= 1 && grad.size(-1) == s1.info.Dm1 && mat2.size(-1) == s1.info.Dm2 &&
-            grad.size(-1) == s2.info.Dm1 && mat1.size(-1) == s2.info.Dm2 && leading(mat1) == heads && leading(mat2) == heads &&
+        if (!t1 && !t2 && grad.dim() >= 1 && grad.size(-1) == s1.info.Dm1 && grad.size(-1) == s2.info.Dm1 &&
             (grad.scalar_type() == at::kHalf || grad.scalar_type() == at::kBFloat16)) {
             g1 = at::empty({heads, s1.info.Dout}, grad.options());
             g2 = at::empty({heads, s2.info.Dout}, grad.options());
@@ -466,6 +473,7 @@ public:
         const Tensor y = saved[0].to(grad.scalar_type());
         const Schedule s = kept_schedule(saved, 4, grad);
         const int64_t H = leading(grad);
+        check_kept(grad, "gradient", grad, H, s.info.Dout); check_kept(y, "result", grad, H, s.info.Dout);
         Tensor dx = at::empty_like(y);
         check_status(ba_blocked_softmax_backward(s.plan.data_ptr(), &s.info, s.info.nseg,
                                                  dtype_code(y, "softmax backward"),
@@ -580,6 +588,11 @@ public:
         const Schedule s = kept_schedule(saved, 5, grad);
         const ba_plan_info &info = s.info;
         const int64_t H = leading(grad);
+        check_kept(grad, "gradient", grad, H, info.Dm1); check_kept(out, "result", grad, H, info.Dm1);
+        check_kept(q, "q", grad, H, info.Dm1); check_kept(k, "k", grad, H, info.Dm2); check_kept(v, "v", grad, H, info.Dm2);
+        check_kept(lse, "row sums", grad, H, ba_attention_rows(&info, info.Dm1));
+        for (const Tensor *t : {&q, &k, &v, &out})
+            TORCH_CHECK(t->scalar_type() == grad.scalar_type(), "backward: a saved operand came back as ", t->toString());
         Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), delta = at::empty_like(lse);
         check_status(ba_varlen_attention_backward(s.plan.data_ptr(), &info, info.nseg, dtype_code(q, "attention backward"),
                                                   q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), grad.data_ptr(),

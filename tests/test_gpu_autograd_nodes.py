@@ -1,4 +1,5 @@
-"""What the operators' autograd nodes keep between the passes: compiled autograd takes it, saved-tensor hooks may move it."""
+"""What the operators' autograd nodes keep between the passes: compiled autograd takes it, saved-tensor hooks may move it,
+and what hooks bring back changed is refused before a kernel sees it."""
 import pytest
 import torch
 
@@ -68,6 +69,36 @@ def test_hooks_that_move_and_copy(dev, op):
                   (lambda t: t.clone(), lambda t: t.clone()),
                   (lambda t: (t.cpu(), t.device), lambda p: p[0].to(p[1]))):
         assert all(torch.equal(a, b) for a, b in zip(gradients(dev, op, hooks=hooks), want))
+
+
+@pytest.mark.parametrize("op", list(OPS))
+@pytest.mark.parametrize("change", ["strided", "short", "wide type"])
+def test_hooks_that_change_are_refused(dev, op, change):
+    shorter = change == "short"
+    change = {"strided": lambda t: torch.stack([t, t], -1)[..., 0], "short": lambda t: t[..., :-1].contiguous(),
+              "wide type": lambda t: t.double() if t.is_floating_point() else t}[change]
+    # one saved tensor at a time (operands, results, row sums, plans, summaries; not the metadata, which no kernel reads):
+    # the backward pass refuses it or makes the same gradients of it
+    f, n = OPS[op]
+    want, counted = gradients(dev, op), []
+    with torch.autograd.graph.saved_tensors_hooks(counted.append, lambda t: t):
+        f(*operands(dev, n), meta(dev))
+    refused = 0
+    for victim in range(len(counted)):
+        seen = []
+
+        def pack(t):
+            seen.append(t)
+            return (t, len(seen) - 1 == victim and t.dtype != torch.int64)
+
+        try:
+            got = gradients(dev, op, hooks=(pack, lambda p: change(p[0]) if p[1] else p[0]))
+        except RuntimeError:
+            refused += 1
+            continue
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), victim
+    if shorter:
+        assert refused == sum(t.dtype != torch.int64 for t in counted)
 
 
 @pytest.mark.parametrize("op", list(OPS))
