@@ -562,7 +562,8 @@ Schedule attention_schedule(const Tensor &q, const Tensor &k, const Tensor &v, c
 }
 
 // Differentiable form.  Between the passes it keeps the operands, the result, the rows' sums and the plan with its
-// summary: nothing of the size M x N, and the backward pass schedules nothing.
+// summary: nothing of the size M x N, and the backward pass schedules nothing.  As with the operators this stands in
+// for, the result may be changed in place before the backward pass.
 class SparseBlockedAttention : public torch::autograd::Function<SparseBlockedAttention> {
 public:
     static variable_list forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &a1,
@@ -571,9 +572,15 @@ public:
         Schedule s = attention_schedule(q, k, v, a1, a2, aO, M, N, K);
         Tensor lse;
         Tensor out = attention_launch(q, k, v, s, scale, &lse);
-        variable_list keep{q, k, v, out, lse};
+        // The result is kept without its version counter, so that a caller may write on it; `watch`, an empty tensor with
+        // that counter, tells the backward pass, which then makes the result again.
+        variable_list keep{q, k, v, out.variable_data(), lse};
         keep_schedule(keep, s);
         ctx->save_for_backward(keep);
+        Tensor watch = at::empty({0}, at::TensorOptions().dtype(at::kByte).device(at::kCPU));
+        torch::autograd::impl::set_version_counter(watch, torch::autograd::impl::version_counter(out));
+        ctx->saved_data["watch"] = watch;
+        ctx->saved_data["version"] = (int64_t)watch._version();
         ctx->saved_data["scale"] = scale;
         ctx->saved_data["lists"] = M.has_value() && N.has_value() && K.has_value();
         return {out};
@@ -582,23 +589,26 @@ public:
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
         TORCH_CHECK(ctx->saved_data["lists"].toBool(), "blockFusedAttention: the backward pass needs MList, NList and KList");
         const auto saved = ctx->get_saved_variables();
-        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4];
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &kept = saved[3], &lse = saved[4];
         const Tensor grad = grads[0].to(q.scalar_type()).contiguous();
         c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
-        const Schedule s = kept_schedule(saved, 5, grad);
+        Schedule s = kept_schedule(saved, 5, grad);
         const ba_plan_info &info = s.info;
         const int64_t H = leading(grad);
-        check_kept(grad, "gradient", grad, H, info.Dm1); check_kept(out, "result", grad, H, info.Dm1);
+        check_kept(grad, "gradient", grad, H, info.Dm1); check_kept(kept, "result", grad, H, info.Dm1);
         check_kept(q, "q", grad, H, info.Dm1); check_kept(k, "k", grad, H, info.Dm2); check_kept(v, "v", grad, H, info.Dm2);
         check_kept(lse, "row sums", grad, H, ba_attention_rows(&info, info.Dm1));
-        for (const Tensor *t : {&q, &k, &v, &out})
+        for (const Tensor *t : {&q, &k, &v, &kept})
             TORCH_CHECK(t->scalar_type() == grad.scalar_type(), "backward: a saved operand came back as ", t->toString());
+        const double scale = ctx->saved_data["scale"].toDouble();
+        const bool changed = (int64_t)ctx->saved_data["watch"].toTensor()._version() != ctx->saved_data["version"].toInt();
+        const Tensor out = changed ? attention_launch(q, k, v, s, scale, nullptr) : kept;
         Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), delta = at::empty_like(lse);
         check_status(ba_varlen_attention_backward(s.plan.data_ptr(), &info, info.nseg, dtype_code(q, "attention backward"),
                                                   q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), grad.data_ptr(),
                                                   lse.data_ptr<float>(), delta.data_ptr<float>(), dq.data_ptr(),
                                                   dk.data_ptr(), dv.data_ptr(), H, info.Dm1, info.Dm2, info.Dout,
-                                                  (float)ctx->saved_data["scale"].toDouble(), current_stream(q)),
+                                                  (float)scale, current_stream(q)),
                      "ba_varlen_attention_backward");
         return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }

@@ -128,3 +128,40 @@ def test_gradients_after_a_call_without(dev, op):
         f(*operands(dev, n), m)
     for _ in range(3):
         assert all(torch.equal(a, b) for a, b in zip(gradients(dev, op, m=m), want))
+
+
+@pytest.mark.parametrize("how", ["plain", "compiled", "checkpoint"])
+def test_attention_result_changed_in_place(dev, how):
+    # masking or dropout on the attention's own result: its value before the change is what the gradients need
+    import torch._dynamo.compiled_autograd as compiled
+    from torch.utils.checkpoint import checkpoint
+
+    mask = (torch.arange(2 * sum(a * b for a, b in zip(M, K)), device=dev) % 3).reshape(2, -1).half()
+
+    def step(in_place):
+        ts, m = operands(dev, 3), meta(dev)
+
+        def layer(*qkv):
+            y = attention(*qkv, m)
+            return y.mul_(mask) if in_place else y * mask
+
+        out = checkpoint(layer, *ts, use_reentrant=False) if how == "checkpoint" else layer(*ts)
+        loss = out.float().pow(2).sum()
+        if how == "compiled":
+            with compiled._enable(torch.compile(backend="eager")):
+                loss.backward()
+        else:
+            loss.backward()
+        return [t.grad for t in ts]
+
+    assert all(torch.equal(a, b) for a, b in zip(step(True), step(False)))
+
+
+def test_attention_result_overwritten(dev):
+    want = gradients(dev, "attention", backward=lambda loss: loss.backward())
+    ts = operands(dev, 3)
+    y = attention(*ts, meta(dev))
+    grad = (2 * y.float()).half()
+    with torch.no_grad():
+        y.zero_()
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(y, ts, grad), want))
