@@ -68,9 +68,13 @@ __global__ __launch_bounds__(kSegThreads, ANY ? (MAXNT <= 8 ? 3 : 2) : MAXNT <= 
             return;
         }
     } else if (!mfma_ok || kind == kSegSlow) {
-        // Element-wise path of the product alone (no fused launch of this build has such segments).
-        if constexpr (!FUSED)
+        // Element-wise path of the product alone.  The fused call gets this build if the summary counts no such segments:
+        // one that is there all the same shows that the summary is another plan's, and is reported.
+        if constexpr (!FUSED) {
             for (int r = first; r < s.M; r += stride) generic_seg_rows<DT>(s, a, r, r + 1, 0, s.N);
+        } else if (blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) {
+            atomicAdd(&reinterpret_cast<PlanHeader *>(a.plan)->run_errors, 1);
+        }
         return;
     }
     if (!ANY && kind == kSegStrip) {
