@@ -78,15 +78,13 @@ def test_one_launch_entry(dev, cols):
 
 
 def test_summary_of_another_plan_is_reported(dev):
-    # equal segment count and totals; the summary counts no unaligned segment, the plan has two of them
-    M, N, K, K2 = np.full(3, 16), np.full(3, 256), np.array([257, 255, 256]), np.full(3, 256)
-    plan, other = make_plan(dev, M, N, K), make_plan(dev, M, N, K2)
-    assert plan.info.slow_items > 0 and other.info.slow_items == 0 and other.info.list_rest == plan.info.list_rest == 3
-    A, B = random_operands(M, N, K, 2, torch.float16, 3)
-    out = torch.full((2, 3 * 16 * 256), 7.0, dtype=torch.float16, device=dev)
+    # equal segment count and totals; the summary counts two packs of tiny segments and no unaligned one, the plan has two of those
+    M = N = np.full(4, 2)
+    plan, other = make_plan(dev, M, N, np.array([9, 7, 16, 16])), make_plan(dev, M, N, np.array([8, 8, 16, 16]))
+    assert plan.info.slow_items == 2 and other.info.slow_items == 0 and other.info.list_rest == other.info.pack_items == 2
+    A = torch.ones((2, 96), dtype=torch.float16, device=dev)
+    out = torch.full((2, 16), 7.0, dtype=torch.float16, device=dev)
     plan.info = other.info
-    capi.gemm_softmax(plan, A.to(dev), B.to(dev), out, 2, 3 * 16 * 256, 3 * 256 * 256, 3 * 16 * 256, 0.05)
+    capi.gemm_softmax(plan, A, A, out, 2, 96, 96, 16, 0.05)
     assert plan.read(raise_on_bad=False).run_errors == 2
-    assert bool((out[:, :2 * 16 * 256] == 7.0).all())
-    ref = oracle.per_segment_torch(A, B, M, N, K, 0.05)[:, 2 * 16 * 256:]
-    assert (out[:, 2 * 16 * 256:].float().cpu() - ref).abs().max() <= 2e-3 * ref.abs().max()
+    assert bool((out[:, :8] == 7.0).all())
