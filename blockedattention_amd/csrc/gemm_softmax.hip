@@ -38,9 +38,16 @@ namespace ba {
 // MAXNT = 8 is the build for batches whose widest segment has N <= 128: half the
 // accumulator registers, half again as many resident wavefronts.  The host picks it from
 // the plan summary; without a summary the 16-tile build runs.
-// ANY: the build of the fused call for batches with segments of any alignment, which runs its strips through any_rows.
-template <int DT, bool FUSED, bool F32OUT, int MAXNT, bool ANY>
-__global__ __launch_bounds__(kSegThreads, ANY ? (MAXNT <= 8 ? 3 : 2) : MAXNT <= 8 ? 6 : 4) void segment_kernel(RunArgs a) {
+// ANY: which fused build takes segments of any alignment.  kAnyKnown, for batches that have some by the summary (or
+// have nothing else), runs all its strips through any_rows at the registers that wants.  kAnyUnknown, without a summary,
+// keeps the registers, the LDS window and the strips of aligned segments, which most batches consist of: its workgroups
+// are nearly all there to find nothing to do, so it counts how many are resident.  any_rows then has panels of 128
+// columns and 30 spilled registers.  Whole calls without a summary, kAnyKnown / kAnyUnknown: 256 x 8 pairs of 32 .. 128
+// rows 43.1 / 42.8 us, 1024 x 4 of 2 .. 512 95.6 / 93.6, the former with K = 61 70.9 / 69.3.
+enum AnyBuild { kAnyNone, kAnyKnown, kAnyUnknown };
+constexpr int kAnyUnknownTiles = 8;
+template <int DT, bool FUSED, bool F32OUT, int MAXNT, AnyBuild ANY>
+__global__ __launch_bounds__(kSegThreads, ANY == kAnyKnown ? (MAXNT <= 8 ? 3 : 2) : MAXNT <= 8 ? 6 : 4) void segment_kernel(RunArgs a) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const PlanRO pv = plan_ro(a.plan, a.nseg);
     const int64_t h = blockIdx.y;
@@ -59,12 +66,12 @@ __global__ __launch_bounds__(kSegThreads, ANY ? (MAXNT <= 8 ? 3 : 2) : MAXNT <= 
     const bool mfma_ok = (a.flags & kFlagMfmaOk) != 0;
     if (kind == kSegEmpty) return;
     if (mfma_ok && a.list < 0 && launch_class(kind, s.M, s.N, s.K) != kListRest) return;   // another kernel's
-    if constexpr (ANY) {
+    if constexpr (ANY != kAnyNone) {
         // With the 16-byte operand loads ruled out for the whole launch this also covers the segments the list
         // kernels would have taken.
-        if (!mfma_ok || kind == kSegSlow || kind == kSegStrip) {
+        if (!mfma_ok || kind == kSegSlow || (ANY == kAnyKnown && kind == kSegStrip)) {
             for (int base = blockIdx.z * kSegWaves * kStripRows; base < s.M; base += stride * kStripRows)
-                any_rows<DT, F32OUT, MAXNT>(s, a, lds, base + wave * kStripRows);
+                any_rows<DT, F32OUT, ANY == kAnyKnown ? MAXNT : kAnyUnknownTiles>(s, a, lds, base + wave * kStripRows);
             return;
         }
     } else if (!mfma_ok || kind == kSegSlow) {
@@ -77,7 +84,7 @@ __global__ __launch_bounds__(kSegThreads, ANY ? (MAXNT <= 8 ? 3 : 2) : MAXNT <= 
         }
         return;
     }
-    if (!ANY && kind == kSegStrip) {
+    if (ANY != kAnyKnown && kind == kSegStrip) {
         // One strip per wavefront; blockIdx.z selects the group of kSegWaves strips.
         const int strips = (s.M + kStripRows - 1) / kStripRows;
         const int nt = (s.N + 15) >> 4;
@@ -335,23 +342,30 @@ static int launch_set(int dtype, const RunArgs &args_in, int64_t nseg, const ba_
             const int64_t nks = ceil_div(std::max<int64_t>(info->max_K, 1), 32);
             blocks = std::max<int64_t>(nt, std::min<int64_t>(nt * nks, 64));
         }
-        if (FUSED && any) blocks = ceil_div(any_rows_lds(lean ? 8 : kMaxTiles), kLdsBlockBytes);
+        const bool unknown = !info && mfma_ok;
+        if (FUSED && any)
+            blocks = unknown ? std::max<int64_t>(blocks, ceil_div(any_rows_lds(kAnyUnknownTiles), kLdsBlockBytes))
+                             : ceil_div(any_rows_lds(lean ? 8 : kMaxTiles), kLdsBlockBytes);
         RunArgs seg_args = args;
         seg_args.list = mfma_ok ? kListRest : -1;
         seg_args.lds_blocks = (int)blocks;
         const dim3 grid((unsigned)n_rest, H, (unsigned)z);
         const size_t lds_bytes = (size_t)blocks * kLdsBlockBytes;
         auto launch = [&](auto any_tag) {
-            constexpr bool ANY = decltype(any_tag)::value;
-            if (lean)
-                hipLaunchKernelGGL((segment_kernel<DT, FUSED, F32OUT, 8, ANY>), grid, dim3(kSegThreads), lds_bytes, stream, seg_args);
-            else
-                hipLaunchKernelGGL((segment_kernel<DT, FUSED, F32OUT, 16, ANY>), grid, dim3(kSegThreads), lds_bytes, stream, seg_args);
+            constexpr AnyBuild ANY = decltype(any_tag)::value;
+            if constexpr (ANY != kAnyUnknown) {
+                if (lean) {
+                    hipLaunchKernelGGL((segment_kernel<DT, FUSED, F32OUT, 8, ANY>), grid, dim3(kSegThreads), lds_bytes, stream, seg_args);
+                    return;
+                }
+            }
+            hipLaunchKernelGGL((segment_kernel<DT, FUSED, F32OUT, 16, ANY>), grid, dim3(kSegThreads), lds_bytes, stream, seg_args);
         };
         if constexpr (FUSED) {
-            if (any) launch(std::true_type{});
-            else launch(std::false_type{});
-        } else launch(std::false_type{});
+            if (unknown) launch(std::integral_constant<AnyBuild, kAnyUnknown>{});
+            else if (any) launch(std::integral_constant<AnyBuild, kAnyKnown>{});
+            else launch(std::integral_constant<AnyBuild, kAnyNone>{});
+        } else launch(std::integral_constant<AnyBuild, kAnyNone>{});
     }
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
 }

@@ -55,7 +55,8 @@ def test_fp32_results_are_fp32_accurate(dev):
     assert ((got - ref).abs() <= torch.as_tensor(rel) * ref + 1e-30).all()
 
 
-def test_among_aligned_segments_and_packs(dev):
+@pytest.mark.parametrize("summary", [True, False])
+def test_among_aligned_segments_and_packs(dev, summary):
     rng = np.random.default_rng(12)
     M = rng.integers(1, 80, 64).astype(np.int64); N = rng.integers(1, 200, 64).astype(np.int64)
     M[::3] = 5; N[::3] = 6
@@ -63,7 +64,7 @@ def test_among_aligned_segments_and_packs(dev):
     K[40:42] = (61, 13)                     # everything behind them starts at odd offsets
     K[42] = 6                               # sums are multiples of eight again further on for some
     A, B = random_operands(M, N, K, 2, torch.float16, 9)
-    assert_probs_close(fused(dev, A, B, M, N, K, 0.2, torch.float16), oracle.per_segment_torch(A, B, M, N, K, 0.2), "mixed")
+    assert_probs_close(fused(dev, A, B, M, N, K, 0.2, torch.float16, summary), oracle.per_segment_torch(A, B, M, N, K, 0.2), "mixed")
 
 
 @pytest.mark.parametrize("cols", [[1, 17, 128], [200, 256, 300]])
