@@ -44,10 +44,10 @@ __host__ __device__ inline bool fast_strip_shape(int N, int K) {
     return b >= 1 && b <= kBigBlocks;
 }
 
-// What the scheduler scans per segment.  The first five are 0/1 class flags whose
-// scan compacts the segment indices into one work list per launch (the arrays of
-// the plan hold those lists); the others are work-item counts of which only the
-// totals are kept (plan summary).
+// What the scheduler counts per segment, totals[] of the header.  The first five are
+// 0/1 class flags whose scan compacts the segments into one work list per launch (the
+// arrays of the plan hold those lists); the others are work-item counts of which only
+// the totals are kept (plan summary).
 constexpr int kRunCols = 256;     // widest row of the softmax lane-run kernel; wider rows take the row kernel
 
 enum PrefixKind {
@@ -64,17 +64,8 @@ enum PrefixKind {
     kPfxRows = 9,   // softmax: M rows
     kPfxPack = 10,  // 1 for the first segment of a pack of tiny segments, else 0
     kPfxSlow = 11,  // ceil(M/16) for segments the 16-byte operand loads cannot serve
-    kPfxAtt64 = 12,   // GEMM plans: ceil(M/64) for every segment with rows (one-pass attention, any-layout GEMM)
-    kPfxAttCols = 13, // GEMM plans: ceil(N/64) for every segment with columns (backward of the one-pass attention)
-    kPfxMini = 14,    // 1 for a segment of the strip kernel's main list that is small enough for one wavefront
-    kNumPrefix = 15
+    kNumTotals = 12
 };
-// Three of the flags share their scanned word with a second one (a pass holds at most 1024 segments, 16 bits suffice):
-//   kPfxMini   2^16 for a segment of the tile list that the pipelined row-block kernel can take (fused call)
-//   kPfxPack   2^16 for a segment with an odd number of row blocks of 64
-//   kListRows  2^16 for a segment with an odd number of column blocks of 64
-// The blocks of 128 before a segment are half of the blocks of 64 and the odd segments before it.
-enum SecondFlag { kTwoPipe = 0, kTwoOddRows = 1, kTwoOddCols = 2, kNumTwo = 3 };
 
 // "Mini" segments: strip-class segments of at most 64 rows whose B_g needs at most kMiniBlocks LDS blocks and at most
 // eight column tiles.  One wavefront can take such a segment on its own (a quarter of a 64 KiB window), so four of
@@ -88,7 +79,7 @@ __host__ __device__ inline bool mini_shape(int M, int N, int K) {
     return M >= 1 && M <= kMiniRows && b >= 1 && b <= kMiniBlocks && fast_strip_tiles(N) <= 8;
 }
 constexpr int kMailboxTicket = 256;   // byte offset of the ticket word in a scheduler mailbox (behind the header copy)
-constexpr int kAttBlockRows = 64;   // kPfxAtt64 counts blocks of this many rows, kPfxAttCols of as many columns
+constexpr int kAttBlockRows = 64;   // rows or columns of the blocks that the row-block and column-block prefixes count
 
 // A segment is "aligned" when K % 8 == 0 and its A and B offsets are multiples
 // of 8 elements: every operand row then starts on a 16-byte boundary (given
@@ -103,13 +94,13 @@ struct PlanHeader {
     int32_t kind;            // 0 = GEMM plan, 1 = softmax plan
     int64_t Dm1, Dm2, Dout;
     int64_t total_rows;
-    int64_t totals[12];      // totals of the scanned quantities (PrefixKind)
+    int64_t totals[kNumTotals];   // see PrefixKind
     int32_t max_M, max_N, max_K;
     int32_t bad_segments;
     int32_t run_errors;      // bumped by kernels that refuse to run
     int32_t small_max_N, small_max_M;   // maxima over the segments of the strip kernel's main launch
     int32_t att_blocks64, att_blocks128;   // row blocks of 64 and of 128 per head: the one-pass attention's work items
-    int32_t mini_count;      // total of kPfxMini
+    int32_t mini_count;      // mini segments
     int32_t pipe_count;      // segments of the tile list that the pipelined row-block kernel can take
     int32_t pipe_groups;     // bumped by every workgroup of the pipelined row-block kernel that found work in this plan
     int32_t min_N, min_K;    // smallest N and K over the segments that have rows and columns (0: there is none)

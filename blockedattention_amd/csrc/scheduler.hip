@@ -29,30 +29,24 @@ struct SchedArgs {
     uint32_t ticket;
 };
 
-// Exclusive scan of NQ quantities over the workgroup.  Wavefront-level DPP
-// scans; the totals of the (up to 16) wavefronts go to LDS as lds[16 q + wavefront] and are scanned four
-// quantities at a time: lane l of every wavefront takes entry 64 b + l of batch b, i.e. quantity 4 b + l / 16 of
-// wavefront l % 16, and one scan inside the rows of 16 lanes serves all four.  lds holds 16 * NQ entries and is
-// free for reuse after the next __syncthreads().  One barrier (none in the one-wavefront build).
+// The level above the wavefronts of a scan over the workgroup: last[q] is, in lane 63, the wavefront's total of quantity q;
+// before[q] = the totals of the wavefronts in front, total[q] = all of them, both the same in every lane.  The totals of
+// the (up to 16) wavefronts go to LDS as lds[16 q + wavefront] and are scanned four quantities at a time: lane l of every
+// wavefront takes entry 64 b + l of batch b, i.e. quantity 4 b + l / 16 of wavefront l % 16, and one scan inside the rows
+// of 16 lanes serves all four.  lds holds 16 * NQ entries and is free for reuse after the next __syncthreads().  One
+// barrier (none in the one-wavefront build; callers still place theirs before reusing lds).
 template <typename T, int NQ, int kSchedWaves>
-__device__ __forceinline__ void block_exclusive_scan(T (&v)[NQ], T (&total)[NQ], T *lds) {
+__device__ __forceinline__ void cross_wave_scan(const T (&last)[NQ], T (&before)[NQ], T (&total)[NQ], T *lds) {
     static_assert(kSchedWaves <= 16, "one row of 16 lanes scans the wavefront totals");
     const int wave = uniform((int)(threadIdx.x >> 6)), lane = lane_id();
-    T incl[NQ];
     if constexpr (kSchedWaves == 1) {
-        // one wavefront: its own scan is the workgroup's (callers still place their barrier before reusing lds)
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            incl[q] = wave_inclusive_scan(v[q]);
-            total[q] = readlane_t(incl[q], 63);
-            v[q] = incl[q] - v[q];
-        }
+        for (int q = 0; q < NQ; ++q) { before[q] = T(0); total[q] = readlane_t(last[q], 63); }
         return;
     }
+    if (lane == 63) {
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        incl[q] = wave_inclusive_scan(v[q]);
-        if (lane == 63) lds[q * 16 + wave] = incl[q];
+        for (int q = 0; q < NQ; ++q) lds[q * 16 + wave] = last[q];
     }
     __syncthreads();
     constexpr int kBatches = (NQ + 3) / 4;
@@ -65,13 +59,25 @@ __device__ __forceinline__ void block_exclusive_scan(T (&v)[NQ], T (&total)[NQ],
         for (int r = 0; r < 4; ++r) {
             const int q = 4 * b + r;
             if (q < NQ) {
-                const T upto = readlane_t(t, 16 * r + kSchedWaves - 1);
-                const T before = wave == 0 ? T(0) : readlane_t(t, 16 * r + wave - 1);
-                v[q] = before + incl[q] - v[q];
-                total[q] = upto;
+                total[q] = readlane_t(t, 16 * r + kSchedWaves - 1);
+                before[q] = wave == 0 ? T(0) : readlane_t(t, 16 * r + wave - 1);
             }
         }
     }
+}
+// Exclusive scan of NQ quantities over the workgroup: DPP scans of the wavefronts and the level above them.
+template <typename T, int NQ, int kSchedWaves>
+__device__ __forceinline__ void block_exclusive_scan(T (&v)[NQ], T (&total)[NQ], T *lds) {
+    T incl[NQ], before[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) incl[q] = wave_inclusive_scan(v[q]);
+    cross_wave_scan<T, NQ, kSchedWaves>(incl, before, total, lds);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) v[q] = before[q] + incl[q] - v[q];
+}
+// Lanes in front of this one whose bit of the ballot is set.
+__device__ __forceinline__ int32_t lanes_before(uint64_t ballot) {
+    return (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(ballot >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ballot, 0u));
 }
 
 __device__ __forceinline__ int64_t isqrt64(int64_t v) {
@@ -117,18 +123,34 @@ struct SchedBatch {
 
 constexpr int kSmallBuckets = 8;                          // work buckets of the main strip launch's list
 
-template <int kSchedThreads>
-__global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedBatch batch) {
-    const SchedArgs a = batch.plan[blockIdx.x];
+// 0/1 flags of a segment: membership of the lists (PrefixKind 0 .. kNumLists - 1, where a main-list segment that is mini
+// counts as kBitMini only) and an odd number of row or column blocks of 64 (the blocks of 128 before a segment are half of
+// the blocks of 64 and the odd segments before it).  A ballot gives a flag's rank in the wavefront and the wavefront's
+// count; two counts share a scanned word (a pass holds at most 1024 segments, 16 bits suffice).
+enum SegBit { kBitMini = kNumLists, kBitOddRows, kBitOddCols, kNumBits };
+enum ScanWord { kWordRows = kNumBits / 2, kWordCols, kNumWords };        // behind the flags: row and column blocks of 64
+static_assert(kNumBits % 2 == 0, "two flags to a word");
+// Per wavefront, for the header: maxima, then sums (counts of a batch that exceed 31 bits come with a weight that rejects it).
+enum Fold { kMaxM, kMaxN, kMaxK, kMaxSmallN, kMaxSmallM, kMaxInvN, kMaxInvK, kSumBad, kSumGemm, kSumStrip, kSumSplit, kSumWide,
+            kSumRows, kSumSlow, kSumPack, kSumPipe, kNumFold };
+
+__device__ __forceinline__ const SchedArgs &plan_args(const SchedArgs &one) { return one; }
+__device__ __forceinline__ const SchedArgs &plan_args(const SchedBatch &batch) { return batch.plan[blockIdx.x]; }
+
+// Args: SchedArgs for one plan, SchedBatch for several (for one plan its 312 bytes of arguments cost up to 0.5 us a call
+// of 64 segments, in some processes and not in others: 5.5 against 5.0).
+template <int kSchedThreads, typename Args>
+__global__ __launch_bounds__(kSchedThreads) void schedule_kernel(Args args) {
+    const SchedArgs a = plan_args(args);
     constexpr int kSchedWaves = kSchedThreads / 64;
     // Only the 256-thread build (65 to 256 segments) orders its list by work: smaller batches are resident at
     // once whatever their order, and in the larger builds, which are bound by instruction issue, the four more
     // scans cost more than the order gains (1024 segments: scheduler +0.8 us, kernels unchanged).
     constexpr bool kBucketed = kSchedThreads == 256;
-    constexpr int kNumScan = kNumPrefix + (kBucketed ? kSmallBuckets / 2 : 0);   // scanned words
+    constexpr int kNumScan = kNumWords + (kBucketed ? kSmallBuckets / 2 : 0);   // scanned words
     __shared__ int64_t sScan64[16 * 3];
     __shared__ int32_t sScan32[16 * kNumScan];
-    __shared__ int32_t sRed[kSchedWaves][8];
+    __shared__ __attribute__((aligned(16))) int32_t sFold[kSchedWaves][kNumFold];
     __shared__ int64_t sWeight[kSchedWaves];
 
     const int tid = threadIdx.x;
@@ -137,10 +159,11 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedBatch batc
     PlanView pv = plan_view(a.plan, nseg);
 
     int64_t base64[3] = {0, 0, 0};
-    int32_t base32[kNumPrefix] = {}, base_two[kNumTwo] = {};
-    int32_t maxM = 0, maxN = 0, maxK = 0, nbad = 0;
-    int32_t maxSmallN = 0, maxSmallM = 0;       // widest / tallest segment of the strip kernel's main launch
-    int32_t maxInvN = 0, maxInvK = 0;           // INT32_MAX - the smallest N and K of the segments that have rows and columns
+    int32_t base_bit[kNumBits] = {}, base_rows = 0, base_cols = 0;
+    // fold[kMaxSmallN / M]: widest / tallest segment of the strip kernel's main launch; fold[kMaxInvN / K]: INT32_MAX - the
+    // smallest N and K of the segments that have rows and columns.  kSumBad, kSumPack and kSumPipe count the wavefront's
+    // segments, the others the thread's.
+    int32_t fold[kNumFold] = {};
     // Every scanned count of a segment is at most max(rows, column blocks, strips x chunks): while the sum of these weights stays
     // below 2^31, none of the int32 scans can overflow; a batch beyond that is rejected as a whole.
     int64_t weight = 0;
@@ -234,30 +257,42 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedBatch batc
                                  : ni <= kSplitCols ? kSegSplit : kSegWide;
         const int cls = a.kind == 0 ? launch_class(seg_kind, mi, ni, ki) : -1;
         const bool mini = cls == kListSmall && mini_shape(mi, ni, ki);     // kept apart from the list's other entries
-        int32_t v32[kNumScan], t32[kNumScan];
-#pragma unroll
-        for (int q = 0; q < kNumLists; ++q) v32[q] = (cls == q && !mini) ? 1 : 0;
-        v32[kPfxMini] = (mini ? 1 : 0) + ((cls == kListTile && pipe_segment(seg_kind, ni, ki)) ? 1 << 16 : 0);
+        const bool gemm = a.kind == 0;
         const bool wide_rows = mi >= 1 && ni > kRunCols;      // the softmax row kernel's, whatever the plan kind
-        const int32_t row_blocks = mi >= 1 ? (mi + kAttBlockRows - 1) / kAttBlockRows : 0;   // of every segment with rows, whatever N and K are
-        const int32_t col_blocks = ni >= 1 ? (ni + kAttBlockRows - 1) / kAttBlockRows : 0;
+        // row blocks of every segment with rows, whatever N and K are; column blocks of those with elements (no one keeps
+        // a batch from having any number of columns without any)
+        const int32_t row_blocks = gemm && mi >= 1 ? (mi + kAttBlockRows - 1) / kAttBlockRows : 0;
+        const int32_t col_blocks = gemm && ni >= 1 && ki >= 1 ? (ni + kAttBlockRows - 1) / kAttBlockRows : 0;
         weight += max(max((int64_t)mi, (int64_t)col_blocks), (int64_t)strips * chunks) + 1;
-        v32[kPfxGemm] = (mfma_ok && ni > kWaveCols) ? strips * chunks : 0;
-        v32[kPfxStrip] = (mfma_ok && ni <= kWaveCols) ? strips : 0;
-        v32[kPfxSplit] = (mfma_ok && ni > kWaveCols && ni <= kSplitCols) ? strips : 0;
-        v32[kPfxWide] = (mfma_ok && ni > kSplitCols) ? strips : 0;
-        v32[kPfxRows] = ni >= 1 ? mi : 0;
-        v32[kListRows] = (wide_rows ? 1 : 0) + ((col_blocks & 1) << 16);
-        v32[kPfxPack] = (pack > 0 ? 1 : 0) + ((row_blocks & 1) << 16);
-        v32[kPfxSlow] = aligned ? 0 : strips;
-        v32[kPfxAtt64] = row_blocks;
-        v32[kPfxAttCols] = col_blocks;
-        if (a.kind == 1) {
-#pragma unroll
-            for (int q = 0; q < kNumPrefix; ++q)
-                if (q >= kNumLists && q != kPfxRows) v32[q] = 0;
-            v32[kListRows] &= 0xffff;
+        if (gemm) {
+            fold[kSumGemm] += (mfma_ok && ni > kWaveCols) ? strips * chunks : 0;
+            fold[kSumStrip] += (mfma_ok && ni <= kWaveCols) ? strips : 0;
+            fold[kSumSplit] += (mfma_ok && ni > kWaveCols && ni <= kSplitCols) ? strips : 0;
+            fold[kSumWide] += (mfma_ok && ni > kSplitCols) ? strips : 0;
+            fold[kSumSlow] += aligned ? 0 : strips;
+            fold[kSumPack] += __popcll(__ballot(pack > 0));
+            fold[kSumPipe] += __popcll(__ballot(cls == kListTile && pipe_segment(seg_kind, ni, ki)));
         }
+        fold[kSumRows] += ni >= 1 ? mi : 0;
+        fold[kSumBad] += __popcll(__ballot(bad));
+
+        bool bit[kNumBits];
+#pragma unroll
+        for (int q = 0; q < kNumLists; ++q) bit[q] = cls == q && !mini;
+        bit[kListRows] = wide_rows;
+        bit[kBitMini] = mini;
+        bit[kBitOddRows] = row_blocks & 1;
+        bit[kBitOddCols] = col_blocks & 1;
+        int32_t pos[kNumBits], last[kNumScan], before[kNumScan], total[kNumScan];
+#pragma unroll
+        for (int w = 0; w < kNumBits / 2; ++w) {
+            const uint64_t lo = __ballot(bit[2 * w]), hi = __ballot(bit[2 * w + 1]);
+            pos[2 * w] = lanes_before(lo);
+            pos[2 * w + 1] = lanes_before(hi);
+            last[w] = __popcll(lo) + (__popcll(hi) << 16);
+        }
+        last[kWordRows] = wave_inclusive_scan(row_blocks);
+        last[kWordCols] = wave_inclusive_scan(col_blocks);
         // The main strip launch's list is kept in eight buckets of decreasing work (16-row strips x column
         // tiles / 8, clipped): workgroups that start together then take about equally long and the longest
         // start first (256 segments x 8 heads of 32..128 rows: fused kernel 16.1 -> 15.4 us).  One counter of
@@ -266,25 +301,25 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedBatch batc
         if constexpr (kBucketed) {
 #pragma unroll
             for (int wd = 0; wd < kSmallBuckets / 2; ++wd)
-                v32[kNumPrefix + wd] = (bucket >> 1) == wd ? 1 << (16 * (bucket & 1)) : 0;
+                last[kNumWords + wd] = wave_inclusive_scan((bucket >> 1) == wd ? 1 << (16 * (bucket & 1)) : 0);
         }
-        block_exclusive_scan<int32_t, kNumScan, kSchedWaves>(v32, t32, sScan32);
-        constexpr int kTwoWord[kNumTwo] = {kPfxMini, kPfxPack, kListRows};
-        int32_t v_two[kNumTwo], t_two[kNumTwo];
+        cross_wave_scan<int32_t, kNumScan, kSchedWaves>(last, before, total, sScan32);
+        int32_t total_bit[kNumBits];
 #pragma unroll
-        for (int q = 0; q < kNumTwo; ++q) {
-            v_two[q] = (int32_t)((uint32_t)v32[kTwoWord[q]] >> 16); v32[kTwoWord[q]] &= 0xffff;
-            t_two[q] = (int32_t)((uint32_t)t32[kTwoWord[q]] >> 16); t32[kTwoWord[q]] &= 0xffff;
+        for (int q = 0; q < kNumBits; ++q) {
+            pos[q] += base_bit[q] + ((before[q / 2] >> (16 * (q & 1))) & 0xffff);
+            total_bit[q] = (total[q / 2] >> (16 * (q & 1))) & 0xffff;
         }
-        int32_t small_pos = v32[kListSmall];                  // position in the list among this pass's entries
         if constexpr (kBucketed) {
-            small_pos = 0;
+            int32_t small_pos = base_bit[kListSmall];
 #pragma unroll
             for (int b = 0; b < kSmallBuckets; ++b) {
-                const int32_t count = (t32[kNumPrefix + (b >> 1)] >> (16 * (b & 1))) & 0xffff;
-                const int32_t rank = (v32[kNumPrefix + (b >> 1)] >> (16 * (b & 1))) & 0xffff;
-                small_pos += b > bucket ? count : b == bucket ? rank : 0;
+                const int32_t count = (total[kNumWords + (b >> 1)] >> (16 * (b & 1))) & 0xffff;
+                // the own entry counts in last[]
+                const int32_t rank = ((before[kNumWords + (b >> 1)] + last[kNumWords + (b >> 1)]) >> (16 * (b & 1))) & 0xffff;
+                small_pos += b > bucket ? count : b == bucket ? rank - 1 : 0;
             }
+            pos[kListSmall] = small_pos;
         }
 
         if (live) {
@@ -295,16 +330,16 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedBatch batc
             rec.index = (int32_t)g;
             pv.recs[g] = rec;
 #pragma unroll
-            for (int q = 0; q < kNumLists; ++q)          // v32 now holds the exclusive scans
-                if (cls == q && !mini) pv.list[q][base32[q] + (q == kListSmall ? small_pos : v32[q])] = rec;
-            if (mini) pv.list[kListSmall][plan_cap(nseg) - 1 - (base32[kPfxMini] + v32[kPfxMini])] = rec;
-            if (wide_rows) pv.list[kListRows][base32[kListRows] + v32[kListRows]] = rec;
-            if (a.kind == 0) {
-                const int32_t rows64 = base32[kPfxAtt64] + v32[kPfxAtt64], cols64 = base32[kPfxAttCols] + v32[kPfxAttCols];
+            for (int q = 0; q < kNumLists; ++q)
+                if (bit[q]) pv.list[q][pos[q]] = rec;
+            if (mini) pv.list[kListSmall][plan_cap(nseg) - 1 - pos[kBitMini]] = rec;
+            if (gemm) {
+                const int32_t rows64 = base_rows + before[kWordRows] + last[kWordRows] - row_blocks;
+                const int32_t cols64 = base_cols + before[kWordCols] + last[kWordCols] - col_blocks;
                 plan_rowblocks(a.plan, nseg, 0)[g] = rows64;
-                plan_rowblocks(a.plan, nseg, 1)[g] = (rows64 + base_two[kTwoOddRows] + v_two[kTwoOddRows]) >> 1;
+                plan_rowblocks(a.plan, nseg, 1)[g] = (rows64 + pos[kBitOddRows]) >> 1;
                 plan_rowblocks(a.plan, nseg, 2)[g] = cols64;
-                plan_rowblocks(a.plan, nseg, 3)[g] = (cols64 + base_two[kTwoOddCols] + v_two[kTwoOddCols]) >> 1;
+                plan_rowblocks(a.plan, nseg, 3)[g] = (cols64 + pos[kBitOddCols]) >> 1;
             }
             if (!offsets_given) {
                 if (a.a1) a.a1[g] = o1;
@@ -317,13 +352,16 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedBatch batc
                 if (a.K) a.K[g] = bad ? -1 : k;
             }
         }
-        maxM = max(maxM, mi); maxN = max(maxN, ni); maxK = max(maxK, ki); nbad += bad ? 1 : 0;
-        if (cls == kListSmall) { maxSmallN = max(maxSmallN, ni); maxSmallM = max(maxSmallM, mi); }
-        if (mi >= 1 && ni >= 1) { maxInvN = max(maxInvN, INT32_MAX - ni); maxInvK = max(maxInvK, INT32_MAX - ki); }
+        fold[kMaxM] = max(fold[kMaxM], mi); fold[kMaxN] = max(fold[kMaxN], ni); fold[kMaxK] = max(fold[kMaxK], ki);
+        if (cls == kListSmall) { fold[kMaxSmallN] = max(fold[kMaxSmallN], ni); fold[kMaxSmallM] = max(fold[kMaxSmallM], mi); }
+        if (mi >= 1 && ni >= 1) {
+            fold[kMaxInvN] = max(fold[kMaxInvN], INT32_MAX - ni);
+            fold[kMaxInvK] = max(fold[kMaxInvK], INT32_MAX - ki);
+        }
 #pragma unroll
-        for (int q = 0; q < kNumPrefix; ++q) base32[q] += t32[q];
-#pragma unroll
-        for (int q = 0; q < kNumTwo; ++q) base_two[q] += t_two[q];
+        for (int q = 0; q < kNumBits; ++q) base_bit[q] += total_bit[q];
+        base_rows += total[kWordRows];
+        base_cols += total[kWordCols];
         if (!offsets_given) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) base64[q] += t64[q];
@@ -332,17 +370,35 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedBatch batc
         __syncthreads();   // the scan scratch is rewritten by the next pass
     }
 
-    // Shape maxima and the count of rejected segments: DPP reduction per
-    // wavefront, then thread 0 folds the 16 partial results.
-    maxM = wave_max_nonneg(maxM); maxN = wave_max_nonneg(maxN); maxK = wave_max_nonneg(maxK);
-    maxSmallN = wave_max_nonneg(maxSmallN); maxSmallM = wave_max_nonneg(maxSmallM);
-    maxInvN = wave_max_nonneg(maxInvN); maxInvK = wave_max_nonneg(maxInvK);
-    nbad = __builtin_amdgcn_readlane(wave_inclusive_scan(nbad), 63);
+    // What only the header needs: reduced per wavefront (results in lane 63), then lane q of the first wavefront folds
+    // quantity q of all of them.
 #pragma unroll
-    for (int msk = 32; msk >= 1; msk >>= 1) weight += __shfl_xor(weight, msk);
-    if (lane == 0) sWeight[wave] = weight;
-    if (lane == 0) { sRed[wave][0] = maxM; sRed[wave][1] = maxN; sRed[wave][2] = maxK; sRed[wave][3] = nbad; sRed[wave][4] = maxSmallN; sRed[wave][5] = maxSmallM; sRed[wave][6] = maxInvN; sRed[wave][7] = maxInvK; }
-    __syncthreads();
+    for (int q = 0; q < kSumBad; ++q) fold[q] = wave_max_nonneg(fold[q]);
+#pragma unroll
+    for (int q = kSumGemm; q < kSumPack; ++q) fold[q] = wave_inclusive_scan(fold[q]);
+    weight = wave_inclusive_scan(weight);
+    int64_t total_weight = readlane_t(weight, 63);
+    if constexpr (kSchedWaves == 1) {
+#pragma unroll
+        for (int q = 0; q < kNumFold; ++q) fold[q] = readlane_t(fold[q], 63);
+    } else {
+        if (lane == 63) {
+#pragma unroll
+            for (int q = 0; q < kNumFold; ++q) sFold[wave][q] = fold[q];
+            sWeight[wave] = total_weight;
+        }
+        __syncthreads();
+        if (wave != 0) return;
+        int32_t folded = 0;
+#pragma unroll
+        for (int w = 0; w < kSchedWaves; ++w) {
+            const int32_t v = sFold[w][lane & (kNumFold - 1)];
+            folded = (lane & (kNumFold - 1)) < kSumBad ? max(folded, v) : folded + v;
+        }
+        total_weight = readlane_t(row16_inclusive_scan(lane < kSchedWaves ? sWeight[lane] : int64_t(0)), 15);
+#pragma unroll
+        for (int q = 0; q < kNumFold; ++q) fold[q] = readlane_t(folded, q);
+    }
 
     if (tid == 0) {
         int64_t D1, D2, DO;
@@ -356,40 +412,37 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(SchedBatch batc
             if (a.a2) a.a2[nseg] = D2;
             if (a.aO) a.aO[nseg] = DO;
         }
-        int32_t rM = 0, rN = 0, rK = 0, rBad = 0, rSN = 0, rSM = 0, rInvN = 0, rInvK = 0;
-        int64_t total_weight = 0;
-        for (int w = 0; w < kSchedWaves; ++w) {
-            rM = max(rM, sRed[w][0]); rN = max(rN, sRed[w][1]); rK = max(rK, sRed[w][2]); rBad += sRed[w][3];
-            total_weight += sWeight[w];
-            rSN = max(rSN, sRed[w][4]); rSM = max(rSM, sRed[w][5]); rInvN = max(rInvN, sRed[w][6]); rInvK = max(rInvK, sRed[w][7]);
-        }
         PlanHeader *h = pv.hdr;
         h->magic = kPlanMagic;
         h->nseg = (int32_t)nseg;
         h->cap = (int32_t)plan_cap(nseg);
         h->kind = a.kind;
         h->Dm1 = D1; h->Dm2 = D2; h->Dout = DO;
-        h->total_rows = base32[kPfxRows];
-        for (int q = 0; q < 12; ++q) h->totals[q] = q < kNumPrefix ? base32[q] : 0;
-        h->max_M = rM; h->max_N = rN; h->max_K = rK;
-        h->small_max_N = rSN; h->small_max_M = rSM;
-        h->bad_segments = rBad + ((D1 < 0 || D2 < 0 || DO < 0) ? 1 : 0) + (total_weight >= (int64_t(1) << 31) ? 1 : 0);
+        h->total_rows = fold[kSumRows];
+#pragma unroll
+        for (int q = 0; q < kNumLists; ++q) h->totals[q] = base_bit[q];
+        h->totals[kPfxGemm] = fold[kSumGemm]; h->totals[kPfxStrip] = fold[kSumStrip]; h->totals[kPfxSplit] = fold[kSumSplit];
+        h->totals[kPfxWide] = fold[kSumWide]; h->totals[kPfxRows] = fold[kSumRows]; h->totals[kPfxPack] = fold[kSumPack];
+        h->totals[kPfxSlow] = fold[kSumSlow];
+        h->max_M = fold[kMaxM]; h->max_N = fold[kMaxN]; h->max_K = fold[kMaxK];
+        h->small_max_N = fold[kMaxSmallN]; h->small_max_M = fold[kMaxSmallM];
+        h->bad_segments = fold[kSumBad] + ((D1 < 0 || D2 < 0 || DO < 0) ? 1 : 0) + (total_weight >= (int64_t(1) << 31) ? 1 : 0);
         h->run_errors = 0;
-        const int32_t rows128 = (base32[kPfxAtt64] + base_two[kTwoOddRows]) >> 1, cols128 = (base32[kPfxAttCols] + base_two[kTwoOddCols]) >> 1;
-        h->att_blocks64 = base32[kPfxAtt64];
+        const int32_t rows128 = (base_rows + base_bit[kBitOddRows]) >> 1, cols128 = (base_cols + base_bit[kBitOddCols]) >> 1;
+        h->att_blocks64 = base_rows;
         h->att_blocks128 = rows128;
-        h->mini_count = base32[kPfxMini];
-        h->pipe_count = base_two[kTwoPipe];
-        h->att_cols64 = base32[kPfxAttCols];
+        h->mini_count = base_bit[kBitMini];
+        h->pipe_count = fold[kSumPipe];
+        h->att_cols64 = base_cols;
         h->att_cols128 = cols128;
         h->pipe_groups = 0;
-        h->min_N = rInvN ? INT32_MAX - rInvN : 0;
-        h->min_K = rInvK ? INT32_MAX - rInvK : 0;
+        h->min_N = fold[kMaxInvN] ? INT32_MAX - fold[kMaxInvN] : 0;
+        h->min_K = fold[kMaxInvK] ? INT32_MAX - fold[kMaxInvK] : 0;
         h->ring_groups = 0;
         h->wide_groups = 0;
-        plan_rowblocks(a.plan, nseg, 0)[nseg] = base32[kPfxAtt64];     // zero for softmax plans
+        plan_rowblocks(a.plan, nseg, 0)[nseg] = base_rows;             // zero for softmax plans
         plan_rowblocks(a.plan, nseg, 1)[nseg] = rows128;
-        plan_rowblocks(a.plan, nseg, 2)[nseg] = base32[kPfxAttCols];
+        plan_rowblocks(a.plan, nseg, 2)[nseg] = base_cols;
         plan_rowblocks(a.plan, nseg, 3)[nseg] = cols128;
         if (a.mailbox) {
             // the summary for a host that waits on the ticket instead of copying and synchronising: the header
@@ -421,18 +474,19 @@ static int schedule_args(SchedArgs &args, void *plan, size_t plan_bytes, int64_t
     return BA_OK;
 }
 
-static int launch_plans(const SchedBatch &args, unsigned plans, int64_t nseg, hipStream_t stream) {
-    if (nseg <= 64) hipLaunchKernelGGL(schedule_kernel<64>, dim3(plans), dim3(64), 0, stream, args);
-    else if (nseg <= 256) hipLaunchKernelGGL(schedule_kernel<256>, dim3(plans), dim3(256), 0, stream, args);
-    else if (nseg <= 512) hipLaunchKernelGGL(schedule_kernel<512>, dim3(plans), dim3(512), 0, stream, args);
-    else hipLaunchKernelGGL(schedule_kernel<kSchedThreadsMax>, dim3(plans), dim3(kSchedThreadsMax), 0, stream, args);
+template <typename Args>
+static int launch_plans(const Args &args, unsigned plans, int64_t nseg, hipStream_t stream) {
+    if (nseg <= 64) hipLaunchKernelGGL((schedule_kernel<64, Args>), dim3(plans), dim3(64), 0, stream, args);
+    else if (nseg <= 256) hipLaunchKernelGGL((schedule_kernel<256, Args>), dim3(plans), dim3(256), 0, stream, args);
+    else if (nseg <= 512) hipLaunchKernelGGL((schedule_kernel<512, Args>), dim3(plans), dim3(512), 0, stream, args);
+    else hipLaunchKernelGGL((schedule_kernel<kSchedThreadsMax, Args>), dim3(plans), dim3(kSchedThreadsMax), 0, stream, args);
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
 }
 
 int launch_schedule(void *plan, size_t plan_bytes, int64_t nseg, int mode, int kind, int64_t *M, int64_t *N,
                     int64_t *K, int64_t *a1, int64_t *a2, int64_t *aO, hipStream_t stream, void *mailbox, uint32_t ticket) {
-    SchedBatch args{};
-    const int st = schedule_args(args.plan[0], plan, plan_bytes, nseg, mode, kind, M, N, K, a1, a2, aO, mailbox, ticket);
+    SchedArgs args{};
+    const int st = schedule_args(args, plan, plan_bytes, nseg, mode, kind, M, N, K, a1, a2, aO, mailbox, ticket);
     return st != BA_OK ? st : launch_plans(args, 1, nseg, stream);
 }
 

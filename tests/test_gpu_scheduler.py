@@ -119,6 +119,38 @@ def test_more_segments_than_one_scheduler_pass(dev):
         assert info[k] == v, (k, info[k], v)
 
 
+@pytest.mark.parametrize("B", [1, 63, 64, 65, 256, 257, 512, 513, 1024, 1025, 2500])
+def test_lists_maxima_and_block_prefixes(dev, B):
+    """Each build of the scheduler at its edges: flags (ranks by ballot), totals folded at the end, the block prefixes."""
+    rng = np.random.default_rng(B)
+    M = rng.integers(0, 70, B); N = np.where(rng.random(B) < 0.1, rng.integers(257, 700, B), rng.integers(0, 200, B))
+    K = rng.choice([0, 8, 64, 61, 136], B)
+    M[B // 2], N[B // 2], K[B // 2] = 300, 301, 64
+    plan = make_plan(dev, M, N, K)
+    info = plan.info.as_dict()
+    both = (M >= 1) & (N >= 1)
+    blocks = {}
+    for i, (v, has) in enumerate(((M, M >= 1), (N, (N >= 1) & (K >= 1)))):
+        for j, rows in enumerate((64, 128)):
+            blocks[2 * i + j] = np.concatenate([[0], np.cumsum(np.where(has, -(-v // rows), 0))])
+    cap = (B + 4) & ~3
+    start = 256 + 6 * cap * 48                       # behind the header, the records and the five lists
+    got = plan.buf[start:start + 16 * (cap + 4)].view(torch.int32).cpu().numpy().reshape(4, cap + 4)[:, :B + 1]
+    for q in range(4):
+        assert np.array_equal(got[q], blocks[q]), q
+    want = dict(expected_items(M, N, K), list_rows=int(((M >= 1) & (N > 256)).sum()), att_blocks64=blocks[0][-1],
+                att_blocks128=blocks[1][-1], att_cols64=blocks[2][-1], max_M=M.max(), max_N=N.max(), max_K=K.max(),
+                min_N=N[both].min(), min_K=K[both].min(), bad_segments=0)
+    for k, v in want.items():
+        assert info[k] == v, (k, info[k], v)
+
+
+def test_columns_without_elements_are_accepted_in_any_number(dev):
+    M = np.zeros(1024, np.int64); N = np.full(1024, (1 << 30) - 1); K = M
+    info = make_plan(dev, M, N, K).info
+    assert info.bad_segments == 0 and info.att_cols64 == 0
+
+
 def test_bad_metadata_is_rejected_and_kernels_refuse_to_run(dev):
     M = dev_i64([4, -1, 3], dev); N = dev_i64([4, 2, 3], dev); K = dev_i64([8, 8, 8], dev)
     plan = capi.plan_gemm(3, dev, M, N, K, mode=capi.META_FROM_LISTS)
