@@ -74,11 +74,12 @@ __global__ __launch_bounds__(kSegThreads, ANY == kAnyKnown ? (MAXNT <= 8 ? 3 : 2
                 any_rows<DT, F32OUT, ANY == kAnyKnown ? MAXNT : kAnyUnknownTiles>(s, a, lds, base + wave * kStripRows);
             return;
         }
-    } else if (!mfma_ok || kind == kSegSlow) {
+    } else if (kind == kSegSlow) {
         // Element-wise path of the product alone.  The fused call gets this build if the summary counts no such segments:
         // one that is there all the same shows that the summary is another plan's, and is reported.
         if constexpr (!FUSED) {
-            for (int r = first; r < s.M; r += stride) generic_seg_rows<DT>(s, a, r, r + 1, 0, s.N);
+            for (int r = first; r < s.M; r += stride)
+                generic_rows<DT>((const uint16_t *)a.A + s.a, (const uint16_t *)a.B + s.b, a.out, s.o, s.N, s.K, r, r + 1);
         } else if (blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) {
             atomicAdd(&reinterpret_cast<PlanHeader *>(a.plan)->run_errors, 1);
         }

@@ -20,36 +20,25 @@ __device__ __forceinline__ u32x4 load_frag_fast(const uint16_t *__restrict__ row
 
 // ------------------------------------------------------------ generic rows
 // The product alone of segments the 16-byte operand loads cannot serve (K % 8
-// != 0, odd segment starts) where they are few among aligned ones: one wavefront
-// walks rows [r_begin, r_end), lanes own columns c_begin + lane + 64*j, fp32
-// multiply-add in k order.  Never inlined, so its registers do not add to the
-// MFMA paths.
-template <int DT> __device__ __forceinline__ float generic_dot(const uint16_t *__restrict__ aseg,
-                                                               const uint16_t *__restrict__ bseg, int r, int col,
-                                                               int M, int N, int K, bool t1, bool t2) {
-    float acc = 0.f;
-    for (int t = 0; t < K; ++t) {
-        const float av = Elem<DT>::to_float(t1 ? aseg[(int64_t)t * M + r] : aseg[(int64_t)r * K + t]);
-        const float bv = Elem<DT>::to_float(t2 ? bseg[(int64_t)t * N + col] : bseg[(int64_t)col * K + t]);
-        acc = fmaf(av, bv, acc);
-    }
-    return acc;
-}
-
+// != 0, odd segment starts) where they are few among aligned ones; transposed
+// operands never come here.  One wavefront walks rows [r_begin, r_end), lanes
+// own columns lane + 64*j, fp32 multiply-add in k order.  Never inlined, so its
+// registers do not add to the MFMA paths.
 template <int DT> __device__ __forceinline__ void store_one(void *out, int64_t e, float v, bool f32out) {
     if (f32out) reinterpret_cast<float *>(out)[e] = v;
     else reinterpret_cast<uint16_t *>(out)[e] = Elem<DT>::from_float(v);
 }
 
 template <int DT>
-__device__ __attribute__((noinline)) void generic_rows(const uint16_t *aseg, const uint16_t *bseg, void *out,
-                                                       int64_t o, int M, int N, int K, int r_begin, int r_end,
-                                                       int c_begin, int c_end, int flags) {
-    const int lane = lane_id();
-    const bool t1 = flags & kFlagTranspose1, t2 = flags & kFlagTranspose2;
+__device__ __attribute__((noinline)) void generic_rows(const uint16_t *__restrict__ aseg, const uint16_t *__restrict__ bseg, void *out,
+                                                       int64_t o, int N, int K, int r_begin, int r_end) {
     for (int r = r_begin; r < r_end; ++r)
-        for (int col = c_begin + lane; col < c_end; col += 64)
-            store_one<DT>(out, o + (int64_t)r * N + col, generic_dot<DT>(aseg, bseg, r, col, M, N, K, t1, t2), false);
+        for (int col = lane_id(); col < N; col += 64) {
+            float acc = 0.f;
+            for (int t = 0; t < K; ++t)
+                acc = fmaf(Elem<DT>::to_float(aseg[(int64_t)r * K + t]), Elem<DT>::to_float(bseg[(int64_t)col * K + t]), acc);
+            store_one<DT>(out, o + (int64_t)r * N + col, acc, false);
+        }
 }
 
 // ------------------------------------------------------------ local softmax
@@ -163,14 +152,6 @@ __device__ __forceinline__ void store_rows(const f32x4 (&acc)[kMaxTiles], int nt
             store_quad<DT, F32OUT>(out, e0 + t * 16, acc[t] * factor, rem - q * 4);
         }
     }
-}
-
-
-template <int DT>
-__device__ __forceinline__ void generic_seg_rows(const Seg &s, const RunArgs &a, int r_begin, int r_end,
-                                                 int c_begin, int c_end) {
-    generic_rows<DT>((const uint16_t *)a.A + s.a, (const uint16_t *)a.B + s.b, a.out, s.o, s.M, s.N, s.K, r_begin,
-                     min(r_end, s.M), c_begin, min(c_end, s.N), a.flags);
 }
 
 // ---------------------------------------------------------------- pack item
