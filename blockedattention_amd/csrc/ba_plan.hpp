@@ -54,7 +54,7 @@ enum PrefixKind {
     kListSmall = 0,  // strip-class segments for the strip kernel's main launch (<= kFastBlocks LDS blocks)
     kListBig = 1,    // strip-class segments for its second launch (<= kBigBlocks)
     kListTile = 2,   // segments of the tile kernel
-    kListRest = 3,   // everything else that has work: pack leaders, element-wise class, leftovers
+    kListRest = 3,   // everything else that has work: pack leaders, unaligned segments, leftovers
     kListRows = 4,   // segments of the softmax row kernel: N > kRunCols, any plan kind (independent of the four above)
     kNumLists = 5,
     kPfxGemm = 5,   // GEMM only, N > 256: ceil(M/16) * ceil(N/256) per segment
@@ -85,7 +85,8 @@ constexpr int kAttBlockRows = 64;   // rows or columns of the blocks that the ro
 // of 8 elements: every operand row then starts on a 16-byte boundary (given
 // 16-byte aligned base pointers and per-head strides that are multiples of 8).
 // Only aligned segments are counted in kPfxGemm/Strip/Split/Wide/Pack; the
-// others are counted in kPfxSlow and take the element-wise path.
+// others are counted in kPfxSlow and take any_rows (fused pair), the any-layout kernel or, few among aligned ones, the
+// element-wise rows (product alone).
 
 struct PlanHeader {
     uint32_t magic;

@@ -27,7 +27,7 @@ namespace ba {
 // ------------------------------------------------------------------ kernels
 // segment_kernel   grid (segment, head, z): one workgroup per segment and head;
 //                  its wavefronts take the segment's 16-row strips (N <= 256, or
-//                  any N where it is not aligned), the pack it leads, or its rows on the element-wise path.
+//                  any N where it is not aligned), the pack it leads, or its rows one by one (product alone).
 //                  No search: the block index is the segment.
 // gemm_large_kernel  GEMM only, N > 256: one wavefront per 16 x 256 piece, found
 //                  by a search in the scanned piece counts.
@@ -200,7 +200,7 @@ static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 //   strip kernel    strip-class segments whose B_g fits its LDS window (main launch: up to 32 KiB;
 //                   second launch: up to 64 KiB, fewer resident workgroups)
 //   tile kernel     large segments (see tile_segment())
-//   segment kernel  packs, the element-wise class, and what the others leave
+//   segment kernel  packs, unaligned segments, and what the others leave
 // With a host copy of the plan summary the grids are exactly the list lengths, empty lists are not
 // launched, and launches are merged where that saves one: the packs ride in the first strip launch
 // when the rest list holds nothing else, and a modest amount of tile-kernel work rides in the 64 KiB

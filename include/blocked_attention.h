@@ -68,7 +68,7 @@ typedef struct ba_plan_info {
     int64_t split_items;    /* 16-row strips with 256 < N <= 4096 */
     int64_t wide_items;     /* 16-row strips with N > 4096 */
     int64_t pack_items;     /* packs of tiny segments sharing one wavefront */
-    int64_t slow_items;     /* 16-row strips of segments that need the element-wise path */
+    int64_t slow_items;     /* 16-row strips of segments whose rows are not 16-byte aligned */
     int32_t max_M, max_N, max_K;
     int32_t bad_segments;   /* segments rejected by the device-side checks */
     int32_t run_errors;     /* kernels that refused to run against this plan */
@@ -76,7 +76,7 @@ typedef struct ba_plan_info {
     int32_t list_small;     /* strip kernel, main launch */
     int32_t list_big;       /* strip kernel, second launch with the 64 KiB window */
     int32_t list_tile;      /* tile kernel (large segments) */
-    int32_t list_rest;      /* segment kernel: packs, element-wise class, leftovers */
+    int32_t list_rest;      /* segment kernel: packs, unaligned segments, leftovers */
     int32_t small_max_N;    /* widest segment of the strip kernel's main launch */
     int32_t small_max_M;    /* tallest segment of the strip kernel's main launch */
     int32_t list_rows;      /* softmax row kernel: segments with N > 256 (GEMM and softmax plans) */
