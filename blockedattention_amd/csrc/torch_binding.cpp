@@ -27,6 +27,7 @@
 #include <mutex>
 
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
+#include <c10/core/InferenceMode.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
@@ -201,6 +202,8 @@ Schedule schedule_gemm(const Tensor &like, const OptTensor &a1, const OptTensor 
     Schedule s;
     const ScheduleKey key = make_key(0, like, {&a1, &a2, &aO, &M, &N, &K});
     if (use_cache && cache_lookup(key, s)) return s;
+    // A schedule made in inference mode may serve a call that saves its tensors for a backward pass.
+    c10::InferenceMode normal_tensors(false);
     s.derived = std::make_shared<Derived>();
     int64_t nseg;
     int mode;
@@ -275,6 +278,7 @@ Schedule schedule_softmax(const Tensor &like, const Tensor &rows, const Tensor &
     const OptTensor rows_o(rows), cols_o(cols), none;
     const ScheduleKey key = make_key(1, like, {&rows_o, &cols_o, &accum, &none, &none, &none});
     if (cache_lookup(key, s)) return s;
+    c10::InferenceMode normal_tensors(false);
     const int64_t nseg = rows.numel();
     check_meta(rows, "rowList", like, nseg); check_meta(cols, "colList", like, nseg);
     s.M = rows; s.N = cols;

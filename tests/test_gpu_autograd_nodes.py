@@ -165,3 +165,14 @@ def test_attention_result_overwritten(dev):
     with torch.no_grad():
         y.zero_()
     assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(y, ts, grad), want))
+
+
+@pytest.mark.parametrize("op", list(OPS))
+def test_metadata_first_seen_in_inference_mode(dev, op):
+    f, n = OPS[op]
+    want = gradients(dev, op)
+    m = meta(dev)
+    with torch.inference_mode():
+        f(*[t.detach() for t in operands(dev, n)], m)
+    for got, ref in zip(gradients(dev, op, m=m), want):          # the schedule kept from the first call
+        assert torch.equal(got, ref)
