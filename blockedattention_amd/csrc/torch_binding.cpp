@@ -86,6 +86,7 @@ struct Schedule;
 struct Derived {
     std::mutex mu;
     std::shared_ptr<Schedule> grad1, grad2;
+    Tensor summary;                                 // of this schedule, as the tensor that autograd nodes keep
 };
 
 struct Schedule {
@@ -245,6 +246,7 @@ Schedule schedule_gemm(const Tensor &like, const OptTensor &a1, const OptTensor 
             // the backward products' plans in the same launch (the same verdict and summaries as if made one by one)
             auto g1 = std::make_shared<Schedule>(), g2 = std::make_shared<Schedule>();
             g1->plan = at::empty_like(s.plan); g2->plan = at::empty_like(s.plan);
+            g1->derived = std::make_shared<Derived>(); g2->derived = std::make_shared<Derived>();
             check_status(ba_plan_gemm_train_notify(s.plan.data_ptr(), g1->plan.data_ptr(), g2->plan.data_ptr(), bytes, nseg,
                                                    mode, m, n, k, o1, o2, oO, mb.mem, ticket, stream),
                          "ba_plan_gemm_train_notify");
@@ -279,6 +281,7 @@ Schedule schedule_softmax(const Tensor &like, const Tensor &rows, const Tensor &
     const ScheduleKey key = make_key(1, like, {&rows_o, &cols_o, &accum, &none, &none, &none});
     if (cache_lookup(key, s)) return s;
     c10::InferenceMode normal_tensors(false);
+    s.derived = std::make_shared<Derived>();
     const int64_t nseg = rows.numel();
     check_meta(rows, "rowList", like, nseg); check_meta(cols, "colList", like, nseg);
     s.M = rows; s.N = cols;
@@ -347,19 +350,24 @@ Schedule &derived_schedule(const Schedule &s, std::shared_ptr<Schedule> Derived:
 
 // What an autograd node keeps of a schedule from its forward to its backward pass: two tensors, the plan and a copy of
 // its summary, saved like the operands (a capsule or raw bytes in the node's other data would shut it out of compiled
-// autograd, which hashes those).
+// autograd, which hashes those).  The copy is made once and shared by the nodes of the schedule.
 void keep_schedule(variable_list &saved, const Schedule &s) {
-    Tensor info = at::empty({(int64_t)sizeof(ba_plan_info)}, at::TensorOptions().dtype(at::kByte).device(at::kCPU));
-    memcpy(info.data_ptr(), &s.info, sizeof(ba_plan_info));
+    std::lock_guard<std::mutex> lock(s.derived->mu);
+    Tensor &summary = s.derived->summary;
+    if (!summary.defined()) {
+        c10::InferenceMode normal_tensors(false);
+        summary = at::empty({(int64_t)sizeof(ba_plan_info)}, at::TensorOptions().dtype(at::kByte).device(at::kCPU));
+        memcpy(summary.data_ptr(), &s.info, sizeof(ba_plan_info));
+    }
     saved.push_back(s.plan);
-    saved.push_back(info);
+    saved.push_back(summary);
 }
 // The schedule of saved[at] and saved[at + 1].  Saved-tensor hooks may have put them anywhere (a summary that comes back
 // on the GPU is copied once more); what is not a plan and its summary any longer is refused.
 Schedule kept_schedule(const variable_list &saved, size_t at, const Tensor &like) {
     Schedule s;
     s.plan = saved[at];
-    const Tensor info = saved[at + 1].to(at::kCPU);
+    const Tensor info = saved[at + 1].is_cpu() ? saved[at + 1] : saved[at + 1].to(at::kCPU);
     TORCH_CHECK(info.scalar_type() == at::kByte && info.is_contiguous() && info.numel() == (int64_t)sizeof(ba_plan_info),
                 "backward: the saved summary of the plan came back as ", info.toString(), info.sizes());
     memcpy(&s.info, info.data_ptr(), sizeof(ba_plan_info));
