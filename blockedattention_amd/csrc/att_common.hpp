@@ -39,6 +39,16 @@ __device__ __forceinline__ uint32_t lds_offset(const void *p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
 }
 
+// The operands that a wavefront keeps for a whole loop have arrived before the loop: without a use in front of it the
+// compiler waits for their loads at their first use inside, in every iteration, and there the wait is for the loads of
+// the next block, issued a moment before.
+template <int A, int B> __device__ __forceinline__ void arrived(u32x4 (&x)[A][B]) {
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+#pragma unroll
+        for (int k = 0; k < B; ++k) asm volatile("" : "+v"(x[i][k]));
+}
+
 // a * b + c for a, b below 2^24: one instruction
 __device__ __forceinline__ uint32_t mad24(uint32_t a, uint32_t b, uint32_t c) { return __umul24(a, b) + c; }
 

@@ -11,9 +11,10 @@
 // and dP are computed in both, seven products instead of five; adding dQ to memory from the second kernel instead
 // would move N / 128 times the size of dQ in fp32 atomics.
 //
-// Measured on 16 segments x 16 heads of 1024 .. 4096 rows, K = 128, bf16: dQ 1.37 ms (1.08 PFLOP/s over its three
-// products), dK and dV 2.10 ms (0.94 over four), 3.5 ms together against 9.3 ms of the chain; every operand read from LDS
-// feeds two matrix instructions, which puts the LDS port at 80 to 100 % of the matrix unit's rate: the next limit.
+// Measured on 16 segments x 16 heads of 1024 .. 4096 rows, K = 128, bf16: dQ 1.33 ms (1.11 PFLOP/s over its three
+// products), dK and dV 1.82 ms (1.08 over four), 3.15 ms together against 9.3 ms of the chain.  The clock falls to 2.0 GHz
+// under them; a 16 x 16 x 32 matrix instruction holds the issue port 8 of its 16 cycles, another vector instruction 4.3, an
+// exponential 8.4, and one operand read takes the LDS port 4 cycles (2.5 for half a transposing one).
 //
 // Operands lie in LDS as rows (one copy of each): a matrix operand whose reduction runs over the head dimension is read
 // 16 bytes per lane, one whose reduction runs over the rows by the transposing read (ds_read_b64_tr_b16).  The lane that
@@ -130,6 +131,8 @@ __device__ __forceinline__ void att_dq_body(const RunArgs &a, const AttBwdArgs &
 #pragma unroll
         for (int t = 0; t < kOutTiles; ++t) acc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
+    arrived(qf);
+    arrived(gf);
     const LdsPtr k_row = lds_ptr(sK) + j * kPitch + rg * 16, v_row = lds_ptr(sV) + j * kPitch + rg * 16;
     const LdsPtr k_col = lds_ptr(sK) + (4 * rg + (j >> 2)) * kPitch + (j & 3) * 8;
 
@@ -325,6 +328,7 @@ __device__ __forceinline__ void att_dkdv_body(const RunArgs &a, const AttBwdArgs
 #pragma unroll
         for (int t = 0; t < kOutTiles; ++t) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
+    arrived(kf);
     // this side's arrays: rows for the scores (Q / dO), columns for the sums (dO / Q)
     const LdsPtr row_base = lds_ptr(lds) + side * kArray + j * kPitch + rg * 16;
     const LdsPtr col_base = lds_ptr(lds) + (1 - side) * kArray + (4 * rg + (j >> 2)) * kPitch + (j & 3) * 8;
@@ -413,7 +417,254 @@ __device__ __forceinline__ void att_dkdv_body(const RunArgs &a, const AttBwdArgs
     }
 }
 
-constexpr int att_dkdv_lds(int nk, int pairs, int qb) { return 2 * (2 * qb * att_pitch(nk) + 8 * qb) + pairs * 64 * qb; }
+// The same for tall segments, eight wavefronts and one barrier a block: side 1 runs half a block behind side 0, so that on
+// every SIMD one wavefront's exponentials stand beside the other's matrix instructions, and neither waits inside a block
+// for what the other makes in it.  In iteration i
+//   side 0   P = 2^(c Q K^T - lse) of block i, packed, handed over; dV^T += dO^T P
+//   side 1   dS = P o (dP - delta) of block i - 1, dK^T += Q^T dS; then dP - delta = dO V^T - delta of block i, kept in registers
+// Three stages (blocks i - 1 and i are read while i + 1 is written), two buffers of the handed probabilities.
+// 16 x 16 pairs of 1024 .. 4096 rows, K = 128, bf16: two barriers a block, both sides in the same block 2.10 ms; one barrier
+// 2.07; LDS reads in flight across the phases 2.01; staging spread over the matrix instructions, delta as their starting
+// value 1.86; a loop for each side without branches in it 1.82.  An iteration takes 3400 cycles, of them 2048 of the
+// matrix unit; 13 % of the time are the ends of a workgroup, which has its compute unit alone.
+template <int DT, int NK, int PAIRS, int QB, bool VEC>
+__device__ __forceinline__ void att_dkdv_pipe_body(const RunArgs &a, const AttBwdArgs &w, const SegRec &rec, int64_t h,
+                                                   int64_t row0, int block, unsigned char *lds) {
+    constexpr int kThreads = 128 * PAIRS;
+    using St = AttStage<NK, kThreads, QB>;
+    constexpr int kTiles = QB / 16;
+    constexpr int kPitch = att_pitch(NK);
+    constexpr int kArray = QB * kPitch;          // bytes of one staged array
+    constexpr int kStage = 2 * kArray + 8 * QB;        // Q, dO, lse, delta
+    constexpr int kHand = 64 * QB;                     // bytes of a pair's probabilities
+    constexpr int kRing = 5;                           // operand reads in flight (the counter of outstanding reads has four bits)
+    constexpr int kOutTiles = 2 * NK;
+    static_assert(QB == 64 && PAIRS % 2 == 0);
+    const int M = rec.M, N = rec.N, K = rec.K;
+    const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = lane_id(), j = lane & 15, rg = lane >> 4;
+    const int side = wave / PAIRS, pair = wave % PAIRS;
+    const int64_t o1 = h * a.Dm1 + rec.off1, o2 = h * a.Dm2 + rec.off2;
+    const RowPieces<VEC> pq((const uint16_t *)a.A + o1, M, K), pg((const uint16_t *)w.dO + o1, M, K);
+    const RowPieces<VEC> pf((const uint16_t *)(side ? w.V : a.B) + o2, N, K);
+    const float c = a.scale * kLog2e;
+
+    // Staging: kPuts pieces a thread and block (Q and dO of kSteps rows); a piece's registers are written to LDS and loaded
+    // again for the block after the next in one place, and these places are spread over the matrix instructions: eight
+    // wavefronts that issue all their loads at once stand in front of the texture unit for 400 cycles an iteration.
+    const int s_row = tid / St::kLpr, s_piece = tid % St::kLpr;
+    const bool stages = (St::kLpr == St::kPieces || s_piece < St::kPieces) && (St::kRowsStep <= QB || s_row < QB);
+    constexpr int kPuts = 2 * St::kSteps;
+    u32x4 piece[kPuts];
+    float aux = 0.f;
+    auto fetch = [&](int x, int qb) {
+        const uint32_t off = pq.offset(qb + (x >> 1) * St::kRowsStep + s_row, s_piece);
+        piece[x] = x & 1 ? pg.load(off) : pq.load(off);
+    };
+    auto put = [&](int x, int qb, int stage) {
+        const int row = (x >> 1) * St::kRowsStep + s_row;
+        const uint32_t off = pq.offset(qb + row, s_piece);
+        const u32x4 done = x & 1 ? pg.finish(piece[x], off, s_piece) : pq.finish(piece[x], off, s_piece);
+        if (stages) *reinterpret_cast<u32x4 *>(lds + stage + (x & 1) * kArray + row * kPitch + s_piece * 16) = done;
+    };
+    // (per-query values: the wavefronts of side 0, those of odd number delta, the two halves of a side the same ones)
+    const int aux_row = tid & (QB - 1);
+    const bool aux_delta = wave & 1;
+    const __amdgpu_buffer_rsrc_t aux_res =
+        __builtin_amdgcn_make_buffer_rsrc((void *)((aux_delta ? w.delta : w.lse) + row0), 0, 4 * M, kRsrcFlags);
+    auto fetch_aux = [&](int qb) { aux = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(aux_res, 4 * (qb + aux_row), 0, 0)); };
+    auto put_aux = [&](int qb, int stage) {
+        // 2^-inf: rows that do not exist have no probabilities
+        const float x = aux_delta ? -aux : qb + aux_row < M ? aux : INFINITY;
+        *reinterpret_cast<float *>(lds + stage + 2 * kArray + (aux_delta ? 4 * QB : 0) + 4 * aux_row) = x;
+    };
+    static_for<kPuts>([&](auto xc) { fetch(decltype(xc)::value, 0); });
+    fetch_aux(0);
+
+    const int key0 = block * 32 * PAIRS + 32 * pair;
+    const bool alive = key0 < N;
+    u32x4 kf[2][NK];
+    f32x4 acc[kOutTiles][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int s = 0; s < NK; ++s) kf[u][s] = pf.get(key0 + 16 * u + j, 4 * s + rg);
+#pragma unroll
+        for (int t = 0; t < kOutTiles; ++t) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    arrived(kf);
+    // this side's arrays: rows for the scores (Q / dO), columns for the sums (dO / Q)
+    const uint32_t row_base = lds_offset(lds) + (uint32_t)(side * kArray + j * kPitch + rg * 16);
+    const uint32_t col_base = lds_offset(lds) + (uint32_t)((1 - side) * kArray + (4 * rg + (j >> 2)) * kPitch + (j & 3) * 8);
+    const uint32_t aux_base = lds_offset(lds) + (uint32_t)(2 * kArray + side * 4 * QB + rg * 16);
+    const uint32_t hand_base = lds_offset(lds) + (uint32_t)(3 * kStage + pair * kHand + lane * 16);   // kTiles 16-byte slots of 64 lanes a pair
+    f32x4 s[kTiles][2];
+    u32x4 pk[kTiles / 2][2];                           // [row tile pair][key tile]
+    u32x4 aux4[kTiles];                                // lse (side 0) or -delta (side 1) of the rows 16 t + 4 rg ..
+    // Two products a block, each a stream of LDS operand reads, kRing of them in flight; towards the end of a stream
+    // (kTail steps before it) the first reads of the next one are issued (`ahead`, kOps of them), so that it starts at once.
+    constexpr int kRows = NK * kTiles, kCols = (kTiles / 2) * kOutTiles, kTail = 3;
+    constexpr int kAheadR = kRing < kRows ? kRing : kRows, kAheadC = kRing < kCols ? kRing : kCols;
+    static_assert(2 * kTail + kTiles + kAheadR <= 15 && kTail + 2 * kAheadC <= 15);      // (the counter has four bits)
+    u32x4 ring[kRing];
+    u32x2 lo[kRing], hi[kRing];
+    auto read_aux = [&](int stage) {
+        static_for<kTiles>([&](auto tc) { lds_read128<64 * decltype(tc)::value>(aux4[decltype(tc)::value], aux_base + stage); });
+    };
+    auto rows_ahead = [&](int stage) {
+        static_for<kAheadR>([&](auto ic) {
+            constexpr int I = decltype(ic)::value;
+            lds_read128<16 * (I % kTiles) * kPitch + 64 * (I / kTiles)>(ring[I], row_base + stage);
+        });
+    };
+    auto cols_ahead = [&](int stage) {
+        static_for<kAheadC>([&](auto ic) {
+            constexpr int I = decltype(ic)::value;
+            lds_read_tr<32 * (I / kOutTiles) * kPitch + 32 * (I % kOutTiles), 16 * kPitch>(lo[I], hi[I], col_base + stage);
+        });
+    };
+    // scores of a stage's rows with the operand held in registers, from zero (side 0) or -delta (side 1) on
+    auto scores = [&](int stage, auto side_tag, auto &&between, auto ops, auto &&ahead) {
+        constexpr bool kDelta = decltype(side_tag)::value == 1;
+        const uint32_t at = row_base + stage;
+        static_for<kRows>([&](auto ic) {
+            constexpr int I = decltype(ic)::value, R = I % kRing, J = I + kRing, t = I % kTiles;
+            constexpr int kBehind = (J < kRows ? J : kRows) - (I + 1) + (I >= kRows - kTail ? decltype(ops)::value : 0);
+            if constexpr (I == kRows - kTail) ahead();
+            if constexpr (kDelta && I < kTiles) lds_wait<kBehind>(aux4[t]);
+            lds_wait<kBehind>(ring[R]);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const f32x4 from = I >= kTiles ? s[t][u] : kDelta ? __builtin_bit_cast(f32x4, aux4[t]) : f32x4{0.f, 0.f, 0.f, 0.f};
+                s[t][u] = Elem<DT>::mfma(ring[R], kf[u][I / kTiles], from);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (J < kRows) lds_read128<16 * (J % kTiles) * kPitch + 64 * (J / kTiles)>(ring[R], at);
+            between(ic, std::integral_constant<int, kRows>{});
+        });
+    };
+    // sums over a stage's rows
+    auto sums = [&](int stage, auto &&between, auto ops, auto &&ahead) {
+        const uint32_t at = col_base + stage;
+        static_for<kCols>([&](auto ic) {
+            constexpr int I = decltype(ic)::value, R = I % kRing, J = I + kRing;
+            constexpr int kBehind = 2 * ((J < kCols ? J : kCols) - (I + 1)) + (I >= kCols - kTail ? decltype(ops)::value : 0);
+            if constexpr (I == kCols - kTail) ahead();
+            lds_wait_tr<kBehind>(lo[R], hi[R]);
+            const u32x4 cf = u32x4{lo[R][0], lo[R][1], hi[R][0], hi[R][1]};
+#pragma unroll
+            for (int u = 0; u < 2; ++u) acc[I % kOutTiles][u] = Elem<DT>::mfma(cf, pk[I / kOutTiles][u], acc[I % kOutTiles][u]);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (J < kCols)
+                lds_read_tr<32 * (J / kOutTiles) * kPitch + 32 * (J % kOutTiles), 16 * kPitch>(lo[R], hi[R], at);
+            between(ic, std::integral_constant<int, kCols>{});
+        });
+    };
+    static_for<kPuts>([&](auto xc) { put(decltype(xc)::value, 0, 0); fetch(decltype(xc)::value, QB); });
+    if (side == 0) { put_aux(0, 0); fetch_aux(QB); }
+    att_lds_barrier();
+
+    // The three kinds of wavefronts have a loop each, one barrier a block.
+    const int blocks = (M + QB - 1) / QB;
+    int now = 0, before = 2 * kStage, next = kStage;   // stages of blocks i, i - 1 and i + 1
+    int i = 0;
+    // (past the last block: a stage that nobody reads, and loads of rows that do not exist)
+    auto exchange = [&](auto xc) {
+        put(decltype(xc)::value, (i + 1) * QB, next);
+        fetch(decltype(xc)::value, (i + 2) * QB);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto spread = [&](auto ic, auto reads) {           // exchange x behind step (x + 1) reads / kPuts - 1
+        constexpr int I = decltype(ic)::value, kEvery = decltype(reads)::value / kPuts;
+        static_assert(kEvery * kPuts == decltype(reads)::value);
+        if constexpr (I % kEvery == kEvery - 1) exchange(std::integral_constant<int, I / kEvery>{});
+    };
+    auto nothing = [](auto...) {};
+    constexpr std::integral_constant<int, 0> zero;
+    constexpr std::integral_constant<int, 1> one;
+    auto turn = [&]() {
+        att_lds_barrier();
+        const int was = before;
+        before = now; now = next; next = was;
+    };
+    auto aux_turn = [&]() { put_aux((i + 1) * QB, next); fetch_aux((i + 2) * QB); };
+    if (!alive) {
+        for (; i < blocks; ++i, turn()) {
+            static_for<kPuts>(exchange);
+            if (side == 0) aux_turn();
+        }
+    } else if (side == 0) {
+        for (; i < blocks; ++i, turn()) {
+            read_aux(now);
+            rows_ahead(now);
+            scores(now, zero, spread, std::integral_constant<int, 2 * kAheadC>{}, [&]() { cols_ahead(now); });
+            static_for<kTiles>([&](auto tc) {
+                constexpr int t = decltype(tc)::value;
+                lds_wait<15>(aux4[t]);                 // (read before the first operand)
+                const f32x4 l = __builtin_bit_cast(f32x4, aux4[t]);
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[t][u][e] = __builtin_amdgcn_exp2f(fmaf(s[t][u][e], c, -l[e]));
+                    pk[t >> 1][u][2 * (t & 1)] = Elem<DT>::pack2(s[t][u][0], s[t][u][1]);
+                    pk[t >> 1][u][2 * (t & 1) + 1] = Elem<DT>::pack2(s[t][u][2], s[t][u][3]);
+                }
+            });
+            unsigned char *hand = lds + 3 * kStage + pair * kHand + lane * 16 + (i & 1) * (PAIRS * kHand);
+#pragma unroll
+            for (int tt = 0; tt < kTiles / 2; ++tt)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) *reinterpret_cast<u32x4 *>(hand + (2 * tt + u) * 1024) = pk[tt][u];
+            sums(now, nothing, zero, nothing);
+            aux_turn();
+        }
+    } else {
+        auto handed = [&]() {                          // dS of block i - 1
+            const uint32_t hand = hand_base + (1 - (i & 1)) * (PAIRS * kHand);
+            static_for<kTiles>([&](auto tc) {
+                constexpr int t = decltype(tc)::value;
+                lds_read128<1024 * t>(pk[t >> 1][t & 1], hand);
+            });
+            cols_ahead(before);
+            static_for<kTiles>([&](auto tc) {          // slot t: row tiles 2 (t / 2) and the next, key tile t % 2
+                constexpr int t = decltype(tc)::value, tt = t >> 1, u = t & 1;
+                lds_wait<kTiles - 1 - t + 2 * kAheadC>(pk[tt][u]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const f32x4 &d = s[2 * tt + (e >> 1)][u];
+                    pk[tt][u][e] = Elem<DT>::pack2(lo16<DT>(pk[tt][u][e]) * d[2 * (e & 1)], hi16<DT>(pk[tt][u][e]) * d[2 * (e & 1) + 1]);
+                }
+            });
+        };
+        auto dp_ahead = [&]() { read_aux(now); rows_ahead(now); };
+        if (blocks > 0) {
+            dp_ahead();
+            scores(now, one, spread, zero, nothing);
+            ++i;
+            turn();
+            for (; i < blocks; ++i, turn()) {
+                handed();
+                sums(before, spread, std::integral_constant<int, kTiles + kAheadR>{}, dp_ahead);
+                scores(now, one, nothing, zero, nothing);
+            }
+            handed();
+            sums(before, nothing, zero, nothing);
+        }
+    }
+    uint16_t *out = (uint16_t *)(side ? w.dK : w.dV) + o2;
+    const float f = side ? a.scale : 1.0f;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int key = key0 + 16 * u + j;
+        if (key >= N) continue;
+#pragma unroll
+        for (int t = 0; t < kOutTiles; ++t) store4<DT>(out + (int64_t)key * K, 16 * t + 4 * rg, K, acc[t][u], f);
+    }
+}
+
+constexpr int att_dkdv_lds(int nk, int pairs, int qb) {
+    return (pairs == 4 ? 3 : 2) * (2 * qb * att_pitch(nk) + 8 * qb) + (pairs == 4 ? 2 : 1) * pairs * 64 * qb;
+}
+static_assert(att_dkdv_lds(4, 4, 64) <= 160 * 1024);
 
 // The build for short segments is bound by the life of a workgroup: three wavefronts per SIMD, not the two that its 197
 // registers at a head dimension of 128 would leave (30 of them spilled), 1024 x 4 pairs of 2 .. 512 rows: 133 -> 110 us.
@@ -431,8 +682,13 @@ __global__ __launch_bounds__(128 * PAIRS, QB == 32 ? 3 : 2) void attention_dkdv_
     const SegRec rec = load_rec(plan_ro(a.plan, a.nseg).recs, g);
     if (rec.N < 1 || rec.K < 1 || !att_fits(a, rec, 32 * NK, h, block)) return;
     const int64_t row0 = att_row_base(w.min_K, a.Dm1, h, rec.off1);
-    if ((rec.K & 7) == 0) att_dkdv_body<DT, NK, PAIRS, QB, true>(a, w, rec, h, row0, block, lds);
-    else att_dkdv_body<DT, NK, PAIRS, QB, false>(a, w, rec, h, row0, block, lds);
+    if constexpr (PAIRS == 4) {
+        if ((rec.K & 7) == 0) att_dkdv_pipe_body<DT, NK, PAIRS, QB, true>(a, w, rec, h, row0, block, lds);
+        else att_dkdv_pipe_body<DT, NK, PAIRS, QB, false>(a, w, rec, h, row0, block, lds);
+    } else {
+        if ((rec.K & 7) == 0) att_dkdv_body<DT, NK, PAIRS, QB, true>(a, w, rec, h, row0, block, lds);
+        else att_dkdv_body<DT, NK, PAIRS, QB, false>(a, w, rec, h, row0, block, lds);
+    }
 }
 
 template <int DT, int NK, int QT, int PAIRS, int QB>
@@ -468,8 +724,8 @@ int launch_attention_backward(int dtype, const RunArgs &args, const void *V, con
     const AttBwdArgs w{V, O, dO, lse, delta, dQ, dK, dV, info->min_K};
     const int nk = std::max(1, (info->max_K + 31) / 32);
     // Segments of 256 rows and more on average: wavefronts of two query strips, and workgroups of 128 keys that stage 64
-    // queries (16 x 16 pairs of 1024 .. 4096 rows: dK and dV 2.10 ms; 64 keys and 32 queries 2.78 ms, 128 keys and 32
-    // queries 2.44 ms: every query block is staged once per workgroup).  Shorter ones: 64 keys and 32 queries, two to
+    // queries, three stages of them (16 x 16 pairs of 1024 .. 4096 rows: dK and dV 1.82 ms; two stages 2.10 ms and there 64 keys
+    // and 32 queries 2.78 ms, 128 keys and 32 queries 2.44 ms: every query block is staged once per workgroup).  Shorter ones: 64 keys and 32 queries, two to
     // three times as many resident workgroups (1024 x 4 pairs of 2 .. 512 rows, at two wavefronts
     // per SIMD: 127 us; 64 queries 184 us, 128 keys 168 us).
     const bool tall = info->total_rows >= 256 * std::max<int64_t>(info->nseg, 1);

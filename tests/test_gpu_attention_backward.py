@@ -96,6 +96,14 @@ def test_tall_segments(dev, K, dtype):
     run(dev, [300, 520, 257], [130, 77, 1025], [K] * 3, 2, dtype, K ** -0.5, seed=7)
 
 
+@pytest.mark.parametrize("K", [24, 64, 96, 128, 101])
+def test_block_counts_beside_a_tall_segment(dev, K):
+    # 128 keys a workgroup, three stages of 64 queries: one, two, three and more blocks, full and ragged, and key blocks
+    # of which one to all four pairs of wavefronts have keys
+    M = [1, 63, 64, 65, 128, 129, 193, 1700]; N = [200, 31, 33, 127, 1, 128, 129, 96]
+    run(dev, M, N, [K] * 8, 2, torch.bfloat16, K ** -0.5, seed=K)
+
+
 def test_empty_segments(dev):
     # no queries: dk and dv are zeros; no keys: dq is zeros
     run(dev, [4, 0, 9, 30, 0], [6, 5, 0, 70, 300], [16, 8, 24, 64, 64], 2, torch.float16, 0.5)
