@@ -49,6 +49,9 @@ template <int A, int B> __device__ __forceinline__ void arrived(u32x4 (&x)[A][B]
         for (int k = 0; k < B; ++k) asm volatile("" : "+v"(x[i][k]));
 }
 
+// Barrier that waits for this wavefront's LDS traffic only (the loads of the next block stay in flight).
+__device__ __forceinline__ void att_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // a * b + c for a, b below 2^24: one instruction
 __device__ __forceinline__ uint32_t mad24(uint32_t a, uint32_t b, uint32_t c) { return __umul24(a, b) + c; }
 

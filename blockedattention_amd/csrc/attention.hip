@@ -45,7 +45,16 @@ static_assert(kAttRows == kAttBlockRows, "the plan's row-block prefixes count bl
 // life of a workgroup: head dimensions up to 64 then fit 128 registers and four wavefronts per SIMD (256 segments of
 // 32..128 rows, 31.3 -> 29.0 us), those up to 128 spill 7 registers instead of 17 at three wavefronts (512 pairs of
 // 16 .. 256 rows and columns, 22.2 -> 21.9 us)
-constexpr int att_ring(int nk, int qt) { return qt == 1 ? 3 : 6; }
+constexpr int att_ring(int nk, int qt) { return qt == 1 ? 3 : 4; }
+constexpr int att_stages(int qt) { return qt == 1 ? 1 : 2; }
+
+// Four accumulators times f, in place: as an assignment under a branch the compiler keeps a second copy of all of them.
+__device__ __forceinline__ void scale_in_place(f32x4 &x, float f) {
+    float a = x[0], b = x[1], c = x[2], d = x[3];
+    asm volatile("v_mul_f32 %0, %0, %4\n\tv_mul_f32 %1, %1, %4\n\tv_mul_f32 %2, %2, %4\n\tv_mul_f32 %3, %3, %4"
+                 : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : "v"(f));
+    x = f32x4{a, b, c, d};
+}
 
 // NK = 32-wide k steps (head dimension padded to 32 * NK).  VEC: the segment's K is a multiple of 8, its
 // rows come as 16-byte loads that need no clearing; otherwise through RowPieces (element by element before: 256 x 8
@@ -53,7 +62,7 @@ constexpr int att_ring(int nk, int qt) { return qt == 1 ? 3 : 6; }
 // separate instances of the whole body so that the clearing does not sit inside the fast path's loops.
 template <int DT, int NK, int QT, bool VEC, bool LSE>
 __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbuf, float *lse_rows, const SegRec &rec, int64_t h,
-                                               int zblock, unsigned char *sK, unsigned char *sV) {
+                                               int zblock, unsigned char *lds) {
     constexpr int KP = 32 * NK;                       // padded head dimension
     constexpr int kPitchK = KP * 2 + 32;              // bytes per LDS row of keys
     constexpr int kPieces = KP / 8;                   // 16-byte pieces per row
@@ -79,7 +88,11 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
     const uint32_t keep = c_signed == 0.f ? 0u : 0xffffffffu;
     const u32x4 zero4 = u32x4{0u, 0u, 0u, 0u};
 
-    // Staging, per thread: kSteps 16-byte pieces of the key rows and of the value rows (kLpr neighbouring lanes share
+    // Staging: one LDS stage for one strip per wavefront; two for two strips, where a block's pieces are written and loaded
+    // again one by one between the matrix instructions of the block before (see below).
+    constexpr int kStages = att_stages(QT);
+    constexpr int kStageBytes = kAttKeys * kPitchK, kValues = kStages * kStageBytes;      // keys' stages, then values' stages
+    // Per thread: kSteps 16-byte pieces of the key rows and of the value rows (kLpr neighbouring lanes share
     // a row; step s takes rows s * kRowsStep ..).  Element offsets inside a segment fit 32 bits (checked by the kernel).
     constexpr int kLpr = NK == 3 ? 16 : kPieces;      // lanes per row (a power of two; 12 pieces: 4 lanes idle)
     constexpr int kSteps = kLpr / 4, kRowsStep = kAttThreads / kLpr;
@@ -97,8 +110,8 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
 
     // operand reads: lane (j, rg) reads 16 bytes of key row 16 t + j at k = 32 s + 8 rg; of the values it addresses four
     // columns of key 4 rg + j / 4 and receives column j of the lane group's four keys
-    const uint32_t k_addr = lds_offset(sK) + (uint32_t)(j * kPitchK + rg * 16);
-    const uint32_t v_addr = lds_offset(sV) + (uint32_t)((4 * rg + (j >> 2)) * kPitchK + (j & 3) * 8);
+    const uint32_t k_addr = lds_offset(lds) + (uint32_t)(j * kPitchK + rg * 16);
+    const uint32_t v_addr = lds_offset(lds) + (uint32_t)(kValues + (4 * rg + (j >> 2)) * kPitchK + (j & 3) * 8);
 
     constexpr int kRoundRows = kAttRows * QT;           // queries per workgroup round
     for (int round = zblock; (int64_t)round * kRoundRows < M; round += a.ride_slots ? (1 << 24) : a.tile_zdim) {
@@ -134,59 +147,108 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
             for (int t = 0; t < kOutTiles; ++t) oacc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
 
-        // The loads run one block ahead of the arithmetic: the loads of block kb + 64 are issued before the
-        // matrix work on block kb and land in registers (kw, vw: this thread's pieces of the key and value
-        // rows) while that work runs.  All loads of a block sit in one branch-free
-        // sequence (index clamped, value selected afterwards): loads behind a branch wait one by one.
-        u32x4 kw[kSteps], vw[kSteps];
-        uint32_t k_byte = k_byte0;
-        auto fetch = [&](int kb) {                     // called for kb = 0, 64, 128, .. in turn
-            if constexpr (VEC) {
-#pragma unroll
-                for (int step = 0; step < kSteps; ++step) {
-                    const uint32_t off = mad24(k_live, (uint32_t)(step * kRowsStep) * row_bytes, k_byte);
-                    kw[step] = __builtin_amdgcn_raw_buffer_load_b128(resK, off, 0, 0);
-                    vw[step] = __builtin_amdgcn_raw_buffer_load_b128(resV, off, 0, 0);
-                }
-                k_byte = mad24(k_live, (uint32_t)kAttKeys * row_bytes, k_byte);
-            } else {
-#pragma unroll
-                for (int step = 0; step < kSteps; ++step) {
-                    const uint32_t off = pk.offset(kb + step * kRowsStep + k_row, k_piece);
-                    kw[step] = pk.load(off);
-                    vw[step] = pv.load(off);
-                }
-            }
+        // The loads run ahead of the arithmetic and land in registers while it runs.  One stage: the loads of block kb + 64
+        // (kw, vw: this thread's pieces of the key and value rows) are issued before the matrix work on block kb; they sit
+        // in one branch-free sequence (index clamped, value selected afterwards): loads behind a branch wait one by one.
+        // Two stages: one barrier a block, and the pieces take turns in one set of registers (kw).  Between the score
+        // products of block kb the value pieces of block kb + 64 go to the other stage and its key pieces are requested;
+        // between the value products these go there and the value pieces of block kb + 128 are requested.
+        u32x4 kw[kSteps], vw[kStages == 1 ? kSteps : 1];
+        uint32_t k_byte = k_byte0;                     // of the block that is loaded next
+        auto offset = [&](auto step_tag, int kb) {
+            constexpr int step = decltype(step_tag)::value;
+            if constexpr (VEC) return mad24(k_live, (uint32_t)(step * kRowsStep) * row_bytes, k_byte);
+            else return pk.offset(kb + step * kRowsStep + k_row, k_piece);
         };
+        auto load_k = [&](uint32_t off) { return VEC ? __builtin_amdgcn_raw_buffer_load_b128(resK, off, 0, 0) : pk.load(off); };
+        auto load_v = [&](uint32_t off) { return VEC ? __builtin_amdgcn_raw_buffer_load_b128(resV, off, 0, 0) : pv.load(off); };
+        auto advance = [&]() { k_byte = mad24(k_live, (uint32_t)kAttKeys * row_bytes, k_byte); };
         // what the loads of block kb brought -> pieces with zeros past the head dimension and past the last key
         // (values: their probabilities are zeros too, but 0 * stale bits could be NaN)
-        auto finish = [&](int kb) {
-            if constexpr (!VEC) {
-#pragma unroll
-                for (int step = 0; step < kSteps; ++step) {
-                    const uint32_t off = pk.offset(kb + step * kRowsStep + k_row, k_piece);
-                    kw[step] = pk.finish(kw[step], off, k_piece);
-                    vw[step] = pv.finish(vw[step], off, k_piece);
-                }
-            }
+        auto finish = [&](auto step_tag, int kb, u32x4 x) {
+            if constexpr (VEC) return x;
+            else return pk.finish(x, pk.offset(kb + decltype(step_tag)::value * kRowsStep + k_row, k_piece), k_piece);
         };
-        if (N > 0) fetch(0);
-
-        for (int kb = 0; kb < N; kb += kAttKeys) {
-            finish(kb);
-            __syncthreads();                           // the previous block (or round) is consumed
-            // ---- one 16-byte piece per thread, array and step, pieces of a row on neighbouring lanes
-            if (kLpr == kPieces || k_piece < kPieces) {
-#pragma unroll
-                for (int step = 0; step < kSteps; ++step) {
-                    const int at = (step * kRowsStep + k_row) * kPitchK + k_piece * 16;
-                    *reinterpret_cast<u32x4 *>(sK + at) = kw[step];
-                    *reinterpret_cast<u32x4 *>(sV + at) = vw[step];
-                }
+        const bool puts = kLpr == kPieces || k_piece < kPieces;
+        unsigned char *const put_at = lds + k_row * kPitchK + k_piece * 16;
+        auto put = [&](auto step_tag, int array, u32x4 x) {
+            if (puts) *reinterpret_cast<u32x4 *>(put_at + array + decltype(step_tag)::value * (kRowsStep * kPitchK)) = x;
+        };
+        int stage = 0;
+        if constexpr (kStages == 2) {
+            if (round != zblock) att_lds_barrier();    // the previous round is consumed
+            if (N > 0) {
+                u32x4 first[kSteps];
+                static_for<kSteps>([&](auto sc) {
+                    const uint32_t off = offset(sc, 0);
+                    kw[decltype(sc)::value] = load_k(off);
+                    first[decltype(sc)::value] = load_v(off);
+                });
+                advance();
+                static_for<kSteps>([&](auto sc) {
+                    constexpr int step = decltype(sc)::value;
+                    put(sc, 0, finish(sc, 0, kw[step]));
+                    put(sc, kValues, finish(sc, 0, first[step]));
+                    kw[step] = load_v(offset(sc, kAttKeys));
+                });
             }
-            __syncthreads();
-            if (kb + kAttKeys < N) fetch(kb + kAttKeys);
-            if (nq == 0) continue;
+            att_lds_barrier();
+        } else if (N > 0) {
+            static_for<kSteps>([&](auto sc) {
+                const uint32_t off = offset(sc, 0);
+                kw[decltype(sc)::value] = load_k(off);
+                vw[decltype(sc)::value] = load_v(off);
+            });
+            advance();
+        }
+
+        int kb = 0;
+        // (past the last block: a stage that nobody reads, rows that do not exist)
+        auto exchange_v = [&](auto sc) {
+            constexpr int step = decltype(sc)::value;
+            put(sc, kStageBytes - stage + kValues, finish(sc, kb + kAttKeys, kw[step]));
+            kw[step] = load_k(offset(sc, kb + kAttKeys));
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto exchange_k = [&](auto sc) {
+            constexpr int step = decltype(sc)::value;
+            put(sc, kStageBytes - stage, finish(sc, kb + kAttKeys, kw[step]));
+            kw[step] = load_v(offset(sc, kb + 2 * kAttKeys));
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if (kStages == 2 && nq == 0) {                 // the wavefront only stages (a loop of its own: in one with the
+            for (; kb < N; kb += kAttKeys) {           // arithmetic the accumulators would be copied where they meet)
+                static_for<kSteps>(exchange_v);
+                advance();
+                static_for<kSteps>(exchange_k);
+                stage = kStageBytes - stage;
+                att_lds_barrier();
+            }
+        }
+        for (; kb < N; kb += kAttKeys) {
+            if constexpr (kStages == 1) {
+                static_for<kSteps>([&](auto sc) {
+                    constexpr int step = decltype(sc)::value;
+                    kw[step] = finish(sc, kb, kw[step]);
+                    vw[step] = finish(sc, kb, vw[step]);
+                });
+                __syncthreads();                       // the previous block (or round) is consumed
+                // ---- one 16-byte piece per thread, array and step, pieces of a row on neighbouring lanes
+                static_for<kSteps>([&](auto sc) {
+                    put(sc, 0, kw[decltype(sc)::value]);
+                    put(sc, kValues, vw[decltype(sc)::value]);
+                });
+                __syncthreads();
+                if (kb + kAttKeys < N) {
+                    static_for<kSteps>([&](auto sc) {
+                        const uint32_t off = offset(sc, kb + kAttKeys);
+                        kw[decltype(sc)::value] = load_k(off);
+                        vw[decltype(sc)::value] = load_v(off);
+                    });
+                    advance();
+                }
+                if (nq == 0) continue;
+            }
             // The arithmetic on one block for NQ live strips, as straight-line code: a branch around every
             // matrix instruction of a strip that may be missing would keep the scheduler from interleaving them.
             auto block_math = [&](auto nq_tag) {
@@ -198,11 +260,12 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
     #pragma unroll
                     for (int t = 0; t < 4; ++t) sacc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
                 u32x4 ring[kAttRing];
+                const uint32_t k_at = k_addr + (kStages == 2 ? stage : 0), v_at = v_addr + (kStages == 2 ? stage : 0);
                 {
                     constexpr int kReads = 4 * NK;         // read i: k step i / 4, key tile i % 4
                     static_for<kAttRing>([&](auto ic) {
                         constexpr int I = decltype(ic)::value;
-                        if constexpr (I < kReads) lds_read128<16 * (I % 4) * kPitchK + 64 * (I / 4)>(ring[I], k_addr);
+                        if constexpr (I < kReads) lds_read128<16 * (I % 4) * kPitchK + 64 * (I / 4)>(ring[I], k_at);
                     });
                     static_for<kReads>([&](auto ic) {
                         constexpr int I = decltype(ic)::value, R = I % kAttRing;
@@ -210,9 +273,26 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                         lds_wait<kBehind>(ring[R]);
     #pragma unroll
                         for (int q = 0; q < NQ; ++q) sacc[q][I % 4] = Elem<DT>::mfma(ring[R], qf[q][I / 4], sacc[q][I % 4]);
+                        if constexpr (kStages == 2) __builtin_amdgcn_sched_barrier(0);
                         if constexpr (I + kAttRing < kReads)
-                            lds_read128<16 * ((I + kAttRing) % 4) * kPitchK + 64 * ((I + kAttRing) / 4)>(ring[R], k_addr);
+                            lds_read128<16 * ((I + kAttRing) % 4) * kPitchK + 64 * ((I + kAttRing) / 4)>(ring[R], k_at);
+                        constexpr int kEvery = kReads / kSteps;
+                        static_assert(kEvery * kSteps == kReads);
+                        if constexpr (kStages == 2 && I % kEvery == kEvery - 1) exchange_v(std::integral_constant<int, I / kEvery>{});
                     });
+                }
+                constexpr int kValueReads = 2 * kOutTiles; // read i: key half i / kOutTiles, output tile i % kOutTiles
+                u32x2 lo[kAttRing], hi[kAttRing];          // keys 4 rg .. + 3 of the half's two key tiles
+                auto values_ahead = [&]() {
+                    static_for<kAttRing>([&](auto ic) {
+                        constexpr int I = decltype(ic)::value;
+                        if constexpr (I < kValueReads)
+                            lds_read_tr<32 * (I / kOutTiles) * kPitchK + 32 * (I % kOutTiles), 16 * kPitchK>(lo[I], hi[I], v_at);
+                    });
+                };
+                if constexpr (kStages == 2) {
+                    advance();
+                    values_ahead();                        // in flight under the softmax
                 }
                 // ---- online softmax; lane holds keys kb + 16 t + 4 rg + e of query j of each strip
                 const int left = N - kb;                   // keys of this block that exist
@@ -223,10 +303,11 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                     // keys past the segment's last: -inf, so that they neither raise the maximum nor count
                     // (their exponentials are zeros)
                     if (left < kAttKeys) {
+                        const int mine = left - 4 * rg;    // (compared with constants: no registers for 16 key numbers)
     #pragma unroll
                         for (int t = 0; t < 4; ++t)
     #pragma unroll
-                            for (int e = 0; e < 4; ++e) sc[t][e] = 16 * t + 4 * rg + e < left ? sc[t][e] : -INFINITY;
+                            for (int e = 0; e < 4; ++e) sc[t][e] = 16 * t + e < mine ? sc[t][e] : -INFINITY;
                     }
                     settle_mfma(sc);                       // max3 reads the scores from inline assembly
                     float bm;                              // one statement: no padding between its instructions
@@ -260,8 +341,9 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                         }
                     lsum[q] = fmaf(lsum[q], alpha, psum);
                     if (__any(raise)) {
+                        // (the matrix instructions that wrote the accumulators are a whole score product away)
     #pragma unroll
-                        for (int t = 0; t < kOutTiles; ++t) oacc[q][t] *= alpha;
+                        for (int t = 0; t < kOutTiles; ++t) scale_in_place(oacc[q][t], alpha);
                     }
                     // probabilities as B operand, 32 keys per step: k = 8 rg + kk is key 32 cc + 4 rg + kk (kk < 4)
                     // or 32 cc + 16 + 4 rg + kk - 4: what the lane holds in sc[2 cc] and sc[2 cc + 1]
@@ -273,31 +355,33 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                 }
                 // ---- O^T += V^T P^T; a value operand read serves every strip
                 {
-                    constexpr int kReads = 2 * kOutTiles;  // read i: key half i / kOutTiles, output tile i % kOutTiles
-                    u32x2 lo[kAttRing], hi[kAttRing];      // keys 4 rg .. + 3 of the half's two key tiles
-                    static_for<kAttRing>([&](auto ic) {
-                        constexpr int I = decltype(ic)::value;
-                        if constexpr (I < kReads)
-                            lds_read_tr<32 * (I / kOutTiles) * kPitchK + 32 * (I % kOutTiles), 16 * kPitchK>(lo[I], hi[I], v_addr);
-                    });
-                    static_for<kReads>([&](auto ic) {
-                        constexpr int I = decltype(ic)::value, R = I % kAttRing;
-                        constexpr int kBehind = (I + kAttRing < kReads ? I + kAttRing : kReads) - (I + 1);
-                        lds_wait_tr<2 * kBehind>(lo[R], hi[R]);
+                    if constexpr (kStages == 1) values_ahead();
+                    static_for<kValueReads>([&](auto ic) {
+                        constexpr int I = decltype(ic)::value, R = I % kAttRing, J = I + kAttRing;
+                        lds_wait_tr<2 * ((J < kValueReads ? J : kValueReads) - (I + 1))>(lo[R], hi[R]);
                         const u32x4 v = u32x4{lo[R][0], lo[R][1], hi[R][0], hi[R][1]};
     #pragma unroll
                         for (int q = 0; q < NQ; ++q)
                             oacc[q][I % kOutTiles] = Elem<DT>::mfma(v, pf[q][I / kOutTiles], oacc[q][I % kOutTiles]);
-                        if constexpr (I + kAttRing < kReads)
-                            lds_read_tr<32 * ((I + kAttRing) / kOutTiles) * kPitchK + 32 * ((I + kAttRing) % kOutTiles), 16 * kPitchK>(
-                                lo[R], hi[R], v_addr);
+                        if constexpr (kStages == 2) __builtin_amdgcn_sched_barrier(0);
+                        if constexpr (J < kValueReads)
+                            lds_read_tr<32 * (J / kOutTiles) * kPitchK + 32 * (J % kOutTiles), 16 * kPitchK>(lo[R], hi[R], v_at);
+                        constexpr int kEvery = kValueReads / kSteps;
+                        static_assert(kEvery * kSteps == kValueReads);
+                        if constexpr (kStages == 2 && I % kEvery == kEvery - 1) exchange_k(std::integral_constant<int, I / kEvery>{});
                     });
                 }
             };
-            if (QT == 1 || nq == 1) block_math(std::integral_constant<int, 1>{});
-            else block_math(std::integral_constant<int, QT>{});
+            block_math(std::integral_constant<int, QT>{});
+            if constexpr (kStages == 2) {
+                stage = kStageBytes - stage;
+                att_lds_barrier();
+            }
         }
         // ---- normalise and store: lane (query j, rg) holds columns 16 t + 4 rg + e.  No key at all: zeros.
+        // (column numbers made here: taken out of the loop over the rounds they would hold registers through the blocks)
+        int own = 4 * rg;
+        asm volatile("" : "+v"(own));
 #pragma unroll
         for (int q = 0; q < QT; ++q) {
             if (q >= nq) continue;
@@ -310,7 +394,7 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                 uint16_t *orow = os + (int64_t)qr * K;
 #pragma unroll
                 for (int t = 0; t < kOutTiles; ++t) {
-                    const int c0 = 16 * t + 4 * rg;
+                    const int c0 = 16 * t + own;
                     if (c0 + 4 <= K) {
                         *reinterpret_cast<u32x2_unaligned *>(orow + c0) =
                             u32x2{Elem<DT>::pack2(oacc[q][t][0] * inv, oacc[q][t][1] * inv),
@@ -331,8 +415,7 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
 template <int DT, int NK, int QT, bool LSE>
 __global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void attention_kernel(RunArgs a, const void *Vbuf, float *lse, int min_K) {
     constexpr int KP = 32 * NK;
-    __shared__ __attribute__((aligned(16))) unsigned char sK[kAttKeys * (KP * 2 + 32)];
-    __shared__ __attribute__((aligned(16))) unsigned char sV[kAttKeys * (KP * 2 + 32)];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * att_stages(QT) * kAttKeys * (KP * 2 + 32)];
     // (the row blocks per head come with the header: one memory round trip less than the prefix's last entry)
     const int64_t per_head = QT == 2 ? ((ConstHdr)(uintptr_t)a.plan)->att_blocks128 : ((ConstHdr)(uintptr_t)a.plan)->att_blocks64;
     // (lse is sized by the min_K of the host's summary)
@@ -382,8 +465,8 @@ __global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void at
         return;
     }
     float *lse_rows = LSE ? lse + att_row_base(min_K, a.Dm1, h, rec.off1) : nullptr;
-    if ((K & 7) == 0) attention_body<DT, NK, QT, true, LSE>(a, Vbuf, lse_rows, rec, h, zblock, sK, sV);
-    else attention_body<DT, NK, QT, false, LSE>(a, Vbuf, lse_rows, rec, h, zblock, sK, sV);
+    if ((K & 7) == 0) attention_body<DT, NK, QT, true, LSE>(a, Vbuf, lse_rows, rec, h, zblock, lds);
+    else attention_body<DT, NK, QT, false, LSE>(a, Vbuf, lse_rows, rec, h, zblock, lds);
 }
 
 template <int DT, int QT, bool LSE>

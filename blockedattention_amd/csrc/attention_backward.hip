@@ -40,9 +40,6 @@ __device__ __forceinline__ u32x4 lds_col8(LdsPtr p, int off, int next) {
     const u32x2 h = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((Ptr)(p + off + next)));
     return u32x4{l[0], l[1], h[0], h[1]};
 }
-// Barrier that waits for this wavefront's LDS traffic only (the loads of the next block stay in flight).
-__device__ __forceinline__ void att_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 template <int DT> __device__ __forceinline__ float lo16(uint32_t w) { return Elem<DT>::to_float((uint16_t)w); }
 template <int DT> __device__ __forceinline__ float hi16(uint32_t w) { return Elem<DT>::to_float((uint16_t)(w >> 16)); }
 
