@@ -41,12 +41,11 @@ static_assert(kAttRows == kAttBlockRows, "the plan's row-block prefixes count bl
 // a time, 512 bytes wide (measured: lane * 16 and 288-byte rows run at 4.75 cycles per wavefront read, 272- and
 // 144-byte rows at 8): the lanes (j, rg) and (j, rg + 1) of sixteen rows j must land in 32 different 16-byte slots
 // modulo 512 bytes, which a pitch of 16 * (2 * odd) bytes does; the transposing reads meet no conflict there either.
-// LDS operand reads in flight per wavefront: six, or three in the builds for short segments, which are bound by the
-// life of a workgroup: head dimensions up to 64 then fit 128 registers and four wavefronts per SIMD (256 segments of
-// 32..128 rows, 31.3 -> 29.0 us), those up to 128 spill 7 registers instead of 17 at three wavefronts (512 pairs of
-// 16 .. 256 rows and columns, 22.2 -> 21.9 us)
-constexpr int att_ring(int nk, int qt) { return qt == 1 ? 3 : 4; }
-constexpr int att_stages(int qt) { return qt == 1 ? 1 : 2; }
+// LDS operand reads in flight per wavefront: six; four with two stages, whose registers hold no more; three in the builds
+// for short segments, which are bound by the life of a workgroup: head dimensions up to 64 then fit 128 registers and
+// four wavefronts per SIMD (256 segments of 32..128 rows, 31.3 -> 29.0 us), those up to 128 spill less at three
+// wavefronts (512 pairs of 16 .. 256 rows and columns, 22.2 -> 21.9 us)
+constexpr int att_ring(int qt, int stages) { return qt == 1 ? 3 : stages == 1 ? 6 : 4; }
 
 // Four accumulators times f, in place: as an assignment under a branch the compiler keeps a second copy of all of them.
 __device__ __forceinline__ void scale_in_place(f32x4 &x, float f) {
@@ -56,18 +55,19 @@ __device__ __forceinline__ void scale_in_place(f32x4 &x, float f) {
     x = f32x4{a, b, c, d};
 }
 
-// NK = 32-wide k steps (head dimension padded to 32 * NK).  VEC: the segment's K is a multiple of 8, its
-// rows come as 16-byte loads that need no clearing; otherwise through RowPieces (element by element before: 256 x 8
-// pairs of 32 .. 128 rows, K = 61: 103 -> 48 us; 16 x 8 pairs of 512 .. 2048, K = 101: 764 -> 279 us).  The two are
-// separate instances of the whole body so that the clearing does not sit inside the fast path's loops.
-template <int DT, int NK, int QT, bool VEC, bool LSE>
+// NK = 32-wide k steps (head dimension padded to 32 * NK).  ST = LDS stages (the rule: launch_attention).  VEC: the
+// segment's K is a multiple of 8, its rows come as 16-byte loads that need no clearing; otherwise through RowPieces
+// (element by element before: 256 x 8 pairs of 32 .. 128 rows, K = 61: 103 -> 48 us; 16 x 8 pairs of 512 .. 2048, K = 101:
+// 764 -> 279 us).  The two are separate instances of the whole body so that the clearing does not sit inside the fast
+// path's loops.
+template <int DT, int NK, int QT, int ST, bool VEC, bool LSE>
 __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbuf, float *lse_rows, const SegRec &rec, int64_t h,
                                                int zblock, unsigned char *lds) {
     constexpr int KP = 32 * NK;                       // padded head dimension
     constexpr int kPitchK = KP * 2 + 32;              // bytes per LDS row of keys
     constexpr int kPieces = KP / 8;                   // 16-byte pieces per row
     constexpr int kOutTiles = KP / 16;
-    constexpr int kAttRing = att_ring(NK, QT);
+    constexpr int kAttRing = att_ring(QT, ST);
     const int M = rec.M, N = rec.N, K = rec.K;
     const int tid = threadIdx.x;
     const int wave = uniform(tid >> 6);
@@ -88,10 +88,9 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
     const uint32_t keep = c_signed == 0.f ? 0u : 0xffffffffu;
     const u32x4 zero4 = u32x4{0u, 0u, 0u, 0u};
 
-    // Staging: one LDS stage for one strip per wavefront; two for two strips, where a block's pieces are written and loaded
-    // again one by one between the matrix instructions of the block before (see below).
-    constexpr int kStages = att_stages(QT);
-    constexpr int kStageBytes = kAttKeys * kPitchK, kValues = kStages * kStageBytes;      // keys' stages, then values' stages
+    // Staging: ST LDS stages.  With two, a block's pieces are written and loaded again one by one between the matrix
+    // instructions of the block before (see below).
+    constexpr int kStageBytes = kAttKeys * kPitchK, kValues = ST * kStageBytes;      // keys' stages, then values' stages
     // Per thread: kSteps 16-byte pieces of the key rows and of the value rows (kLpr neighbouring lanes share
     // a row; step s takes rows s * kRowsStep ..).  Element offsets inside a segment fit 32 bits (checked by the kernel).
     constexpr int kLpr = NK == 3 ? 16 : kPieces;      // lanes per row (a power of two; 12 pieces: 4 lanes idle)
@@ -153,7 +152,7 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
         // Two stages: one barrier a block, and the pieces take turns in one set of registers (kw).  Between the score
         // products of block kb the value pieces of block kb + 64 go to the other stage and its key pieces are requested;
         // between the value products these go there and the value pieces of block kb + 128 are requested.
-        u32x4 kw[kSteps], vw[kStages == 1 ? kSteps : 1];
+        u32x4 kw[kSteps], vw[ST == 1 ? kSteps : 1];
         uint32_t k_byte = k_byte0;                     // of the block that is loaded next
         auto offset = [&](auto step_tag, int kb) {
             constexpr int step = decltype(step_tag)::value;
@@ -175,7 +174,7 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
             if (puts) *reinterpret_cast<u32x4 *>(put_at + array + decltype(step_tag)::value * (kRowsStep * kPitchK)) = x;
         };
         int stage = 0;
-        if constexpr (kStages == 2) {
+        if constexpr (ST == 2) {
             if (round != zblock) att_lds_barrier();    // the previous round is consumed
             if (N > 0) {
                 u32x4 first[kSteps];
@@ -216,7 +215,7 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
             kw[step] = load_v(offset(sc, kb + 2 * kAttKeys));
             __builtin_amdgcn_sched_barrier(0);
         };
-        if (kStages == 2 && nq == 0) {                 // the wavefront only stages (a loop of its own: in one with the
+        if (ST == 2 && nq == 0) {                 // the wavefront only stages (a loop of its own: in one with the
             for (; kb < N; kb += kAttKeys) {           // arithmetic the accumulators would be copied where they meet)
                 static_for<kSteps>(exchange_v);
                 advance();
@@ -226,7 +225,7 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
             }
         }
         for (; kb < N; kb += kAttKeys) {
-            if constexpr (kStages == 1) {
+            if constexpr (ST == 1) {
                 static_for<kSteps>([&](auto sc) {
                     constexpr int step = decltype(sc)::value;
                     kw[step] = finish(sc, kb, kw[step]);
@@ -260,7 +259,7 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
     #pragma unroll
                     for (int t = 0; t < 4; ++t) sacc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
                 u32x4 ring[kAttRing];
-                const uint32_t k_at = k_addr + (kStages == 2 ? stage : 0), v_at = v_addr + (kStages == 2 ? stage : 0);
+                const uint32_t k_at = k_addr + (ST == 2 ? stage : 0), v_at = v_addr + (ST == 2 ? stage : 0);
                 {
                     constexpr int kReads = 4 * NK;         // read i: k step i / 4, key tile i % 4
                     static_for<kAttRing>([&](auto ic) {
@@ -273,12 +272,12 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                         lds_wait<kBehind>(ring[R]);
     #pragma unroll
                         for (int q = 0; q < NQ; ++q) sacc[q][I % 4] = Elem<DT>::mfma(ring[R], qf[q][I / 4], sacc[q][I % 4]);
-                        if constexpr (kStages == 2) __builtin_amdgcn_sched_barrier(0);
+                        if constexpr (ST == 2) __builtin_amdgcn_sched_barrier(0);
                         if constexpr (I + kAttRing < kReads)
                             lds_read128<16 * ((I + kAttRing) % 4) * kPitchK + 64 * ((I + kAttRing) / 4)>(ring[R], k_at);
                         constexpr int kEvery = kReads / kSteps;
                         static_assert(kEvery * kSteps == kReads);
-                        if constexpr (kStages == 2 && I % kEvery == kEvery - 1) exchange_v(std::integral_constant<int, I / kEvery>{});
+                        if constexpr (ST == 2 && I % kEvery == kEvery - 1) exchange_v(std::integral_constant<int, I / kEvery>{});
                     });
                 }
                 constexpr int kValueReads = 2 * kOutTiles; // read i: key half i / kOutTiles, output tile i % kOutTiles
@@ -290,7 +289,7 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                             lds_read_tr<32 * (I / kOutTiles) * kPitchK + 32 * (I % kOutTiles), 16 * kPitchK>(lo[I], hi[I], v_at);
                     });
                 };
-                if constexpr (kStages == 2) {
+                if constexpr (ST == 2) {
                     advance();
                     values_ahead();                        // in flight under the softmax
                 }
@@ -343,7 +342,10 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                     if (__any(raise)) {
                         // (the matrix instructions that wrote the accumulators are a whole score product away)
     #pragma unroll
-                        for (int t = 0; t < kOutTiles; ++t) scale_in_place(oacc[q][t], alpha);
+                        for (int t = 0; t < kOutTiles; ++t) {
+                            if constexpr (ST == 2) scale_in_place(oacc[q][t], alpha);
+                            else oacc[q][t] *= alpha;
+                        }
                     }
                     // probabilities as B operand, 32 keys per step: k = 8 rg + kk is key 32 cc + 4 rg + kk (kk < 4)
                     // or 32 cc + 16 + 4 rg + kk - 4: what the lane holds in sc[2 cc] and sc[2 cc + 1]
@@ -355,7 +357,7 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                 }
                 // ---- O^T += V^T P^T; a value operand read serves every strip
                 {
-                    if constexpr (kStages == 1) values_ahead();
+                    if constexpr (ST == 1) values_ahead();
                     static_for<kValueReads>([&](auto ic) {
                         constexpr int I = decltype(ic)::value, R = I % kAttRing, J = I + kAttRing;
                         lds_wait_tr<2 * ((J < kValueReads ? J : kValueReads) - (I + 1))>(lo[R], hi[R]);
@@ -363,17 +365,19 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
     #pragma unroll
                         for (int q = 0; q < NQ; ++q)
                             oacc[q][I % kOutTiles] = Elem<DT>::mfma(v, pf[q][I / kOutTiles], oacc[q][I % kOutTiles]);
-                        if constexpr (kStages == 2) __builtin_amdgcn_sched_barrier(0);
+                        if constexpr (ST == 2) __builtin_amdgcn_sched_barrier(0);
                         if constexpr (J < kValueReads)
                             lds_read_tr<32 * (J / kOutTiles) * kPitchK + 32 * (J % kOutTiles), 16 * kPitchK>(lo[R], hi[R], v_at);
                         constexpr int kEvery = kValueReads / kSteps;
                         static_assert(kEvery * kSteps == kValueReads);
-                        if constexpr (kStages == 2 && I % kEvery == kEvery - 1) exchange_k(std::integral_constant<int, I / kEvery>{});
+                        if constexpr (ST == 2 && I % kEvery == kEvery - 1) exchange_k(std::integral_constant<int, I / kEvery>{});
                     });
                 }
             };
-            block_math(std::integral_constant<int, QT>{});
-            if constexpr (kStages == 2) {
+            // (two stages: a strip that does not exist is computed along, a second body would not fit the registers)
+            if (ST == 1 && QT == 2 && nq == 1) block_math(std::integral_constant<int, 1>{});
+            else block_math(std::integral_constant<int, QT>{});
+            if constexpr (ST == 2) {
                 stage = kStageBytes - stage;
                 att_lds_barrier();
             }
@@ -381,7 +385,7 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
         // ---- normalise and store: lane (query j, rg) holds columns 16 t + 4 rg + e.  No key at all: zeros.
         // (column numbers made here: taken out of the loop over the rounds they would hold registers through the blocks)
         int own = 4 * rg;
-        asm volatile("" : "+v"(own));
+        if constexpr (ST == 2) asm volatile("" : "+v"(own));
 #pragma unroll
         for (int q = 0; q < QT; ++q) {
             if (q >= nq) continue;
@@ -412,10 +416,10 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
 
 // LSE: the build for training, which also writes the rows' sums (as a run-time choice it cost the plain one 2 % on 512
 // segments of 16 .. 256 rows and columns: 23.1 -> 23.6 us).
-template <int DT, int NK, int QT, bool LSE>
+template <int DT, int NK, int QT, int ST, bool LSE>
 __global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void attention_kernel(RunArgs a, const void *Vbuf, float *lse, int min_K) {
     constexpr int KP = 32 * NK;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * att_stages(QT) * kAttKeys * (KP * 2 + 32)];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * ST * kAttKeys * (KP * 2 + 32)];
     // (the row blocks per head come with the header: one memory round trip less than the prefix's last entry)
     const int64_t per_head = QT == 2 ? ((ConstHdr)(uintptr_t)a.plan)->att_blocks128 : ((ConstHdr)(uintptr_t)a.plan)->att_blocks64;
     // (lse is sized by the min_K of the host's summary)
@@ -465,25 +469,25 @@ __global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void at
         return;
     }
     float *lse_rows = LSE ? lse + att_row_base(min_K, a.Dm1, h, rec.off1) : nullptr;
-    if ((K & 7) == 0) attention_body<DT, NK, QT, true, LSE>(a, Vbuf, lse_rows, rec, h, zblock, lds);
-    else attention_body<DT, NK, QT, false, LSE>(a, Vbuf, lse_rows, rec, h, zblock, lds);
+    if ((K & 7) == 0) attention_body<DT, NK, QT, ST, true, LSE>(a, Vbuf, lse_rows, rec, h, zblock, lds);
+    else attention_body<DT, NK, QT, ST, false, LSE>(a, Vbuf, lse_rows, rec, h, zblock, lds);
 }
 
-template <int DT, int QT, bool LSE>
+template <int DT, int QT, int ST, bool LSE>
 static void launch_nk(int nk, dim3 grid, hipStream_t stream, const RunArgs &args, const void *V, float *lse, int min_K) {
     // args.ride_slots = 1: work items from the plan's row-block prefix; else args.tile_zdim = row blocks per
     // (segment, head) pair, tile_groups = pairs per die
-    switch (nk) {
-        case 1: hipLaunchKernelGGL((attention_kernel<DT, 1, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
-        case 2: hipLaunchKernelGGL((attention_kernel<DT, 2, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
-        case 3: hipLaunchKernelGGL((attention_kernel<DT, 3, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
-        default: hipLaunchKernelGGL((attention_kernel<DT, 4, QT, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
+    switch (nk) {                                      // (two stages: never with nk = 1)
+        case 1: hipLaunchKernelGGL((attention_kernel<DT, 1, QT, 1, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
+        case 2: hipLaunchKernelGGL((attention_kernel<DT, 2, QT, ST, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
+        case 3: hipLaunchKernelGGL((attention_kernel<DT, 3, QT, ST, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
+        default: hipLaunchKernelGGL((attention_kernel<DT, 4, QT, ST, LSE>), grid, dim3(kAttThreads), 0, stream, args, V, lse, min_K); break;
     }
 }
-template <int DT, int QT>
+template <int DT, int QT, int ST>
 static void launch_build(int nk, dim3 grid, hipStream_t stream, const RunArgs &args, const void *V, float *lse, int min_K) {
-    if (lse) launch_nk<DT, QT, true>(nk, grid, stream, args, V, lse, min_K);
-    else launch_nk<DT, QT, false>(nk, grid, stream, args, V, lse, min_K);
+    if (lse) launch_nk<DT, QT, ST, true>(nk, grid, stream, args, V, lse, min_K);
+    else launch_nk<DT, QT, ST, false>(nk, grid, stream, args, V, lse, min_K);
 }
 
 // Strips per wavefront: two where segments are tall (each operand read from LDS then feeds two matrix
@@ -503,6 +507,12 @@ int launch_attention(int dtype, const RunArgs &args, const void *V, float *lse, 
         if (info->total_rows >= 256 * std::max<int64_t>(nseg, 1)) qt = 2;   // mean segment height >= 256 (136: one strip is 6 % faster)
     }
     if (forced == 1 || forced == 2) qt = forced;
+    // LDS stages for two strips.  Two keep the matrix unit busier in the steady state (16 x 16 segments of 1024 .. 4096,
+    // K = 128, 1068 -> 1037 us; 48 x 4 of 1000 .. 2000, K = 64, 184 -> 173; of 600 .. 900, K = 128, 90 -> 83), but the first
+    // block waits for its successor's values and a missing strip is computed along: with 507 keys per query (the mean over
+    // the queries) 34.0 -> 32.9 us at K = 64 and 50.8 -> 48.3 at K = 128, with 311 18.1 -> 20.1 and 27.1 -> 28.8.  At K <= 32
+    // there are too few matrix instructions to hide an exchange behind (1000 .. 2000: 117 -> 121 us).
+    const bool deep = qt == 2 && nk > 1 && info && info->Dout >= 400 * info->total_rows;
     // Row blocks per pair: enough for the tallest segment, but no more than four times what the mean segment
     // needs (a workgroup takes every Z-th block of its pair; blocks that do not exist cost a launch each).
     const int64_t round_rows = kAttRows * qt;
@@ -529,8 +539,14 @@ int launch_attention(int dtype, const RunArgs &args, const void *V, float *lse, 
         run.tile_groups = (int)pairs8;
         grid = flat_grid(pairs8 * z * 8);
     }
-    if (dtype == BA_F16) { if (qt == 2) launch_build<0, 2>(nk, grid, stream, run, V, lse, min_K); else launch_build<0, 1>(nk, grid, stream, run, V, lse, min_K); }
-    else { if (qt == 2) launch_build<1, 2>(nk, grid, stream, run, V, lse, min_K); else launch_build<1, 1>(nk, grid, stream, run, V, lse, min_K); }
+    auto build = [&](auto dt) {
+        constexpr int DT = decltype(dt)::value;
+        if (qt == 1) launch_build<DT, 1, 1>(nk, grid, stream, run, V, lse, min_K);
+        else if (deep) launch_build<DT, 2, 2>(nk, grid, stream, run, V, lse, min_K);
+        else launch_build<DT, 2, 1>(nk, grid, stream, run, V, lse, min_K);
+    };
+    if (dtype == BA_F16) build(std::integral_constant<int, 0>{});
+    else build(std::integral_constant<int, 1>{});
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
 }
 

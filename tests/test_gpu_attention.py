@@ -114,6 +114,15 @@ def test_long_segments_many_key_blocks(dev):
     run(dev, [70], [2000], [64], 1, torch.float16, 1.0, sigma=2.0, seed=3)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K", [40, 64, 96, 128, 101])
+def test_two_stages_block_edges(dev, K, dtype):
+    # more than 400 keys per query and tall segments: two LDS stages.  One key, one, two and three blocks, full and ragged;
+    # rounds in which one to all four wavefronts have queries, one strip or two
+    M = [513, 300, 640, 257, 130, 400]; N = [2000, 1, 449, 64, 129, 192]
+    run(dev, M, N, [K] * 6, 2, dtype, K ** -0.5, seed=K)
+
+
 @pytest.mark.parametrize("seed", [11, 12, 13, 14])
 def test_random_batches(dev, seed):
     # random batches: segment counts, heights, widths and head dimensions drawn anew (multiples of 8 or anything),
