@@ -11,8 +11,8 @@
 // and dP are computed in both, seven products instead of five; adding dQ to memory from the second kernel instead
 // would move N / 128 times the size of dQ in fp32 atomics.
 //
-// Measured on 16 segments x 16 heads of 1024 .. 4096 rows, K = 128, bf16: dQ 1.33 ms (1.11 PFLOP/s over its three
-// products), dK and dV 1.82 ms (1.08 over four), 3.15 ms together against 9.3 ms of the chain.  The clock falls to 2.0 GHz
+// Measured on 16 segments x 16 heads of 1024 .. 4096 rows, K = 128, bf16: dQ 1.24 ms (1.19 PFLOP/s over its three
+// products), dK and dV 1.82 ms (1.08 over four), 3.06 ms together against 9.3 ms of the chain.  The clock falls to 2.0 GHz
 // under them; a 16 x 16 x 32 matrix instruction holds the issue port 8 of its 16 cycles, another vector instruction 4.3, an
 // exponential 8.4, and one operand read takes the LDS port 4 cycles (2.5 for half a transposing one).
 //
@@ -215,6 +215,193 @@ __device__ __forceinline__ void att_dq_body(const RunArgs &a, const AttBwdArgs &
     }
 }
 
+// The same for two strips a wavefront and many keys: two LDS stages and one barrier a block.  Each half of a block is one
+// stream of operand reads, kRing of them in flight across its three products (and into the next half); the exponentials
+// stand between the matrix instructions of dP, and the pieces of the next block are written, and those of the block after
+// it requested, between all of them: its values during the first half, its keys during the second, in one set of registers.
+// Before, staging stood between two barriers a block and every product began with an LDS round trip.  16 x 16 pairs of
+// 1024 .. 4096 rows, K = 128, bf16: 1378 -> 1241 us a launch; forward and backward 4104 -> 4025..4081 (the other kernels
+// clock lower then), of 24 x 4 pairs of 1000 .. 2000 634 -> 610, of 48 x 4 of 200 .. 400 104 -> 101, K = 64 79 -> 78.
+template <int DT, int NK, bool VEC>
+__device__ __forceinline__ void att_dq_pipe_body(const RunArgs &a, const AttBwdArgs &w, const SegRec &rec, int64_t h, int64_t row0,
+                                                 int block, unsigned char *lds) {
+    using St = AttStage<NK, 256>;
+    constexpr int QT = 2;
+    constexpr int kPitch = att_pitch(NK);
+    constexpr int kArray = kAttKeys * kPitch, kStage = 2 * kArray;       // keys, then values
+    constexpr int kOutTiles = 2 * NK;
+    constexpr int kRing = 4, kTail = 3;
+    const int M = rec.M, N = rec.N, K = rec.K;
+    const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = lane_id(), j = lane & 15, rg = lane >> 4;
+    const int64_t o1 = h * a.Dm1 + rec.off1, o2 = h * a.Dm2 + rec.off2;
+    const RowPieces<VEC> pq((const uint16_t *)a.A + o1, M, K), pg((const uint16_t *)w.dO + o1, M, K), po((const uint16_t *)w.O + o1, M, K);
+    const RowPieces<VEC> pk((const uint16_t *)a.B + o2, N, K), pv((const uint16_t *)w.V + o2, N, K);
+    const float c = a.scale * kLog2e;
+
+    const int s_row = tid / St::kLpr, s_piece = tid % St::kLpr;
+    const bool stages = St::kLpr == St::kPieces || s_piece < St::kPieces;
+    u32x4 piece[St::kSteps];
+    auto offset = [&](int s, int kb) { return pk.offset(kb + s * St::kRowsStep + s_row, s_piece); };
+    auto put = [&](int s, int kb, int at, u32x4 x) {
+        x = pk.finish(x, offset(s, kb), s_piece);
+        if (stages) *reinterpret_cast<u32x4 *>(lds + at + (s * St::kRowsStep + s_row) * kPitch + s_piece * 16) = x;
+    };
+    {
+        u32x4 values[St::kSteps];
+#pragma unroll
+        for (int s = 0; s < St::kSteps; ++s) {
+            piece[s] = pk.load(offset(s, 0));
+            values[s] = pv.load(offset(s, 0));
+        }
+#pragma unroll
+        for (int s = 0; s < St::kSteps; ++s) {
+            put(s, 0, 0, piece[s]);
+            put(s, 0, kArray, values[s]);
+            piece[s] = pv.load(offset(s, kAttKeys));
+        }
+    }
+    const int r0 = block * kAttBlockRows * QT + wave * 16;
+    u32x4 qf[QT][NK], gf[QT][NK];
+    float lse[QT], delta[QT];
+    f32x4 acc[QT][kOutTiles];
+#pragma unroll
+    for (int q = 0; q < QT; ++q) {
+        const int row = r0 + kAttBlockRows * q + j;
+        float d = 0.f;
+#pragma unroll
+        for (int s = 0; s < NK; ++s) {
+            qf[q][s] = pq.get(row, 4 * s + rg);
+            gf[q][s] = pg.get(row, 4 * s + rg);
+            const u32x4 of = po.get(row, 4 * s + rg);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                d = fmaf(lo16<DT>(gf[q][s][i]), lo16<DT>(of[i]), d);
+                d = fmaf(hi16<DT>(gf[q][s][i]), hi16<DT>(of[i]), d);
+            }
+        }
+        delta[q] = quad_column_sum(d);
+        lse[q] = row < M && N > 0 ? w.lse[row0 + row] : INFINITY;        // 2^-inf: rows that do not exist have no probabilities
+        if (row < M && N > 0 && rg == 0) w.delta[row0 + row] = delta[q];
+#pragma unroll
+        for (int t = 0; t < kOutTiles; ++t) acc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    arrived(qf);
+    arrived(gf);
+    att_lds_barrier();
+
+    int kb = 0, stage = 0;
+    // (past the last block: a stage that nobody reads, and loads of rows that do not exist)
+    auto exchange = [&](auto sc, auto half_tag) {
+        constexpr int s = decltype(sc)::value, H0 = decltype(half_tag)::value;
+        put(s, kb + kAttKeys, (kStage - stage) + (H0 ? 0 : kArray), piece[s]);
+        piece[s] = H0 ? pv.load(offset(s, kb + 2 * kAttKeys)) : pk.load(offset(s, kb + kAttKeys));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr std::integral_constant<int, 0> first;
+    constexpr std::integral_constant<int, 1> second;
+    auto turn = [&]() {
+        stage = kStage - stage;
+        att_lds_barrier();
+    };
+    if (r0 >= M) {                                     // the wavefront only stages
+        for (; kb < N; kb += kAttKeys, turn()) {
+            static_for<St::kSteps>([&](auto sc) { exchange(sc, first); });
+            static_for<St::kSteps>([&](auto sc) { exchange(sc, second); });
+        }
+        return;
+    }
+    const uint32_t row_base = lds_offset(lds) + (uint32_t)(j * kPitch + rg * 16);
+    const uint32_t col_base = lds_offset(lds) + (uint32_t)((4 * rg + (j >> 2)) * kPitch + (j & 3) * 8);
+    constexpr int kRows = 4 * NK, kCols = kOutTiles, kSteps = kRows + kCols;
+    constexpr int kAheadC = kRing < kCols ? kRing : kCols;
+    static_assert(kTail + 2 * kAheadC <= 15 && 2 * kTail + kRing <= 15);  // (the counter of outstanding reads has four bits)
+    u32x4 ring[kRing];
+    u32x2 lo[kRing], hi[kRing];
+    // read I of half H0: scores (key row tiles 2 H0 and the next, step by step), then dP (value rows)
+    auto read_row = [&](auto ic, auto half_tag) {
+        constexpr int I = decltype(ic)::value, H0 = decltype(half_tag)::value;
+        lds_read128<(I >= 2 * NK ? kArray : 0) + 16 * (2 * H0 + I % 2) * kPitch + 64 * (I % (2 * NK) / 2)>(ring[I % kRing], row_base + stage);
+    };
+    auto read_col = [&](auto ic, auto half_tag) {
+        constexpr int I = decltype(ic)::value, H0 = decltype(half_tag)::value;
+        lds_read_tr<32 * H0 * kPitch + 32 * I, 16 * kPitch>(lo[I % kRing], hi[I % kRing], col_base + stage);
+    };
+    auto half = [&](auto half_tag, int left) {         // (a strip whose rows do not exist runs along: one code path)
+        constexpr int H0 = decltype(half_tag)::value;
+        f32x4 s[QT][2], dp[QT][2];
+        auto spread = [&](auto ic) {                   // the half's exchanges, evenly behind its steps
+            constexpr int I = decltype(ic)::value, now = I * St::kSteps / kSteps, then = (I + 1) * St::kSteps / kSteps;
+            if constexpr (then > now) exchange(std::integral_constant<int, now>{}, half_tag);
+        };
+        static_for<kRows>([&](auto ic) {
+            constexpr int I = decltype(ic)::value, R = I % kRing, J = I + kRing, t = I % 2, st = I % (2 * NK) / 2;
+            constexpr int kBehind = (J < kRows ? J : kRows) - (I + 1) + (I >= kRows - kTail ? 2 * kAheadC : 0);
+            if constexpr (I == kRows - kTail) static_for<kAheadC>([&](auto xc) { read_col(xc, half_tag); });
+            lds_wait<kBehind>(ring[R]);
+#pragma unroll
+            for (int q = 0; q < QT; ++q) {
+                if constexpr (I < 2 * NK) s[q][t] = Elem<DT>::mfma(ring[R], qf[q][st], st ? s[q][t] : f32x4{0.f, 0.f, 0.f, 0.f});
+                else dp[q][t] = Elem<DT>::mfma(ring[R], gf[q][st], st ? dp[q][t] : f32x4{-delta[q], -delta[q], -delta[q], -delta[q]});
+            }
+            // (from the second step of dP on: the scores have left the matrix unit)
+            if constexpr (I > 2 * NK) {
+                constexpr int kParts = 2 * NK - 1, from = (I - 2 * NK - 1) * 16 / kParts, to = (I - 2 * NK) * 16 / kParts;
+                static_for<to - from>([&](auto xc) {
+                    constexpr int x = from + decltype(xc)::value, tt = x / 8, q = x / 4 % 2, e = x % 4;
+                    s[q][tt][e] = __builtin_amdgcn_exp2f(fmaf(s[q][tt][e], c, -lse[q]));
+                });
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (J < kRows) read_row(std::integral_constant<int, (J < kRows ? J : 0)>{}, half_tag);
+            spread(ic);
+        });
+        if (left < kAttKeys) {                         // keys past the last one (their scores are zeros, lse may be anything)
+            const int mine = left - 4 * rg;
+#pragma unroll
+            for (int q = 0; q < QT; ++q)
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[q][t][e] = 16 * (2 * H0 + t) + e < mine ? s[q][t][e] : 0.f;
+        }
+        u32x4 ds[QT];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int q = 0; q < QT; ++q) {
+                ds[q][2 * t] = Elem<DT>::pack2(s[q][t][0] * dp[q][t][0], s[q][t][1] * dp[q][t][1]);
+                ds[q][2 * t + 1] = Elem<DT>::pack2(s[q][t][2] * dp[q][t][2], s[q][t][3] * dp[q][t][3]);
+            }
+        static_for<kCols>([&](auto ic) {
+            constexpr int I = decltype(ic)::value, R = I % kRing, J = I + kRing;
+            constexpr int kBehind = 2 * ((J < kCols ? J : kCols) - (I + 1)) + (H0 == 0 && I >= kCols - kTail ? kRing : 0);
+            if constexpr (H0 == 0 && I == kCols - kTail) static_for<kRing>([&](auto xc) { read_row(xc, second); });
+            lds_wait_tr<kBehind>(lo[R], hi[R]);
+            const u32x4 kc = u32x4{lo[R][0], lo[R][1], hi[R][0], hi[R][1]};
+#pragma unroll
+            for (int q = 0; q < QT; ++q) acc[q][I] = Elem<DT>::mfma(kc, ds[q], acc[q][I]);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (J < kCols) read_col(std::integral_constant<int, (J < kCols ? J : 0)>{}, half_tag);
+            spread(std::integral_constant<int, kRows + I>{});
+        });
+    };
+    for (; kb < N; kb += kAttKeys, turn()) {
+        const int left = N - kb;
+        static_for<kRing>([&](auto xc) { read_row(xc, first); });
+        half(first, left);
+        if (left > 32) half(second, left);
+        else static_for<kRing>([&](auto xc) { lds_wait<0>(ring[decltype(xc)::value]); });     // (what was read for it)
+    }
+    uint16_t *dq = (uint16_t *)w.dQ + o1;
+#pragma unroll
+    for (int q = 0; q < QT; ++q) {
+        const int row = r0 + kAttBlockRows * q + j;
+        if (row >= M) continue;
+#pragma unroll
+        for (int t = 0; t < kOutTiles; ++t) store4<DT>(dq + (int64_t)row * K, 16 * t + 4 * rg, K, acc[q][t], a.scale);
+    }
+}
+
 // Work item of a workgroup: item u of the (head, segment, block) items, head-major, cut into eight contiguous shares, one
 // per die (as in attention_kernel: the blocks of a pair read the same rows and run side by side on one die).
 // prefix: blocks of the segments before each segment; per_head: all of them.
@@ -242,8 +429,8 @@ __device__ __forceinline__ bool att_fits(const RunArgs &a, const SegRec &rec, in
 
 template <int DT, int NK, int QT>
 __global__ __launch_bounds__(256, 2) void attention_dq_kernel(RunArgs a, AttBwdArgs w) {
-    __shared__ __attribute__((aligned(16))) unsigned char sK[kAttKeys * att_pitch(NK)];
-    __shared__ __attribute__((aligned(16))) unsigned char sV[kAttKeys * att_pitch(NK)];
+    constexpr bool kPipe = QT == 2 && NK > 1;          // (K <= 32: too few matrix instructions to spread the staging over)
+    __shared__ __attribute__((aligned(16))) unsigned char lds[(kPipe ? 4 : 2) * kAttKeys * att_pitch(NK)];
     const ConstHdr hdr = (ConstHdr)(uintptr_t)a.plan;
     const int64_t per_head = QT == 2 ? hdr->att_blocks128 : hdr->att_blocks64;
     const bool rows_ok = hdr->min_K == w.min_K;
@@ -254,8 +441,14 @@ __global__ __launch_bounds__(256, 2) void attention_dq_kernel(RunArgs a, AttBwdA
     const SegRec rec = load_rec(plan_ro(a.plan, a.nseg).recs, g);
     if (rec.M < 1 || rec.K < 1 || !att_fits(a, rec, 32 * NK, h, block)) return;
     const int64_t row0 = att_row_base(w.min_K, a.Dm1, h, rec.off1);
-    if ((rec.K & 7) == 0) att_dq_body<DT, NK, QT, true>(a, w, rec, h, row0, block, sK, sV);
-    else att_dq_body<DT, NK, QT, false>(a, w, rec, h, row0, block, sK, sV);
+    if constexpr (kPipe) {
+        if ((rec.K & 7) == 0) att_dq_pipe_body<DT, NK, true>(a, w, rec, h, row0, block, lds);
+        else att_dq_pipe_body<DT, NK, false>(a, w, rec, h, row0, block, lds);
+    } else {
+        unsigned char *values = lds + kAttKeys * att_pitch(NK);
+        if ((rec.K & 7) == 0) att_dq_body<DT, NK, QT, true>(a, w, rec, h, row0, block, lds, values);
+        else att_dq_body<DT, NK, QT, false>(a, w, rec, h, row0, block, lds, values);
+    }
 }
 
 // ------------------------------------------------------------------------------------------------------- dK and dV
