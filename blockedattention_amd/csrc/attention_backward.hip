@@ -913,16 +913,23 @@ int launch_attention_backward(int dtype, const RunArgs &args, const void *V, con
     if (info->max_K > 128 || info->nseg <= 0) return info->nseg <= 0 ? BA_OK : BA_ERR_UNSUPPORTED;
     const AttBwdArgs w{V, O, dO, lse, delta, dQ, dK, dV, info->min_K};
     const int nk = std::max(1, (info->max_K + 31) / 32);
-    // Segments of 256 rows and more on average: wavefronts of two query strips, and workgroups of 128 keys that stage 64
-    // queries, three stages of them (16 x 16 pairs of 1024 .. 4096 rows: dK and dV 1.82 ms; two stages 2.10 ms and there 64 keys
-    // and 32 queries 2.78 ms, 128 keys and 32 queries 2.44 ms: every query block is staged once per workgroup).  Shorter ones: 64 keys and 32 queries, two to
-    // three times as many resident workgroups (1024 x 4 pairs of 2 .. 512 rows, at two wavefronts
-    // per SIMD: 127 us; 64 queries 184 us, 128 keys 168 us).
-    const bool tall = info->total_rows >= 256 * std::max<int64_t>(info->nseg, 1);
-    if (dtype == BA_F16)
-        return tall ? launch_bwd_nk<0, 2, 4, 64>(nk, args, w, info, stream) : launch_bwd_nk<0, 1, 2, 32>(nk, args, w, info, stream);
-    if (dtype == BA_BF16)
-        return tall ? launch_bwd_nk<1, 2, 4, 64>(nk, args, w, info, stream) : launch_bwd_nk<1, 1, 2, 32>(nk, args, w, info, stream);
+    // Rows per segment on average: from 256 on wavefronts of two query strips (dQ); from 768 on workgroups of 128 keys that
+    // stage 64 queries, three stages of them (every query block is staged once per workgroup, which has its compute unit
+    // alone; 16 x 16 pairs of 1024 .. 4096 rows, K = 128: dK and dV 1.82 ms, 64 keys and 32 queries 2.78 ms).  Below, 64 keys
+    // and 32 queries, two to three times as many resident workgroups: forward and backward at 311 rows and K = 64
+    // 203 -> 184 us, K = 128 350 -> 331; at 507 204 -> 193 and 339 -> 334; at 760 263 -> 250 and 427 -> 430.  Rows at any
+    // alignment, where the small build has too few registers, keep the line at 256 (K = 101, 100 .. 300 rows: 128 keys 316 us,
+    // 64 keys 369 us).
+    const int64_t mean = info->total_rows / std::max<int64_t>(info->nseg, 1);
+    const bool strips2 = mean >= 256, keys128 = mean >= (((info->min_K | info->max_K) & 7) ? 256 : 768);
+    auto launch = [&](auto dt) {
+        constexpr int DT = decltype(dt)::value;
+        if (keys128) return launch_bwd_nk<DT, 2, 4, 64>(nk, args, w, info, stream);
+        if (strips2) return launch_bwd_nk<DT, 2, 2, 32>(nk, args, w, info, stream);
+        return launch_bwd_nk<DT, 1, 2, 32>(nk, args, w, info, stream);
+    };
+    if (dtype == BA_F16) return launch(std::integral_constant<int, 0>{});
+    if (dtype == BA_BF16) return launch(std::integral_constant<int, 1>{});
     return BA_ERR_UNSUPPORTED;
 }
 

@@ -101,7 +101,7 @@ def test_block_counts_beside_a_tall_segment(dev, K):
     # 128 keys a workgroup, three stages of 64 queries: one, two, three and more blocks, full and ragged, and key blocks
     # of which one to all four pairs of wavefronts have keys
     # (dQ: 64 keys a block in two halves of which the last may have none, wavefronts without rows, no keys at all)
-    M = [1, 63, 64, 65, 128, 129, 193, 1700, 260]; N = [200, 31, 33, 127, 1, 128, 129, 96, 0]
+    M = [1, 63, 64, 65, 128, 129, 193, 6400, 260]; N = [200, 31, 33, 127, 1, 128, 129, 96, 0]
     run(dev, M, N, [K] * 9, 2, torch.bfloat16, K ** -0.5, seed=K)
 
 
