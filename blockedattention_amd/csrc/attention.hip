@@ -137,15 +137,6 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
                                  (qf[q][s][3] ^ flip) & keep};
             }
         }
-        float m[QT], lsum[QT];
-        f32x4 oacc[QT][kOutTiles];
-#pragma unroll
-        for (int q = 0; q < QT; ++q) {
-            m[q] = -INFINITY; lsum[q] = 0.f;
-#pragma unroll
-            for (int t = 0; t < kOutTiles; ++t) oacc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-
         // The loads run ahead of the arithmetic and land in registers while it runs.  One stage: the loads of block kb + 64
         // (kw, vw: this thread's pieces of the key and value rows) are issued before the matrix work on block kb; they sit
         // in one branch-free sequence (index clamped, value selected afterwards): loads behind a branch wait one by one.
@@ -215,200 +206,215 @@ __device__ __forceinline__ void attention_body(const RunArgs &a, const void *Vbu
             kw[step] = load_v(offset(sc, kb + 2 * kAttKeys));
             __builtin_amdgcn_sched_barrier(0);
         };
-        if (ST == 2 && nq == 0) {                 // the wavefront only stages (a loop of its own: in one with the
-            for (; kb < N; kb += kAttKeys) {           // arithmetic the accumulators would be copied where they meet)
+        // All blocks and the results of a wavefront with S strips.  Two stages: a wavefront of one strip has a walk of its own
+        // from its accumulators to its results (as a choice inside the loop the accumulators would be copied where the two
+        // meet); computing the missing strip along instead cost 5 % on 100 x 8 segments of 320 rows and 500 keys.
+        auto walk = [&](auto s_tag) {
+            constexpr int S = decltype(s_tag)::value;
+            float m[S], lsum[S];
+            f32x4 oacc[S][kOutTiles];
+#pragma unroll
+            for (int q = 0; q < S; ++q) {
+                m[q] = -INFINITY; lsum[q] = 0.f;
+#pragma unroll
+                for (int t = 0; t < kOutTiles; ++t) oacc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+            for (; kb < N; kb += kAttKeys) {
+                if constexpr (ST == 1) {
+                    static_for<kSteps>([&](auto sc) {
+                        constexpr int step = decltype(sc)::value;
+                        kw[step] = finish(sc, kb, kw[step]);
+                        vw[step] = finish(sc, kb, vw[step]);
+                    });
+                    __syncthreads();                       // the previous block (or round) is consumed
+                    // ---- one 16-byte piece per thread, array and step, pieces of a row on neighbouring lanes
+                    static_for<kSteps>([&](auto sc) {
+                        put(sc, 0, kw[decltype(sc)::value]);
+                        put(sc, kValues, vw[decltype(sc)::value]);
+                    });
+                    __syncthreads();
+                    if (kb + kAttKeys < N) {
+                        static_for<kSteps>([&](auto sc) {
+                            const uint32_t off = offset(sc, kb + kAttKeys);
+                            kw[decltype(sc)::value] = load_k(off);
+                            vw[decltype(sc)::value] = load_v(off);
+                        });
+                        advance();
+                    }
+                    if (nq == 0) continue;
+                }
+                // The arithmetic on one block for NQ live strips, as straight-line code: a branch around every
+                // matrix instruction of a strip that may be missing would keep the scheduler from interleaving them.
+                auto block_math = [&](auto nq_tag) {
+                    constexpr int NQ = decltype(nq_tag)::value;
+                    // ---- scores of 64 keys x 16 queries per strip; a key operand read serves every strip
+                    f32x4 sacc[NQ][4];
+        #pragma unroll
+                    for (int q = 0; q < NQ; ++q)
+        #pragma unroll
+                        for (int t = 0; t < 4; ++t) sacc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    u32x4 ring[kAttRing];
+                    const uint32_t k_at = k_addr + (ST == 2 ? stage : 0), v_at = v_addr + (ST == 2 ? stage : 0);
+                    {
+                        constexpr int kReads = 4 * NK;         // read i: k step i / 4, key tile i % 4
+                        static_for<kAttRing>([&](auto ic) {
+                            constexpr int I = decltype(ic)::value;
+                            if constexpr (I < kReads) lds_read128<16 * (I % 4) * kPitchK + 64 * (I / 4)>(ring[I], k_at);
+                        });
+                        static_for<kReads>([&](auto ic) {
+                            constexpr int I = decltype(ic)::value, R = I % kAttRing;
+                            constexpr int kBehind = (I + kAttRing < kReads ? I + kAttRing : kReads) - (I + 1);
+                            lds_wait<kBehind>(ring[R]);
+        #pragma unroll
+                            for (int q = 0; q < NQ; ++q) sacc[q][I % 4] = Elem<DT>::mfma(ring[R], qf[q][I / 4], sacc[q][I % 4]);
+                            if constexpr (ST == 2) __builtin_amdgcn_sched_barrier(0);
+                            if constexpr (I + kAttRing < kReads)
+                                lds_read128<16 * ((I + kAttRing) % 4) * kPitchK + 64 * ((I + kAttRing) / 4)>(ring[R], k_at);
+                            constexpr int kEvery = kReads / kSteps;
+                            static_assert(kEvery * kSteps == kReads);
+                            if constexpr (ST == 2 && I % kEvery == kEvery - 1) exchange_v(std::integral_constant<int, I / kEvery>{});
+                        });
+                    }
+                    constexpr int kValueReads = 2 * kOutTiles; // read i: key half i / kOutTiles, output tile i % kOutTiles
+                    u32x2 lo[kAttRing], hi[kAttRing];          // keys 4 rg .. + 3 of the half's two key tiles
+                    auto values_ahead = [&]() {
+                        static_for<kAttRing>([&](auto ic) {
+                            constexpr int I = decltype(ic)::value;
+                            if constexpr (I < kValueReads)
+                                lds_read_tr<32 * (I / kOutTiles) * kPitchK + 32 * (I % kOutTiles), 16 * kPitchK>(lo[I], hi[I], v_at);
+                        });
+                    };
+                    if constexpr (ST == 2) {
+                        advance();
+                        values_ahead();                        // in flight under the softmax
+                    }
+                    // ---- online softmax; lane holds keys kb + 16 t + 4 rg + e of query j of each strip
+                    const int left = N - kb;                   // keys of this block that exist
+                    u32x4 pf[NQ][2];
+        #pragma unroll
+                    for (int q = 0; q < NQ; ++q) {
+                        f32x4(&sc)[4] = sacc[q];
+                        // keys past the segment's last: -inf, so that they neither raise the maximum nor count
+                        // (their exponentials are zeros)
+                        if (left < kAttKeys) {
+                            const int mine = left - 4 * rg;    // (compared with constants: no registers for 16 key numbers)
+        #pragma unroll
+                            for (int t = 0; t < 4; ++t)
+        #pragma unroll
+                                for (int e = 0; e < 4; ++e) sc[t][e] = 16 * t + e < mine ? sc[t][e] : -INFINITY;
+                        }
+                        settle_mfma(sc);                       // max3 reads the scores from inline assembly
+                        float bm;                              // one statement: no padding between its instructions
+                        asm volatile("v_max3_f32 %0, %1, %2, %3\n\tv_max3_f32 %0, %0, %4, %5\n\tv_max3_f32 %0, %0, %6, %7\n\t"
+                                     "v_max3_f32 %0, %0, %8, %9\n\tv_max3_f32 %0, %0, %10, %11\n\tv_max3_f32 %0, %0, %12, %13\n\t"
+                                     "v_max3_f32 %0, %0, %14, %15\n\tv_max_f32 %0, %0, %16"
+                                     : "=&v"(bm)
+                                     : "v"(sc[0][0]), "v"(sc[0][1]), "v"(sc[0][2]), "v"(sc[0][3]), "v"(sc[1][0]), "v"(sc[1][1]),
+                                       "v"(sc[1][2]), "v"(sc[1][3]), "v"(sc[2][0]), "v"(sc[2][1]), "v"(sc[2][2]), "v"(sc[2][3]),
+                                       "v"(sc[3][0]), "v"(sc[3][1]), "v"(sc[3][2]), "v"(sc[3][3]));
+                        bm = quad_column_max_swap(bm);
+                        // m is the reference the exponentials are taken against, not necessarily the maximum: it is
+                        // raised (and the sums so far rescaled) only when a block's maximum passes it by more than
+                        // 2^8 in the exponent, so probabilities stay below 256 (fine for both 16-bit types and the
+                        // fp32 sums) and most blocks skip the rescale.  The comparison is false, i.e. raises, for the
+                        // first block (m = -inf).
+                        const bool raise = !((bm - m[q]) * c <= 8.0f);
+                        const float m_new = raise ? bm : m[q];
+                        const float m_use = m_new == -INFINITY ? 0.f : m_new;
+                        const float alpha = !raise ? 1.0f : m[q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m[q] - m_use) * c);
+                        m[q] = m_new;
+                        const float bias = -m_use * c;
+                        float psum = 0.f;
+        #pragma unroll
+                        for (int t = 0; t < 4; ++t)
+        #pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                float p = __builtin_amdgcn_exp2f(fmaf(sc[t][e], c, bias));
+                                sc[t][e] = p;
+                                psum += p;
+                            }
+                        lsum[q] = fmaf(lsum[q], alpha, psum);
+                        if (__any(raise)) {
+                            // (the matrix instructions that wrote the accumulators are a whole score product away)
+        #pragma unroll
+                            for (int t = 0; t < kOutTiles; ++t) {
+                                if constexpr (ST == 2) scale_in_place(oacc[q][t], alpha);
+                                else oacc[q][t] *= alpha;
+                            }
+                        }
+                        // probabilities as B operand, 32 keys per step: k = 8 rg + kk is key 32 cc + 4 rg + kk (kk < 4)
+                        // or 32 cc + 16 + 4 rg + kk - 4: what the lane holds in sc[2 cc] and sc[2 cc + 1]
+        #pragma unroll
+                        for (int cc = 0; cc < 2; ++cc)
+                            pf[q][cc] = u32x4{Elem<DT>::pack2(sc[2 * cc][0], sc[2 * cc][1]), Elem<DT>::pack2(sc[2 * cc][2], sc[2 * cc][3]),
+                                              Elem<DT>::pack2(sc[2 * cc + 1][0], sc[2 * cc + 1][1]),
+                                              Elem<DT>::pack2(sc[2 * cc + 1][2], sc[2 * cc + 1][3])};
+                    }
+                    // ---- O^T += V^T P^T; a value operand read serves every strip
+                    {
+                        if constexpr (ST == 1) values_ahead();
+                        static_for<kValueReads>([&](auto ic) {
+                            constexpr int I = decltype(ic)::value, R = I % kAttRing, J = I + kAttRing;
+                            lds_wait_tr<2 * ((J < kValueReads ? J : kValueReads) - (I + 1))>(lo[R], hi[R]);
+                            const u32x4 v = u32x4{lo[R][0], lo[R][1], hi[R][0], hi[R][1]};
+        #pragma unroll
+                            for (int q = 0; q < NQ; ++q)
+                                oacc[q][I % kOutTiles] = Elem<DT>::mfma(v, pf[q][I / kOutTiles], oacc[q][I % kOutTiles]);
+                            if constexpr (ST == 2) __builtin_amdgcn_sched_barrier(0);
+                            if constexpr (J < kValueReads)
+                                lds_read_tr<32 * (J / kOutTiles) * kPitchK + 32 * (J % kOutTiles), 16 * kPitchK>(lo[R], hi[R], v_at);
+                            constexpr int kEvery = kValueReads / kSteps;
+                            static_assert(kEvery * kSteps == kValueReads);
+                            if constexpr (ST == 2 && I % kEvery == kEvery - 1) exchange_k(std::integral_constant<int, I / kEvery>{});
+                        });
+                    }
+                };
+                if (ST == 1 && QT == 2 && nq == 1) block_math(std::integral_constant<int, 1>{});
+                else block_math(std::integral_constant<int, S>{});
+                if constexpr (ST == 2) {
+                    stage = kStageBytes - stage;
+                    att_lds_barrier();
+                }
+            }
+            // ---- normalise and store: lane (query j, rg) holds columns 16 t + 4 rg + e.  No key at all: zeros.
+            // (column numbers made here: taken out of the loop over the rounds they would hold registers through the blocks)
+            int own = 4 * rg;
+            if constexpr (ST == 2) asm volatile("" : "+v"(own));
+#pragma unroll
+            for (int q = 0; q < S; ++q) {
+                if (q >= nq) continue;
+                const int qr = r0 + kAttRows * q + j;
+                const float l = quad_column_sum(lsum[q]);
+                const float inv = N > 0 ? 1.0f / l : 0.f;
+                // base-2 logarithm of the row's sum of exponentials, for the backward pass
+                if (LSE && rg == 0 && qr < M && N > 0) lse_rows[qr] = fmaf(m[q], c, __builtin_amdgcn_logf(l));
+                if (qr < M) {
+                    uint16_t *orow = os + (int64_t)qr * K;
+#pragma unroll
+                    for (int t = 0; t < kOutTiles; ++t) {
+                        const int c0 = 16 * t + own;
+                        if (c0 + 4 <= K) {
+                            *reinterpret_cast<u32x2_unaligned *>(orow + c0) =
+                                u32x2{Elem<DT>::pack2(oacc[q][t][0] * inv, oacc[q][t][1] * inv),
+                                      Elem<DT>::pack2(oacc[q][t][2] * inv, oacc[q][t][3] * inv)};
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                if (c0 + e < K) orow[c0 + e] = Elem<DT>::from_float(oacc[q][t][e] * inv);
+                        }
+                    }
+                }
+            }
+        };
+        if (ST == 1 || nq == QT) walk(std::integral_constant<int, QT>{});
+        else if (nq == 1) walk(std::integral_constant<int, 1>{});
+        else {                                         // the wavefront only stages
+            for (; kb < N; kb += kAttKeys) {
                 static_for<kSteps>(exchange_v);
                 advance();
                 static_for<kSteps>(exchange_k);
                 stage = kStageBytes - stage;
                 att_lds_barrier();
-            }
-        }
-        for (; kb < N; kb += kAttKeys) {
-            if constexpr (ST == 1) {
-                static_for<kSteps>([&](auto sc) {
-                    constexpr int step = decltype(sc)::value;
-                    kw[step] = finish(sc, kb, kw[step]);
-                    vw[step] = finish(sc, kb, vw[step]);
-                });
-                __syncthreads();                       // the previous block (or round) is consumed
-                // ---- one 16-byte piece per thread, array and step, pieces of a row on neighbouring lanes
-                static_for<kSteps>([&](auto sc) {
-                    put(sc, 0, kw[decltype(sc)::value]);
-                    put(sc, kValues, vw[decltype(sc)::value]);
-                });
-                __syncthreads();
-                if (kb + kAttKeys < N) {
-                    static_for<kSteps>([&](auto sc) {
-                        const uint32_t off = offset(sc, kb + kAttKeys);
-                        kw[decltype(sc)::value] = load_k(off);
-                        vw[decltype(sc)::value] = load_v(off);
-                    });
-                    advance();
-                }
-                if (nq == 0) continue;
-            }
-            // The arithmetic on one block for NQ live strips, as straight-line code: a branch around every
-            // matrix instruction of a strip that may be missing would keep the scheduler from interleaving them.
-            auto block_math = [&](auto nq_tag) {
-                constexpr int NQ = decltype(nq_tag)::value;
-                // ---- scores of 64 keys x 16 queries per strip; a key operand read serves every strip
-                f32x4 sacc[NQ][4];
-    #pragma unroll
-                for (int q = 0; q < NQ; ++q)
-    #pragma unroll
-                    for (int t = 0; t < 4; ++t) sacc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-                u32x4 ring[kAttRing];
-                const uint32_t k_at = k_addr + (ST == 2 ? stage : 0), v_at = v_addr + (ST == 2 ? stage : 0);
-                {
-                    constexpr int kReads = 4 * NK;         // read i: k step i / 4, key tile i % 4
-                    static_for<kAttRing>([&](auto ic) {
-                        constexpr int I = decltype(ic)::value;
-                        if constexpr (I < kReads) lds_read128<16 * (I % 4) * kPitchK + 64 * (I / 4)>(ring[I], k_at);
-                    });
-                    static_for<kReads>([&](auto ic) {
-                        constexpr int I = decltype(ic)::value, R = I % kAttRing;
-                        constexpr int kBehind = (I + kAttRing < kReads ? I + kAttRing : kReads) - (I + 1);
-                        lds_wait<kBehind>(ring[R]);
-    #pragma unroll
-                        for (int q = 0; q < NQ; ++q) sacc[q][I % 4] = Elem<DT>::mfma(ring[R], qf[q][I / 4], sacc[q][I % 4]);
-                        if constexpr (ST == 2) __builtin_amdgcn_sched_barrier(0);
-                        if constexpr (I + kAttRing < kReads)
-                            lds_read128<16 * ((I + kAttRing) % 4) * kPitchK + 64 * ((I + kAttRing) / 4)>(ring[R], k_at);
-                        constexpr int kEvery = kReads / kSteps;
-                        static_assert(kEvery * kSteps == kReads);
-                        if constexpr (ST == 2 && I % kEvery == kEvery - 1) exchange_v(std::integral_constant<int, I / kEvery>{});
-                    });
-                }
-                constexpr int kValueReads = 2 * kOutTiles; // read i: key half i / kOutTiles, output tile i % kOutTiles
-                u32x2 lo[kAttRing], hi[kAttRing];          // keys 4 rg .. + 3 of the half's two key tiles
-                auto values_ahead = [&]() {
-                    static_for<kAttRing>([&](auto ic) {
-                        constexpr int I = decltype(ic)::value;
-                        if constexpr (I < kValueReads)
-                            lds_read_tr<32 * (I / kOutTiles) * kPitchK + 32 * (I % kOutTiles), 16 * kPitchK>(lo[I], hi[I], v_at);
-                    });
-                };
-                if constexpr (ST == 2) {
-                    advance();
-                    values_ahead();                        // in flight under the softmax
-                }
-                // ---- online softmax; lane holds keys kb + 16 t + 4 rg + e of query j of each strip
-                const int left = N - kb;                   // keys of this block that exist
-                u32x4 pf[NQ][2];
-    #pragma unroll
-                for (int q = 0; q < NQ; ++q) {
-                    f32x4(&sc)[4] = sacc[q];
-                    // keys past the segment's last: -inf, so that they neither raise the maximum nor count
-                    // (their exponentials are zeros)
-                    if (left < kAttKeys) {
-                        const int mine = left - 4 * rg;    // (compared with constants: no registers for 16 key numbers)
-    #pragma unroll
-                        for (int t = 0; t < 4; ++t)
-    #pragma unroll
-                            for (int e = 0; e < 4; ++e) sc[t][e] = 16 * t + e < mine ? sc[t][e] : -INFINITY;
-                    }
-                    settle_mfma(sc);                       // max3 reads the scores from inline assembly
-                    float bm;                              // one statement: no padding between its instructions
-                    asm volatile("v_max3_f32 %0, %1, %2, %3\n\tv_max3_f32 %0, %0, %4, %5\n\tv_max3_f32 %0, %0, %6, %7\n\t"
-                                 "v_max3_f32 %0, %0, %8, %9\n\tv_max3_f32 %0, %0, %10, %11\n\tv_max3_f32 %0, %0, %12, %13\n\t"
-                                 "v_max3_f32 %0, %0, %14, %15\n\tv_max_f32 %0, %0, %16"
-                                 : "=&v"(bm)
-                                 : "v"(sc[0][0]), "v"(sc[0][1]), "v"(sc[0][2]), "v"(sc[0][3]), "v"(sc[1][0]), "v"(sc[1][1]),
-                                   "v"(sc[1][2]), "v"(sc[1][3]), "v"(sc[2][0]), "v"(sc[2][1]), "v"(sc[2][2]), "v"(sc[2][3]),
-                                   "v"(sc[3][0]), "v"(sc[3][1]), "v"(sc[3][2]), "v"(sc[3][3]));
-                    bm = quad_column_max_swap(bm);
-                    // m is the reference the exponentials are taken against, not necessarily the maximum: it is
-                    // raised (and the sums so far rescaled) only when a block's maximum passes it by more than
-                    // 2^8 in the exponent, so probabilities stay below 256 (fine for both 16-bit types and the
-                    // fp32 sums) and most blocks skip the rescale.  The comparison is false, i.e. raises, for the
-                    // first block (m = -inf).
-                    const bool raise = !((bm - m[q]) * c <= 8.0f);
-                    const float m_new = raise ? bm : m[q];
-                    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-                    const float alpha = !raise ? 1.0f : m[q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m[q] - m_use) * c);
-                    m[q] = m_new;
-                    const float bias = -m_use * c;
-                    float psum = 0.f;
-    #pragma unroll
-                    for (int t = 0; t < 4; ++t)
-    #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            float p = __builtin_amdgcn_exp2f(fmaf(sc[t][e], c, bias));
-                            sc[t][e] = p;
-                            psum += p;
-                        }
-                    lsum[q] = fmaf(lsum[q], alpha, psum);
-                    if (__any(raise)) {
-                        // (the matrix instructions that wrote the accumulators are a whole score product away)
-    #pragma unroll
-                        for (int t = 0; t < kOutTiles; ++t) {
-                            if constexpr (ST == 2) scale_in_place(oacc[q][t], alpha);
-                            else oacc[q][t] *= alpha;
-                        }
-                    }
-                    // probabilities as B operand, 32 keys per step: k = 8 rg + kk is key 32 cc + 4 rg + kk (kk < 4)
-                    // or 32 cc + 16 + 4 rg + kk - 4: what the lane holds in sc[2 cc] and sc[2 cc + 1]
-    #pragma unroll
-                    for (int cc = 0; cc < 2; ++cc)
-                        pf[q][cc] = u32x4{Elem<DT>::pack2(sc[2 * cc][0], sc[2 * cc][1]), Elem<DT>::pack2(sc[2 * cc][2], sc[2 * cc][3]),
-                                          Elem<DT>::pack2(sc[2 * cc + 1][0], sc[2 * cc + 1][1]),
-                                          Elem<DT>::pack2(sc[2 * cc + 1][2], sc[2 * cc + 1][3])};
-                }
-                // ---- O^T += V^T P^T; a value operand read serves every strip
-                {
-                    if constexpr (ST == 1) values_ahead();
-                    static_for<kValueReads>([&](auto ic) {
-                        constexpr int I = decltype(ic)::value, R = I % kAttRing, J = I + kAttRing;
-                        lds_wait_tr<2 * ((J < kValueReads ? J : kValueReads) - (I + 1))>(lo[R], hi[R]);
-                        const u32x4 v = u32x4{lo[R][0], lo[R][1], hi[R][0], hi[R][1]};
-    #pragma unroll
-                        for (int q = 0; q < NQ; ++q)
-                            oacc[q][I % kOutTiles] = Elem<DT>::mfma(v, pf[q][I / kOutTiles], oacc[q][I % kOutTiles]);
-                        if constexpr (ST == 2) __builtin_amdgcn_sched_barrier(0);
-                        if constexpr (J < kValueReads)
-                            lds_read_tr<32 * (J / kOutTiles) * kPitchK + 32 * (J % kOutTiles), 16 * kPitchK>(lo[R], hi[R], v_at);
-                        constexpr int kEvery = kValueReads / kSteps;
-                        static_assert(kEvery * kSteps == kValueReads);
-                        if constexpr (ST == 2 && I % kEvery == kEvery - 1) exchange_k(std::integral_constant<int, I / kEvery>{});
-                    });
-                }
-            };
-            // (two stages: a strip that does not exist is computed along, a second body would not fit the registers)
-            if (ST == 1 && QT == 2 && nq == 1) block_math(std::integral_constant<int, 1>{});
-            else block_math(std::integral_constant<int, QT>{});
-            if constexpr (ST == 2) {
-                stage = kStageBytes - stage;
-                att_lds_barrier();
-            }
-        }
-        // ---- normalise and store: lane (query j, rg) holds columns 16 t + 4 rg + e.  No key at all: zeros.
-        // (column numbers made here: taken out of the loop over the rounds they would hold registers through the blocks)
-        int own = 4 * rg;
-        if constexpr (ST == 2) asm volatile("" : "+v"(own));
-#pragma unroll
-        for (int q = 0; q < QT; ++q) {
-            if (q >= nq) continue;
-            const int qr = r0 + kAttRows * q + j;
-            const float l = quad_column_sum(lsum[q]);
-            const float inv = N > 0 ? 1.0f / l : 0.f;
-            // base-2 logarithm of the row's sum of exponentials, for the backward pass
-            if (LSE && rg == 0 && qr < M && N > 0) lse_rows[qr] = fmaf(m[q], c, __builtin_amdgcn_logf(l));
-            if (qr < M) {
-                uint16_t *orow = os + (int64_t)qr * K;
-#pragma unroll
-                for (int t = 0; t < kOutTiles; ++t) {
-                    const int c0 = 16 * t + own;
-                    if (c0 + 4 <= K) {
-                        *reinterpret_cast<u32x2_unaligned *>(orow + c0) =
-                            u32x2{Elem<DT>::pack2(oacc[q][t][0] * inv, oacc[q][t][1] * inv),
-                                  Elem<DT>::pack2(oacc[q][t][2] * inv, oacc[q][t][3] * inv)};
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (c0 + e < K) orow[c0 + e] = Elem<DT>::from_float(oacc[q][t][e] * inv);
-                    }
-                }
             }
         }
     }

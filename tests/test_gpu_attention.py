@@ -123,6 +123,16 @@ def test_two_stages_block_edges(dev, K, dtype):
     run(dev, M, N, [K] * 6, 2, dtype, K ** -0.5, seed=K)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K", [64, 96, 128, 101])
+def test_two_stages_raise_the_reference_late(dev, K, dtype):
+    # scaled scores of standard deviation 9: in most rows a later block's maximum passes the first one's by more than 2^8 in
+    # the exponent, so sums and accumulators are rescaled in the middle, in both strips of a wavefront (two in the first
+    # wavefront and one in the others: 80 rows past a whole block) and in the only one.  Scores of either sign, and no scale
+    for scale in (K ** -0.5, -(K ** -0.5), 0.0):
+        run(dev, [336, 520, 300], [2000, 1025, 700], [K] * 3, 2, dtype, scale, seed=K, sigma=3.0)
+
+
 @pytest.mark.parametrize("seed", [11, 12, 13, 14])
 def test_random_batches(dev, seed):
     # random batches: segment counts, heights, widths and head dimensions drawn anew (multiples of 8 or anything),
