@@ -21,6 +21,11 @@ template <int OFF> __device__ __forceinline__ void lds_read128(u32x4 &dst, uint3
 template <int N> __device__ __forceinline__ void lds_wait(u32x4 &x) {
     asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(x) : "n"(N) : "memory");
 }
+// Reads that turn out not to be needed arrive before their registers are free for something else.  One statement that names
+// them all and hands none on: of one for each the compiler copied the registers before the first wait.
+__device__ __forceinline__ void lds_drain(const u32x4 (&x)[4]) {
+    asm volatile("s_waitcnt lgkmcnt(0)" : : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]) : "memory");
+}
 // The same for the transposing read: four elements of one column from each of two groups of rows NEXT bytes apart.
 template <int OFF, int NEXT> __device__ __forceinline__ void lds_read_tr(u32x2 &lo, u32x2 &hi, uint32_t addr) {
     asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(lo) : "v"(addr), "n"(OFF) : "memory");

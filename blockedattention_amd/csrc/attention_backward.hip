@@ -390,7 +390,7 @@ __device__ __forceinline__ void att_dq_pipe_body(const RunArgs &a, const AttBwdA
         static_for<kRing>([&](auto xc) { read_row(xc, first); });
         half(first, left);
         if (left > 32) half(second, left);
-        else static_for<kRing>([&](auto xc) { lds_wait<0>(ring[decltype(xc)::value]); });     // (what was read for it)
+        else lds_drain(ring);                          // (what was read for it)
     }
     uint16_t *dq = (uint16_t *)w.dQ + o1;
 #pragma unroll
