@@ -851,14 +851,14 @@ __device__ __forceinline__ void att_dkdv_pipe_body(const RunArgs &a, const AttBw
     }
 }
 
-constexpr int att_dkdv_lds(int nk, int pairs, int qb) {
-    return (pairs == 4 ? 3 : 2) * (2 * qb * att_pitch(nk) + 8 * qb) + (pairs == 4 ? 2 : 1) * pairs * 64 * qb;
+constexpr int att_dkdv_lds(int nk, int pairs, int qb, bool pipe) {
+    return (pipe ? 3 : 2) * (2 * qb * att_pitch(nk) + 8 * qb) + (pipe ? 2 : 1) * pairs * 64 * qb;
 }
-static_assert(att_dkdv_lds(4, 4, 64) <= 160 * 1024);
+static_assert(att_dkdv_lds(4, 4, 64, true) <= 160 * 1024);
 
 // The build for short segments is bound by the life of a workgroup: three wavefronts per SIMD, not the two that its 197
 // registers at a head dimension of 128 would leave (30 of them spilled), 1024 x 4 pairs of 2 .. 512 rows: 133 -> 110 us.
-template <int DT, int NK, int PAIRS, int QB>
+template <int DT, int NK, int PAIRS, int QB, bool PIPE>
 __global__ __launch_bounds__(128 * PAIRS, QB == 32 ? 3 : 2) void attention_dkdv_kernel(RunArgs a, AttBwdArgs w) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     static_assert(PAIRS == 2 || PAIRS == 4, "the plan's column-block prefixes count blocks of 64 and of 128");
@@ -872,7 +872,7 @@ __global__ __launch_bounds__(128 * PAIRS, QB == 32 ? 3 : 2) void attention_dkdv_
     const SegRec rec = load_rec(plan_ro(a.plan, a.nseg).recs, g);
     if (rec.N < 1 || rec.K < 1 || !att_fits(a, rec, 32 * NK, h, block)) return;
     const int64_t row0 = att_row_base(w.min_K, a.Dm1, h, rec.off1);
-    if constexpr (PAIRS == 4) {
+    if constexpr (PIPE) {
         if ((rec.K & 7) == 0) att_dkdv_pipe_body<DT, NK, PAIRS, QB, true>(a, w, rec, h, row0, block, lds);
         else att_dkdv_pipe_body<DT, NK, PAIRS, QB, false>(a, w, rec, h, row0, block, lds);
     } else {
@@ -881,30 +881,32 @@ __global__ __launch_bounds__(128 * PAIRS, QB == 32 ? 3 : 2) void attention_dkdv_
     }
 }
 
-template <int DT, int NK, int QT, int PAIRS, int QB>
+// Blocks of 128 columns a head: at most half of the blocks of 64 and a half more for every segment.
+static int64_t att_cols128_most(const ba_plan_info *info) { return ((int64_t)info->att_cols64 + info->nseg) / 2; }
+
+template <int DT, int NK, int QT, int PAIRS, int QB, bool PIPE>
 static int launch_bwd(const RunArgs &args, const AttBwdArgs &w, const ba_plan_info *info, hipStream_t stream) {
-    constexpr int kLds = att_dkdv_lds(NK, PAIRS, QB);
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&attention_dkdv_kernel<DT, NK, PAIRS, QB>),
+    constexpr int kLds = att_dkdv_lds(NK, PAIRS, QB, PIPE);
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&attention_dkdv_kernel<DT, NK, PAIRS, QB, PIPE>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (attr != hipSuccess) return BA_ERR_LAUNCH;
     const int64_t rows = ((QT == 2 ? info->att_blocks128 : info->att_blocks64) * args.H + 7) / 8 * 8;
-    // (blocks of 128 columns: at most half of the blocks of 64 and a half more for every segment)
-    const int64_t blocks = PAIRS == 4 ? ((int64_t)info->att_cols64 + info->nseg) / 2 : info->att_cols64;
+    const int64_t blocks = PAIRS == 4 ? att_cols128_most(info) : info->att_cols64;
     const int64_t cols = (blocks * args.H + 7) / 8 * 8;
     if (rows > 0x7fffffff || cols > 0x7fffffff) return BA_ERR_UNSUPPORTED;
     if (rows > 0) hipLaunchKernelGGL((attention_dq_kernel<DT, NK, QT>), flat_grid(rows), dim3(256), 0, stream, args, w);
     if (cols > 0)
-        hipLaunchKernelGGL((attention_dkdv_kernel<DT, NK, PAIRS, QB>), flat_grid(cols), dim3(128 * PAIRS), kLds, stream, args, w);
+        hipLaunchKernelGGL((attention_dkdv_kernel<DT, NK, PAIRS, QB, PIPE>), flat_grid(cols), dim3(128 * PAIRS), kLds, stream, args, w);
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;
 }
 
-template <int DT, int QT, int PAIRS, int QB>
+template <int DT, int QT, int PAIRS, int QB, bool PIPE>
 static int launch_bwd_nk(int nk, const RunArgs &args, const AttBwdArgs &w, const ba_plan_info *info, hipStream_t stream) {
     switch (nk) {
-        case 1: return launch_bwd<DT, 1, QT, PAIRS, QB>(args, w, info, stream);
-        case 2: return launch_bwd<DT, 2, QT, PAIRS, QB>(args, w, info, stream);
-        case 3: return launch_bwd<DT, 3, QT, PAIRS, QB>(args, w, info, stream);
-        default: return launch_bwd<DT, 4, QT, PAIRS, QB>(args, w, info, stream);
+        case 1: return launch_bwd<DT, 1, QT, PAIRS, QB, PIPE>(args, w, info, stream);
+        case 2: return launch_bwd<DT, 2, QT, PAIRS, QB, PIPE>(args, w, info, stream);
+        case 3: return launch_bwd<DT, 3, QT, PAIRS, QB, PIPE>(args, w, info, stream);
+        default: return launch_bwd<DT, 4, QT, PAIRS, QB, PIPE>(args, w, info, stream);
     }
 }
 
@@ -922,11 +924,17 @@ int launch_attention_backward(int dtype, const RunArgs &args, const void *V, con
     // 64 keys 369 us).
     const int64_t mean = info->total_rows / std::max<int64_t>(info->nseg, 1);
     const bool strips2 = mean >= 256, keys128 = mean >= (((info->min_K | info->max_K) & 7) ? 256 : 768);
+    // K <= 32: the pipeline's LDS leaves room for one workgroup a compute unit where its two-stage form has two, and there are
+    // too few matrix instructions to hide the exchanges behind: the pipeline only where a compute unit gets no second one.
+    // Backward of 16 x 16 pairs of 1024 .. 4096 rows, K = 16 1273 us, two stages 1185; K = 32 1308, 1227; of 32 x 8 of 768 ..
+    // 1100 190, 175; of 2 x 2 of 1000 .. 2000 49, 56; 32 x 8 of 768 .. 1100 rows with 64 keys 33, 37.
+    const bool few = att_cols128_most(info) * args.H <= device_cu_count();
     auto launch = [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
-        if (keys128) return launch_bwd_nk<DT, 2, 4, 64>(nk, args, w, info, stream);
-        if (strips2) return launch_bwd_nk<DT, 2, 2, 32>(nk, args, w, info, stream);
-        return launch_bwd_nk<DT, 1, 2, 32>(nk, args, w, info, stream);
+        if (keys128 && nk == 1 && !few) return launch_bwd<DT, 1, 2, 4, 64, false>(args, w, info, stream);
+        if (keys128) return launch_bwd_nk<DT, 2, 4, 64, true>(nk, args, w, info, stream);
+        if (strips2) return launch_bwd_nk<DT, 2, 2, 32, false>(nk, args, w, info, stream);
+        return launch_bwd_nk<DT, 1, 2, 32, false>(nk, args, w, info, stream);
     };
     if (dtype == BA_F16) return launch(std::integral_constant<int, 0>{});
     if (dtype == BA_BF16) return launch(std::integral_constant<int, 1>{});

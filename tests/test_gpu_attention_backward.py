@@ -105,6 +105,15 @@ def test_block_counts_beside_a_tall_segment(dev, K):
     run(dev, M, N, [K] * 9, 2, torch.bfloat16, K ** -0.5, seed=K)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K", [8, 32, 29])
+def test_small_head_dimensions_many_workgroups(dev, K, dtype):
+    # head dimensions up to 32, tall segments, more workgroups of 128 keys than compute units: two stages of 64 queries; one
+    # block and more, full and ragged, key blocks of which one to all four pairs of wavefronts have keys
+    M = [1, 63, 64, 65, 129, 193, 2500, 3200]; N = [200, 31, 33, 127, 1, 128, 129, 300]
+    run(dev, M, N, [K] * 8, 20, dtype, K ** -0.5, seed=K)
+
+
 def test_empty_segments(dev):
     # no queries: dk and dv are zeros; no keys: dq is zeros
     run(dev, [4, 0, 9, 30, 0], [6, 5, 0, 70, 300], [16, 8, 24, 64, 64], 2, torch.float16, 0.5)
