@@ -915,20 +915,24 @@ int launch_attention_backward(int dtype, const RunArgs &args, const void *V, con
     if (info->max_K > 128 || info->nseg <= 0) return info->nseg <= 0 ? BA_OK : BA_ERR_UNSUPPORTED;
     const AttBwdArgs w{V, O, dO, lse, delta, dQ, dK, dV, info->min_K};
     const int nk = std::max(1, (info->max_K + 31) / 32);
-    // Rows per segment on average: from 256 on wavefronts of two query strips (dQ); from 768 on workgroups of 128 keys that
-    // stage 64 queries, three stages of them (every query block is staged once per workgroup, which has its compute unit
-    // alone; 16 x 16 pairs of 1024 .. 4096 rows, K = 128: dK and dV 1.82 ms, 64 keys and 32 queries 2.78 ms).  Below, 64 keys
-    // and 32 queries, two to three times as many resident workgroups: forward and backward at 311 rows and K = 64
-    // 203 -> 184 us, K = 128 350 -> 331; at 507 204 -> 193 and 339 -> 334; at 760 263 -> 250 and 427 -> 430.  Rows at any
-    // alignment, where the small build has too few registers, keep the line at 256 (K = 101, 100 .. 300 rows: 128 keys 316 us,
-    // 64 keys 369 us).
+    // Rows per segment on average: from 256 on wavefronts of two query strips (dQ), and for dK and dV a choice of workgroup
+    // that is timed in backward passes, us, bf16.  128 keys that stage 64 queries, three stages of them: every query block is
+    // staged once per workgroup, which has its compute unit alone.  64 keys and 32 queries: two to three times as many
+    // resident workgroups.
+    // - All workgroups of 128 keys find a compute unit of their own: these, they do twice the work at a time (10 x 4 of 400 ..
+    //   600 rows, K = 32 / 64 / 128: 64 keys 31 / 36 / 54, 128 keys 25 / 30 / 47; 8 x 4 of 256 .. 300 18.3 / 21.8, 16.7 / 20.8).
+    // - Otherwise where segments are tall enough for the stages to pay.  K <= 64 768 rows (24 x 8 of 750 .. 900 158, 168; 16 x 8
+    //   of 1000 .. 1300 199, 194; 10 x 4 of 1500 .. 2500 213, 202).  Above 576, K = 96 / 128: 50 x 8 of 450 .. 600 216 / 285,
+    //   217 / 291; 64 x 8 of 600 .. 900 499 / 626, 484 / 613; 32 x 8 of 500 .. 750 rows and 100 .. 300 keys 91 / 114, 82 / 104.
+    // - Rows at any alignment, for which the small build has too few registers: always (64 x 8 of 200 .. 400, K = 101: 314, 230).
     const int64_t mean = info->total_rows / std::max<int64_t>(info->nseg, 1);
-    const bool strips2 = mean >= 256, keys128 = mean >= (((info->min_K | info->max_K) & 7) ? 256 : 768);
+    const bool few = att_cols128_most(info) * args.H <= device_cu_count();
+    const bool unaligned = (info->min_K | info->max_K) & 7;
+    const bool strips2 = mean >= 256, keys128 = mean >= (unaligned || few ? 256 : nk > 2 ? 576 : 768);
     // K <= 32: the pipeline's LDS leaves room for one workgroup a compute unit where its two-stage form has two, and there are
     // too few matrix instructions to hide the exchanges behind: the pipeline only where a compute unit gets no second one.
     // Backward of 16 x 16 pairs of 1024 .. 4096 rows, K = 16 1273 us, two stages 1185; K = 32 1308, 1227; of 32 x 8 of 768 ..
     // 1100 190, 175; of 2 x 2 of 1000 .. 2000 49, 56; 32 x 8 of 768 .. 1100 rows with 64 keys 33, 37.
-    const bool few = att_cols128_most(info) * args.H <= device_cu_count();
     auto launch = [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
         if (keys128 && nk == 1 && !few) return launch_bwd<DT, 1, 2, 4, 64, false>(args, w, info, stream);

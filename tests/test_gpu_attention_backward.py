@@ -96,6 +96,13 @@ def test_tall_segments(dev, K, dtype):
     run(dev, [300, 520, 257], [130, 77, 1025], [K] * 3, 2, dtype, K ** -0.5, seed=7)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K", [24, 64, 96, 128])
+def test_two_strips_beside_workgroups_of_64_keys(dev, K, dtype):
+    # the same heights, more workgroups of 128 keys than compute units: 64 keys a workgroup
+    run(dev, [300, 520, 257], [130, 77, 1025], [K] * 3, 24, dtype, K ** -0.5, seed=8)
+
+
 @pytest.mark.parametrize("K", [24, 64, 96, 128, 101])
 def test_block_counts_beside_a_tall_segment(dev, K):
     # 128 keys a workgroup, three stages of 64 queries: one, two, three and more blocks, full and ragged, and key blocks
