@@ -103,6 +103,14 @@ def test_two_strips_beside_workgroups_of_64_keys(dev, K, dtype):
     run(dev, [300, 520, 257], [130, 77, 1025], [K] * 3, 24, dtype, K ** -0.5, seed=8)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 101])
+def test_scales_and_missing_queries_in_tall_segments(dev, K, dtype):
+    # above every line of heights: 128 keys a workgroup; scores of either sign and none; without queries dK and dV are zeros
+    for scale in (K ** -0.5, -0.3, 0.0):
+        run(dev, [2100, 0, 1500, 700], [130, 300, 77, 1025], [K] * 4, 1, dtype, scale, seed=K)
+
+
 @pytest.mark.parametrize("K", [24, 64, 96, 128, 101])
 def test_block_counts_beside_a_tall_segment(dev, K):
     # 128 keys a workgroup, three stages of 64 queries: one, two, three and more blocks, full and ragged, and key blocks
@@ -126,14 +134,10 @@ def test_empty_segments(dev):
     run(dev, [4, 0, 9, 30, 0], [6, 5, 0, 70, 300], [16, 8, 24, 64, 64], 2, torch.float16, 0.5)
 
 
-def test_negative_zero_and_large_scale(dev):
-    # large scores of both signs: probabilities close to 0 and 1, sums far below 2^-128 for a padding key of score zero
-    for scale in (-0.3, 0.0):
-        run(dev, [9, 70], [100, 17], [16, 64], 2, torch.float16, scale)
-        run(dev, [300, 520], [130, 77], [128, 64], 1, torch.bfloat16, scale)
-    M, N, K = np.array([40, 300]), np.array([50, 270]), np.array([64, 64])
-    q, k = torch.full((1, 340 * 64), -2.0), torch.full((1, 320 * 64), 2.0)      # every score is -256
-    v = torch.randn((1, 320 * 64), generator=torch.Generator("cpu").manual_seed(1))
+def all_scores_far_below_zero(dev, M, N):
+    K, rows, keys = np.full_like(M, 64), int(M.sum()), int(N.sum())
+    q, k = torch.full((1, rows * 64), -2.0), torch.full((1, keys * 64), 2.0)      # every score is -256
+    v = torch.randn((1, keys * 64), generator=torch.Generator("cpu").manual_seed(1))
     plan = make_plan(dev, M, N, K)
     q, k, v = (t.to(torch.bfloat16).to(dev) for t in (q, k, v))
     out = torch.empty_like(q); lse = torch.empty((1, capi.attention_rows(plan, q.shape[1])), device=dev)
@@ -142,7 +146,20 @@ def test_negative_zero_and_large_scale(dev):
     grads = [torch.empty_like(t) for t in (q, k, v)]
     capi.varlen_attention_backward(plan, q, k, v, out, torch.ones_like(q), lse, torch.empty_like(lse), *grads, *dims)
     assert all(bool(torch.isfinite(g).all()) for g in grads)
-    assert torch.allclose(grads[2][0, : 50 * 64].float(), torch.full((50 * 64,), 40 / 50, device=dev), rtol=2 ** -8)
+    assert torch.allclose(grads[2][0, : N[0] * 64].float(), torch.full((int(N[0]) * 64,), M[0] / N[0], device=dev), rtol=2 ** -8)
+
+
+def test_negative_zero_and_large_scale(dev):
+    # large scores of both signs: probabilities close to 0 and 1, sums far below 2^-128 for a padding key of score zero
+    for scale in (-0.3, 0.0):
+        run(dev, [9, 70], [100, 17], [16, 64], 2, torch.float16, scale)
+        run(dev, [300, 520], [130, 77], [128, 64], 1, torch.bfloat16, scale)
+    all_scores_far_below_zero(dev, np.array([40, 300]), np.array([50, 270]))
+
+
+def test_scores_far_below_zero_in_tall_segments(dev):
+    # two strips a wavefront and 128 keys a workgroup, the last of them ragged
+    all_scores_far_below_zero(dev, np.array([1000, 900, 1100]), np.array([50, 270, 1025]))
 
 
 @pytest.mark.parametrize("seed", [21, 22, 23, 24])
