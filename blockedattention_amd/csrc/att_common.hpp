@@ -10,6 +10,14 @@ namespace ba {
 
 constexpr int kAttKeys = 64;                          // keys (backward: or queries) staged in LDS at a time
 
+// Rows past a segment's last one that a kernel asks for, at most: the pipelines request two blocks ahead, where rows that
+// do not exist read as zeros by their byte offset, which must not wrap.  Dimensions and areas of a plan's segments are below
+// 2^30 (the scheduler refuses others) and head dimensions at most 128: every such segment fits.
+constexpr int kAttAhead = 3 * kAttKeys;
+__host__ __device__ constexpr bool att_offsets_fit(int64_t rows, int K) { return (rows + kAttAhead) * K < (int64_t(1) << 31); }
+static_assert(att_offsets_fit((1 << 30) - 1, 1) && att_offsets_fit(((1 << 30) - 1) / 128, 128));
+static_assert(!att_offsets_fit((int64_t(1) << 31) - kAttAhead, 1) && !att_offsets_fit((1 << 24) - kAttAhead, 128));
+
 // LDS operand reads as inline assembly, so that kAttRing of them are in flight under the matrix instructions
 // (left to itself the compiler, short of registers, issues each read right before its use and every matrix
 // instruction waits a full LDS round trip).  The compiler does not count these reads: lds_wait<n> waits until at

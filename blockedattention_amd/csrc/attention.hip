@@ -469,7 +469,7 @@ __global__ __launch_bounds__(kAttThreads, QT == 2 ? 2 : NK <= 2 ? 4 : 3) void at
     if (M < 1 || K < 1) return;
     // the launch was sized for a smaller head dimension, or byte offsets inside the segment (of a last block of
     // keys that reaches past the segment's end, too) pass 32 bits
-    if (K > KP || ((int64_t)max(M, rec.N) + kAttKeys) * K >= (int64_t(1) << 31)) {
+    if (K > KP || !att_offsets_fit(max(M, rec.N), K)) {
         if (h == 0 && zblock == 0 && threadIdx.x == 0)
             atomicAdd(&reinterpret_cast<PlanHeader *>(a.plan)->run_errors, 1);
         return;

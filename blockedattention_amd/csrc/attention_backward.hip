@@ -422,7 +422,7 @@ __device__ __forceinline__ bool att_item(const RunArgs &a, int which, int64_t pe
 }
 // The head dimension fits the build and every byte offset inside the segment fits 32 bits.
 __device__ __forceinline__ bool att_fits(const RunArgs &a, const SegRec &rec, int kp, int64_t h, int block) {
-    if (rec.K <= kp && ((int64_t)max(rec.M, rec.N) + kAttKeys) * rec.K < (int64_t(1) << 31)) return true;
+    if (rec.K <= kp && att_offsets_fit(max(rec.M, rec.N), rec.K)) return true;
     if (h == 0 && block == 0 && threadIdx.x == 0) atomicAdd(&reinterpret_cast<PlanHeader *>(a.plan)->run_errors, 1);
     return false;
 }
@@ -660,11 +660,11 @@ __device__ __forceinline__ void att_dkdv_pipe_body(const RunArgs &a, const AttBw
     const int aux_row = tid & (QB - 1);
     const bool aux_delta = wave & 1;
     const __amdgpu_buffer_rsrc_t aux_res =
-        __builtin_amdgcn_make_buffer_rsrc((void *)((aux_delta ? w.delta : w.lse) + row0), 0, 4 * M, kRsrcFlags);
-    auto fetch_aux = [&](int qb) { aux = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(aux_res, 4 * (qb + aux_row), 0, 0)); };
+        __builtin_amdgcn_make_buffer_rsrc((void *)((aux_delta ? w.delta : w.lse) + row0), 0, 4u * (uint32_t)M, kRsrcFlags);
+    auto fetch_aux = [&](int qb) { aux = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(aux_res, 4u * (uint32_t)(qb + aux_row), 0, 0)); };
     auto put_aux = [&](int qb, int stage) {
-        // 2^-inf: rows that do not exist have no probabilities
-        const float x = aux_delta ? -aux : qb + aux_row < M ? aux : INFINITY;
+        // 2^-inf: rows that do not exist have no probabilities (past 2^30 rows the offset wraps: delta is not taken as read either)
+        const float x = qb + aux_row < M ? (aux_delta ? -aux : aux) : (aux_delta ? 0.f : INFINITY);
         *reinterpret_cast<float *>(lds + stage + 2 * kArray + (aux_delta ? 4 * QB : 0) + 4 * aux_row) = x;
     };
     static_for<kPuts>([&](auto xc) { fetch(decltype(xc)::value, 0); });
