@@ -215,7 +215,7 @@ __device__ __forceinline__ void att_dq_body(const RunArgs &a, const AttBwdArgs &
     }
 }
 
-// The same for two strips a wavefront and many keys: two LDS stages and one barrier a block.  Each half of a block is one
+// The same for two strips a wavefront: two LDS stages and one barrier a block.  Each half of a block is one
 // stream of operand reads, kRing of them in flight across its three products (and into the next half); the exponentials
 // stand between the matrix instructions of dP, and the pieces of the next block are written, and those of the block after
 // it requested, between all of them: its values during the first half, its keys during the second, in one set of registers.
@@ -427,10 +427,9 @@ __device__ __forceinline__ bool att_fits(const RunArgs &a, const SegRec &rec, in
     return false;
 }
 
-template <int DT, int NK, int QT>
+template <int DT, int NK, int QT, bool PIPE>
 __global__ __launch_bounds__(256, 2) void attention_dq_kernel(RunArgs a, AttBwdArgs w) {
-    constexpr bool kPipe = QT == 2 && NK > 1;          // (K <= 32: too few matrix instructions to spread the staging over)
-    __shared__ __attribute__((aligned(16))) unsigned char lds[(kPipe ? 4 : 2) * kAttKeys * att_pitch(NK)];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[(PIPE ? 4 : 2) * kAttKeys * att_pitch(NK)];
     const ConstHdr hdr = (ConstHdr)(uintptr_t)a.plan;
     const int64_t per_head = QT == 2 ? hdr->att_blocks128 : hdr->att_blocks64;
     const bool rows_ok = hdr->min_K == w.min_K;
@@ -441,7 +440,7 @@ __global__ __launch_bounds__(256, 2) void attention_dq_kernel(RunArgs a, AttBwdA
     const SegRec rec = load_rec(plan_ro(a.plan, a.nseg).recs, g);
     if (rec.M < 1 || rec.K < 1 || !att_fits(a, rec, 32 * NK, h, block)) return;
     const int64_t row0 = att_row_base(w.min_K, a.Dm1, h, rec.off1);
-    if constexpr (kPipe) {
+    if constexpr (PIPE) {
         if ((rec.K & 7) == 0) att_dq_pipe_body<DT, NK, true>(a, w, rec, h, row0, block, lds);
         else att_dq_pipe_body<DT, NK, false>(a, w, rec, h, row0, block, lds);
     } else {
@@ -894,7 +893,22 @@ static int launch_bwd(const RunArgs &args, const AttBwdArgs &w, const ba_plan_in
     const int64_t blocks = PAIRS == 4 ? att_cols128_most(info) : info->att_cols64;
     const int64_t cols = (blocks * args.H + 7) / 8 * 8;
     if (rows > 0x7fffffff || cols > 0x7fffffff) return BA_ERR_UNSUPPORTED;
-    if (rows > 0) hipLaunchKernelGGL((attention_dq_kernel<DT, NK, QT>), flat_grid(rows), dim3(256), 0, stream, args, w);
+    if (rows > 0) {
+        auto dq = [&](auto pipe) {
+            hipLaunchKernelGGL((attention_dq_kernel<DT, NK, QT, decltype(pipe)::value>), flat_grid(rows), dim3(256), 0, stream, args, w);
+        };
+        // K <= 32: too few matrix instructions to spread the staging over.  Rows at any alignment and fewer than 256 keys a query
+        // (the mean over the queries): the first blocks, which nothing overlaps, weigh more than the others gain (backward of
+        // 48 x 8 pairs of 900 .. 1400 rows, K = 101, us: 64 keys 253, one stage 239; 128 281, 269; 256 385, 381; 64 x 8 of 256 ..
+        // 400 267, 273).  Aligned rows within 2 % either way below 256 keys (K = 64, 128 keys 107, 106; K = 128, 64 keys 178, 177).
+        const bool unaligned = (info->min_K | info->max_K) & 7;
+        if constexpr (QT == 2 && NK > 1) {
+            if (unaligned && info->Dout < 256 * info->total_rows) dq(std::false_type{});
+            else dq(std::true_type{});
+        } else {
+            dq(std::false_type{});
+        }
+    }
     if (cols > 0)
         hipLaunchKernelGGL((attention_dkdv_kernel<DT, NK, PAIRS, QB, PIPE>), flat_grid(cols), dim3(128 * PAIRS), kLds, stream, args, w);
     return hipGetLastError() == hipSuccess ? BA_OK : BA_ERR_LAUNCH;

@@ -111,6 +111,14 @@ def test_scales_and_missing_queries_in_tall_segments(dev, K, dtype):
         run(dev, [2100, 0, 1500, 700], [130, 300, 77, 1025], [K] * 4, 1, dtype, scale, seed=K)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K", [61, 90, 127])
+def test_two_strips_at_any_alignment(dev, K, dtype):
+    # dQ in one stage (fewer than 256 keys a query) and in two
+    run(dev, [300, 520, 257], [130, 77, 33], [K] * 3, 2, dtype, K ** -0.5, seed=9)
+    run(dev, [300, 520, 257], [330, 577, 1], [K] * 3, 2, dtype, K ** -0.5, seed=9)
+
+
 @pytest.mark.parametrize("K", [24, 64, 96, 128, 101])
 def test_block_counts_beside_a_tall_segment(dev, K):
     # 128 keys a workgroup, three stages of 64 queries: one, two, three and more blocks, full and ragged, and key blocks
