@@ -39,7 +39,9 @@ template <bool VEC> struct RowPieces {
     __device__ __forceinline__ u32x4 finish(u32x4 x, uint32_t off, int piece) const {
         if constexpr (VEC) return x;
         if (bytes >= 16) {
-            const uint32_t behind = off <= bytes - 16 ? 0u : (min(off, bytes) - (bytes - 16)) >> 1;    // elements 0 .. 8
+            // (elements 0 .. 8; a piece past the row's end is cleared below: shifting those too would run for every block of a
+            // head dimension with lanes to spare, 16 x 4 pairs of 1000 .. 2000 rows, K = 101: forward 187 -> 159 us, backward 423 -> 378)
+            const uint32_t behind = 8 * piece >= K || off <= bytes - 16 ? 0u : (min(off, bytes) - (bytes - 16)) >> 1;
             if (__any(behind != 0)) {
                 if (behind & 8) x = u32x4{0u, 0u, 0u, 0u};
                 if (behind & 4) x = u32x4{x[2], x[3], 0u, 0u};
