@@ -513,12 +513,16 @@ int launch_attention(int dtype, const RunArgs &args, const void *V, float *lse, 
         if (info->total_rows >= 256 * std::max<int64_t>(nseg, 1)) qt = 2;   // mean segment height >= 256 (136: one strip is 6 % faster)
     }
     if (forced == 1 || forced == 2) qt = forced;
-    // LDS stages for two strips.  Two keep the matrix unit busier in the steady state (16 x 16 segments of 1024 .. 4096,
-    // K = 128, 1068 -> 1037 us; 48 x 4 of 1000 .. 2000, K = 64, 184 -> 173; of 600 .. 900, K = 128, 90 -> 83), but the first
-    // block waits for its successor's values and a missing strip is computed along: with 507 keys per query (the mean over
-    // the queries) 34.0 -> 32.9 us at K = 64 and 50.8 -> 48.3 at K = 128, with 311 18.1 -> 20.1 and 27.1 -> 28.8.  At K <= 32
-    // there are too few matrix instructions to hide an exchange behind (1000 .. 2000: 117 -> 121 us).
-    const bool deep = qt == 2 && nk > 1 && info && info->Dout >= 400 * info->total_rows;
+    // LDS stages for two strips.  Two keep the matrix unit busier in the steady state, but the first block waits for its
+    // successor's values.  Keys per query (the mean over the queries) from which they are faster, us, one stage and two:
+    // - 400 (48 x 8 segments of 600 .. 900 rows, K = 64 / 128: 128 keys 35.4 / 53.1, 36.3 / 55.9; 300 keys 56.1 / 83.7, 56.1 /
+    //   81.5; 400 keys 69.0 / 103.6, 68.2 / 99.2; 800 keys 109 / 171, 106 / 165);
+    // - 800 for rows at any alignment up to K = 96, where one stage leaves registers for six reads in flight and clears its
+    //   pieces in one place (K = 61 / 70 / 95: 64 x 8 of 300 .. 500 71 / 93 / 102, 73 / 97 / 107; 16 x 4 of 1000 .. 2000 111 / 148 /
+    //   159, 110 / 152 / 157; above, K = 101: 110 and 175, 109 and 159);
+    // - K <= 32: never, too few matrix instructions to hide an exchange behind (1000 .. 2000 rows: 117, 121).
+    const int64_t deep_keys = info && nk < 4 && ((info->min_K | info->max_K) & 7) ? 800 : 400;
+    const bool deep = qt == 2 && nk > 1 && info && info->Dout / deep_keys >= info->total_rows;
     // Row blocks per pair: enough for the tallest segment, but no more than four times what the mean segment
     // needs (a workgroup takes every Z-th block of its pair; blocks that do not exist cost a launch each).
     const int64_t round_rows = kAttRows * qt;

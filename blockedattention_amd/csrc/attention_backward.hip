@@ -899,8 +899,9 @@ static int launch_bwd(const RunArgs &args, const AttBwdArgs &w, const ba_plan_in
         };
         // K <= 32: too few matrix instructions to spread the staging over.  Rows at any alignment and fewer than 256 keys a query
         // (the mean over the queries): the first blocks, which nothing overlaps, weigh more than the others gain (backward of
-        // 48 x 8 pairs of 900 .. 1400 rows, K = 101, us: 64 keys 253, one stage 239; 128 281, 269; 256 385, 381; 64 x 8 of 256 ..
-        // 400 267, 273).  Aligned rows within 2 % either way below 256 keys (K = 64, 128 keys 107, 106; K = 128, 64 keys 178, 177).
+        // 48 x 8 pairs of 900 .. 1400 rows, K = 61 / 77 / 101, us, two stages and one: 64 keys 132 / 194 / 238, 128 / 182 / 225; 192 keys
+        // 186 / 277 / 333, 184 / 270 / 324; 16 x 4 of 1000 .. 2000 242 / 334 / 378, 249 / 354 / 404).  Aligned rows are within 2 %
+        // either way below 256 keys (K = 64, 128 keys 107, 106; K = 128, 64 keys 178, 177).
         const bool unaligned = (info->min_K | info->max_K) & 7;
         if constexpr (QT == 2 && NK > 1) {
             if (unaligned && info->Dout < 256 * info->total_rows) dq(std::false_type{});

@@ -124,6 +124,14 @@ def test_two_stages_block_edges(dev, K, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K", [33, 61, 70, 95])
+def test_two_strips_at_any_alignment(dev, K, dtype):
+    # up to 96 columns: two LDS stages from 800 keys per query on, one below
+    run(dev, [513, 300, 640, 257], [2000, 1, 1449, 64], [K] * 4, 2, dtype, K ** -0.5, seed=K)
+    run(dev, [513, 300, 640, 257], [500, 1, 449, 64], [K] * 4, 2, dtype, K ** -0.5, seed=K)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("K", [64, 96, 128, 101])
 def test_two_stages_raise_the_reference_late(dev, K, dtype):
     # scaled scores of standard deviation 9: in most rows a later block's maximum passes the first one's by more than 2^8 in
