@@ -11,10 +11,10 @@
 // and dP are computed in both, seven products instead of five; adding dQ to memory from the second kernel instead
 // would move N / 128 times the size of dQ in fp32 atomics.
 //
-// Measured on 16 segments x 16 heads of 1024 .. 4096 rows, K = 128, bf16: dQ 1.24 ms (1.19 PFLOP/s over its three
-// products), dK and dV 1.82 ms (1.08 over four), 3.06 ms together against 9.3 ms of the chain.  The clock falls to 2.0 GHz
-// under them; a 16 x 16 x 32 matrix instruction holds the issue port 8 of its 16 cycles, another vector instruction 4.3, an
-// exponential 8.4, and one operand read takes the LDS port 4 cycles (2.5 for half a transposing one).
+// Measured on 16 segments x 16 heads of 1024 .. 4096 rows, K = 128, bf16: dQ 1.21 ms (1.22 PFLOP/s over its three
+// products), dK and dV 1.75 ms (1.13 over four), 2.96 ms together against 9.3 ms of the chain.  By counters the clock is 2.0
+// GHz under dQ and 2.2 under dK and dV, and of the cycles the matrix unit is busy 59 and 50 %, the vector issue port 43 and
+// 36 %, LDS 39 and 39 %, no bank conflicts: the phases of a block still follow each other in part.
 //
 // Operands lie in LDS as rows (one copy of each): a matrix operand whose reduction runs over the head dimension is read
 // 16 bytes per lane, one whose reduction runs over the rows by the transposing read (ds_read_b64_tr_b16).  The lane that
@@ -614,8 +614,8 @@ __device__ __forceinline__ void att_dkdv_body(const RunArgs &a, const AttBwdArgs
 // Three stages (blocks i - 1 and i are read while i + 1 is written), two buffers of the handed probabilities.
 // 16 x 16 pairs of 1024 .. 4096 rows, K = 128, bf16: two barriers a block, both sides in the same block 2.10 ms; one barrier
 // 2.07; LDS reads in flight across the phases 2.01; staging spread over the matrix instructions, delta as their starting
-// value 1.86; a loop for each side without branches in it 1.82.  An iteration takes 3400 cycles, of them 2048 of the
-// matrix unit; 13 % of the time are the ends of a workgroup, which has its compute unit alone.
+// value 1.86; a loop for each side without branches in it 1.82.  An iteration takes 4100 cycles, of them 2048 of the matrix unit
+// (counters; the ends of a workgroup, which has its compute unit alone, included).
 template <int DT, int NK, int PAIRS, int QB, bool VEC>
 __device__ __forceinline__ void att_dkdv_pipe_body(const RunArgs &a, const AttBwdArgs &w, const SegRec &rec, int64_t h,
                                                    int64_t row0, int block, unsigned char *lds) {
