@@ -936,14 +936,16 @@ int launch_attention_backward(int dtype, const RunArgs &args, const void *V, con
     // resident workgroups.
     // - All workgroups of 128 keys find a compute unit of their own: these, they do twice the work at a time (10 x 4 of 400 ..
     //   600 rows, K = 32 / 64 / 128: 64 keys 31 / 36 / 54, 128 keys 25 / 30 / 47; 8 x 4 of 256 .. 300 18.3 / 21.8, 16.7 / 20.8).
-    // - Otherwise where segments are tall enough for the stages to pay.  K <= 64 768 rows (24 x 8 of 750 .. 900 158, 168; 16 x 8
-    //   of 1000 .. 1300 199, 194; 10 x 4 of 1500 .. 2500 213, 202).  Above 576, K = 96 / 128: 50 x 8 of 450 .. 600 216 / 285,
+    // - Otherwise where segments are tall enough for the stages to pay.  32 < K <= 64: 768 rows (24 x 8 of 750 .. 900 158, 168;
+    //   16 x 8 of 1000 .. 1300 199, 194; 10 x 4 of 1500 .. 2500 213, 202).  Above, 576, K = 96 / 128: 50 x 8 of 450 .. 600 216 / 285,
     //   217 / 291; 64 x 8 of 600 .. 900 499 / 626, 484 / 613; 32 x 8 of 500 .. 750 rows and 100 .. 300 keys 91 / 114, 82 / 104.
+    //   K <= 32 (two stages, below): 400 (K = 16 / 32: 64 x 8 of 256 .. 400 63 / 67, 65 / 70; of 400 .. 500 95 / 98, 92 / 96; 16 x 8
+    //   of 600 .. 760 62.5 / 65, 57 / 59).
     // - Rows at any alignment, for which the small build has too few registers: always (64 x 8 of 200 .. 400, K = 101: 314, 230).
     const int64_t mean = info->total_rows / std::max<int64_t>(info->nseg, 1);
     const bool few = att_cols128_most(info) * args.H <= device_cu_count();
     const bool unaligned = (info->min_K | info->max_K) & 7;
-    const bool strips2 = mean >= 256, keys128 = mean >= (unaligned || few ? 256 : nk > 2 ? 576 : 768);
+    const bool strips2 = mean >= 256, keys128 = mean >= (unaligned || few ? 256 : nk == 1 ? 400 : nk == 2 ? 768 : 576);
     // K <= 32: the pipeline's LDS leaves room for one workgroup a compute unit where its two-stage form has two, and there are
     // too few matrix instructions to hide the exchanges behind: the pipeline only where a compute unit gets no second one.
     // Backward of 16 x 16 pairs of 1024 .. 4096 rows, K = 16 1273 us, two stages 1185; K = 32 1308, 1227; of 32 x 8 of 768 ..
