@@ -128,13 +128,10 @@ __device__ __forceinline__ void att_dq_body(const RunArgs &a, const AttBwdArgs &
 #pragma unroll
         for (int t = 0; t < kOutTiles; ++t) acc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    arrived(qf);
-    arrived(gf);
     const LdsPtr k_row = lds_ptr(sK) + j * kPitch + rg * 16, v_row = lds_ptr(sV) + j * kPitch + rg * 16;
     const LdsPtr k_col = lds_ptr(sK) + (4 * rg + (j >> 2)) * kPitch + (j & 3) * 8;
 
-    for (int kb = 0; kb < N; kb += kAttKeys) {
-        att_lds_barrier();                             // the previous block is consumed
+    auto put = [&](int kb) {
         if (St::kLpr == St::kPieces || s_piece < St::kPieces) {
 #pragma unroll
             for (int s = 0; s < St::kSteps; ++s) {
@@ -144,7 +141,25 @@ __device__ __forceinline__ void att_dq_body(const RunArgs &a, const AttBwdArgs &
                 *reinterpret_cast<u32x4 *>(sV + row * kPitch + s_piece * 16) = pv.finish(vw[s], off, s_piece);
             }
         }
+    };
+    // The operands and delta's rows arrive under the first block's way into LDS: waited for in front of it, 64 x 8 segments of
+    // 8 .. 32 rows, K = 128, took 13.6 us backward instead of 13.0, 338 x 14 of 5 .. 28 74 instead of 72.  Not at 32 < K <= 64,
+    // where that costs 16 registers and the fifth wavefront per SIMD (512 x 8 of 100 .. 120 rows and 30 .. 60 keys 111 -> 115 us),
+    // nor for rows that are cleared on that way (51 segments of 13 .. 43, K = 31: 11.1 -> 11.5).
+    constexpr bool kPeeled = VEC && NK != 2;
+    if constexpr (kPeeled) {
+        if (N > 0) put(0);
         att_lds_barrier();
+    }
+    arrived(qf);
+    arrived(gf);
+
+    for (int kb = 0; kb < N; kb += kAttKeys) {
+        if (!kPeeled || kb > 0) {
+            att_lds_barrier();                         // the previous block is consumed
+            put(kb);
+            att_lds_barrier();
+        }
         if (kb + kAttKeys < N) fetch(kb + kAttKeys);
         if (r0 >= M) continue;                         // the wavefront only stages
         const int left = N - kb;
@@ -517,14 +532,17 @@ __device__ __forceinline__ void att_dkdv_body(const RunArgs &a, const AttBwdArgs
 #pragma unroll
         for (int t = 0; t < kOutTiles; ++t) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    arrived(kf);
     // this side's arrays: rows for the scores (Q / dO), columns for the sums (dO / Q)
     const LdsPtr row_base = lds_ptr(lds) + side * kArray + j * kPitch + rg * 16;
     const LdsPtr col_base = lds_ptr(lds) + (1 - side) * kArray + (4 * rg + (j >> 2)) * kPitch + (j & 3) * 8;
     const LdsPtr aux_base = lds_ptr(lds) + 2 * kArray + side * 4 * QB + rg * 16;
     unsigned char *hand = lds + 2 * kStage + pair * (64 * QB) + lane * 16;        // kTiles 16-byte slots of 64 lanes a pair
+    // (the operands arrive under the first block's way into LDS: backward of 338 x 14 segments of 5 .. 28 rows, K = 128, 73 -> 72
+    // us; before it at 32 < K <= 64, 16 x 8 of 600 .. 760 85 us against 86, and for rows that are cleared on that way)
+    if constexpr (!VEC || NK == 2) arrived(kf);
     if (M > 0) put(0, lds);
     att_lds_barrier();
+    if constexpr (VEC && NK != 2) arrived(kf);
 
     for (int qb = 0, stage = 0; qb < M; qb += QB, stage ^= 1) {
         const bool more = qb + QB < M;
